@@ -102,6 +102,18 @@ extern "C" {
  * Workspace and scratch as for MEC_DTYPE_F32_BF16X3 (one term instead of
  * three). */
 #define MEC_DTYPE_F32_BF16 4
+/* fp32 inputs and outputs with every value of the similarity GEMMs and the
+ * contractions (x^, y^, G') held as a pair of fp16 values, hi = fp16(v) and lo
+ * = fp16(v - hi) (about 22 significant bits, after a power-of-two scaling that
+ * keeps lo within fp16's range), and every product formed as hi_a hi_b + lo_a
+ * hi_b + hi_a lo_b on the fp16 MFMA, accumulated in fp32.  The loss and the
+ * gradients are as close to the 64-bit values as those of MEC_DTYPE_F32 (the
+ * rounding of the fp32 sums is larger than what the pairs leave out), at a
+ * multiple of its speed for larger problems.  n <= 2^20.  Workspace
+ * (mec_workspace_floats_for, 16-byte aligned) and scratch are larger; any row
+ * stride and alignment is accepted.  mec_product_dtype names the problems that
+ * are better run this way.  No counterpart dtype in the reference. */
+#define MEC_DTYPE_F32_PAIRS 6
 
 #define MEC_MODE_CLIP 0 /* symmetric image<->text loss, gradients for x and y */
 #define MEC_MODE_LIT 1  /* text->image only (x = text), gradient for x only */
@@ -180,6 +192,12 @@ int64_t mec_workspace_floats_for(int64_t n, int64_t d, int dtype);
  * args, or for MEC_FLAG_KEEP_EXP with a dtype other than MEC_DTYPE_F32 or
  * n > MEC_KEEP_EXP_MAX_N.  No counterpart in the reference. */
 int64_t mec_workspace_floats_mode(int64_t n, int64_t d, int dtype, int mode);
+
+/* The dtype code to run MEC_DTYPE_F32 or MEC_DTYPE_F32_BF16X3 data of this
+ * size with: MEC_DTYPE_F32_PAIRS where that is faster (it is as exact as the
+ * first and more exact than the second), else `dtype` itself (any other dtype
+ * is returned as it is).  Host-only.  No counterpart in the reference. */
+int mec_product_dtype(int64_t n, int64_t d, int dtype);
 
 /* 1 if mec_forward / mec_backward accept MEC_FLAG_KEEP_EXP for these inputs
  * (MEC_DTYPE_F32, n <= MEC_KEEP_EXP_MAX_N, 16-byte aligned rows: x and y

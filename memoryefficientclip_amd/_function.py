@@ -16,9 +16,11 @@ This mirrors the glue of the reference's autograd Functions
   are bitwise reproducible (the reference's relaxed atomics are not,
   ``clip_loss.py:63-64,155-156``);
 * fp32 inputs follow ``torch.get_float32_matmul_precision()``: "highest" (the
-  default) multiplies in IEEE fp32 on the fp32 MFMA; "high" forms each product
-  from bf16 terms (hi*hi + lo*hi + hi*lo, about 16 significant bits per
-  operand) on the bf16 MFMA and keeps the fp32 tolerances; "medium" multiplies
+  default) has the accuracy of IEEE fp32 products, on the fp32 MFMA or, for
+  the larger problems (``mec_product_dtype``), on the fp16 MFMA from pairs of
+  fp16 terms of about 22 significant bits, whose sums are as close to the
+  64-bit values; "high" allows less (at least three bf16 terms per product)
+  and always runs the pairs, up to their size limit; "medium" multiplies
   bf16-rounded values (the bf16 tolerances).  These are PyTorch's meanings of
   the three settings.  The reference's fp32 dot products are TF32 on NVIDIA
   (``tl.dot`` without ``input_precision``, ``clip_loss.py:53,113,148-149``).
@@ -112,7 +114,8 @@ def refuse_graph_capture() -> None:
 def compute_dtype(dtype: torch.dtype) -> int:
     """C-ABI dtype code for inputs of `dtype` under the current
     ``torch.get_float32_matmul_precision()`` (fp32 only: "high" selects the
-    three-term bf16 products, "medium" plain bf16 products)."""
+    three-term bf16 products, "medium" plain bf16 products), before
+    ``mec_product_dtype`` has its say."""
     code = _DTYPES[dtype]
     if code == _lib.DTYPE_F32:
         p = torch.get_float32_matmul_precision()
@@ -137,6 +140,7 @@ def forward(ctx, x: torch.Tensor, y: torch.Tensor, temperature: float, mode: int
     di = x.get_device()
     dt = compute_dtype(x.dtype)
     lib = _lib.load()
+    dt = lib.mec_product_dtype(n, d, dt)
     # small fp32 problems keep the similarity matrix for the backward (three
     # launches per step instead of six, no gradient scratch), when a gradient
     # will be asked for
@@ -174,7 +178,7 @@ def backward(ctx, grad_output: torch.Tensor, need_x: bool, need_y: bool):
         go = go.detach().to(device=dev, dtype=torch.float32).reshape(())
     acc_x = torch.empty((n, d), dtype=torch.float32, device=dev) if need_x else None
     acc_y = torch.empty((n, d), dtype=torch.float32, device=dev) if need_y else None
-    if dt in (_lib.DTYPE_F32, _lib.DTYPE_F32_BF16X3, _lib.DTYPE_F32_BF16):
+    if x.dtype == torch.float32:
         dx, dy = acc_x, acc_y  # the post-pass runs in place
     else:
         dx = torch.empty((n, d), dtype=x.dtype, device=dev) if need_x else None

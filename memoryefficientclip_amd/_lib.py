@@ -23,6 +23,7 @@ DTYPE_BF16 = 1
 DTYPE_F16 = 2
 DTYPE_F32_BF16X3 = 3  # fp32 data, products as three bf16 MFMA terms
 DTYPE_F32_BF16 = 4  # fp32 data, bf16 products
+DTYPE_F32_PAIRS = 6  # fp32 data as fp16 pairs, products as three fp16 MFMA terms
 MODE_CLIP = 0
 MODE_LIT = 1
 FLAG_DETERMINISTIC = 0x100  # OR into the mode of mec_sumexp / mec_forward
@@ -43,6 +44,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "mec_workspace_floats": (_i64, [_i64]),
     "mec_workspace_floats_for": (_i64, [_i64, _i64, _int]),
     "mec_workspace_floats_mode": (_i64, [_i64, _i64, _int, _int]),
+    "mec_product_dtype": (_int, [_i64, _i64, _int]),
     "mec_keep_exp_supported": (_int, [_vp, _i64, _vp, _i64, _i64, _i64, _int]),
     "mec_grad_scratch_bytes": (_i64, [_i64, _i64, _int]),
     "mec_grad_scratch_bytes_for": (_i64, [_i64, _i64, _int, _int, _int]),

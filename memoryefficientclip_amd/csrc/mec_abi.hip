@@ -123,8 +123,14 @@ constexpr int64_t kMaxD = int64_t(1) << 20;
 
 bool known_dtype(int dtype) {
   return dtype == MEC_DTYPE_F32 || dtype == MEC_DTYPE_BF16 || dtype == MEC_DTYPE_F16 ||
-         dtype == MEC_DTYPE_F32_BF16X3 || dtype == MEC_DTYPE_F32_BF16;
+         dtype == MEC_DTYPE_F32_BF16X3 || dtype == MEC_DTYPE_F32_BF16 || dtype == MEC_DTYPE_F32_PAIRS;
 }
+// fp32 data as fp16 pairs (F16S): every value takes two 16-bit elements
+bool is_pairs(int dtype) { return dtype == MEC_DTYPE_F32_PAIRS; }
+// a 256-row panel of their transposed inputs, 256 x 2 ldt elements, must span
+// less than 2^31 bytes: n <= 2^20 leaves a factor of two
+constexpr int64_t kMaxNPairs = int64_t(1) << 20;
+int64_t max_n(int dtype) { return is_pairs(dtype) ? kMaxNPairs : kMaxN; }
 // fp32 data with bf16 products: bf16 terms per operand value in the
 // similarity GEMMs (3: hi, lo; 1: hi), 0 for the other dtypes
 int split_terms(int dtype) {
@@ -133,12 +139,16 @@ int split_terms(int dtype) {
 bool is_split(int dtype) { return split_terms(dtype) > 0; }
 bool is_x3(int dtype) { return dtype == MEC_DTYPE_F32_BF16X3; }
 // element type of the caller's x, y, dx, dy (the split modes read and write fp32)
-int data_dtype(int dtype) { return is_split(dtype) ? MEC_DTYPE_F32 : dtype; }
+int data_dtype(int dtype) { return is_split(dtype) || is_pairs(dtype) ? MEC_DTYPE_F32 : dtype; }
+// dtypes whose workspace holds 16-byte vectors
+bool ws_copies(int dtype) { return is_split(dtype) || is_pairs(dtype); }
 
 int check_common(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d,
                  int dtype) {
   if (n < 1) return fail(MEC_ERR_INVALID, "n=%lld must be >= 1", (long long)n);
   if (n > kMaxN) return fail(MEC_ERR_UNSUPPORTED, "n=%lld exceeds the supported maximum 2^22", (long long)n);
+  if (n > max_n(dtype))
+    return fail(MEC_ERR_UNSUPPORTED, "n=%lld exceeds the maximum 2^20 of MEC_DTYPE_F32_PAIRS", (long long)n);
   if (d < 1 || d > kMaxD) return fail(MEC_ERR_INVALID, "d=%lld out of range [1, 2^20]", (long long)d);
   if (ldx < d || ldy < d)
     return fail(MEC_ERR_INVALID, "row strides ldx=%lld ldy=%lld must be >= d=%lld", (long long)ldx,
@@ -185,7 +195,21 @@ int64_t base_workspace_floats(int64_t n) { return det_partials_offset(n) + (int6
 int64_t split_dp(int64_t d) { return (d + 7) & ~int64_t(7); }
 int64_t split_ld(int64_t d, int dtype) { return split_terms(dtype) * split_dp(d); }
 int64_t split_offset_floats(int64_t n) { return (base_workspace_floats(n) + 3) & ~int64_t(3); }
+// Split pairs: the scales (4 of PAIR_SCL floats), then the pairs of the x rows
+// and of the y rows, n rows of 2 dp fp16 each, dp = d rounded up to 32
+// (k_pair_prepass).
+constexpr int64_t PAIR_SCL = 64;
+int64_t pair_dp(int64_t d) { return (d + 31) & ~int64_t(31); }
+int64_t pair_scl_offset(int64_t n) { return (base_workspace_floats(n) + 63) & ~int64_t(63); }
+float* pair_scl(const float* ws, int64_t n) { return const_cast<float*>(ws) + pair_scl_offset(n); }
+PairRows pair_rows(const float* ws, int64_t n, int64_t d) {
+  float* scl = pair_scl(ws, n);
+  uint16_t* a = (uint16_t*)(scl + PAIR_SCL);
+  const int64_t dp = pair_dp(d);
+  return PairRows{a, a + n * 2 * dp, scl, (int)dp};
+}
 int64_t workspace_floats_for(int64_t n, int64_t d, int dtype) {
+  if (is_pairs(dtype)) return pair_scl_offset(n) + PAIR_SCL + 2 * n * pair_dp(d);
   if (!is_split(dtype)) return base_workspace_floats(n);
   return split_offset_floats(n) + n * split_ld(d, dtype);  // 2 n ld bf16 = n ld floats
 }
@@ -312,11 +336,16 @@ int check_keep(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n
 // blocks and few launches) and at most 16 GiB; it wins over the 1024-row
 // target.
 int g_planes(int dtype) { return is_x3(dtype) ? 2 : 1; }
-int64_t g_elem(int dtype) { return dtype == MEC_DTYPE_F32 ? 4 : 2; }
+int64_t g_elem(int dtype) { return dtype == MEC_DTYPE_F32 || is_pairs(dtype) ? 4 : 2; }
+// Diagonals held: two, except with one block, and for the pairs, whose
+// contractions of one diagonal end before the next one's tiles begin (two
+// launches on one stream): at 4 bytes per value, one buffer of twice the block
+// rows takes the same memory and half the launches.
+int g_nbuf(int dtype, int64_t nb) { return nb > 1 && !is_pairs(dtype) ? 2 : 1; }
 // bytes of the gradient-matrix buffers for blocks of tb quanta
 int64_t g_bytes(int64_t tiles, int64_t q, int64_t tb, int dtype) {
   const int64_t nb = (tiles + tb - 1) / tb, bs = tb * q;
-  return (nb > 1 ? 2 : 1) * g_planes(dtype) * nb * bs * bs * g_elem(dtype);
+  return g_nbuf(dtype, nb) * g_planes(dtype) * nb * bs * bs * g_elem(dtype);
 }
 constexpr int64_t kGradBudgetCap = int64_t(16) << 30;
 constexpr int64_t kGradBudgetMin = int64_t(256) << 20;
@@ -334,14 +363,15 @@ void grad_blocks_budget(int64_t n, int64_t d, int dtype, int64_t gbudget, int* b
   // offsets ((bs - 1) * bs + 128 floats within 2^31 bytes: bs <= 16384); the
   // 16-bit contractions read a transposed block as a direct-to-LDS operand
   // ((bs - 1) * bs + 256 elements within 2^31 bytes: bs <= 127 * 256).
-  int64_t cap = dtype == MEC_DTYPE_F32 ? 128 : 127;
+  // (pairs: 4 bs^2 bytes within 2^31: bs <= 90 * 256)
+  int64_t cap = dtype == MEC_DTYPE_F32 ? 128 : is_pairs(dtype) ? 90 : 127;
   if (cap > tiles) cap = tiles;
   // the longest blocks within the budget (at least one quantum): an
   // estimate from the double-buffered size, then a short walk down
   {
     int64_t tb = cap;
     if (g_bytes(tiles, q, tb, dtype) > gbudget) {
-      const int64_t per_tb = 2 * (int64_t)g_planes(dtype) * tiles * q * q * g_elem(dtype);
+      const int64_t per_tb = g_nbuf(dtype, 2) * (int64_t)g_planes(dtype) * tiles * q * q * g_elem(dtype);
       if (gbudget / per_tb < tb) tb = gbudget / per_tb;
       if (tb < 1) tb = 1;
       while (tb > 1 && g_bytes(tiles, q, tb, dtype) > gbudget) --tb;
@@ -349,7 +379,7 @@ void grad_blocks_budget(int64_t n, int64_t d, int dtype, int64_t gbudget, int* b
     cap = tb;
   }
   int64_t mult = dtype == MEC_DTYPE_F32 ? 4 : 8;
-  if (dtype != MEC_DTYPE_F32 && n >= 8192 && n < 16 * 8 * d) mult = 16;
+  if (dtype != MEC_DTYPE_F32 && !is_pairs(dtype) && n >= 8192 && n < 16 * 8 * d) mult = 16;
   // at least 1024 rows (below that the pipeline's launches and accumulator
   // updates dominate), where the budget allows
   const int64_t target_rows = mult * d > kTargetMinRows ? mult * d : kTargetMinRows;
@@ -394,6 +424,7 @@ constexpr int kSideX = MEC_SIDE_X, kSideY = MEC_SIDE_Y;
 //   fp32:                  [H0 | H1]
 //   bf16, fp16, fp32/bf16: [GT0 | GT1 | XT | YT]
 //   bf16x3:                [GT0 | GT1 | GTlo0 | GTlo1 | XT | XTlo | YT | YTlo]
+//   pairs:                 [GT | XT | YT], 4 bytes per value, one diagonal
 // H0/H1 double-buffer one block diagonal of H = diag(rx) G' diag(ry) (nb
 // blocks of bs x bs, row-major); GT0/GT1 the 16-bit types' transposed blocks
 // of G' in the blocked layout gdma::gb_offset (bf16x3: hi and lo planes).
@@ -416,7 +447,7 @@ ScratchLayout scratch_layout_blocks(int64_t n, int64_t d, int dtype, int sides, 
   L.bs = bs;
   L.nb = nb;
   const int64_t elem = g_elem(dtype);
-  L.nbuf = nb > 1 ? 2 : 1;
+  L.nbuf = g_nbuf(dtype, nb);
   L.planes = g_planes(dtype);
   L.ntp = dtype == MEC_DTYPE_F32 ? 0 : (is_x3(dtype) ? 2 : 1);
   L.ldt = (n + 127) / 128 * 128;
@@ -532,7 +563,7 @@ BlockGrid block_grid(int64_t d, int dtype, int sides, int bs, int nb, int64_t ld
   const int D = (int)d;
   BlockGrid bg{bs, nb, bs / tf.bm, bs / tf.bn, bs / tc.bm, (D + tc.bn - 1) / tc.bn, 0};
   *w384 = false;
-  if (separate_contractions(dtype)) {
+  if (separate_contractions(dtype) && !is_pairs(dtype)) {
     const int64_t nsides = ((sides & kSideX) ? 1 : 0) + ((sides & kSideY) ? 1 : 0);
     const int64_t wide = nsides * nb * bg.ctm * bg.ctd;
     int64_t tiles = wide;
@@ -581,6 +612,29 @@ BlockGrid block_grid(int64_t d, int dtype, int sides, int bs, int nb, int64_t ld
     }                                  \
   } while (0)
 
+// fp32 data that runs as fp16 pairs.
+// "high" precision (bf16x3): always (three products as well, more exact, fewer
+// operand bytes; step at 2048 x 512 248 -> 201 us, 4999 x 640 655 -> 567 us,
+// 8192 x 768 1194 -> 1127 us, 32768 x 1152 the same).
+// fp32: where the products dominate.  Measured, CLIP step, fp32 MFMA -> pairs:
+// 2500 x 512 285 -> 228 us, 4096 x 512 554 -> 361 us, 4999 x 640 1171 -> 567
+// us, 8192 x 768 3028 -> 1127 us, 32768 x 1152 71.9 -> 24.4 ms, 32768 x 128 9.7
+// -> 5.4 ms; but 2500 x 64 134 -> 201 us, 4096 x 64 153 -> 326 us, 8192 x 128
+// 698 -> 723 us (at a small d the contractions' 256-feature tiles are mostly
+// empty and their few workgroups run over all n rows), and up to n = 2048 the
+// kept similarity matrix takes three launches (2048 x 512 131 -> 201 us).
+bool pairs_preferred(int64_t n, int64_t d, int dtype) {
+  if (dtype != MEC_DTYPE_F32 && dtype != MEC_DTYPE_F32_BF16X3) return false;
+  if (n < 1 || d < 1 || n > kMaxNPairs || d > kMaxD) return false;
+  if (const char* env = std::getenv("MEC_F32_PAIRS")) {  // (tests)
+    if (env[0] == '0') return false;
+    if (env[0] == '1') return true;
+  }
+  if (dtype == MEC_DTYPE_F32_BF16X3) return true;
+  if (small_tiles_env() >= 0) return false;  // (the fp32 tiles are asked for)
+  return n > 2048 && n * n * d >= 3000000000LL && (d >= 192 || n > 12288);
+}
+
 }  // namespace
 
 extern "C" {
@@ -595,15 +649,19 @@ int64_t mec_workspace_floats(int64_t n) {
 }
 
 int64_t mec_workspace_floats_for(int64_t n, int64_t d, int dtype) {
-  if (n < 1 || n > kMaxN || d < 1 || d > kMaxD || !known_dtype(dtype)) return -1;
+  if (n < 1 || n > max_n(dtype) || d < 1 || d > kMaxD || !known_dtype(dtype)) return -1;
   return workspace_floats_for(n, d, dtype);
 }
 
 int64_t mec_workspace_floats_mode(int64_t n, int64_t d, int dtype, int mode) {
-  if (n < 1 || n > kMaxN || d < 1 || d > kMaxD || !known_dtype(dtype)) return -1;
+  if (n < 1 || n > max_n(dtype) || d < 1 || d > kMaxD || !known_dtype(dtype)) return -1;
   if (check_mode(mode) != MEC_OK) return -1;
   if (keep_flag(mode) && !keep_shape_ok(n, dtype)) return -1;
   return workspace_floats_mode(n, d, dtype, mode);
+}
+
+int mec_product_dtype(int64_t n, int64_t d, int dtype) {
+  return pairs_preferred(n, d, dtype) ? MEC_DTYPE_F32_PAIRS : dtype;
 }
 
 int mec_keep_exp_supported(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d,
@@ -612,13 +670,13 @@ int mec_keep_exp_supported(const void* x, int64_t ldx, const void* y, int64_t ld
 }
 
 int64_t mec_grad_scratch_bytes(int64_t n, int64_t d, int dtype) {
-  if (n < 1 || n > kMaxN || d < 1 || d > kMaxD) return -1;
+  if (n < 1 || n > max_n(dtype) || d < 1 || d > kMaxD) return -1;
   if (!known_dtype(dtype)) return -1;
   return scratch_layout(n, d, dtype, kSideX | kSideY).total;
 }
 
 int64_t mec_grad_scratch_bytes_for(int64_t n, int64_t d, int dtype, int mode, int sides) {
-  if (n < 1 || n > kMaxN || d < 1 || d > kMaxD || !known_dtype(dtype)) return -1;
+  if (n < 1 || n > max_n(dtype) || d < 1 || d > kMaxD || !known_dtype(dtype)) return -1;
   if (check_mode(mode) != MEC_OK) return -1;
   if (is_lit(mode)) sides &= kSideX;
   if (sides < 1 || sides > (kSideX | kSideY)) return -1;
@@ -630,6 +688,7 @@ int mec_backward_plan(int64_t n, int64_t d, int dtype, int mode, int sides, int 
   g_err.clear();
   if (n < 1 || d < 1 || d > kMaxD) return fail(MEC_ERR_INVALID, "n or d out of range");
   if (n > kMaxN) return fail(MEC_ERR_UNSUPPORTED, "n=%lld exceeds the supported maximum 2^22", (long long)n);
+  if (n > max_n(dtype)) return fail(MEC_ERR_UNSUPPORTED, "n=%lld exceeds the maximum 2^20 of MEC_DTYPE_F32_PAIRS", (long long)n);
   if (!known_dtype(dtype)) return fail(MEC_ERR_INVALID, "unknown dtype %d", dtype);
   int rc = check_mode(mode);
   if (rc) return rc;
@@ -657,7 +716,7 @@ int mec_backward_plan(int64_t n, int64_t d, int dtype, int mode, int sides, int 
   plan->num_blocks = L.nb;
   plan->scratch_bytes = L.total;
   // the tiles of a launch with contractions (16-byte rows assumed)
-  const int gdt = is_split(dtype) ? MEC_DTYPE_BF16 : dtype;
+  const int gdt = is_split(dtype) ? MEC_DTYPE_BF16 : dtype;  // (block_grid: no special tiles for the pairs)
   const bool small = gdt == MEC_DTYPE_F32 && f32_small_bwd_tiles(n, d, L.bs, cus);
   bool w384 = false;
   const BlockGrid bg = block_grid(d, gdt, sides, L.bs, L.nb, L.ldt, cus, fwd_tile_dims(gdt, true, small),
@@ -678,13 +737,26 @@ int mec_prepass(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t 
   int rc = check_common(x, ldx, y, ldy, n, d, dtype);
   if (rc) return rc;
   if (!workspace) return fail(MEC_ERR_INVALID, "workspace must be non-null");
-  if (is_split(dtype) && !aligned16(workspace))
-    return fail(MEC_ERR_INVALID, "workspace must be 16-byte aligned for the bf16-product modes");
+  if (ws_copies(dtype) && !aligned16(workspace))
+    return fail(MEC_ERR_INVALID, "workspace must be 16-byte aligned for the modes that keep 16-bit copies in it");
   rc = check_not_capturing(stream);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   const int N = (int)n, D = (int)d;
   dim3 grid((unsigned)((n + 3) / 4));
+  if (is_pairs(dtype)) {
+    const PairRows pr = pair_rows(workspace, n, d);
+    const bool vec = aligned16(x) && aligned16(y) && ldx % 4 == 0 && ldy % 4 == 0;
+    if (normalize) {
+      k_pair_prepass<true><<<grid, 256, 0, s>>>((const float*)x, ldx, (const float*)y, ldy, N, D, vec, workspace, pr);
+    } else {
+      k_pair_prepass<false><<<grid, 256, 0, s>>>((const float*)x, ldx, (const float*)y, ldy, N, D, vec, workspace, pr);
+      // (every workgroup reads the maxima: a bounded number of them)
+      k_pair_rows<<<grid.x < 1024 ? grid.x : 1024, 256, 0, s>>>((const float*)x, ldx, (const float*)y, ldy, N, D, vec,
+                                                               workspace, pr, (int)grid.x);
+    }
+    return check_launch("prepass");
+  }
   DISPATCH_DTYPE(data_dtype(dtype), T, DISPATCH_BOOL(normalize, NORM,
       k_prepass<T, NORM><<<grid, 256, 0, s>>>((const T*)x, ldx, (const T*)y, ldy, N, D, workspace)));
   if (is_split(dtype)) {
@@ -713,6 +785,38 @@ int mec_prepass(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t 
   return check_launch("prepass");
 }
 
+}  // extern "C"
+
+// The forward sums without atomics: one pass over the tile grid in P x Q
+// blocks, then the partials in order.  (D: K of the operands as stored; scl:
+// split pairs.)
+template <typename T>
+static int sumexp_det_run(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int D, bool lit,
+                          bool normalize, bool vec, float c, float* workspace, const float* scl, int tiles_m,
+                          int tiles_n, hipStream_t s) {
+  const int N = (int)n;
+  float* rowpart = workspace + det_partials_offset(n);
+  float* colpart = rowpart + (int64_t)DET_Q * n;
+  const int P = tiles_m < DET_P ? tiles_m : DET_P, Q = tiles_n < DET_Q ? tiles_n : DET_Q;
+  const unsigned sum_grid = (unsigned)((n + 255) / 256);
+  auto run = [&](auto lit_c, auto norm_c, auto vec_c) {
+    constexpr bool LIT = decltype(lit_c)::value, NORM = decltype(norm_c)::value, VEC = decltype(vec_c)::value;
+    if constexpr (!IsSplit<T>::value || (VEC && !NORM)) {
+      k_sumexp_det<T, LIT, NORM, VEC><<<(unsigned)(P * Q), FwdTile<T, VEC>::NT, 0, s>>>(
+          (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace + WS_RX * n, workspace + WS_RY * n, rowpart,
+          colpart, tiles_m, tiles_n, P, Q, scl);
+      k_det_reduce<LIT><<<sum_grid, 256, 0, s>>>(rowpart, Q, colpart, P, N, workspace + WS_ROW_OFF * n,
+                                                 workspace + WS_COL_OFF * n);
+    }
+  };
+  DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(vec, VEC,
+      run(std::integral_constant<bool, LIT>{}, std::integral_constant<bool, NORM>{},
+          std::integral_constant<bool, VEC>{}))));
+  return check_launch("sumexp (deterministic)");
+}
+
+extern "C" {
+
 int mec_sumexp(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
                int mode, int normalize, float temperature, float* workspace, void* stream) {
   g_err.clear();
@@ -722,8 +826,8 @@ int mec_sumexp(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n
   if (!rc) rc = check_temperature(temperature);
   if (rc) return rc;
   if (!workspace) return fail(MEC_ERR_INVALID, "workspace must be non-null");
-  if (is_split(dtype) && !aligned16(workspace))
-    return fail(MEC_ERR_INVALID, "workspace must be 16-byte aligned for the bf16-product modes");
+  if (ws_copies(dtype) && !aligned16(workspace))
+    return fail(MEC_ERR_INVALID, "workspace must be 16-byte aligned for the modes that keep 16-bit copies in it");
   rc = check_not_capturing(stream);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
@@ -734,6 +838,12 @@ int mec_sumexp(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n
   if (is_split(dtype)) {
     g = split_operands(workspace, n, d, dtype);
     normalize = 0;
+  }
+  if (is_pairs(dtype)) {
+    const PairRows pr = pair_rows(workspace, n, d);
+    const int tiles = (int)((n + 255) / 256), dk = 2 * pr.dp;
+    return sumexp_det_run<F16S>(pr.a, dk, pr.b, dk, n, dk, is_lit(mode), false, true, c, workspace, pr.scl, tiles,
+                                tiles, s);
   }
   x = g.x, ldx = g.ldx, y = g.y, ldy = g.ldy, d = g.d, dtype = g.dtype;
   const int N = (int)n, D = (int)d;
@@ -758,20 +868,9 @@ int mec_sumexp(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n
   if (nwg > 0x7fffffff) return fail(MEC_ERR_UNSUPPORTED, "forward grid too large");
   const bool lit = is_lit(mode);
   if (det) {
-    // one pass over the tile grid in P x Q blocks, then the partials in order
-    const int64_t n64 = n;
-    float* rowpart = workspace + det_partials_offset(n);
-    float* colpart = rowpart + (int64_t)DET_Q * n64;
-    const int P = tiles_m < DET_P ? tiles_m : DET_P, Q = tiles_n < DET_Q ? tiles_n : DET_Q;
-    const unsigned sum_grid = (unsigned)((n + 255) / 256);
-    DISPATCH_DTYPE(dtype, T, DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(vec, VEC, {
-      k_sumexp_det<T, LIT, NORM, VEC><<<(unsigned)(P * Q), FwdTile<T, VEC>::NT, 0, s>>>(
-          (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace + WS_RX * n64, workspace + WS_RY * n64, rowpart,
-          colpart, tiles_m, tiles_n, P, Q);
-      k_det_reduce<LIT><<<sum_grid, 256, 0, s>>>(rowpart, Q, colpart, P, N, workspace + WS_ROW_OFF * n64,
-                                                 workspace + WS_COL_OFF * n64);
-    }))));
-    return check_launch("sumexp (deterministic)");
+    DISPATCH_DTYPE(dtype, T, rc = sumexp_det_run<T>(x, ldx, y, ldy, n, D, lit, normalize != 0, vec, c, workspace,
+                                                    nullptr, tiles_m, tiles_n, s));
+    return rc;
   }
   dim3 grid((unsigned)nwg);
   DISPATCH_DTYPE(dtype, T, DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(vec, VEC, {
@@ -863,6 +962,7 @@ int mec_grad_blocking(int64_t n, int64_t d, int dtype, int64_t* block_rows, int6
   g_err.clear();
   if (n < 1 || d < 1 || d > kMaxD) return fail(MEC_ERR_INVALID, "n or d out of range");
   if (n > kMaxN) return fail(MEC_ERR_UNSUPPORTED, "n=%lld exceeds the supported maximum 2^22", (long long)n);
+  if (n > max_n(dtype)) return fail(MEC_ERR_UNSUPPORTED, "n=%lld exceeds the maximum 2^20 of MEC_DTYPE_F32_PAIRS", (long long)n);
   if (!known_dtype(dtype)) return fail(MEC_ERR_INVALID, "unknown dtype %d", dtype);
   if (!block_rows || !num_blocks) return fail(MEC_ERR_INVALID, "block_rows and num_blocks must be non-null");
   int bs, nb;
@@ -904,8 +1004,8 @@ static int check_step_args(StepArgs& a) {
   if (!a.workspace) return fail(MEC_ERR_INVALID, "workspace must be non-null");
   if (!a.acc_x && !a.acc_y)
     return fail(MEC_ERR_INVALID, "no gradient requested (acc_x%s null)", lit ? "" : " and acc_y");
-  if (is_split(a.dtype) && !aligned16(a.workspace))
-    return fail(MEC_ERR_INVALID, "workspace must be 16-byte aligned for the bf16-product modes");
+  if (ws_copies(a.dtype) && !aligned16(a.workspace))
+    return fail(MEC_ERR_INVALID, "workspace must be 16-byte aligned for the modes that keep 16-bit copies in it");
   if (a.dtype == MEC_DTYPE_F32 && (a.ldx > kMaxLdF32 || a.ldy > kMaxLdF32))
     return fail(MEC_ERR_UNSUPPORTED, "row strides ldx=%lld ldy=%lld: the fp32 backward supports up to 2^24",
                 (long long)a.ldx, (long long)a.ldy);
@@ -930,10 +1030,10 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
   if (rc) return rc;
   const int N = (int)n, D = (int)d;
   const float c = (float)(1.4426950408889634 / (double)temperature);
-  const bool x3 = is_x3(dtype), split = is_split(dtype);
+  const bool x3 = is_x3(dtype), split = is_split(dtype), pairs = is_pairs(dtype);
   // operands of the gradient-matrix tiles (split modes: the copies, K = terms * dp)
   const GemmOperands go = split ? split_operands(workspace, n, d, dtype) : GemmOperands{x, ldx, y, ldy, d, dtype};
-  const bool vec = vec_ok(go.x, go.ldx, go.y, go.ldy, go.d, go.dtype);
+  const bool vec = pairs || vec_ok(go.x, go.ldx, go.y, go.ldy, go.d, go.dtype);
   if (split && !vec) return fail(MEC_ERR_UNSUPPORTED, "split operands beyond the direct-load range");
   const bool small = dtype == MEC_DTYPE_F32 && vec && f32_small_bwd_tiles(n, d, bs, cus);
   bool w384 = false;  // 16-bit contractions in 256 x 384 tiles
@@ -983,6 +1083,7 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
     if (x3) gb.yt_lo = base + L.yt + L.tbuf;
   }
   gb.ldt = L.ldt;
+  if (pairs) gb.scl = pair_scl(workspace, n);
   hipStream_t s = (hipStream_t)stream;
   if (step == 0 && dtype != MEC_DTYPE_F32) {
     // transposed normalised operands of the 16-bit contractions: YT for the
@@ -992,7 +1093,14 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
     // XT when the y side is
     const unsigned nsides = (acc_x ? 1u : 0u) + (acc_y ? 1u : 0u);
     dim3 tgrid((unsigned)(L.ldt / 64), (unsigned)((d + 63) / 64), nsides);
-    if (split) {
+    if (pairs) {
+      using TS = TransSide<float, uint16_t>;
+      const TS ty{(const float*)y, ldy, workspace + WS_RY * n64, (uint16_t*)gb.yt, nullptr};
+      const TS tx{(const float*)x, ldx, workspace + WS_RX * n64, (uint16_t*)gb.xt, nullptr};
+      DISPATCH_BOOL(normalize, NORM, k_transpose_pairs<NORM><<<tgrid, 256, 0, s>>>(
+                                         acc_x ? ty : tx, tx, N, D, L.ldt, gb.scl + (acc_x ? SCL_Y : SCL_X),
+                                         gb.scl + SCL_X));
+    } else if (split) {
       using TS = TransSide<float, uint16_t>;
       const TS ty{(const float*)y, ldy, workspace + WS_RY * n64, (uint16_t*)gb.yt, (uint16_t*)gb.yt_lo};
       const TS tx{(const float*)x, ldx, workspace + WS_RX * n64, (uint16_t*)gb.xt, (uint16_t*)gb.xt_lo};
@@ -1010,6 +1118,22 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
     }
     rc = check_launch("transpose");
     if (rc) return rc;
+  }
+  if (pairs) {
+    using T = F16S;
+    const PairRows pr = pair_rows(workspace, n, d);
+    const int dk = 2 * pr.dp;
+    if (grid_c > 0) {
+      k_grad_contract<T><<<(unsigned)grid_c, ConTileX<T>::NT, 0, s>>>(N, D, gb, bg, sp_c, acc_x, acc_y);
+      rc = check_launch("grad_contract");
+    }
+    if (!rc && grid > 0) {
+      DISPATCH_BOOL(lit, LIT,
+          k_grad_g_chain<T, LIT, false><<<(unsigned)(grid < cus ? grid : cus), FwdTile<T, true>::NT, 0, s>>>(
+              (const T*)pr.a, dk, (const T*)pr.b, dk, N, dk, dk, c, workspace, gb, bg, sp_g));
+      rc = check_launch("grad_step");
+    }
+    return rc;
   }
   if (split) {
     // the bf16 kernels on the split operands (bf16x3: with hi/lo planes of

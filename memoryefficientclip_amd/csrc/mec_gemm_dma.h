@@ -88,7 +88,7 @@ __host__ __device__ constexpr int64_t gb_offset(int j, int i, int bs) {
 }
 
 template <int BM_, int BN_, bool TA_ = false, int WM_ = 2, int WN_ = 2, int KIND_ = K_BF16, int SA_ = 2,
-          bool GB_ = false, int TB_ = 0, int S_ = 2, int KS_ = 1>
+          bool GB_ = false, int TB_ = 0, int S_ = 2, int KS_ = 1, bool SPL_ = false>
 struct Geo {
   static constexpr int BM = BM_, BN = BN_;
   static constexpr int KIND = KIND_;
@@ -131,9 +131,22 @@ struct Geo {
   // k-step (blocked) or vector h * NS + s (row-major operands).
   static constexpr bool GB = GB_;
   static_assert(!GB || (ESZ == 2 && BK == 64), "blocked A: 16-bit, 64 k per chunk");
-  static __device__ __forceinline__ int kvec(int s, int h) { return GB ? 2 * s + h : h * NS + s; }
+  // SPL: split operands (mainloop_split).  Every 32 values of a row are stored
+  // as 64, their hi parts and then their lo parts (blocked A: every 32 columns
+  // i as four 1 KB blocks, hi of i-blocks 0 and 1, then lo), so a chunk of 64
+  // stored k is 32 values in both parts: k-steps 0 and 1 are their hi parts,
+  // 2 and 3 their lo parts.
+  static constexpr bool SPL = SPL_;
+  static_assert(!SPL || ESZ == 2, "split operands are pairs of 16-bit values");
+  static __device__ __forceinline__ int kvec(int s, int h) { return GB || SPL ? 2 * s + h : h * NS + s; }
   static __device__ __forceinline__ void gb_block(int b, int& jb, int& ib) {
-    if (TA) {
+    if (TA && SPL) {
+      // one row of blocks; stage block b holds part b / (BM / 16) of i-block
+      // b % (BM / 16), stored at block 4 (i / 2) + 2 part + i % 2 of the row
+      const int part = b / (BM / 16), i = b - part * (BM / 16);
+      jb = 0;
+      ib = (i >> 1) * 4 + part * 2 + (i & 1);
+    } else if (TA) {
       jb = b / (BM / 16);
       ib = b - jb * (BM / 16);
     } else if (SA == 4) {
@@ -250,8 +263,11 @@ struct LoadPlan {
     if constexpr (G::GB) {
       // the tile's blocks: TA, i-blocks [0, BM/16) of the j-block rows up to
       // kmax; else its BM/32 j-block rows (every i-block)
-      const int64_t rows32 = ((int64_t)A.kmax + 31) / 32;
-      const int64_t elems = G::TA ? (rows32 > 0 ? (rows32 - 1) * 32 * A.ld + G::BM * 32 : 0) : (int64_t)G::BM * A.ld;
+      // (split TA: 64 stored k and 2 ld stored columns per j-block row)
+      const int64_t rows32 = G::SPL ? (int64_t)A.kmax / 64 : ((int64_t)A.kmax + 31) / 32;
+      const int64_t rowe = (G::SPL ? 64 : 32) * A.ld;
+      const int64_t elems =
+          G::TA ? (rows32 > 0 ? (rows32 - 1) * rowe + G::BM * (G::SPL ? 64 : 32) : 0) : (int64_t)G::BM * A.ld;
       return __builtin_amdgcn_make_buffer_rsrc((void*)A.base, 0, (int)(elems * 2), 0x00020000);
     } else {
       return G::TA ? make_rsrc_t<G::BM, G::ESZ>(A) : make_rsrc<G::ESZ>(A);
@@ -345,7 +361,11 @@ struct LoadPlan {
       int jb, ib;
       G::gb_block(I * G::NW + w, jb, ib);
       const int lane = threadIdx.x & 63;
-      if (G::TA) {
+      if (G::TA && G::SPL) {
+        // whole chunks (kmax a multiple of 64): one row of blocks each
+        off = k0 < kmax_a ? voff[I] : OOB;
+        soff = (uint32_t)(k0 * lda);
+      } else if (G::TA) {
         // k = j: this lane's row of the block; a chunk is k0 / 32 j-block rows down
         const int jj = (lane & 31) ^ (8 * kr + 4 * (ib & 1));
         off = (k0 + 32 * jb + jj < kmax_a) ? voff[I] : OOB;
@@ -533,30 +553,34 @@ struct FragReader {
   }
   template <int R>
   __device__ __forceinline__ void read(Frags<G>& f) const {
+    read_to<R>(f.a, f.b);
+  }
+  template <int R>
+  __device__ __forceinline__ void read_to(i16x8 (&fa)[G::FM], i16x8 (&fb)[G::FN]) const {
     constexpr int NA = frag_reads_a<G>();
     if constexpr (R < NA) {
       if constexpr (TA16) {
         i16x4_t v;
         asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(v) : "v"(ta[R / 2][R % 2]) : "memory");
         if constexpr (R % 2 == 0)
-          f.a[R / 2].lo = v;
+          fa[R / 2].lo = v;
         else
-          f.a[R / 2].hi = v;
+          fa[R / 2].hi = v;
       } else if constexpr (TA32) {
-        f32x4 v = __builtin_bit_cast(f32x4, f.a[R / 4]);
+        f32x4 v = __builtin_bit_cast(f32x4, fa[R / 4]);
         v[R % 4] = lds_read_b32<(R % 4) * G::BM * 4>(a32[R / 4]);
-        f.a[R / 4] = __builtin_bit_cast(i16x8, v);
+        fa[R / 4] = __builtin_bit_cast(i16x8, v);
       } else {
-        f.a[R] = lds_read_b128<R * 32 * G::ROWB>(abase);
+        fa[R] = lds_read_b128<R * 32 * G::ROWB>(abase);
       }
     } else {
       constexpr int RB = R - NA;
       if constexpr (G::TB) {
-        f32x4 v = __builtin_bit_cast(f32x4, f.b[RB / 4]);
+        f32x4 v = __builtin_bit_cast(f32x4, fb[RB / 4]);
         v[RB % 4] = lds_read_b32<(RB % 4) * G::BN * 4>(b32[RB / 4]);
-        f.b[RB / 4] = __builtin_bit_cast(i16x8, v);
+        fb[RB / 4] = __builtin_bit_cast(i16x8, v);
       } else {
-        f.b[RB] = lds_read_b128<RB * 32 * G::ROWB>(bbase);
+        fb[RB] = lds_read_b128<RB * 32 * G::ROWB>(bbase);
       }
     }
   }
@@ -922,6 +946,143 @@ __device__ __forceinline__ void mainloop_ks2(LoadPlan<G>& lp, int K, char* lds, 
   mfma_step<G, 0, 0, FH>(f1, acc, lp, 0, lds, lds, fh);
 }
 
+// ------------------------------------------------------- split operands
+// The k-loop of split operands (Geo::SPL): an fp32 value v is the pair hi =
+// fp16(v), lo = fp16(v - hi), and the product of two of them hi hi + lo hi +
+// hi lo.  Per 16 k the fragments of both parts are read once and used in three
+// products,
+//   P1 = A.hi B.hi,  P2 = A.lo B.hi,  P3 = A.hi B.lo,
+// i.e. 2 (FM + FN) fragment reads for 3 FM FN MFMAs, and one chunk (64 KB of
+// a 256 x 256 tile) feeds 1.5 times the MFMAs of a chunk of plain 16-bit
+// operands: the same three products as one GEMM over [hi | lo | hi] and
+// [hi | hi | lo] rows cost a third more LDS reads and half more global loads
+// per MFMA.  Registers hold A's hi and lo fragments in two sets that swap
+// roles every 16 k, and B's in one set each: a set is read again during the
+// product after the last one that used it,
+//   P3 (the 16 k before): next A.hi, B.hi;  P1: A.lo, B.lo;  P2: nothing,
+// so every read has a product (FM FN MFMAs) of lead.  As in mainloop_core the
+// last product of a chunk runs after the next chunk's barrier, under the
+// first reads of that chunk; the chunk's loads go out during that product and
+// the next one.  CHAIN, hook, VMF and the stages are mainloop_core's.
+// Measured at 32768 x 1152: forward 5.6-5.8 ms (1273-1325 TFLOP/s of fp16
+// products), 83% MFMA busy at 1.47 GHz; what bounds it is the card's power (the
+// bf16 kernels run 59-67% busy at 1.65-1.8 GHz), so a busier loop buys little
+// time at the largest sizes.
+template <class G>
+__device__ __forceinline__ void lgkm_wait_ab(i16x8 (&a)[G::FM], i16x8 (&b)[G::FN]) {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < G::FM; ++i) asm volatile("" : "+v"(a[i]));
+#pragma unroll
+  for (int j = 0; j < G::FN; ++j) asm volatile("" : "+v"(b[j]));
+}
+// one product of fragments a, b; READ: the reads of `rd` into na, nb spread
+// two per MFMA over the first MFMAs, loads [L0, L1) over all of them
+template <class G, int L0, int L1, bool READ>
+__device__ __forceinline__ void split_step(const i16x8 (&a)[G::FM], const i16x8 (&b)[G::FN],
+                                           f32x16 (&acc)[G::FM][G::FN], const LoadPlan<G>& lp, int k0, char* ad,
+                                           char* bd, const FragReader<G>& rd, i16x8 (&na)[G::FM],
+                                           i16x8 (&nb)[G::FN]) {
+  constexpr int NR = frag_reads<G>();
+  static_assert((NR + 1) / 2 <= G::NMF, "read slots");
+  static_for<G::NMF>([&](auto mc) {
+    constexpr int m = mc;
+    acc[m / G::FN][m % G::FN] =
+        mfma16_32x32x16<G::F16>(a[m / G::FN], b[m % G::FN], acc[m / G::FN][m % G::FN]);
+    if constexpr (READ && 2 * m < NR) {
+      sched_fence();
+      rd.template read_to<2 * m>(na, nb);
+      if constexpr (2 * m + 1 < NR) rd.template read_to<2 * m + 1>(na, nb);
+      sched_fence();
+    }
+    LoadSlots<G, L0, L1>::template after<m>(lp, k0, ad, bd);
+  });
+  sched_fence();
+}
+template <class G, bool ZERO, bool CHAIN, class Hook = NoHook, int VMF = 0>
+__device__ __forceinline__ void mainloop_split(LoadPlan<G>& lp, __amdgpu_buffer_rsrc_t ra_next,
+                                               __amdgpu_buffer_rsrc_t rb_next, bool has_next, int K, char* lds,
+                                               int& p0, f32x16 (&acc)[G::FM][G::FN], const Hook& hook = Hook(),
+                                               bool vmf_first = false) {
+  static_assert(G::SPL && G::NS == 4 && G::MPB == 1 && G::S == 2, "16-bit pairs, four k-steps, two stages");
+  static_assert(G::SA == 2 || (G::SA == 3 && !CHAIN && VMF == 0), "three A stages: one tile per call");
+  if constexpr (ZERO) {
+#pragma unroll
+    for (int i = 0; i < G::FM; ++i)
+#pragma unroll
+      for (int j = 0; j < G::FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  }
+  constexpr int BK = G::BK;
+  constexpr int LA = LoadPlan<G>::A_LOADS;
+  constexpr int L1 = G::SA == 2 ? G::IPW / 2 : LA, L2 = G::IPW;
+  // as mainloop_core: two A stages, chunk kt + 1's first and second half of
+  // the loads; three, chunk kt + 1's B loads, then chunk kt + 2's A loads
+  constexpr int S0A = G::SA == 2 ? 0 : LA, S0B = G::SA == 2 ? L1 : L2;
+  constexpr int S1A = G::SA == 2 ? L1 : 0, S1B = G::SA == 2 ? L2 : LA;
+  const int nk = (K + BK - 1) / BK;
+  i16x8 a0[G::FM], a1[G::FM], bh[G::FN], bl[G::FN];
+  for (int kt = 0; kt < nk; ++kt) {
+    if constexpr (G::SA == 3)
+      wait_barrier<LA>();
+    else if (VMF > 0 && kt == 0 && vmf_first)
+      wait_barrier<VMF>();
+    else
+      wait_barrier<0>();
+    lgkm_wait_ab<G>(a0, bl);
+    sched_fence();
+    char *ca, *cb, *na, *nb;
+    if constexpr (G::SA == 2) {
+      ca = G::a_stage(lds, (kt + p0) & 1);
+      cb = G::b_stage(lds, (kt + p0) & 1);
+      na = G::a_stage(lds, (kt + p0 + 1) & 1);
+      nb = G::b_stage(lds, (kt + p0 + 1) & 1);
+    } else {
+      ca = G::a_stage(lds, kt % 3);
+      cb = G::b_stage(lds, kt & 1);
+      na = G::a_stage(lds, (kt + 2) % 3);
+      nb = G::b_stage(lds, (kt + 1) & 1);
+    }
+    int k1 = (kt + 1) * BK;
+    if constexpr (CHAIN) {
+      if (kt + 1 == nk && has_next) {
+        lp.ra = ra_next;
+        lp.rb = rb_next;
+        k1 = 0;
+      }
+    }
+    const int k2 = G::SA == 2 ? k1 : (kt + 2) * BK;
+    const FragReader<G> h0(ca, cb, 0), h1(ca, cb, 1), l0(ca, cb, 2), l1(ca, cb, 3);
+    if (kt > 0) {
+      split_step<G, S0A, S0B, true>(a0, bl, acc, lp, k1, na, nb, h0, a1, bh);  // P3 of the chunk before
+    } else {
+      static_for<frag_reads<G>()>([&](auto r) { h0.template read_to<r>(a1, bh); });
+      static_for<S0B - S0A>([&](auto i) { lp.template issue<S0A + i>(k1, na, nb); });
+      hook();
+    }
+    lgkm_wait_ab<G>(a1, bh);
+    sched_fence();
+    split_step<G, S1A, S1B, true>(a1, bh, acc, lp, k2, na, nb, l0, a0, bl);  // P1, values 0-15
+    lgkm_wait_ab<G>(a0, bl);
+    sched_fence();
+    split_step<G, 0, 0, false>(a0, bh, acc, lp, 0, lds, lds, l0, a0, bl);  // P2
+    split_step<G, 0, 0, true>(a1, bl, acc, lp, 0, lds, lds, h1, a0, bh);  // P3
+    lgkm_wait_ab<G>(a0, bh);
+    sched_fence();
+    split_step<G, 0, 0, true>(a0, bh, acc, lp, 0, lds, lds, l1, a1, bl);  // P1, values 16-31
+    lgkm_wait_ab<G>(a1, bl);
+    sched_fence();
+    split_step<G, 0, 0, false>(a1, bh, acc, lp, 0, lds, lds, l1, a1, bl);  // P2
+  }
+  static_for<G::NMF>([&](auto mc) {
+    constexpr int m = mc;
+    acc[m / G::FN][m % G::FN] =
+        mfma16_32x32x16<G::F16>(a0[m / G::FN], bl[m % G::FN], acc[m / G::FN][m % G::FN]);
+  });
+  if constexpr (CHAIN) p0 = (p0 + nk) & 1;
+}
+
 // Split k: k-group 1's accumulators added to k-group 0's through LDS (over
 // the ring, after every wave's last ring read and load), acc(0) + acc(1) in
 // that order; the waves of group 0 then hold the tile's sums.  The ring is
@@ -964,7 +1125,10 @@ __device__ __forceinline__ void mainloop(const Operand& A, const Operand& B, int
     ks_reduce<G>(lds, acc);
   } else {
     int p0 = 0;
-    mainloop_core<G, ZERO, false>(lp, lp.ra, lp.rb, false, K, lds, p0, acc);
+    if constexpr (G::SPL)
+      mainloop_split<G, ZERO, false>(lp, lp.ra, lp.rb, false, K, lds, p0, acc);
+    else
+      mainloop_core<G, ZERO, false>(lp, lp.ra, lp.rb, false, K, lds, p0, acc);
     drain_loads();
   }
 }

@@ -75,7 +75,7 @@ template <bool F16>
 struct Tile16V : Pack16<F16> {
   using Elem = uint16_t;
   using Op = g16::Operand;
-  static constexpr bool TA = false, GB = false;
+  static constexpr bool TA = false, GB = false, SPL = false;
   static constexpr int TB = 0;
   static constexpr int BM = 128, BN = 128, TM = 64, TN = 64, FM = 2, FN = 2, WM = 2, WN = 2, NT = 256;
   static constexpr int LDS_BYTES = g16::Cfg<MEC_16BIT_BK>::LDS_ELEMS * 2;
@@ -103,12 +103,12 @@ template <> struct PackOf<gdma::K_F32> { using type = PackF32; };
 // k-row-major (fp32 raw input rows; 1: 16-byte lanes, 2: 4-byte lanes); S_:
 // stages of the LDS ring (gdma::Geo::S)
 template <int BM_, int BN_, bool TA_, int WM_, int WN_, int KIND, int SA_ = 2, bool GB_ = false, bool ROLL_ = false,
-          int TB_ = 0, int S_ = 2, int KS_ = 1>
+          int TB_ = 0, int S_ = 2, int KS_ = 1, bool SPL_ = false>
 struct TileD : PackOf<KIND>::type {
   using Elem = typename std::conditional<KIND == gdma::K_F32, float, uint16_t>::type;
   using Op = gdma::Operand;
-  using G = gdma::Geo<BM_, BN_, TA_, WM_, WN_, KIND, SA_, GB_, TB_, S_, KS_>;
-  static constexpr bool TA = TA_, GB = GB_, ROLL = ROLL_;
+  using G = gdma::Geo<BM_, BN_, TA_, WM_, WN_, KIND, SA_, GB_, TB_, S_, KS_, SPL_>;
+  static constexpr bool TA = TA_, GB = GB_, ROLL = ROLL_, SPL = SPL_;
   static constexpr int TB = TB_;
   static constexpr int BM = G::BM, BN = G::BN, TM = G::TM, TN = G::TN, FM = G::FM, FN = G::FN;
   static constexpr int WM = G::WM, WN = G::WN, NT = G::NT;
@@ -151,15 +151,30 @@ struct TileD : PackOf<KIND>::type {
   static __device__ __forceinline__ void chain(Plan& lp, const Op& an, const Op& bn, bool has_next, int K, void* lds,
                                                int& p0, f32x16 (&acc)[FM][FN], const Hook& hook,
                                                bool vmf_first = false) {
-    gdma::mainloop_core<G, true, true, Hook, VMF>(lp, Plan::rsrc_a(an), Plan::rsrc_b(bn), has_next, K, (char*)lds,
-                                                  p0, acc, hook, vmf_first);
+    if constexpr (SPL_)
+      gdma::mainloop_split<G, true, true, Hook, VMF>(lp, Plan::rsrc_a(an), Plan::rsrc_b(bn), has_next, K, (char*)lds,
+                                                     p0, acc, hook, vmf_first);
+    else
+      gdma::mainloop_core<G, true, true, Hook, VMF>(lp, Plan::rsrc_a(an), Plan::rsrc_b(bn), has_next, K, (char*)lds,
+                                                    p0, acc, hook, vmf_first);
   }
   static constexpr int STAGE_BYTES = G::STAGE;  // one ring stage
 };
 
 // Input element types: float, bf16 bits (uint16_t), fp16 (_Float16).  The
 // 16-bit types share every tile and kernel; F16 selects the MFMA and packing.
+// F16S: an fp32 value as the pair of fp16 values hi, lo (fp32 data on the fp16
+// MFMA, three products each; the layout of gdma::Geo::SPL).  The fp16 MFMA has
+// 16 times the rate of the fp32 one, so three products are still several times
+// faster: the CLIP step at 32768 x 1152 took 70.8 ms on the fp32 kernels (89% of
+// their peak) and takes 23.9 ms, 4999 x 640 1166 -> 520 us.  The off-diagonal
+// gradient sums come out at 0.6-1.0 times the fp32 kernels' distance from 64
+// bits (n = 300-65536, d = 64-1500): 16 products round once, and the pairs
+// leave out less than the fp32 sums round off.
+struct F16S { uint16_t bits; };
+template <typename T> struct IsSplit { static constexpr bool value = std::is_same<T, F16S>::value; };
 template <typename T> struct Is16 { static constexpr bool value = false, f16 = false; };
+template <> struct Is16<F16S> { static constexpr bool value = true, f16 = true; };
 template <> struct Is16<uint16_t> { static constexpr bool value = true, f16 = false; };
 template <> struct Is16<_Float16> { static constexpr bool value = true, f16 = true; };
 template <typename T> constexpr int kind16() { return Is16<T>::f16 ? gdma::K_F16 : gdma::K_BF16; }
@@ -168,7 +183,9 @@ template <typename T> constexpr int kind16() { return Is16<T>::f16 ? gdma::K_F16
 template <typename T, bool VEC, bool IS16 = Is16<T>::value> struct FwdTileSel;
 template <typename T> struct FwdTileSel<T, false, false> { using type = TileF32; };
 template <typename T> struct FwdTileSel<T, true, false> { using type = TileD<128, 128, false, 2, 2, gdma::K_F32>; };
-template <typename T> struct FwdTileSel<T, true, true> { using type = TileD<256, 256, false, 4, 2, kind16<T>()>; };
+template <typename T> struct FwdTileSel<T, true, true> {
+  using type = TileD<256, 256, false, 4, 2, kind16<T>(), 2, false, false, 0, 2, 1, IsSplit<T>::value>;
+};
 template <typename T> struct FwdTileSel<T, false, true> { using type = Tile16V<Is16<T>::f16>; };
 template <typename T, bool VEC> using FwdTile = typename FwdTileSel<T, VEC>::type;
 // fp32 at a small N (few 128 x 128 tiles for the CUs): 64 x 64 direct-to-LDS
@@ -218,6 +235,15 @@ template <typename T, bool VEC> struct ConTileSel<T, VEC, true> {
   using wx = TileD<256, 384, true, 2, 4, kind16<T>(), 4, true, true>;
   using wy = TileD<256, 384, false, 2, 4, kind16<T>(), 4, true, true>;
 };
+// (split pairs: 256 x 256, three A stages; a chunk of them has 1.5 times the MFMAs)
+template <bool VEC> struct ConTileSel<F16S, VEC, true> {
+  using x = TileD<256, 256, true, 4, 2, gdma::K_F16, 3, true, false, 0, 2, 1, true>;
+  using y = TileD<256, 256, false, 4, 2, gdma::K_F16, 3, true, false, 0, 2, 1, true>;
+  using nx = x;
+  using ny = y;
+  using wx = x;
+  using wy = y;
+};
 template <typename T, bool VEC = true> using ConTileX = typename ConTileSel<T, VEC>::x;
 template <typename T, bool VEC = true> using ConTileY = typename ConTileSel<T, VEC>::y;
 template <typename T> using ConTileNX = typename ConTileSel<T, true>::nx;
@@ -238,6 +264,20 @@ template <typename T> struct GtOnly { static constexpr bool value = Is16<T>::val
 // the fp16 maximum 65504) and the contractions scale back by 2^-14 (exact).
 template <typename T> struct GScale { static constexpr float value = 1.f; };
 template <> struct GScale<_Float16> { static constexpr float value = 16384.f; };
+template <> struct GScale<F16S> { static constexpr float value = 16384.f; };
+
+// The scales of the split pairs: x and y are multiplied by the powers of two
+// scl[0] and scl[1] before they are split (so that the lo parts stay within
+// fp16's range), scl[2] and scl[3] are their inverses.  Exponent multiplier of
+// the accumulated similarities: c, times the inverse scales of split pairs.
+enum { SCL_X = 0, SCL_Y = 1, SCL_INVX = 2, SCL_INVY = 3 };
+template <typename T>
+__device__ __forceinline__ float exp_mul(float c, const float* __restrict__ scl) {
+  if constexpr (IsSplit<T>::value)
+    return c * scl[SCL_INVX] * scl[SCL_INVY];
+  else
+    return c;
+}
 
 // workgroups per CU the launch bounds promise (the 16-bit direct-load tiles
 // use 96 KB of LDS or more: one per CU)
@@ -254,16 +294,16 @@ __device__ __forceinline__ typename TL::Op tile_op(const T* p, int64_t ld, int r
 template <int A, int B> struct CMax { static constexpr int value = A > B ? A : B; };
 
 // ---------------------------------------------------------------- forward
-// E = exp2(S c - c) of this wave's TM x TN accumulators (S scaled by rx_i ry_j
-// when NORM); rowv[bm * 16 + r] and colv[bn] collect this lane's partial row
+// E = exp2(S cm - c) of this wave's TM x TN accumulators (S scaled by rx_i ry_j
+// when NORM; cm = c, exp_mul of split pairs); rowv[bm * 16 + r] and colv[bn] collect this lane's partial row
 // and column sums.  MASK zeroes the diagonal and entries outside [0, N).
 // Eb (not null): every entry of the tile, masked ones as 0, is also stored at
 // Eb[row * ldE + column] (tile-relative; each 32-lane half writes 128 bytes
 // of one row); STORE_S stores the exponent's row-scaled similarity S_ij rx_i
 // there instead (unmasked), from which E is exp2(s c ry_j - c) as here.
 template <class TL, bool NORM, bool MASK, bool STORE_S = false>
-__device__ __forceinline__ void sumexp_epilogue(const f32x16 (&acc)[TL::FM][TL::FN], float c, int m0, int n0, int N,
-                                                const float* s_rx, const float* s_ry, float (&rowv)[TL::FM * 16],
+__device__ __forceinline__ void sumexp_epilogue(const f32x16 (&acc)[TL::FM][TL::FN], float cm, float c, int m0,
+                                                int n0, int N, const float* s_rx, const float* s_ry, float (&rowv)[TL::FM * 16],
                                                 float (&colv)[TL::FN], float* __restrict__ Eb = nullptr,
                                                 int ldE = 0) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w / TL::WN, wn = w % TL::WN;
@@ -274,7 +314,7 @@ __device__ __forceinline__ void sumexp_epilogue(const f32x16 (&acc)[TL::FM][TL::
   for (int bn = 0; bn < TL::FN; ++bn) {
     const int nl = wn * TL::TN + bn * 32 + (lane & 31);
     const int j = n0 + nl;
-    const float cy = NORM ? c * s_ry[nl] : c;
+    const float cy = NORM ? cm * s_ry[nl] : cm;
     float cs = 0.f;
 #pragma unroll
     for (int bm = 0; bm < TL::FM; ++bm) {
@@ -347,9 +387,9 @@ __device__ __forceinline__ void sumexp_tile(const f32x16 (&acc)[TL::FM][TL::FN],
     // interior tiles (no diagonal entry, no row or column beyond N) need no mask
     const bool diag = m0 < n0 + TL::BN && n0 < m0 + TL::BM;
     if (!diag && m0 + TL::BM <= N && n0 + TL::BN <= N)
-      sumexp_epilogue<TL, NORM, false, STORE_S>(acc, c, m0, n0, N, s_rx, s_ry, rowv, colv, Eb, ldE);
+      sumexp_epilogue<TL, NORM, false, STORE_S>(acc, c, c, m0, n0, N, s_rx, s_ry, rowv, colv, Eb, ldE);
     else
-      sumexp_epilogue<TL, NORM, true, STORE_S>(acc, c, m0, n0, N, s_rx, s_ry, rowv, colv, Eb, ldE);
+      sumexp_epilogue<TL, NORM, true, STORE_S>(acc, c, c, m0, n0, N, s_rx, s_ry, rowv, colv, Eb, ldE);
     if constexpr (TL::FM == 1) {
       // one 32-row block: its 16 row sums padded to the 32 of the reduction
       float v[32];
@@ -457,8 +497,9 @@ template <typename T, bool LIT, bool NORM, bool VEC>
 __global__ __launch_bounds__((FwdTile<T, VEC>::NT), (Occ<T, VEC>::fwd)) void k_sumexp_det(
     const T* __restrict__ X, int64_t ldx, const T* __restrict__ Y, int64_t ldy, int N, int D, int kmax, float c,
     const float* __restrict__ rx, const float* __restrict__ ry, float* __restrict__ rowpart,
-    float* __restrict__ colpart, int tiles_m, int tiles_n, int P, int Q) {
+    float* __restrict__ colpart, int tiles_m, int tiles_n, int P, int Q, const float* __restrict__ scl) {
   using TL = FwdTile<T, VEC>;
+  const float cm = exp_mul<T>(c, scl);
   static_assert(TL::FM == 2, "row reduction assumes 64-row wave sub-tiles");
   static_assert(TL::WN == 2, "two row-sum slots per row");
   static_assert(TL::NT >= TL::BM && TL::NT >= TL::BN, "one row and one column per thread");
@@ -511,9 +552,9 @@ __global__ __launch_bounds__((FwdTile<T, VEC>::NT), (Occ<T, VEC>::fwd)) void k_s
     float colv[TL::FN];
     const bool diag = m0 < n0 + TL::BN && n0 < m0 + TL::BM;
     if (!diag && m0 + TL::BM <= N && n0 + TL::BN <= N)
-      sumexp_epilogue<TL, NORM, false>(acc, c, m0, n0, N, s_rx, s_ry, rowv, colv);
+      sumexp_epilogue<TL, NORM, false>(acc, cm, c, m0, n0, N, s_rx, s_ry, rowv, colv);
     else
-      sumexp_epilogue<TL, NORM, true>(acc, c, m0, n0, N, s_rx, s_ry, rowv, colv);
+      sumexp_epilogue<TL, NORM, true>(acc, cm, c, m0, n0, N, s_rx, s_ry, rowv, colv);
     s_row[wn][my_row] = transpose_reduce32(rowv, lane);
     if (!LIT) {
 #pragma unroll
@@ -635,7 +676,8 @@ struct BlockGrid {
 //          up to 128 and zero columns [N, ldt): element (d, i) = rx_i x_i[d].
 // Every contraction operand is then K-major (k contiguous).  The bf16x3 mode
 // keeps GT, XT and YT as bf16 hi planes (gt, xt, yt) and lo planes (gt_lo,
-// xt_lo, yt_lo), all null otherwise.
+// xt_lo, yt_lo), all null otherwise.  Split pairs (F16S) keep both parts in
+// gt, xt and yt, every 32 values as 64 (gdma::Geo::SPL), scaled by scl.
 struct GradBufs {
   void* g[2];
   void* gt[2];
@@ -645,6 +687,7 @@ struct GradBufs {
   void* gt_lo[2];
   const void* xt_lo;
   const void* yt_lo;
+  const float* scl;  // scales of split pairs (F16S)
 };
 
 // One pipeline step of the backward (launch t = 0 .. nb):
@@ -712,20 +755,22 @@ constexpr int gt_chain_stores() {
   return TL::FM * TL::FN * 2;
 }
 // X3 (bf16x3): a second plane bf16(G' - bf16(G')) at GTl, the same way.
+// TL::SPL (split pairs): the lo part fp16(G' - fp16(G')) two blocks after the hi part.
 template <class TL, bool LIT, bool NORM, bool MASK, int GSC, bool X3 = false>
-__device__ __forceinline__ void grad_gt_store_direct(const f32x16 (&acc)[TL::FM][TL::FN], float c, int i0, int j0,
-                                                     int N, uint16_t* __restrict__ GTb, int bs, const float* s_rx,
+__device__ __forceinline__ void grad_gt_store_direct(const f32x16 (&acc)[TL::FM][TL::FN], float cm, float c, int i0,
+                                                     int j0, int N, uint16_t* __restrict__ GTb, int bs, const float* s_rx,
                                                      const float* s_ry, const float* s_ir, const float* s_ic,
                                                      uint16_t* __restrict__ GTl = nullptr) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  constexpr int NP = X3 ? 2 : 1;  // planes
+  constexpr bool SPL = TL::SPL;
+  constexpr int NP = X3 || SPL ? 2 : 1;  // planes
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w / TL::WN, wn = w % TL::WN;
-  const int64_t rowb = (int64_t)(bs >> 4) * 512;  // elements per row of blocks
+  const int64_t rowb = (int64_t)(bs >> 4) * (SPL ? 1024 : 512);  // elements per row of blocks
   // Non-temporal stores through buffer descriptors at the tile's planes (the
   // write-once G'^T should not displace the operand panels from the caches).
   // __builtin_nontemporal_store lost its hint in this function for the
   // one-plane case (no nt bit in the stores); the buffer store's cache-policy
-  // operand (2: nt) keeps it.  A tile's offsets stay below 8 * bs * 64 bytes.
+  // operand (2: nt) keeps it.  A tile's offsets stay below 8 * bs * 64 bytes (twice that for split pairs).
   const __amdgpu_buffer_rsrc_t rs_hi = __builtin_amdgcn_make_buffer_rsrc((void*)GTb, 0, 0x7fffffff, 0x00020000);
   const __amdgpu_buffer_rsrc_t rs_lo =
       __builtin_amdgcn_make_buffer_rsrc((void*)(X3 ? GTl : GTb), 0, 0x7fffffff, 0x00020000);
@@ -733,7 +778,7 @@ __device__ __forceinline__ void grad_gt_store_direct(const f32x16 (&acc)[TL::FM]
   for (int bn = 0; bn < TL::FN; ++bn) {
     const int nl = wn * TL::TN + bn * 32 + (lane & 31);
     const int j = j0 + nl;
-    const float cy = NORM ? c * s_ry[nl] : c;
+    const float cy = NORM ? cm * s_ry[nl] : cm;
     const float icj = s_ic[nl];
     const int64_t jrow = ((wn * TL::TN + bn * 32) >> 5) * rowb;
 #pragma unroll
@@ -763,9 +808,14 @@ __device__ __forceinline__ void grad_gt_store_direct(const f32x16 (&acc)[TL::FM]
             for (int e = 0; e < 4; ++e) gv[e] -= bf16_to_f32(f32_to_bf16(gv[e]));
             pk[NP - 1][q][0] = TL::pack2(gv[0], gv[1]);
             pk[NP - 1][q][1] = TL::pack2(gv[2], gv[3]);
+          } else if constexpr (SPL) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) gv[e] -= (float)(_Float16)gv[e];
+            pk[NP - 1][q][0] = TL::pack2(gv[0], gv[1]);
+            pk[NP - 1][q][1] = TL::pack2(gv[2], gv[3]);
           }
         }
-        const int ib = (wm * TL::TM + bm * 32) / 16 + p;
+        const int ib = SPL ? (wm * TL::TM + bm * 32) / 8 + p : (wm * TL::TM + bm * 32) / 16 + p;
         const int64_t off = jrow + ib * 512 + gdma::gb_slot(lane & 31, lane >> 5, p) * 8;
 #pragma unroll
         for (int pl = 0; pl < NP; ++pl) {
@@ -776,7 +826,8 @@ __device__ __forceinline__ void grad_gt_store_direct(const f32x16 (&acc)[TL::FM]
             pk[pl][1][d] = sw[1];
           }
           const u32x4 u = u32x4{pk[pl][0][0], pk[pl][0][1], pk[pl][1][0], pk[pl][1][1]};
-          __builtin_amdgcn_raw_buffer_store_b128(u, pl ? rs_lo : rs_hi, (uint32_t)(off * 2), 0, 2);
+          __builtin_amdgcn_raw_buffer_store_b128(u, X3 && pl ? rs_lo : rs_hi,
+                                                 (uint32_t)(off * 2) + (SPL ? pl * 2048 : 0), 0, 2);
         }
       }
     }
@@ -818,15 +869,15 @@ __device__ __forceinline__ void grad_g_tile(const T* __restrict__ X, int64_t ldx
   if constexpr (X3) {
     static_assert(std::is_same<T, uint16_t>::value, "bf16x3 runs on bf16 split operands");
     if (!diag && i0 + TL::BM <= N && j0 + TL::BN <= N)
-      grad_gt_store_direct<TL, LIT, NORM, false, 1, true>(acc, c, i0, j0, N, GTb, bs, s_rx, s_ry, s_ir, s_ic, GTl);
+      grad_gt_store_direct<TL, LIT, NORM, false, 1, true>(acc, c, c, i0, j0, N, GTb, bs, s_rx, s_ry, s_ir, s_ic, GTl);
     else
-      grad_gt_store_direct<TL, LIT, NORM, true, 1, true>(acc, c, i0, j0, N, GTb, bs, s_rx, s_ry, s_ir, s_ic, GTl);
+      grad_gt_store_direct<TL, LIT, NORM, true, 1, true>(acc, c, c, i0, j0, N, GTb, bs, s_rx, s_ry, s_ir, s_ic, GTl);
   } else if constexpr (GtOnly<T>::value) {
     // (s_ir, s_ic carry the storage scale)
     if (!diag && i0 + TL::BM <= N && j0 + TL::BN <= N)
-      grad_gt_store_direct<TL, LIT, NORM, false, 1>(acc, c, i0, j0, N, (uint16_t*)GTb, bs, s_rx, s_ry, s_ir, s_ic);
+      grad_gt_store_direct<TL, LIT, NORM, false, 1>(acc, c, c, i0, j0, N, (uint16_t*)GTb, bs, s_rx, s_ry, s_ir, s_ic);
     else
-      grad_gt_store_direct<TL, LIT, NORM, true, 1>(acc, c, i0, j0, N, (uint16_t*)GTb, bs, s_rx, s_ry, s_ir, s_ic);
+      grad_gt_store_direct<TL, LIT, NORM, true, 1>(acc, c, c, i0, j0, N, (uint16_t*)GTb, bs, s_rx, s_ry, s_ir, s_ic);
   } else {
     if (!diag && i0 + TL::BM <= N && j0 + TL::BN <= N)
       grad_g_store<TL, LIT, NORM, false>(acc, c, i0, j0, N, (float*)Gb, bs, s_rx, s_ry, s_ir, s_ic);
@@ -851,27 +902,31 @@ __device__ __forceinline__ void grad_g_tile(const T* __restrict__ X, int64_t ldx
 // atomics, clip_loss.py:148-156).
 // X3 (bf16x3): Gblk/OT are the hi planes and Glo/OTlo the lo planes; the
 // tile is hi.hi + hi.lo + lo.hi, three passes over K into one accumulator.
+// osc: the inverse of the operands' storage scales (a power of two).
 template <class TC, typename T, bool X3 = false>
 __device__ __forceinline__ void grad_contract_tile(int N, int D, const T* __restrict__ Gblk,
                                                    const T* __restrict__ Glo, const T* __restrict__ OT,
                                                    const T* __restrict__ OTlo, int64_t ldt, const BlockGrid& bg,
                                                    int P, int Q, int tm, int td, bool accumulate,
-                                                   float* __restrict__ out, char* lds) {
+                                                   float* __restrict__ out, char* lds, float osc) {
   const int r0 = P * bg.bs + tm * TC::BM;
   if (r0 >= N) return;
   const int d0 = td * TC::BN;
   const int q0 = Q * bg.bs;
   const int qn = min(bg.bs, N - q0);
-  // entries of G' and XT/YT at k in [qn, round8(qn)) are stored zeros
-  const int kq = (qn + 7) & ~7;
+  // entries of G' and XT/YT at k in [qn, round8(qn)) (split pairs: round32)
+  // are stored zeros; split pairs store every 32 k as 64
+  constexpr bool SPL = IsSplit<T>::value;
+  constexpr int E = SPL ? 2 : 1;
+  const int kq = SPL ? 2 * ((qn + 31) & ~31) : (qn + 7) & ~7;
   // A: rows tm*BM.. of the block (K-major), or columns tm*BM.. of a transposed
   // block (blocked layout: i-block tm*BM/16 of the first j-block row)
-  const int64_t a_off = TC::TA ? (int64_t)(tm * TC::BM) * (TC::GB ? 32 : 1) : (int64_t)(tm * TC::BM) * bg.bs;
-  const auto A = tile_op<TC>(Gblk + a_off, bg.bs, TC::BM, kq);
+  const int64_t a_off = E * (TC::TA ? (int64_t)(tm * TC::BM) * (TC::GB ? 32 : 1) : (int64_t)(tm * TC::BM) * bg.bs);
+  const auto A = tile_op<TC>(Gblk + a_off, SPL && !TC::TA ? 2 * (int64_t)bg.bs : bg.bs, TC::BM, kq);
   // the feature operand: transposed copy (rows d, k = q0 + j) or, fp32, the
   // raw rows q0 + k (only the block's qn valid rows)
-  const int64_t b_off = TC::TB ? (int64_t)q0 * ldt + d0 : (int64_t)d0 * ldt + q0;
-  const auto B = tile_op<TC>(OT + b_off, ldt, min(D - d0, TC::BN), TC::TB ? qn : kq);
+  const int64_t b_off = TC::TB ? (int64_t)q0 * ldt + d0 : E * ((int64_t)d0 * ldt + q0);
+  const auto B = tile_op<TC>(OT + b_off, E * ldt, min(D - d0, TC::BN), TC::TB ? qn : kq);
   f32x16 acc[TC::FM][TC::FN];
   TC::template run<true, true>(A, B, kq, lds, acc);
   if constexpr (X3) {
@@ -894,7 +949,7 @@ __device__ __forceinline__ void grad_contract_tile(int N, int D, const T* __rest
           // a fire-and-forget add in L2 instead of a load-add-store round trip;
           // the tile has one owner per launch, so the summation order (launch
           // order) and the result are deterministic
-          const float v = acc[bm][bn][r] * (1.f / GScale<T>::value);
+          const float v = acc[bm][bn][r] * osc;
           if (accumulate)
             __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           else
@@ -913,8 +968,10 @@ __device__ __forceinline__ void grad_contract_dispatch(int sub, int N, int D, co
                                                        const StepPlan& sp, float* __restrict__ acc_x,
                                                        float* __restrict__ acc_y, char* lds, const T* X = nullptr,
                                                        int64_t ldx = 0, const T* Y = nullptr, int64_t ldy = 0) {
-  const int64_t blk = (int64_t)bg.bs * bg.bs;  // elements per G' block
+  const int64_t blk = (int64_t)bg.bs * bg.bs * (IsSplit<T>::value ? 2 : 1);  // elements per G' block
   const bool is_x = sub < sp.cx_pad;
+  float osc = 1.f / GScale<T>::value;
+  if constexpr (IsSplit<T>::value) osc *= gb.scl[is_x ? SCL_INVY : SCL_INVX];
   if (!is_x) sub -= sp.cx_pad;
   const int pid = xcd_remap(sub, is_x ? sp.cx_pad : sp.cy_pad);
   if (pid >= (is_x ? sp.cx_n : sp.cy_n)) return;
@@ -953,26 +1010,26 @@ __device__ __forceinline__ void grad_contract_dispatch(int sub, int N, int D, co
     const T* gxl = X3 ? (const T*)gb.gt_lo[buf] + P * blk : nullptr;
     if (narrow)
       grad_contract_tile<TNX, T, X3>(N, D, gx, gxl, (const T*)gb.yt, (const T*)gb.yt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_x, lds);
+                                     sp.accumulate != 0, acc_x, lds, osc);
     else if constexpr (TCX::TB)
       grad_contract_tile<TCX, T, X3>(N, D, gx, gxl, Y, nullptr, ldy, bg, P, Q, tm, td, sp.accumulate != 0, acc_x,
-                                     lds);
+                                     lds, osc);
     else
       grad_contract_tile<TCX, T, X3>(N, D, gx, gxl, (const T*)gb.yt, (const T*)gb.yt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_x, lds);
+                                     sp.accumulate != 0, acc_x, lds, osc);
   } else {
     const int Q = (P - sp.diag_c + bg.nb) % bg.nb;
     const T* gy = (const T*)(GtOnly<T>::value ? gb.gt[buf] : gb.g[buf]) + Q * blk;
     const T* gyl = X3 ? (const T*)gb.gt_lo[buf] + Q * blk : nullptr;
     if (narrow)
       grad_contract_tile<TNY, T, X3>(N, D, gy, gyl, (const T*)gb.xt, (const T*)gb.xt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_y, lds);
+                                     sp.accumulate != 0, acc_y, lds, osc);
     else if constexpr (TCY::TB)
       grad_contract_tile<TCY, T, X3>(N, D, gy, gyl, X, nullptr, ldx, bg, P, Q, tm, td, sp.accumulate != 0, acc_y,
-                                     lds);
+                                     lds, osc);
     else
       grad_contract_tile<TCY, T, X3>(N, D, gy, gyl, (const T*)gb.xt, (const T*)gb.xt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_y, lds);
+                                     sp.accumulate != 0, acc_y, lds, osc);
   }
 }
 
@@ -990,7 +1047,7 @@ __global__ __launch_bounds__(ConTileX<T>::NT, 1) void k_grad_contract(int N, int
   using TNY = typename std::conditional<W, TCY, typename Sel::ny>::type;
   static_assert(TCX::BM == TCY::BM && TCX::BN == TCY::BN && TCX::NT == TCY::NT && TCX::NT == ConTileX<T>::NT,
                 "one contraction tile shape and workgroup size");
-  static_assert(W || (TNX::NT == TCX::NT && TNY::NT == TCX::NT && TNX::BM == 2 * TCX::BM && 2 * TNX::BN == TCX::BN),
+  static_assert(W || IsSplit<T>::value || (TNX::NT == TCX::NT && TNY::NT == TCX::NT && TNX::BM == 2 * TCX::BM && 2 * TNX::BN == TCX::BN),
                 "narrow tiles: two row tiles high, half a feature tile wide");
   __shared__ __attribute__((aligned(1024)))
   char lds[CMax<CMax<TCX::LDS_BYTES, TCY::LDS_BYTES>::value, CMax<TNX::LDS_BYTES, TNY::LDS_BYTES>::value>::value];
@@ -1063,10 +1120,12 @@ __global__ __launch_bounds__((FwdTile<T, true>::NT), 1) void k_grad_g_chain(
   enum { V_RX = 0, V_RY = 1, V_IR = 2, V_IC = 3 };
   __shared__ __attribute__((aligned(1024))) char lds[TL::LDS_BYTES];
   __shared__ __attribute__((aligned(16))) float s_vec[2][4][TL::BM];
-  constexpr int NST = gt_chain_stores<TL>() * (X3 ? 2 : 1);  // G'^T stores per lane and tile (X3: two planes)
+  constexpr int NST = gt_chain_stores<TL>() * (X3 || IsSplit<T>::value ? 2 : 1);  // G'^T stores per lane and tile (two parts)
   const int64_t n64 = N;
-  const int64_t blk = (int64_t)bg.bs * bg.bs;
+  constexpr int E = IsSplit<T>::value ? 2 : 1;  // stored elements per value
+  const int64_t blk = (int64_t)bg.bs * bg.bs * E;
   const int buf = sp.diag_g & 1;
+  const float cm = exp_mul<T>(c, gb.scl);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   // tile -> (i0, j0, its place in the G'^T block); false for padding ids and tiles wholly past N
   auto coords = [&](int tile, int& i0, int& j0, uint16_t*& gt) {
@@ -1078,7 +1137,7 @@ __global__ __launch_bounds__((FwdTile<T, true>::NT), 1) void k_grad_g_chain(
     const int J = (I + sp.diag_g) % bg.nb;
     i0 = I * bg.bs + tm * TL::BM;
     j0 = J * bg.bs + tn * TL::BN;
-    gt = (uint16_t*)gb.gt[buf] + I * blk + gdma::gb_offset(tn * TL::BN, tm * TL::BM, bg.bs);
+    gt = (uint16_t*)gb.gt[buf] + I * blk + E * gdma::gb_offset(tn * TL::BN, tm * TL::BM, bg.bs);
     return i0 < N && j0 < N;
   };
   auto next_valid = [&](int tile, int& i0, int& j0, uint16_t*& gt) {
@@ -1135,11 +1194,11 @@ __global__ __launch_bounds__((FwdTile<T, true>::NT), 1) void k_grad_g_chain(
     uint16_t* gtl = X3 ? (uint16_t*)gb.gt_lo[buf] + (gt - (uint16_t*)gb.gt[buf]) : nullptr;
     if (!diag && i0 + TL::BM <= N && j0 + TL::BN <= N)
       grad_gt_store_direct<TL, LIT, NORM, false, (int)GScale<T>::value, X3>(
-          acc, c, i0, j0, N, gt, bg.bs, sv + V_RX * TL::BM, sv + V_RY * TL::BM, sv + V_IR * TL::BM,
+          acc, cm, c, i0, j0, N, gt, bg.bs, sv + V_RX * TL::BM, sv + V_RY * TL::BM, sv + V_IR * TL::BM,
           sv + V_IC * TL::BM, gtl);
     else
       grad_gt_store_direct<TL, LIT, NORM, true, (int)GScale<T>::value, X3>(
-          acc, c, i0, j0, N, gt, bg.bs, sv + V_RX * TL::BM, sv + V_RY * TL::BM, sv + V_IR * TL::BM,
+          acc, cm, c, i0, j0, N, gt, bg.bs, sv + V_RX * TL::BM, sv + V_RY * TL::BM, sv + V_IR * TL::BM,
           sv + V_IC * TL::BM, gtl);
     if (!has_next) break;
     tile = next;

@@ -433,4 +433,246 @@ __global__ __launch_bounds__(256) void k_transpose_split(TransSide<float, uint16
   }
 }
 
+// ------------------------------------------------------- fp16 split pairs
+// fp32 as the sum of two fp16 terms, v = hi + lo + r with hi = fp16(v), lo =
+// fp16(v - hi), both rounded to nearest even: |r| <= 2^-23 |v| while lo is a
+// normal number, and never more than 2^-25 (half of fp16's smallest step).  The
+// values are first scaled by a power of two that puts the largest one into
+// [2^14, 2^15), so the second bound is 2^-39 of the largest value: what is lost
+// below it is far smaller than the rounding of an fp32 sum.  The products hi hi
+// + lo hi + hi lo leave out lo lo, at most 2^-22 of a product and of either
+// sign.
+__device__ __forceinline__ void split_pair4(const f32x4& v, uint2& hi, uint2& lo) {
+  float h[4], l[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    h[e] = (float)(_Float16)v[e];
+    // (an infinite value stays hi = inf, lo = 0)
+    l[e] = __builtin_isinf(h[e]) ? 0.f : v[e] - h[e];
+  }
+  hi = uint2{pack2_f16(h[0], h[1]), pack2_f16(h[2], h[3])};
+  lo = uint2{pack2_f16(l[0], l[1]), pack2_f16(l[2], l[3])};
+}
+// the power of two that puts m (the largest finite magnitude) into [2^14,
+// 2^15), kept between 2^-100 and 2^100 (its square must be a number); 1 for 0
+__device__ __forceinline__ float pair_scale(float m) {
+  if (!(m > 0.f)) return 1.f;
+  int s = 14 - ((int)(__float_as_uint(m) >> 23) - 127);
+  s = s < -100 ? -100 : s > 100 ? 100 : s;
+  return __uint_as_float((uint32_t)(s + 127) << 23);
+}
+constexpr float PAIR_UNIT_SCALE = 16384.f;  // of rows that are normalized here (|v| <= 1)
+
+// features d .. d + 3 of a row, zero from D on (vec: 16-byte aligned rows)
+__device__ __forceinline__ f32x4 row_load4(const float* __restrict__ p, int d, int D, bool vec) {
+  if (vec && d + 3 < D) return *(const f32x4*)(p + d);
+  f32x4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = d + e < D ? p[d + e] : 0.f;
+  return v;
+}
+// v (features d .. d + 3) into a row of pairs: every 32 features as 32 hi and
+// then 32 lo values
+__device__ __forceinline__ void pair_store4(uint16_t* __restrict__ out, int d, const f32x4& v) {
+  uint2 hi, lo;
+  split_pair4(v, hi, lo);
+  uint16_t* o = out + (d >> 5) * 64 + (d & 31);
+  *(uint2*)o = hi;
+  *(uint2*)(o + 32) = lo;
+}
+
+struct PairRows {
+  uint16_t* a;     // x rows as pairs, pitch 2 dp (dp = D rounded up to 32, zeros past D)
+  uint16_t* b;     // y rows
+  float* scl;      // the scales (SCL_X ..)
+  int dp;
+};
+
+// Pre-pass of the split pairs, one wave per row: k_prepass's norms and
+// diagonal.  NORM: also the pairs of x_i rx_i and y_i ry_i (one launch instead
+// of a pre-pass and a split per side: rows of up to PAIR_REG x 256 features
+// stay in registers between the reduction and the stores).  Otherwise the rows
+// are split as they are, once the largest finite magnitude of each side is
+// known: this launch leaves each workgroup's in the slots 1/R and 1/C (which
+// the finalize fills later) for k_pair_rows.
+constexpr int PAIR_REG = 8;
+template <bool NORM>
+__global__ __launch_bounds__(256) void k_pair_prepass(const float* __restrict__ X, int64_t ldx,
+                                                      const float* __restrict__ Y, int64_t ldy, int N, int D, bool vec,
+                                                      float* __restrict__ ws, PairRows pr) {
+  __shared__ float s_mx[2][4];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int row = blockIdx.x * 4 + w;
+  const int64_t n = N;
+  float mx = 0.f, my = 0.f;
+  if (row < N) {
+    const float* x = X + (int64_t)row * ldx;
+    const float* y = Y + (int64_t)row * ldy;
+    f32x4 xv[PAIR_REG], yv[PAIR_REG];
+    float sx = 0.f, sy = 0.f, sxy = 0.f;
+    auto add = [&](const f32x4& a, const f32x4& b) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sx = fmaf(a[e], a[e], sx);
+        sy = fmaf(b[e], b[e], sy);
+        sxy = fmaf(a[e], b[e], sxy);
+        if (!NORM) {
+          const float p = fabsf(a[e]), q = fabsf(b[e]);
+          mx = p < __builtin_inff() ? fmaxf(mx, p) : mx;
+          my = q < __builtin_inff() ? fmaxf(my, q) : my;
+        }
+      }
+    };
+    const bool inreg = pr.dp <= PAIR_REG * 256;
+    if (inreg) {
+#pragma unroll
+      for (int k = 0; k < PAIR_REG; ++k) {
+        const int d = 4 * lane + 256 * k;
+        if (256 * k < D) {
+          xv[k] = row_load4(x, d, D, vec);
+          yv[k] = row_load4(y, d, D, vec);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < PAIR_REG; ++k)
+        if (256 * k < D) add(xv[k], yv[k]);
+    } else {
+      for (int d = 4 * lane; d < D; d += 256) add(row_load4(x, d, D, vec), row_load4(y, d, D, vec));
+    }
+    sx = wave_sum(sx);
+    sy = wave_sum(sy);
+    sxy = wave_sum(sxy);
+    float rx = 1.f, ry = 1.f;
+    if (NORM) {
+      rx = 1.f / fmaxf(sqrtf(sx), 1e-12f);
+      ry = 1.f / fmaxf(sqrtf(sy), 1e-12f);
+    }
+    if (lane == 0) {
+      ws[WS_RX * n + row] = rx;
+      ws[WS_RY * n + row] = ry;
+      ws[WS_DIAG * n + row] = sxy;
+      ws[WS_ROW_OFF * n + row] = 0.f;
+      ws[WS_COL_OFF * n + row] = 0.f;
+    }
+    if constexpr (NORM) {
+      uint16_t* oa = pr.a + (int64_t)row * (2 * pr.dp);
+      uint16_t* ob = pr.b + (int64_t)row * (2 * pr.dp);
+      // (the power of two is exact: as x_i rx_i scaled)
+      if (inreg) {
+#pragma unroll
+        for (int k = 0; k < PAIR_REG; ++k) {
+          const int d = 4 * lane + 256 * k;
+          if (d < pr.dp) {
+            pair_store4(oa, d, xv[k] * rx * PAIR_UNIT_SCALE);
+            pair_store4(ob, d, yv[k] * ry * PAIR_UNIT_SCALE);
+          }
+        }
+      } else {
+        for (int d = 4 * lane; d < pr.dp; d += 256) {
+          pair_store4(oa, d, row_load4(x, d, D, vec) * rx * PAIR_UNIT_SCALE);
+          pair_store4(ob, d, row_load4(y, d, D, vec) * ry * PAIR_UNIT_SCALE);
+        }
+      }
+    }
+  }
+  if constexpr (NORM) {
+    if (blockIdx.x == 0 && threadIdx.x < 4) pr.scl[threadIdx.x] = threadIdx.x < 2 ? PAIR_UNIT_SCALE : 1.f / PAIR_UNIT_SCALE;
+  } else {
+    for (int m = 32; m >= 1; m >>= 1) {
+      mx = fmaxf(mx, __shfl_xor(mx, m, 64));
+      my = fmaxf(my, __shfl_xor(my, m, 64));
+    }
+    if (lane == 0) {
+      s_mx[0][w] = mx;
+      s_mx[1][w] = my;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+      const float* s = s_mx[threadIdx.x];
+      ws[(threadIdx.x ? WS_INV_COL : WS_INV_ROW) * n + blockIdx.x] = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+    }
+  }
+}
+
+// Pairs of rows that come normalized (k_pair_prepass<false> ran before): every
+// workgroup takes the largest magnitudes from the nmax = ceil(N / 4) it left
+// per side, and its share of the rows, one wave per row.
+__global__ __launch_bounds__(256) void k_pair_rows(const float* __restrict__ X, int64_t ldx,
+                                                   const float* __restrict__ Y, int64_t ldy, int N, int D, bool vec,
+                                                   const float* __restrict__ ws, PairRows pr, int nmax) {
+  __shared__ float s_mx[2][4];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t n = N;
+  float mx = 0.f, my = 0.f;
+  for (int k = threadIdx.x; k < nmax; k += 256) {
+    mx = fmaxf(mx, ws[WS_INV_ROW * n + k]);
+    my = fmaxf(my, ws[WS_INV_COL * n + k]);
+  }
+  for (int m = 32; m >= 1; m >>= 1) {
+    mx = fmaxf(mx, __shfl_xor(mx, m, 64));
+    my = fmaxf(my, __shfl_xor(my, m, 64));
+  }
+  if (lane == 0) {
+    s_mx[0][w] = mx;
+    s_mx[1][w] = my;
+  }
+  __syncthreads();
+  const float sx = pair_scale(fmaxf(fmaxf(s_mx[0][0], s_mx[0][1]), fmaxf(s_mx[0][2], s_mx[0][3])));
+  const float sy = pair_scale(fmaxf(fmaxf(s_mx[1][0], s_mx[1][1]), fmaxf(s_mx[1][2], s_mx[1][3])));
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    pr.scl[0] = sx;
+    pr.scl[1] = sy;
+    pr.scl[2] = 1.f / sx;
+    pr.scl[3] = 1.f / sy;
+  }
+  for (int row = blockIdx.x * 4 + w; row < N; row += gridDim.x * 4) {
+    const float* x = X + (int64_t)row * ldx;
+    const float* y = Y + (int64_t)row * ldy;
+    for (int d = 4 * lane; d < pr.dp; d += 256) {
+      pair_store4(pr.a + (int64_t)row * (2 * pr.dp), d, row_load4(x, d, D, vec) * sx);
+      pair_store4(pr.b + (int64_t)row * (2 * pr.dp), d, row_load4(y, d, D, vec) * sy);
+    }
+  }
+}
+
+// k_transpose_split into pairs: row d of XT (pitch 2 ldt) holds, for every 32
+// rows i, 32 hi and then 32 lo values of scale_i x_i[d] (NORM) times the side's
+// pair scale, zero for N <= i < ldt (ldt a multiple of 64).  Two values of i
+// per thread: 4-byte stores, 64 contiguous bytes per part.
+template <bool NORM>
+__global__ __launch_bounds__(256) void k_transpose_pairs(TransSide<float, uint16_t> s0, TransSide<float, uint16_t> s1,
+                                                         int N, int D, int64_t ldt, const float* scl0,
+                                                         const float* scl1) {
+  const TransSide<float, uint16_t>& sd = blockIdx.z ? s1 : s0;
+  const float ps = blockIdx.z ? *scl1 : *scl0;
+  const float* __restrict__ X = sd.X;
+  const int64_t ldx = sd.ldx;
+  const float* __restrict__ scale = sd.scale;
+  uint16_t* __restrict__ XT = sd.XT;
+  __shared__ float tile[64][65];
+  const int i0 = blockIdx.x * 64, d0 = blockIdx.y * 64;
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+  for (int r = ty; r < 64; r += 4) {
+    const int i = i0 + r, d = d0 + tx;
+    float v = 0.f;
+    if (i < N && d < D) {
+      v = X[(int64_t)i * ldx + d];
+      if (NORM) v *= scale[i];
+      v *= ps;
+    }
+    tile[r][tx] = v;
+  }
+  __syncthreads();
+  const int il = 2 * (threadIdx.x & 31);
+  for (int r = threadIdx.x >> 5; r < 64; r += 8) {
+    const int d = d0 + r;
+    if (d >= D) break;
+    const float a = tile[il][r], b = tile[il + 1][r];
+    const float ha = (float)(_Float16)a, hb = (float)(_Float16)b;
+    uint16_t* o = XT + (int64_t)d * (2 * ldt) + (int64_t)(i0 + (il & 32)) * 2 + (il & 31);
+    *(uint32_t*)o = pack2_f16(ha, hb);
+    *(uint32_t*)(o + 32) = pack2_f16(__builtin_isinf(ha) ? 0.f : a - ha, __builtin_isinf(hb) ? 0.f : b - hb);
+  }
+}
+
 }  // namespace mec

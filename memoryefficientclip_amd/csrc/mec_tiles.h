@@ -38,6 +38,7 @@ constexpr int kDtypeBF16 = 1;
 constexpr int kDtypeF16 = 2;
 constexpr int kDtypeX3 = 3;   // fp32 data, products as three bf16 MFMA terms
 constexpr int kDtypeF32B = 4;  // fp32 data, bf16 products
+constexpr int kDtypePairs = 6;  // fp32 data as fp16 pairs (hi, lo), three products each
 
 // fp32 direct-to-LDS problems whose 128 x 128 grid has fewer than two tiles
 // per CU of a 256-CU device (n <= 2816) run 64 x 64 tiles instead (`small`)
@@ -74,7 +75,7 @@ inline bool f32_small_bwd(int64_t n, int64_t d, int64_t bs, int cus) {
 }
 // forward sums and gradient-matrix tiles (x rows x y rows)
 inline TileDims fwd_tile_dims(int dtype, bool vec, bool small = false) {
-  if (dtype == kDtypeX3 || dtype == kDtypeF32B) return {256, 256};
+  if (dtype == kDtypeX3 || dtype == kDtypeF32B || dtype == kDtypePairs) return {256, 256};
   if (dtype == kDtypeF32 && vec && small) return {64, 64};
   if (dtype == kDtypeF32 || !vec) return {128, 128};
   return {256, 256};

@@ -555,3 +555,45 @@ def test_graph_capture_is_refused_before_any_launch(monkeypatch):
         assert "graph" in _lib.last_error(), (name, _lib.last_error())
     # argument errors still come first
     assert lib.mec_prepass(16, d, 16, d, 0, d, 0, 1, 16, None) == _lib.MEC_ERR_INVALID
+
+
+def test_pairs_sizes_and_rule(monkeypatch):
+    # fp32 data as fp16 pairs: scales and pairs of both inputs in the
+    # workspace (4 bytes per value, d rounded up to 32), scratch with one
+    # diagonal of 4-byte entries and the transposed pairs, n up to 2^20
+    lib = _lib.load()
+    P = _lib.DTYPE_F32_PAIRS
+    for n, d in [(1000, 3), (32768, 1152), (777, 130)]:
+        base = (lib.mec_workspace_floats(n) + 63) // 64 * 64
+        assert lib.mec_workspace_floats_for(n, d, P) == base + 64 + 2 * n * ((d + 31) // 32 * 32)
+        bs, nb = _lib.grad_blocking(n, d, P)
+        assert bs % 256 == 0 and nb * bs >= n > (nb - 1) * bs and 4 * bs * bs < 2 ** 31
+        ldt = (n + 127) // 128 * 128
+        for sides in (1, 2, 3):
+            want = 4 * nb * bs * bs + bin(sides).count("1") * 4 * d * ldt
+            assert lib.mec_grad_scratch_bytes_for(n, d, P, 0, sides) == want
+    # the scratch of the README's shape is the fp32 kernels' and the transposed pairs
+    assert _lib.grad_blocking(32768, 1152, P) == (8192, 4)
+    assert lib.mec_workspace_floats_for((1 << 20) + 1, 64, P) < 0
+    assert lib.mec_grad_scratch_bytes((1 << 20) + 1, 64, P) < 0
+    rc = lib.mec_prepass(16, 64, 16, 64, (1 << 20) + 1, 64, P, 1, 16, None)
+    assert rc == _lib.MEC_ERR_UNSUPPORTED and "2^20" in _lib.last_error()
+    rc = lib.mec_prepass(16, 64, 16, 64, 10, 64, P, 1, 8, None)
+    assert rc == _lib.MEC_ERR_INVALID and "16-byte" in _lib.last_error()
+    # which problems run as pairs
+    for v in ("MEC_F32_PAIRS", "MEC_F32_SMALL_TILES"):
+        monkeypatch.delenv(v, raising=False)
+    x3 = _lib.DTYPE_F32_BF16X3
+    for dt in (1, 2, 4, P, 7):
+        assert lib.mec_product_dtype(32768, 1152, dt) == dt
+    assert lib.mec_product_dtype(32768, 1152, 0) == P and lib.mec_product_dtype(1024, 512, 0) == 0
+    assert lib.mec_product_dtype(10, 3, x3) == P
+    for dt in (0, x3):
+        assert lib.mec_product_dtype((1 << 20) + 1, 1152, dt) == dt
+        assert lib.mec_product_dtype(0, 1152, dt) == dt
+    monkeypatch.setenv("MEC_F32_SMALL_TILES", "1")
+    assert lib.mec_product_dtype(32768, 1152, 0) == 0
+    monkeypatch.setenv("MEC_F32_PAIRS", "1")
+    assert lib.mec_product_dtype(1, 1, 0) == P
+    monkeypatch.setenv("MEC_F32_PAIRS", "0")
+    assert lib.mec_product_dtype(10, 3, x3) == x3
