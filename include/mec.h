@@ -233,6 +233,15 @@ int64_t mec_grad_scratch_bytes_for(int64_t n, int64_t d, int dtype, int mode, in
  * enough for every mode and side. */
 int64_t mec_grad_scratch_bytes(int64_t n, int64_t d, int dtype);
 
+/* Bytes of scratch with which mec_backward runs fastest: as
+ * mec_grad_scratch_bytes_for, plus, where the 16-bit contractions have too few
+ * tiles for the device, room for further parts of the accumulators (at most
+ * 256 MiB): the contractions are then split over k, each part with its own
+ * n x d sums, which the post-pass adds in order (deterministic).  With less
+ * scratch mec_backward runs unsplit.  On the current device (256 compute units
+ * are assumed where there is none).  No counterpart in the reference. */
+int64_t mec_backward_scratch_bytes(int64_t n, int64_t d, int dtype, int mode, int sides);
+
 /* The backward's plan for (n, d, dtype, mode, sides) on a device of
  * `compute_units` CUs (<= 0: the current device's), for 16-byte aligned rows.
  * No counterpart in the reference; for callers sizing buffers and for tests

@@ -189,7 +189,7 @@ def backward(ctx, grad_output: torch.Tensor, need_x: bool, need_y: bool):
     # torch.use_deterministic_algorithms(True) (gigabytes at large N) would
     # be wasted work.
     sides = (_lib.SIDE_X if need_x else 0) | (_lib.SIDE_Y if need_y else 0)
-    nbytes = lib.mec_grad_scratch_bytes_for(n, d, dt, mode, sides)  # 0 with the kept exponentials
+    nbytes = lib.mec_backward_scratch_bytes(n, d, dt, mode, sides)  # 0 with the kept exponentials
 
     def ptr(t):
         return None if t is None else t.data_ptr()

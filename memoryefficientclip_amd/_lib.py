@@ -48,6 +48,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "mec_keep_exp_supported": (_int, [_vp, _i64, _vp, _i64, _i64, _i64, _int]),
     "mec_grad_scratch_bytes": (_i64, [_i64, _i64, _int]),
     "mec_grad_scratch_bytes_for": (_i64, [_i64, _i64, _int, _int, _int]),
+    "mec_backward_scratch_bytes": (_i64, [_i64, _i64, _int, _int, _int]),
     "mec_backward_plan": (_int, [_i64, _i64, _int, _int, _int, _int, _vp]),
     "mec_grad_blocking": (_int, [_i64, _i64, _int, _vp, _vp]),
     "mec_prepass": (_int, [_vp, _i64, _vp, _i64, _i64, _i64, _int, _int, _vp, _vp]),

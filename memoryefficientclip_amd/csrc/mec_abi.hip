@@ -382,7 +382,11 @@ void grad_blocks_budget(int64_t n, int64_t d, int dtype, int64_t gbudget, int* b
   if (dtype != MEC_DTYPE_F32 && !is_pairs(dtype) && n >= 8192 && n < 16 * 8 * d) mult = 16;
   // at least 1024 rows (below that the pipeline's launches and accumulator
   // updates dominate), where the budget allows
-  const int64_t target_rows = mult * d > kTargetMinRows ? mult * d : kTargetMinRows;
+  // (pairs: twice the fp32 kernels' rows throughout.  A sum over more rows
+  // rounds more, and at twice the rows their sums are still no further from 64
+  // bits than the fp32 kernels', at four times 1.5 times as far: 4097 x 192)
+  const int64_t min_rows = is_pairs(dtype) ? 2 * kTargetMinRows : kTargetMinRows;
+  const int64_t target_rows = mult * d > min_rows ? mult * d : min_rows;
   int64_t target = (target_rows + q - 1) / q;
   if (const char* env = std::getenv("MEC_GRAD_BLOCK_TILES")) {
     long v = std::strtol(env, nullptr, 10);
@@ -585,6 +589,88 @@ BlockGrid block_grid(int64_t d, int dtype, int sides, int bs, int nb, int64_t ld
   return bg;
 }
 
+// Contractions split over k (16-bit kernels): ks parts of kl k-rows each, in
+// their own n x d sums, which the post-pass adds in order.  A contraction tile
+// runs over all bs rows of a block, so where a launch has fewer tiles than the
+// device has CUs (or a nearly empty last round), its time is one tile's k-loop
+// whatever n is.  The cost of a choice, in us: rounds of tiles, each its k rows
+// at 20 ns per 256 x 256 tile (measured: 1.3 us per 64-row chunk; pairs three
+// products; a 384-wide tile 1.4 times that) and 4 us around them, and the parts,
+// written by every launch and read once, at 2.5 TB/s.  Parts are taken where they
+// save at least 7%.  Measured, whole CLIP step with 1, 2, 3, 4 and 8 parts: bf16
+// 4096 x 768 (96 tiles) 177, 157, 166, 178 and 230 us; 8192 x 256 (four blocks)
+// 307, 264, 272, 300 and 378 us; 8192 x 1024 544, 571, 625, 696 and 544 (8 do not
+// fit) us; pairs 2500 x 64 177, 122, 106, 95 and 84 us, 4096 x 512 340, 259, 244,
+// 243 and 266 us, 4999 x 640 529, 460, 503, 474 and 523 us.
+struct ConSplit {
+  int ks, kl;
+  bool w384;
+};
+constexpr int kMaxParts = 8;
+constexpr int64_t kPartsBytes = int64_t(256) << 20;  // at most this much for the parts
+bool contract_forced() { return std::getenv("MEC_NARROW_CONTRACT") || std::getenv("MEC_WIDE_CONTRACT"); }
+// bg, w384: the unsplit choice (block_grid)
+ConSplit contract_split(int64_t n, int64_t d, int dtype, int sides, const BlockGrid& bg, bool w384, int64_t ldt,
+                        int cus) {
+  ConSplit best{1, bg.bs, w384};
+  if (!separate_contractions(dtype) || is_x3(dtype) || cus <= 0) return best;
+  int force = 0;
+  if (const char* env = std::getenv("MEC_CONTRACT_PARTS")) force = std::atoi(env);  // (tests)
+  if (contract_forced() && force <= 0) return best;
+  const int nsides = ((sides & kSideX) ? 1 : 0) + ((sides & kSideY) ? 1 : 0);
+  const int64_t rows = n < bg.bs ? n : bg.bs;  // k rows of a block
+  const double per_k = is_pairs(dtype) ? 0.060 : 0.020;
+  const int64_t tiles1 = (int64_t)nsides * bg.nb * (bg.cnw ? (bg.ctm / 2) * (2 * bg.ctd + 1) : bg.ctm * bg.ctd);
+  const int64_t t384 = (int64_t)nsides * bg.nb * bg.ctm * ((d + 383) / 384);
+  const bool can384 = !is_pairs(dtype) && wide_contract_fits(ldt, bg.bs);
+  auto cost = [&](int ks, bool w) {
+    const int64_t tiles = (w && !w384 ? t384 : tiles1) * ks;
+    const double k = (double)((rows + ks - 1) / ks) * per_k * (w ? 1.4 : 1.0);
+    return (double)bg.nb * ((double)((tiles + cus - 1) / cus) * (k + 4.0) +
+                            (double)(ks - 1) * n * d * nsides * 4.0 * (1.0 + 1.0 / bg.nb) / 2.5e6);
+  };
+  const int most = force > 0 ? (force < kMaxParts ? force : kMaxParts) : kMaxParts;
+  double c = force > 0 ? 1e300 : 0.93 * cost(1, w384);
+  for (int ks = force > 0 ? most : 2; ks <= most; ++ks) {
+    const int64_t kl = ((rows + ks - 1) / ks + 63) / 64 * 64;
+    if (kl * (ks - 1) >= rows || (kl < 256 && force <= 0)) continue;
+    if ((int64_t)(ks - 1) * n * d * 4 * nsides > kPartsBytes) continue;
+    // (where the unsplit choice is 384 wide, so are the parts)
+    for (int w = w384 ? 1 : 0; w <= (w384 || can384 ? 1 : 0); ++w) {
+      const double v = cost(ks, w != 0);
+      if (v < c) {
+        c = v;
+        best = ConSplit{ks, (int)kl, w != 0};
+      }
+    }
+  }
+  return best;
+}
+int64_t parts_bytes(int64_t n, int64_t d, int sides, int ks) {
+  const int nsides = ((sides & kSideX) ? 1 : 0) + ((sides & kSideY) ? 1 : 0);
+  return (int64_t)(ks - 1) * n * d * 4 * nsides;
+}
+int64_t align256(int64_t b) { return (b + 255) & ~int64_t(255); }
+// the parts of mec_backward on a scratch laid out as L (they follow it)
+ConSplit backward_split(int64_t n, int64_t d, int dtype, int sides, const ScratchLayout& L, int cus) {
+  if (!separate_contractions(dtype) || is_x3(dtype)) return ConSplit{1, L.bs, false};
+  const int gdt = is_split(dtype) ? MEC_DTYPE_BF16 : dtype;
+  bool w384 = false;
+  const BlockGrid bg = block_grid(d, gdt, sides, L.bs, L.nb, L.ldt, cus, fwd_tile_dims(gdt, true, false),
+                                  con_tile_dims(gdt, false), &w384);
+  return contract_split(n, d, dtype, sides, bg, w384, L.ldt, cus);
+}
+// compute units of the device for the size queries (which also run without one)
+int plan_units() {
+  int cus = 0;
+  if (compute_units(&cus) != MEC_OK) {
+    (void)hipGetLastError();
+    g_err.clear();
+    cus = 256;
+  }
+  return cus;
+}
+
 // T = element type of dtype: float, bf16 bits (uint16_t) or fp16 (_Float16);
 // callers map the split modes to float first (data_dtype)
 #define DISPATCH_DTYPE(dtype, T, ...)       \
@@ -616,13 +702,14 @@ BlockGrid block_grid(int64_t d, int dtype, int sides, int bs, int nb, int64_t ld
 // "high" precision (bf16x3): always (three products as well, more exact, fewer
 // operand bytes; step at 2048 x 512 248 -> 201 us, 4999 x 640 655 -> 567 us,
 // 8192 x 768 1194 -> 1127 us, 32768 x 1152 the same).
-// fp32: where the products dominate.  Measured, CLIP step, fp32 MFMA -> pairs:
-// 2500 x 512 285 -> 228 us, 4096 x 512 554 -> 361 us, 4999 x 640 1171 -> 567
-// us, 8192 x 768 3028 -> 1127 us, 32768 x 1152 71.9 -> 24.4 ms, 32768 x 128 9.7
-// -> 5.4 ms; but 2500 x 64 134 -> 201 us, 4096 x 64 153 -> 326 us, 8192 x 128
-// 698 -> 723 us (at a small d the contractions' 256-feature tiles are mostly
-// empty and their few workgroups run over all n rows), and up to n = 2048 the
-// kept similarity matrix takes three launches (2048 x 512 131 -> 201 us).
+// fp32: above the kept similarity matrix's range.  Measured, CLIP step, fp32
+// MFMA -> pairs: 2500 x 64 129 -> 131 us, 4096 x 64 153 -> 126 us, 8192 x 128
+// 695 -> 384 us, 4096 x 512 554 -> 243 us, 4999 x 640 1171 -> 460 us, 8192 x 768
+// 3028 -> 1090 us, 32768 x 1152 71.9 -> 23.8 ms; the loss alone, 16384 x 64 390
+// -> 164 us, 2500 x 512 80 -> 52 us.  Up to n = 2048 the kept matrix takes three
+// launches (1024 x 512 107 -> 150 us, 1500 x 768 140 -> 156 us, 2048 x 512 131 ->
+// 137 us; only its corner past 1800 x 1152 is slower, 258 -> 234 us), and the
+// loss alone is no faster (2048 x 512 50 us either way).
 bool pairs_preferred(int64_t n, int64_t d, int dtype) {
   if (dtype != MEC_DTYPE_F32 && dtype != MEC_DTYPE_F32_BF16X3) return false;
   if (n < 1 || d < 1 || n > kMaxNPairs || d > kMaxD) return false;
@@ -632,7 +719,7 @@ bool pairs_preferred(int64_t n, int64_t d, int dtype) {
   }
   if (dtype == MEC_DTYPE_F32_BF16X3) return true;
   if (small_tiles_env() >= 0) return false;  // (the fp32 tiles are asked for)
-  return n > 2048 && n * n * d >= 3000000000LL && (d >= 192 || n > 12288);
+  return n > MEC_KEEP_EXP_MAX_N;
 }
 
 }  // namespace
@@ -682,6 +769,14 @@ int64_t mec_grad_scratch_bytes_for(int64_t n, int64_t d, int dtype, int mode, in
   if (sides < 1 || sides > (kSideX | kSideY)) return -1;
   if (keep_flag(mode)) return keep_shape_ok(n, dtype) ? 0 : -1;  // contracts the kept matrix
   return scratch_layout(n, d, dtype, sides).total;
+}
+
+int64_t mec_backward_scratch_bytes(int64_t n, int64_t d, int dtype, int mode, int sides) {
+  const int64_t base = mec_grad_scratch_bytes_for(n, d, dtype, mode, sides);
+  if (base <= 0 || keep_flag(mode)) return base;
+  if (is_lit(mode)) sides &= kSideX;
+  const ConSplit cs = backward_split(n, d, dtype, sides, scratch_layout(n, d, dtype, sides), plan_units());
+  return cs.ks > 1 ? align256(base) + parts_bytes(n, d, sides, cs.ks) : base;
 }
 
 int mec_backward_plan(int64_t n, int64_t d, int dtype, int mode, int sides, int cus, mec_backward_plan_t* plan) {
@@ -972,6 +1067,11 @@ int mec_grad_blocking(int64_t n, int64_t d, int dtype, int64_t* block_rows, int6
   return MEC_OK;
 }
 
+static int postpass_run(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
+                        int mode, int normalize, float grad_scale, const float* workspace, const float* grad_output,
+                        const float* acc_x, const float* acc_y, void* dx, void* dy, int nparts, const float* parts,
+                        void* stream);
+
 // Arguments of one backward pipeline step, checked by the entry points.
 struct StepArgs {
   const void* x;
@@ -1014,7 +1114,9 @@ static int check_step_args(StepArgs& a) {
 
 // Pipeline step `step` of a checked problem on the scratch at `scratch`
 // (16-byte aligned, laid out as L for the problem's sides: L.total bytes).
-static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L, void* scratch, void* stream) {
+// cs: the contractions' parts (null: not split), parts: where they go.
+static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L, void* scratch, void* stream,
+                         const ConSplit* cs = nullptr, float* parts = nullptr) {
   const void *x = a.x, *y = a.y;
   const int64_t ldx = a.ldx, ldy = a.ldy, n = a.n, d = a.d;
   const int dtype = a.dtype, mode = a.mode, normalize = a.normalize;
@@ -1037,12 +1139,22 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
   if (split && !vec) return fail(MEC_ERR_UNSUPPORTED, "split operands beyond the direct-load range");
   const bool small = dtype == MEC_DTYPE_F32 && vec && f32_small_bwd_tiles(n, d, bs, cus);
   bool w384 = false;  // 16-bit contractions in 256 x 384 tiles
-  const BlockGrid bg = block_grid(d, dtype, a.sides(), bs, nb, L.ldt, cus, fwd_tile_dims(dtype, vec, small),
-                                  con_tile_dims(dtype, small), &w384);
+  BlockGrid bg = block_grid(d, dtype, a.sides(), bs, nb, L.ldt, cus, fwd_tile_dims(dtype, vec, small),
+                            con_tile_dims(dtype, small), &w384);
+  if (cs && cs->ks > 1 && cs->w384 && !w384) {
+    w384 = true;
+    bg.ctd = (D + 383) / 384;
+    bg.cnw = 0;
+  }
   const bool sep = separate_contractions(dtype);
   // contraction tiles per block and side
-  const int ct_blk = bg.cnw ? (bg.ctm / 2) * (2 * bg.ctd + 1) : bg.ctm * bg.ctd;
+  const int ks = cs ? cs->ks : 1;
+  const int ct_blk = (bg.cnw ? (bg.ctm / 2) * (2 * bg.ctd + 1) : bg.ctm * bg.ctd) * ks;
   StepPlan sp{};
+  sp.ks = ks;
+  sp.kl = cs ? cs->kl : bs;
+  sp.px = parts;
+  sp.py = parts ? parts + (acc_x ? (int64_t)(ks - 1) * n * d : 0) : nullptr;
   sp.diag_g = step < nb ? (int)step : -1;
   sp.diag_c = step > 0 ? (int)step - 1 : -1;
   sp.accumulate = step > 1;
@@ -1322,6 +1434,18 @@ int mec_backward_noalloc(const void* x, int64_t ldx, const void* y, int64_t ldy,
 int mec_postpass(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
                  int mode, int normalize, float grad_scale, const float* workspace, const float* grad_output,
                  const float* acc_x, const float* acc_y, void* dx, void* dy, void* stream) {
+  return postpass_run(x, ldx, y, ldy, n, d, dtype, mode, normalize, grad_scale, workspace, grad_output, acc_x, acc_y,
+                      dx, dy, 1, nullptr, stream);
+}
+
+}  // extern "C"
+
+// mec_postpass on accumulators in `nparts` parts, the parts after the first
+// at `parts` (n d floats each, the x side's and then the y side's)
+static int postpass_run(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
+                        int mode, int normalize, float grad_scale, const float* workspace, const float* grad_output,
+                        const float* acc_x, const float* acc_y, void* dx, void* dy, int nparts, const float* parts,
+                        void* stream) {
   g_err.clear();
   int rc = check_common(x, ldx, y, ldy, n, d, dtype);
   if (!rc) rc = check_mode(mode);
@@ -1353,17 +1477,20 @@ int mec_postpass(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t
                     aligned16(x) && aligned16(y) && aligned16(acc_x) && aligned16(acc_y) && aligned16(dx) &&
                     aligned16(dy);
   DISPATCH_DTYPE(data_dtype(dtype), T, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(accr, ACCR, {
-    const PostSide<T> px{(const T*)x, ldx, (const T*)y, ldy, rx, ry, acc_x, (T*)dx};
-    const PostSide<T> py{(const T*)y, ldy, (const T*)x, ldx, ry, rx, acc_y, (T*)dy};
+    const PostSide<T> px{(const T*)x, ldx, (const T*)y, ldy, rx, ry, acc_x, (T*)dx, parts};
+    const PostSide<T> py{(const T*)y, ldy, (const T*)x, ldx, ry, rx, acc_y, (T*)dy,
+                         parts ? parts + (acc_x ? (nparts - 1) * n * d : 0) : nullptr};
     if constexpr (std::is_same<T, float>::value) {
       DISPATCH_BOOL(pvec, VEC,
-          k_postpass<T, NORM, ACCR, VEC><<<grid, 256, 0, s>>>(acc_x ? px : py, py, N, D, kap, a, grad_output));
+          k_postpass<T, NORM, ACCR, VEC><<<grid, 256, 0, s>>>(acc_x ? px : py, py, N, D, kap, a, grad_output, nparts));
     } else if constexpr (!ACCR) {
-      k_postpass<T, NORM, ACCR><<<grid, 256, 0, s>>>(acc_x ? px : py, py, N, D, kap, a, grad_output);
+      k_postpass<T, NORM, ACCR><<<grid, 256, 0, s>>>(acc_x ? px : py, py, N, D, kap, a, grad_output, nparts);
     }
   })));
   return check_launch("postpass");
 }
+
+extern "C" {
 
 int mec_backward(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
                  int mode, int normalize, float temperature, float grad_scale, const float* workspace,
@@ -1376,9 +1503,35 @@ int mec_backward(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t
     const int rc = check_step_args(a);
     return rc ? rc : keep_backward(a, grad_scale, grad_output, dx, dy, stream);
   }
-  int rc = mec_grad(x, ldx, y, ldy, n, d, dtype, mode, normalize, temperature, workspace, scratch,
-                    scratch_bytes, acc_x, acc_y, stream);
+  StepArgs a{x, ldx, y, ldy, n, d, dtype, mode, normalize, temperature, workspace, acc_x, acc_y};
+  int rc = check_step_args(a);
+  ScratchLayout L;
+  if (!rc) rc = check_scratch(a, scratch, scratch_bytes, &L);
+  if (!rc) rc = check_not_capturing(stream);
   if (rc) return rc;
+  // split contractions where the scratch has room for their parts
+  ConSplit cs{1, L.bs, false};
+  const int64_t off = align256(L.total);
+  if (scratch_bytes > off) {
+    int cus = 0;
+    rc = compute_units(&cus);
+    if (rc) return rc;
+    cs = backward_split(n, d, dtype, a.sides(), L, cus);
+    if (cs.ks > 1 && scratch_bytes < off + parts_bytes(n, d, a.sides(), cs.ks)) cs.ks = 1;
+  }
+  if (cs.ks > 1) {
+    float* parts = (float*)((char*)scratch + off);
+    for (int t = 0; t <= L.nb; ++t) {
+      rc = grad_step_run(a, t, L, scratch, stream, &cs, parts);
+      if (rc) return rc;
+    }
+    return postpass_run(x, ldx, y, ldy, n, d, dtype, mode, normalize, grad_scale, workspace, grad_output, a.acc_x,
+                        a.acc_y, dx, is_lit(mode) ? nullptr : dy, cs.ks, parts, stream);
+  }
+  for (int t = 0; t <= L.nb; ++t) {
+    rc = grad_step_run(a, t, L, scratch, stream);
+    if (rc) return rc;
+  }
   return mec_postpass(x, ldx, y, ldy, n, d, dtype, mode, normalize, grad_scale, workspace, grad_output, acc_x,
                       acc_y, dx, dy, stream);
 }

@@ -704,6 +704,11 @@ struct StepPlan {
   int g_n, g_pad;    // G' tiles (nb * gtm * gtn or 0), padded to a multiple of 8
   int cx_n, cx_pad;  // x-side contraction tiles (nb * ctm * ctd; cnw: nb * ctm / 2 * (2 ctd + 1); or 0), padded
   int cy_n, cy_pad;  // y-side contraction tiles, padded
+  // contractions split over k (16-bit tiles; ks = 1: not): part p of ks takes
+  // k rows [p kl, (p + 1) kl) of the block, part 0 into the accumulators and
+  // part p into px / py + (p - 1) N D
+  int ks, kl;
+  float *px, *py;
 };
 
 // fp32 gradient-matrix tile: H_ij = rx_i G'_ij ry_j (G'_ij without the norm
@@ -908,7 +913,8 @@ __device__ __forceinline__ void grad_contract_tile(int N, int D, const T* __rest
                                                    const T* __restrict__ Glo, const T* __restrict__ OT,
                                                    const T* __restrict__ OTlo, int64_t ldt, const BlockGrid& bg,
                                                    int P, int Q, int tm, int td, bool accumulate,
-                                                   float* __restrict__ out, char* lds, float osc) {
+                                                   float* __restrict__ out, char* lds, float osc, int kbeg = 0,
+                                                   int klen = 1 << 30) {
   const int r0 = P * bg.bs + tm * TC::BM;
   if (r0 >= N) return;
   const int d0 = td * TC::BN;
@@ -918,17 +924,31 @@ __device__ __forceinline__ void grad_contract_tile(int N, int D, const T* __rest
   // are stored zeros; split pairs store every 32 k as 64
   constexpr bool SPL = IsSplit<T>::value;
   constexpr int E = SPL ? 2 : 1;
-  const int kq = SPL ? 2 * ((qn + 31) & ~31) : (qn + 7) & ~7;
+  // (k rows [kbeg, kbeg + klen) of them: multiples of a chunk)
+  const int qk = min(qn - kbeg, klen);
+  const int kq = SPL ? 2 * ((qk + 31) & ~31) : (qk + 7) & ~7;
   // A: rows tm*BM.. of the block (K-major), or columns tm*BM.. of a transposed
   // block (blocked layout: i-block tm*BM/16 of the first j-block row)
-  const int64_t a_off = E * (TC::TA ? (int64_t)(tm * TC::BM) * (TC::GB ? 32 : 1) : (int64_t)(tm * TC::BM) * bg.bs);
+  int64_t a_off = E * (TC::TA ? (int64_t)(tm * TC::BM) * (TC::GB ? 32 : 1) : (int64_t)(tm * TC::BM) * bg.bs);
+  if constexpr (TC::GB) a_off += (int64_t)E * kbeg * (TC::TA ? bg.bs : 32);
   const auto A = tile_op<TC>(Gblk + a_off, SPL && !TC::TA ? 2 * (int64_t)bg.bs : bg.bs, TC::BM, kq);
   // the feature operand: transposed copy (rows d, k = q0 + j) or, fp32, the
   // raw rows q0 + k (only the block's qn valid rows)
-  const int64_t b_off = TC::TB ? (int64_t)q0 * ldt + d0 : E * ((int64_t)d0 * ldt + q0);
+  const int64_t b_off = TC::TB ? (int64_t)q0 * ldt + d0 : E * ((int64_t)d0 * ldt + q0 + kbeg);
   const auto B = tile_op<TC>(OT + b_off, E * ldt, min(D - d0, TC::BN), TC::TB ? qn : kq);
   f32x16 acc[TC::FM][TC::FN];
-  TC::template run<true, true>(A, B, kq, lds, acc);
+  if (GtOnly<T>::value && qk <= 0) {
+    // a part past a short last block
+    if (accumulate) return;
+#pragma unroll
+    for (int bm = 0; bm < TC::FM; ++bm)
+#pragma unroll
+      for (int bn = 0; bn < TC::FN; ++bn)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[bm][bn][r] = 0.f;
+  } else {
+    TC::template run<true, true>(A, B, kq, lds, acc);
+  }
   if constexpr (X3) {
     __syncthreads();  // every wave is past its last read of the ring
     TC::template run<true, true, false>(A, tile_op<TC>(OTlo + b_off, ldt, min(D - d0, TC::BN), kq), kq, lds, acc);
@@ -975,6 +995,7 @@ __device__ __forceinline__ void grad_contract_dispatch(int sub, int N, int D, co
   if (!is_x) sub -= sp.cx_pad;
   const int pid = xcd_remap(sub, is_x ? sp.cx_pad : sp.cy_pad);
   if (pid >= (is_x ? sp.cx_n : sp.cy_n)) return;
+  int part = 0;  // of ks parts of k
   int tmg, td, rows = bg.ctm;  // rows: row tiles per block of this tile's height
   bool narrow = false;
   if constexpr (GtOnly<T>::value) {
@@ -999,37 +1020,49 @@ __device__ __forceinline__ void grad_contract_dispatch(int sub, int N, int D, co
       tmg = pid / bg.ctd;
       td = pid - tmg * bg.ctd;
     }
+    if (sp.ks > 1) {
+      // (the tiles of one panel and part stay side by side)
+      const int per = bg.cnw ? 2 * bg.ctd + 1 : bg.ctd;
+      const int grp = pid / per, g0 = grp / sp.ks;
+      part = grp - g0 * sp.ks;
+      tmg += (g0 - grp) * (bg.cnw && !narrow ? 2 : 1);
+    }
   } else {
     group_tile(pid, bg.nb * bg.ctm, bg.ctd, 8, tmg, td);
   }
   const int P = tmg / rows, tm = tmg - P * rows;  // P: block owning the output rows
   const int buf = sp.diag_c & 1;
+  const int kbeg = part * sp.kl, klen = sp.ks > 1 ? sp.kl : 1 << 30;
+  if (part > 0) {
+    acc_x = sp.px + (int64_t)(part - 1) * N * D;
+    acc_y = sp.py + (int64_t)(part - 1) * N * D;
+  }
   if (is_x) {
     const int Q = (P + sp.diag_c) % bg.nb;
     const T* gx = (const T*)(GtOnly<T>::value ? gb.gt[buf] : gb.g[buf]) + P * blk;
     const T* gxl = X3 ? (const T*)gb.gt_lo[buf] + P * blk : nullptr;
     if (narrow)
       grad_contract_tile<TNX, T, X3>(N, D, gx, gxl, (const T*)gb.yt, (const T*)gb.yt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_x, lds, osc);
+                                     sp.accumulate != 0, acc_x, lds, osc, kbeg, klen);
     else if constexpr (TCX::TB)
       grad_contract_tile<TCX, T, X3>(N, D, gx, gxl, Y, nullptr, ldy, bg, P, Q, tm, td, sp.accumulate != 0, acc_x,
-                                     lds, osc);
+                                     lds, osc, kbeg, klen);
     else
       grad_contract_tile<TCX, T, X3>(N, D, gx, gxl, (const T*)gb.yt, (const T*)gb.yt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_x, lds, osc);
+                                     sp.accumulate != 0, acc_x, lds, osc, kbeg, klen);
   } else {
     const int Q = (P - sp.diag_c + bg.nb) % bg.nb;
     const T* gy = (const T*)(GtOnly<T>::value ? gb.gt[buf] : gb.g[buf]) + Q * blk;
     const T* gyl = X3 ? (const T*)gb.gt_lo[buf] + Q * blk : nullptr;
     if (narrow)
       grad_contract_tile<TNY, T, X3>(N, D, gy, gyl, (const T*)gb.xt, (const T*)gb.xt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_y, lds, osc);
+                                     sp.accumulate != 0, acc_y, lds, osc, kbeg, klen);
     else if constexpr (TCY::TB)
       grad_contract_tile<TCY, T, X3>(N, D, gy, gyl, X, nullptr, ldx, bg, P, Q, tm, td, sp.accumulate != 0, acc_y,
-                                     lds, osc);
+                                     lds, osc, kbeg, klen);
     else
       grad_contract_tile<TCY, T, X3>(N, D, gy, gyl, (const T*)gb.xt, (const T*)gb.xt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_y, lds, osc);
+                                     sp.accumulate != 0, acc_y, lds, osc, kbeg, klen);
   }
 }
 

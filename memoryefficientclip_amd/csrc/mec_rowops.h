@@ -170,6 +170,7 @@ struct PostSide {
   const float* r_oth;
   const float* acc;
   T* out;
+  const float* part;  // nparts - 1 further parts of the accumulators, n x D each (contractions split over k)
 };
 // ACCR (fp32 data on the fp32 kernels): the accumulator row carries the
 // row's own inverse norm, acc = r_i (sum_j G'_ij y^_j), since the
@@ -182,7 +183,7 @@ struct PostSide {
 template <typename T, bool NORM, bool ACCR = false, bool VEC = false>
 __global__ __launch_bounds__(256) void k_postpass(PostSide<T> s0, PostSide<T> s1, int N, int D,
                                                   const float* __restrict__ kappa, float a,
-                                                  const float* __restrict__ grad_output) {
+                                                  const float* __restrict__ grad_output, int nparts) {
   static_assert(!VEC || std::is_same<T, float>::value, "16-byte vectors of fp32");
   const PostSide<T>& sd = blockIdx.y ? s1 : s0;
   const T* __restrict__ own = sd.own;
@@ -199,6 +200,19 @@ __global__ __launch_bounds__(256) void k_postpass(PostSide<T> s0, PostSide<T> s1
   const T* xo = own + (int64_t)row * ld_own;
   const T* yo = oth + (int64_t)row * ld_oth;
   const float* ac = acc + (int64_t)row * D;
+  const float* pt = sd.part + (int64_t)row * D;
+  const int64_t ps = (int64_t)N * D;
+  // accumulated sums of feature d (or d .. d + 3): the parts in order
+  auto accv = [&](int d) {
+    float v = ac[d];
+    for (int p = 0; p + 1 < nparts; ++p) v += pt[p * ps + d];
+    return v;
+  };
+  auto accv4 = [&](int d) {
+    f32x4 v = *(const f32x4*)(ac + d);
+    for (int p = 0; p + 1 < nparts; ++p) v += *(const f32x4*)(pt + p * ps + d);
+    return v;
+  };
   T* o = out + (int64_t)row * D;
   const float ro = r_own[row];
   const float kq = kappa[row] * r_oth[row] * (ACCR ? ro : 1.f);
@@ -215,7 +229,7 @@ __global__ __launch_bounds__(256) void k_postpass(PostSide<T> s0, PostSide<T> s1
         g[k] = f32x4{0.f, 0.f, 0.f, 0.f};
         xr[k] = g[k];
         if (d < D) {
-          const f32x4 yv = *(const f32x4*)(yo + d), av = *(const f32x4*)(ac + d), xv = *(const f32x4*)(xo + d);
+          const f32x4 yv = *(const f32x4*)(yo + d), av = accv4(d), xv = *(const f32x4*)(xo + d);
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             g[k][u] = a * fmaf(kq, yv[u], av[u]);
@@ -248,7 +262,7 @@ __global__ __launch_bounds__(256) void k_postpass(PostSide<T> s0, PostSide<T> s1
         g[k] = 0.f;
         xr[k] = 0.f;
         if (d < D) {
-          g[k] = a * fmaf(kq, Elem<T>::load(yo, d), ac[d]);
+          g[k] = a * fmaf(kq, Elem<T>::load(yo, d), accv(d));
           xr[k] = Elem<T>::load(xo, d) * ro;
           dot = fmaf(xr[k], g[k], dot);
         }
@@ -265,19 +279,19 @@ __global__ __launch_bounds__(256) void k_postpass(PostSide<T> s0, PostSide<T> s1
       return;
     }
     for (int d = lane; d < D; d += 64) {
-      float g = a * fmaf(kq, Elem<T>::load(yo, d), ac[d]);
+      float g = a * fmaf(kq, Elem<T>::load(yo, d), accv(d));
       dot = fmaf(Elem<T>::load(xo, d) * ro, g, dot);
     }
     dot = wave_sum(dot);
     for (int d = lane; d < D; d += 64) {
-      float g = a * fmaf(kq, Elem<T>::load(yo, d), ac[d]);
+      float g = a * fmaf(kq, Elem<T>::load(yo, d), accv(d));
       const float xh = Elem<T>::load(xo, d) * ro;
       float v = ACCR ? (clamped ? g : g - xh * dot) : (clamped ? ro * g : ro * (g - xh * dot));
       Elem<T>::store(o, d, go * v);
     }
   } else {
     for (int d = lane; d < D; d += 64) {
-      float g = a * fmaf(kq, Elem<T>::load(yo, d), ac[d]);
+      float g = a * fmaf(kq, Elem<T>::load(yo, d), accv(d));
       Elem<T>::store(o, d, go * g);
     }
   }

@@ -586,7 +586,8 @@ def test_pairs_sizes_and_rule(monkeypatch):
     x3 = _lib.DTYPE_F32_BF16X3
     for dt in (1, 2, 4, P, 7):
         assert lib.mec_product_dtype(32768, 1152, dt) == dt
-    assert lib.mec_product_dtype(32768, 1152, 0) == P and lib.mec_product_dtype(1024, 512, 0) == 0
+    assert lib.mec_product_dtype(32768, 1152, 0) == P and lib.mec_product_dtype(2048, 512, 0) == 0
+    assert lib.mec_product_dtype(2049, 3, 0) == P
     assert lib.mec_product_dtype(10, 3, x3) == P
     for dt in (0, x3):
         assert lib.mec_product_dtype((1 << 20) + 1, 1152, dt) == dt

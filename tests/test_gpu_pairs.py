@@ -172,7 +172,9 @@ def test_off_diagonal_sums_are_as_exact_as_in_fp32(n, d, t):
 
 
 def test_noalloc_and_one_side(pairs):
-    """mec_backward_noalloc and a frozen tower, bitwise as mec_backward with both sides."""
+    """mec_backward_noalloc and a frozen tower, bitwise as mec_backward with both
+    sides (unsplit: each chooses its own split of the contractions)."""
+    pairs.setenv("MEC_CONTRACT_PARTS", "1")
     n, d, t = 1100, 72, 0.07
     a, b = randn_pair(n, d, seed=5)
     ga, gb = a.to(DEV).requires_grad_(True), b.to(DEV).requires_grad_(True)
@@ -193,7 +195,7 @@ def test_noalloc_and_one_side(pairs):
 
 def test_rule_reaches_the_module():
     os.environ.pop("MEC_F32_PAIRS", None)
-    for n, d, want in [(2048, 512, _lib.DTYPE_F32), (4999, 64, _lib.DTYPE_F32), (4999, 640, _lib.DTYPE_F32_PAIRS)]:
+    for n, d, want in [(2048, 512, _lib.DTYPE_F32), (2049, 64, _lib.DTYPE_F32_PAIRS), (4999, 640, _lib.DTYPE_F32_PAIRS)]:
         x = torch.randn(n, d, device=DEV).requires_grad_(True)
         loss = MemoryEfficientCLIPLoss()(x, torch.randn(n, d, device=DEV))
         assert loss.grad_fn.mec[4] == want, (n, d)
