@@ -826,8 +826,11 @@ int mec_backward_plan(int64_t n, int64_t d, int dtype, int mode, int sides, int 
   return MEC_OK;
 }
 
-int mec_prepass(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
-                int normalize, float* workspace, void* stream) {
+}  // extern "C"
+
+// mec_prepass; counter (or null): the word that k_finalize_all counts in, zeroed
+static int prepass_run(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
+                       int normalize, float* workspace, void* stream, uint32_t* counter) {
   g_err.clear();
   int rc = check_common(x, ldx, y, ldy, n, d, dtype);
   if (rc) return rc;
@@ -843,9 +846,11 @@ int mec_prepass(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t 
     const PairRows pr = pair_rows(workspace, n, d);
     const bool vec = aligned16(x) && aligned16(y) && ldx % 4 == 0 && ldy % 4 == 0;
     if (normalize) {
-      k_pair_prepass<true><<<grid, 256, 0, s>>>((const float*)x, ldx, (const float*)y, ldy, N, D, vec, workspace, pr);
+      k_pair_prepass<true><<<grid, 256, 0, s>>>((const float*)x, ldx, (const float*)y, ldy, N, D, vec, workspace, pr,
+                                                  counter);
     } else {
-      k_pair_prepass<false><<<grid, 256, 0, s>>>((const float*)x, ldx, (const float*)y, ldy, N, D, vec, workspace, pr);
+      k_pair_prepass<false><<<grid, 256, 0, s>>>((const float*)x, ldx, (const float*)y, ldy, N, D, vec, workspace, pr,
+                                                 counter);
       // (every workgroup reads the maxima: a bounded number of them)
       k_pair_rows<<<grid.x < 1024 ? grid.x : 1024, 256, 0, s>>>((const float*)x, ldx, (const float*)y, ldy, N, D, vec,
                                                                workspace, pr, (int)grid.x);
@@ -853,7 +858,7 @@ int mec_prepass(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t 
     return check_launch("prepass");
   }
   DISPATCH_DTYPE(data_dtype(dtype), T, DISPATCH_BOOL(normalize, NORM,
-      k_prepass<T, NORM><<<grid, 256, 0, s>>>((const T*)x, ldx, (const T*)y, ldy, N, D, workspace)));
+      k_prepass<T, NORM><<<grid, 256, 0, s>>>((const T*)x, ldx, (const T*)y, ldy, N, D, workspace, counter)));
   if (is_split(dtype)) {
     // bf16 (split) copies of x and y for the similarity GEMMs (the norms and
     // the diagonal above come from the fp32 inputs)
@@ -880,15 +885,27 @@ int mec_prepass(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t 
   return check_launch("prepass");
 }
 
+extern "C" {
+
+int mec_prepass(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
+                int normalize, float* workspace, void* stream) {
+  return prepass_run(x, ldx, y, ldy, n, d, dtype, normalize, workspace, stream, nullptr);
+}
+
 }  // extern "C"
 
 // The forward sums without atomics: one pass over the tile grid in P x Q
 // blocks, then the partials in order.  (D: K of the operands as stored; scl:
-// split pairs.)
+// split pairs; dp: not null, the partials are left to the finalize and described
+// there.)
+struct DetPartials {
+  const float *rowpart, *colpart;
+  int P, Q;  // 0: no partials
+};
 template <typename T>
 static int sumexp_det_run(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int D, bool lit,
                           bool normalize, bool vec, float c, float* workspace, const float* scl, int tiles_m,
-                          int tiles_n, hipStream_t s) {
+                          int tiles_n, hipStream_t s, DetPartials* dp) {
   const int N = (int)n;
   float* rowpart = workspace + det_partials_offset(n);
   float* colpart = rowpart + (int64_t)DET_Q * n;
@@ -900,8 +917,11 @@ static int sumexp_det_run(const void* x, int64_t ldx, const void* y, int64_t ldy
       k_sumexp_det<T, LIT, NORM, VEC><<<(unsigned)(P * Q), FwdTile<T, VEC>::NT, 0, s>>>(
           (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace + WS_RX * n, workspace + WS_RY * n, rowpart,
           colpart, tiles_m, tiles_n, P, Q, scl);
-      k_det_reduce<LIT><<<sum_grid, 256, 0, s>>>(rowpart, Q, colpart, P, N, workspace + WS_ROW_OFF * n,
-                                                 workspace + WS_COL_OFF * n);
+      if (dp)
+        *dp = DetPartials{rowpart, colpart, P, Q};
+      else
+        k_det_reduce<LIT><<<sum_grid, 256, 0, s>>>(rowpart, Q, colpart, P, N, workspace + WS_ROW_OFF * n,
+                                                   workspace + WS_COL_OFF * n);
     }
   };
   DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(vec, VEC,
@@ -910,11 +930,11 @@ static int sumexp_det_run(const void* x, int64_t ldx, const void* y, int64_t ldy
   return check_launch("sumexp (deterministic)");
 }
 
-extern "C" {
-
-int mec_sumexp(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
-               int mode, int normalize, float temperature, float* workspace, void* stream) {
+// mec_sumexp; dp: as sumexp_det_run (P = Q = 0 where the sums are added by atomics)
+static int sumexp_run(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
+                      int mode, int normalize, float temperature, float* workspace, void* stream, DetPartials* dp) {
   g_err.clear();
+  if (dp) *dp = DetPartials{};
   int rc = check_common(x, ldx, y, ldy, n, d, dtype);
   if (!rc) rc = check_mode(mode);
   if (!rc) rc = check_no_keep(mode, "mec_sumexp");
@@ -938,7 +958,7 @@ int mec_sumexp(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n
     const PairRows pr = pair_rows(workspace, n, d);
     const int tiles = (int)((n + 255) / 256), dk = 2 * pr.dp;
     return sumexp_det_run<F16S>(pr.a, dk, pr.b, dk, n, dk, is_lit(mode), false, true, c, workspace, pr.scl, tiles,
-                                tiles, s);
+                                tiles, s, dp);
   }
   x = g.x, ldx = g.ldx, y = g.y, ldy = g.ldy, d = g.d, dtype = g.dtype;
   const int N = (int)n, D = (int)d;
@@ -964,7 +984,7 @@ int mec_sumexp(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n
   const bool lit = is_lit(mode);
   if (det) {
     DISPATCH_DTYPE(dtype, T, rc = sumexp_det_run<T>(x, ldx, y, ldy, n, D, lit, normalize != 0, vec, c, workspace,
-                                                    nullptr, tiles_m, tiles_n, s));
+                                                    nullptr, tiles_m, tiles_n, s, dp));
     return rc;
   }
   dim3 grid((unsigned)nwg);
@@ -981,6 +1001,13 @@ int mec_sumexp(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n
     }
   }))));
   return check_launch("sumexp");
+}
+
+extern "C" {
+
+int mec_sumexp(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
+               int mode, int normalize, float temperature, float* workspace, void* stream) {
+  return sumexp_run(x, ldx, y, ldy, n, d, dtype, mode, normalize, temperature, workspace, stream, nullptr);
 }
 
 int mec_finalize(int64_t n, int mode, float temperature, float* workspace, float* loss, void* stream) {
@@ -1047,10 +1074,21 @@ int mec_forward(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t 
     }));
     return check_launch("forward (kept exponentials)");
   }
-  rc = mec_prepass(x, ldx, y, ldy, n, d, dtype, normalize, workspace, stream);
-  if (!rc) rc = mec_sumexp(x, ldx, y, ldy, n, d, dtype, mode, normalize, temperature, workspace, stream);
-  if (!rc) rc = mec_finalize(n, mode, temperature, workspace, loss, stream);
-  return rc;
+  if (reinterpret_cast<uintptr_t>(workspace) & 7u) return fail(MEC_ERR_INVALID, "workspace must be 8-byte aligned");
+  // the loss word counts the finalize's workgroups until the last one writes the loss
+  uint32_t* counter = reinterpret_cast<uint32_t*>(loss);
+  DetPartials dp;
+  rc = prepass_run(x, ldx, y, ldy, n, d, dtype, normalize, workspace, stream, counter);
+  if (!rc) rc = sumexp_run(x, ldx, y, ldy, n, d, dtype, mode, normalize, temperature, workspace, stream, &dp);
+  if (rc) return rc;
+  const double inv_t = 1.0 / (double)temperature;
+  const unsigned blocks = (unsigned)((n + FIN_ROWS - 1) / FIN_ROWS);
+  double* partial = (double*)(workspace + (int64_t)WS_NSLOTS * n);
+  DISPATCH_BOOL(is_lit(mode), LIT, DISPATCH_BOOL(dp.Q > 0, DET, {
+    k_finalize_all<LIT, DET><<<blocks, DET ? 4 * FIN_ROWS : FIN_ROWS, 0, (hipStream_t)stream>>>(
+        (int)n, inv_t, workspace, dp.rowpart, dp.Q, dp.colpart, dp.P, partial, counter, loss);
+  }));
+  return check_launch("finalize");
 }
 
 int mec_grad_blocking(int64_t n, int64_t d, int dtype, int64_t* block_rows, int64_t* num_blocks) {

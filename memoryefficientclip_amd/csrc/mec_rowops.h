@@ -27,7 +27,8 @@ template <> struct Elem<_Float16> {
 template <typename T, bool NORM>
 __global__ __launch_bounds__(256) void k_prepass(const T* __restrict__ X, int64_t ldx,
                                                  const T* __restrict__ Y, int64_t ldy, int N, int D,
-                                                 float* __restrict__ ws) {
+                                                 float* __restrict__ ws, uint32_t* __restrict__ counter) {
+  if (counter && blockIdx.x == 0 && threadIdx.x == 0) *counter = 0u;  // (k_finalize_all)
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= N) return;
@@ -143,6 +144,80 @@ __global__ __launch_bounds__(1024) void k_finalize_sum(int N, int nparts, const 
   if (threadIdx.x == 0) {
     double tot = 0.0;
     for (int k = 0; k < (int)(blockDim.x >> 6); ++k) tot += red[k];
+    *loss = (float)(tot / (LIT ? (double)N : 2.0 * (double)N));
+  }
+}
+
+// The finalize of mec_forward in one launch: DET: the partial sums of the
+// deterministic forward first (row i's Q row partials and P column partials,
+// four threads per row, partials k, k + 4, ... each, then the four in order);
+// finalize_row on FIN_ROWS rows; the workgroup's fp64 loss sum to partial[];
+// and the last workgroup to arrive at `counter` (zeroed by the pre-pass) adds
+// the partials in order and writes the loss.  The counter is the loss word
+// itself, which nobody reads before the launch ends.  The handshake is a
+// release / acquire of one thread per workgroup.  Latency-bound: as separate
+// launches (k_det_reduce with one thread per row adding 48 partials one after
+// the other, rows, sum) it took 11 + 5 + 5 us at n = 6001, 16 + 5 + 5 us at 8192.
+template <bool LIT, bool DET>
+__global__ __launch_bounds__(DET ? 4 * FIN_ROWS : FIN_ROWS) void k_finalize_all(
+    int N, double inv_t, float* __restrict__ ws, const float* __restrict__ rowpart, int Q,
+    const float* __restrict__ colpart, int P, double* partial, uint32_t* counter, float* loss) {
+  constexpr int NT = DET ? 4 * FIN_ROWS : FIN_ROWS;
+  constexpr int MQ = DET_Q / 4, MP = DET_P / 4;
+  __shared__ float s_r[DET ? 4 : 1][FIN_ROWS], s_c[DET ? 4 : 1][FIN_ROWS];
+  __shared__ double red[NT / 64];
+  __shared__ bool s_last;
+  const int64_t n = N;
+  const int r = threadIdx.x % FIN_ROWS, q = threadIdx.x / FIN_ROWS;
+  const int i = blockIdx.x * FIN_ROWS + r;
+  if constexpr (DET) {
+    // every load at a valid address, issued back to back
+    const int ic = min(i, N - 1);
+    float rv[MQ], cv[LIT ? 1 : MP];
+#pragma unroll
+    for (int k = 0; k < MQ; ++k) rv[k] = rowpart[min(4 * k + q, Q - 1) * n + ic];
+    if constexpr (!LIT) {
+#pragma unroll
+      for (int k = 0; k < MP; ++k) cv[k] = colpart[min(4 * k + q, P - 1) * n + ic];
+    }
+    float a = 0.f, b = 0.f;
+#pragma unroll
+    for (int k = 0; k < MQ; ++k) a += 4 * k + q < Q ? rv[k] : 0.f;
+    s_r[q][r] = a;
+    if constexpr (!LIT) {
+#pragma unroll
+      for (int k = 0; k < MP; ++k) b += 4 * k + q < P ? cv[k] : 0.f;
+      s_c[q][r] = b;
+    }
+    __syncthreads();
+    if (q == 0 && i < N) {
+      ws[WS_ROW_OFF * n + i] = (s_r[0][r] + s_r[1][r]) + (s_r[2][r] + s_r[3][r]);
+      if (!LIT) ws[WS_COL_OFF * n + i] = (s_c[0][r] + s_c[1][r]) + (s_c[2][r] + s_c[3][r]);
+    }
+  }
+  // (the same thread reads back what it wrote)
+  double acc = q == 0 && i < N ? finalize_row<LIT>(i, n, inv_t, ws) : 0.0;
+  acc = wave_sum_f64(acc);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (lane == 0) red[w] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double tot = 0.0;
+    for (int k = 0; k < FIN_ROWS / 64; ++k) tot += red[k];
+    __hip_atomic_store(&partial[blockIdx.x], tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  double sum = 0.0;
+  for (int k = threadIdx.x; k < (int)gridDim.x; k += NT)
+    sum += __hip_atomic_load(&partial[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  sum = wave_sum_f64(sum);
+  if (lane == 0) red[w] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double tot = 0.0;
+    for (int k = 0; k < NT / 64; ++k) tot += red[k];
     *loss = (float)(tot / (LIT ? (double)N : 2.0 * (double)N));
   }
 }
@@ -513,8 +588,10 @@ constexpr int PAIR_REG = 8;
 template <bool NORM>
 __global__ __launch_bounds__(256) void k_pair_prepass(const float* __restrict__ X, int64_t ldx,
                                                       const float* __restrict__ Y, int64_t ldy, int N, int D, bool vec,
-                                                      float* __restrict__ ws, PairRows pr) {
+                                                      float* __restrict__ ws, PairRows pr,
+                                                      uint32_t* __restrict__ counter) {
   __shared__ float s_mx[2][4];
+  if (counter && blockIdx.x == 0 && threadIdx.x == 0) *counter = 0u;  // (k_finalize_all)
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int row = blockIdx.x * 4 + w;
   const int64_t n = N;
