@@ -242,13 +242,18 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 int64_t dma_max_elems(int dtype) { return ((int64_t(1) << 31) - 1) / (dtype == MEC_DTYPE_F32 ? 4 : 2); }
 int64_t dma_rows(int dtype) { return dtype == MEC_DTYPE_F32 ? 128 : 256; }
 
+// every row of x and y a whole number of 16-byte vectors
+bool rows_vec16(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t d, int dtype) {
+  const int64_t per = dtype == MEC_DTYPE_F32 ? 4 : 8;
+  return aligned16(x) && aligned16(y) && d % per == 0 && ldx % per == 0 && ldy % per == 0;
+}
+
 // 16-byte vector loads are legal when every row start is 16-byte aligned and
 // rows hold a whole number of vectors; this also selects the direct-to-LDS
 // core for the forward and gradient-matrix tiles, whose panels must fit its
 // 32-bit offsets.
 bool vec_ok(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t d, int dtype) {
-  const int64_t per = dtype == MEC_DTYPE_F32 ? 4 : 8;
-  if (!(aligned16(x) && aligned16(y) && d % per == 0 && ldx % per == 0 && ldy % per == 0)) return false;
+  if (!rows_vec16(x, ldx, y, ldy, d, dtype)) return false;
   const int64_t ld = ldx > ldy ? ldx : ldy;
   return (dma_rows(dtype) - 1) * ld + d <= dma_max_elems(dtype);
 }
@@ -858,7 +863,8 @@ static int prepass_run(const void* x, int64_t ldx, const void* y, int64_t ldy, i
     return check_launch("prepass");
   }
   DISPATCH_DTYPE(data_dtype(dtype), T, DISPATCH_BOOL(normalize, NORM,
-      k_prepass<T, NORM><<<grid, 256, 0, s>>>((const T*)x, ldx, (const T*)y, ldy, N, D, workspace, counter)));
+      DISPATCH_BOOL(rows_vec16(x, ldx, y, ldy, d, data_dtype(dtype)), VEC,
+          k_prepass<T, NORM, VEC><<<grid, 256, 0, s>>>((const T*)x, ldx, (const T*)y, ldy, N, D, workspace, counter))));
   if (is_split(dtype)) {
     // bf16 (split) copies of x and y for the similarity GEMMs (the norms and
     // the diagonal above come from the fp32 inputs)
@@ -1262,7 +1268,9 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
           using TS = TransSide<T>;
           const TS ty{(const T*)y, ldy, workspace + WS_RY * n64, (T*)gb.yt, nullptr};
           const TS tx{(const T*)x, ldx, workspace + WS_RX * n64, (T*)gb.xt, nullptr};
-          k_transpose<T, NORM><<<tgrid, 256, 0, s>>>(acc_x ? ty : tx, tx, N, D, L.ldt);
+          const dim3 g128((unsigned)(L.ldt / 128), tgrid.y, nsides);
+          DISPATCH_BOOL(rows_vec16(x, ldx, y, ldy, d, dtype), VEC,
+              k_transpose<T, NORM, VEC><<<g128, 256, 0, s>>>(acc_x ? ty : tx, tx, N, D, L.ldt));
         }
       }));
     }
@@ -1514,6 +1522,27 @@ static int postpass_run(const void* x, int64_t ldx, const void* y, int64_t ldy, 
   const bool pvec = data_dtype(dtype) == MEC_DTYPE_F32 && d % 4 == 0 && ldx % 4 == 0 && ldy % 4 == 0 &&
                     aligned16(x) && aligned16(y) && aligned16(acc_x) && aligned16(acc_y) && aligned16(dx) &&
                     aligned16(dy);
+  // both sides, 16-byte rows throughout (the accumulators' rows are n d floats:
+  // D a multiple of the vector), up to 2048 features: one wave takes a row of
+  // both.  Measured against a launch over (row, side): see k_postpass_both.
+  const bool both = acc_x && acc_y && d <= 2048 && rows_vec16(x, ldx, y, ldy, d, data_dtype(dtype)) &&
+                    aligned16(acc_x) && aligned16(acc_y) && aligned16(dx) && aligned16(dy) && aligned16(parts);
+  if (both) {
+    const dim3 rows((unsigned)((n + 3) / 4));
+    DISPATCH_DTYPE(data_dtype(dtype), T, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(accr, ACCR, {
+      if constexpr (std::is_same<T, float>::value || !ACCR) {
+        const PostSide<T> px{(const T*)x, ldx, (const T*)y, ldy, rx, ry, acc_x, (T*)dx, parts};
+        const PostSide<T> py{(const T*)y, ldy, (const T*)x, ldx, ry, rx, acc_y, (T*)dy,
+                             parts ? parts + (nparts - 1) * n * d : nullptr};
+        constexpr int per = 16 / kVec16<T>;  // vectors of 16 features
+        if (d <= 1024)
+          k_postpass_both<T, NORM, ACCR, per><<<rows, 256, 0, s>>>(px, py, N, D, kap, a, grad_output, nparts);
+        else
+          k_postpass_both<T, NORM, ACCR, 2 * per><<<rows, 256, 0, s>>>(px, py, N, D, kap, a, grad_output, nparts);
+      }
+    })));
+    return check_launch("postpass");
+  }
   DISPATCH_DTYPE(data_dtype(dtype), T, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(accr, ACCR, {
     const PostSide<T> px{(const T*)x, ldx, (const T*)y, ldy, rx, ry, acc_x, (T*)dx, parts};
     const PostSide<T> py{(const T*)y, ldy, (const T*)x, ldx, ry, rx, acc_y, (T*)dy,

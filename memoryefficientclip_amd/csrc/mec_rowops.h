@@ -2,6 +2,8 @@
 // diagonal pre-pass, the loss finalize, and the gradient post-pass.  These are
 // HBM-bound; one 64-lane wave owns one feature row.
 #pragma once
+#include <type_traits>
+
 #include "mec_common.h"
 
 namespace mec {
@@ -20,11 +22,45 @@ template <> struct Elem<_Float16> {
   static __device__ __forceinline__ void store(_Float16* p, int64_t i, float v) { p[i] = (_Float16)v; }
 };
 
+// V consecutive elements of a row as floats, and back: one 16-byte vector (fp32
+// V = 4, 16-bit V = 8; 16-byte aligned)
+template <typename T> constexpr int kVec16 = 16 / (int)sizeof(T);
+template <typename T>
+__device__ __forceinline__ void load_vec(const T* __restrict__ p, float (&v)[kVec16<T>]) {
+  if constexpr (sizeof(T) == 4) {
+    const f32x4 u = *(const f32x4*)p;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = u[e];
+  } else {
+    typedef T tvec __attribute__((ext_vector_type(8)));
+    const tvec u = *(const tvec*)p;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const T t = u[e];
+      v[e] = Elem<T>::load(&t, 0);
+    }
+  }
+}
+template <typename T>
+__device__ __forceinline__ void store_vec(T* __restrict__ p, const float (&v)[kVec16<T>]) {
+  if constexpr (sizeof(T) == 4) {
+    *(f32x4*)p = f32x4{v[0], v[1], v[2], v[3]};
+  } else {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      u[e] = std::is_same<T, uint16_t>::value ? pack2_bf16(v[2 * e], v[2 * e + 1]) : pack2_f16(v[2 * e], v[2 * e + 1]);
+    *(u32x4*)p = u;
+  }
+}
+
 // Per row i: rx = 1/max(||x_i||, 1e-12) (or 1), ry likewise, diag = x_i . y_i.
 // Also clears the off-diagonal sum accumulators used by the sum-exp kernel.
 // Follows F.normalize(dim=1) as applied at clip_loss.py:266-268 and the
 // einsum('bi,bi->b') diagonal at clip_loss.py:206.
-template <typename T, bool NORM>
+// VEC: 16-byte aligned rows, D a multiple of the vector.
+template <typename T, bool NORM, bool VEC>
 __global__ __launch_bounds__(256) void k_prepass(const T* __restrict__ X, int64_t ldx,
                                                  const T* __restrict__ Y, int64_t ldy, int N, int D,
                                                  float* __restrict__ ws, uint32_t* __restrict__ counter) {
@@ -35,11 +71,38 @@ __global__ __launch_bounds__(256) void k_prepass(const T* __restrict__ X, int64_
   const T* x = X + (int64_t)row * ldx;
   const T* y = Y + (int64_t)row * ldy;
   float sx = 0.f, sy = 0.f, sxy = 0.f;
-  for (int d = lane; d < D; d += 64) {
-    float a = Elem<T>::load(x, d), b = Elem<T>::load(y, d);
-    sx = fmaf(a, a, sx);
-    sy = fmaf(b, b, sy);
-    sxy = fmaf(a, b, sxy);
+  if constexpr (VEC) {
+    // (16-byte vectors; up to four of each row in flight)
+    constexpr int V = kVec16<T>;
+    for (int d0 = V * lane; d0 < D; d0 += 256 * V) {
+      float a[4][V], b[4][V];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int d = d0 + 64 * V * k;
+        if (d < D) {
+          load_vec<T>(x + d, a[k]);
+          load_vec<T>(y + d, b[k]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < V; ++e) a[k][e] = b[k][e] = 0.f;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+          sx = fmaf(a[k][e], a[k][e], sx);
+          sy = fmaf(b[k][e], b[k][e], sy);
+          sxy = fmaf(a[k][e], b[k][e], sxy);
+        }
+    }
+  } else {
+    for (int d = lane; d < D; d += 64) {
+      float a = Elem<T>::load(x, d), b = Elem<T>::load(y, d);
+      sx = fmaf(a, a, sx);
+      sy = fmaf(b, b, sy);
+      sxy = fmaf(a, b, sxy);
+    }
   }
   sx = wave_sum(sx);
   sy = wave_sum(sy);
@@ -372,6 +435,106 @@ __global__ __launch_bounds__(256) void k_postpass(PostSide<T> s0, PostSide<T> s1
   }
 }
 
+// k_postpass of both sides at once, on 16-byte vectors: one wave per row takes x_i,
+// y_i and both accumulator rows (with their parts), so that x and y are read once
+// instead of once per side.  HBM-bound.  Rows of up to NV x 64 vectors, 16-byte
+// aligned (own, other, accumulators, parts and outputs; D a multiple of the
+// vector).  The same arithmetic as k_postpass; only the order of the feature sum
+// <x^, h> differs.  NV sizes the registers: 16 features per lane up to D = 1024,
+// 32 up to D = 2048.
+template <typename T, bool NORM, bool ACCR, int NV>
+__global__ __launch_bounds__(256) void k_postpass_both(PostSide<T> s0, PostSide<T> s1, int N, int D,
+                                                       const float* __restrict__ kappa, float a,
+                                                       const float* __restrict__ grad_output, int nparts) {
+  constexpr int V = kVec16<T>;
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= N) return;
+  const T* x = s0.own + (int64_t)row * s0.ld_own;
+  const T* y = s1.own + (int64_t)row * s1.ld_own;
+  const int64_t ps = (int64_t)N * D, ro = (int64_t)row * D;
+  const float rx = s0.r_own[row], ry = s1.r_own[row], kap = kappa[row];
+  const float kx = kap * ry * (ACCR ? rx : 1.f), ky = kap * rx * (ACCR ? ry : 1.f);
+  const float go = grad_output ? *grad_output : 1.f;
+  float xv[NV][V], yv[NV][V], hx[NV][V], hy[NV][V];
+  auto load_acc = [&](const float* p, float (&v)[V]) {
+#pragma unroll
+    for (int q = 0; q < V / 4; ++q) {
+      const f32x4 u = *(const f32x4*)(p + 4 * q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * q + e] = u[e];
+    }
+  };
+  // (an accumulator may be its side's output: every element is read before the
+  // same lane writes it)
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int d = V * (lane + 64 * k);
+    if (64 * V * k < D && d < D) {
+      load_vec<T>(x + d, xv[k]);
+      load_vec<T>(y + d, yv[k]);
+      load_acc(s0.acc + ro + d, hx[k]);
+      load_acc(s1.acc + ro + d, hy[k]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < V; ++e) xv[k][e] = yv[k][e] = hx[k][e] = hy[k][e] = 0.f;
+    }
+  }
+  for (int p = 0; p + 1 < nparts; ++p) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int d = V * (lane + 64 * k);
+      if (64 * V * k < D && d < D) {
+        float u[V], w[V];
+        load_acc(s0.part + p * ps + ro + d, u);
+        load_acc(s1.part + p * ps + ro + d, w);
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+          hx[k][e] += u[e];
+          hy[k][e] += w[e];
+        }
+      }
+    }
+  }
+  float dx = 0.f, dy = 0.f;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      hx[k][e] = a * fmaf(kx, yv[k][e], hx[k][e]);
+      hy[k][e] = a * fmaf(ky, xv[k][e], hy[k][e]);
+      if (NORM) {
+        xv[k][e] *= rx;
+        yv[k][e] *= ry;
+        dx = fmaf(xv[k][e], hx[k][e], dx);
+        dy = fmaf(yv[k][e], hy[k][e], dy);
+      }
+    }
+  }
+  if (NORM) {
+    dx = wave_sum(dx);
+    dy = wave_sum(dy);
+  }
+  const bool cx = rx >= 1e12f, cy = ry >= 1e12f;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int d = V * (lane + 64 * k);
+    if (64 * V * k < D && d < D) {
+      float u[V], w[V];
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        u[e] = NORM && !cx ? hx[k][e] - xv[k][e] * dx : hx[k][e];
+        w[e] = NORM && !cy ? hy[k][e] - yv[k][e] * dy : hy[k][e];
+        // (grad_output last, as k_postpass)
+        u[e] = NORM && !ACCR ? go * (rx * u[e]) : go * u[e];
+        w[e] = NORM && !ACCR ? go * (ry * w[e]) : go * w[e];
+      }
+      store_vec<T>(s0.out + ro + d, u);
+      store_vec<T>(s1.out + ro + d, w);
+    }
+  }
+}
+
 // One feature matrix to transpose: X (row pitch ldx), its row scales and the
 // destination plane(s) (pitch ldt).  The transposes of the two sides share
 // one launch: blockIdx.z picks the side.
@@ -386,31 +549,69 @@ struct TransSide {
 
 // Transposed, normalised copy of one feature matrix for the backward's
 // contractions: XT[d, i] = scale_i * X[i, d] (scale = 1/max(||x_i||, 1e-12)
-// when NORM) for i < N and 0 for N <= i < ldt, rounded to T once.  64 x 64
-// tiles through LDS; both the loads and the stores are coalesced.
-template <typename T, bool NORM>
+// when NORM) for i < N and 0 for N <= i < ldt, rounded to T once.  64 features x
+// 128 rows through LDS.  VEC (16-byte aligned rows, D a multiple of 8): 16-byte
+// loads, 8 features per lane; the stores are 16-byte either way (8 rows i per
+// lane, 256 contiguous bytes per feature).  HBM-bound.
+// LDS: [i][d] with an odd pitch in 4-byte words: the 16 row groups of a
+// feature's gather fall on 8 banks, two lanes each.
+template <typename T, bool NORM, bool VEC>
 __global__ __launch_bounds__(256) void k_transpose(TransSide<T> s0, TransSide<T> s1, int N, int D, int64_t ldt) {
   const TransSide<T>& sd = blockIdx.z ? s1 : s0;
   const T* __restrict__ X = sd.X;
   const int64_t ldx = sd.ldx;
   const float* __restrict__ scale = sd.scale;
   T* __restrict__ XT = sd.XT;
-  __shared__ float tile[64][65];
-  const int i0 = blockIdx.x * 64, d0 = blockIdx.y * 64;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  for (int r = ty; r < 64; r += 4) {
-    const int i = i0 + r, d = d0 + tx;
-    float v = 0.f;
-    if (i < N && d < D) {
-      v = Elem<T>::load(X, (int64_t)i * ldx + d);
-      if (NORM) v *= scale[i];
+  static_assert(sizeof(T) == 2, "16-bit types");
+  constexpr int TI = 128, TD = 64, P = TD + 2;
+  __shared__ __attribute__((aligned(16))) uint16_t tile[TI * P];
+  const int i0 = blockIdx.x * TI, d0 = blockIdx.y * TD;
+  if constexpr (VEC) {
+#pragma unroll
+    for (int u = 0; u < TI * TD / 8 / 256; ++u) {
+      const int v = threadIdx.x + 256 * u, r = v >> 3, c = (v & 7) * 8;
+      const int i = i0 + r, d = d0 + c;
+      float f[8];
+      if (i < N && d < D) {
+        load_vec<T>(X + (int64_t)i * ldx + d, f);
+        if (NORM) {
+          const float s = scale[i];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) f[e] *= s;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = 0.f;
+      }
+      uint32_t* o = (uint32_t*)&tile[r * P + c];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        o[e] = std::is_same<T, uint16_t>::value ? pack2_bf16(f[2 * e], f[2 * e + 1]) : pack2_f16(f[2 * e], f[2 * e + 1]);
     }
-    tile[r][tx] = v;
+  } else {
+    for (int r = threadIdx.x >> 6; r < TI; r += 4) {
+      const int c = threadIdx.x & 63, i = i0 + r, d = d0 + c;
+      float v = 0.f;
+      if (i < N && d < D) {
+        v = Elem<T>::load(X, (int64_t)i * ldx + d);
+        if (NORM) v *= scale[i];
+      }
+      T t;
+      Elem<T>::store(&t, 0, v);
+      tile[r * P + c] = __builtin_bit_cast(uint16_t, t);
+    }
   }
   __syncthreads();
-  for (int r = ty; r < 64; r += 4) {
-    const int d = d0 + r, i = i0 + tx;
-    if (d < D && i < ldt) Elem<T>::store(XT, (int64_t)d * ldt + i, tile[tx][r]);
+  typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+#pragma unroll
+  for (int u = 0; u < TI * TD / 8 / 256; ++u) {
+    const int v = threadIdx.x + 256 * u, g = v & 15, c = v >> 4;
+    const int d = d0 + c;
+    if (d >= D) break;
+    u16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = tile[(8 * g + e) * P + c];
+    *(u16x8*)(XT + (int64_t)d * ldt + i0 + 8 * g) = o;
   }
 }
 
