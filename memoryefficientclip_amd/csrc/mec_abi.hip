@@ -393,6 +393,14 @@ void grad_blocks_budget(int64_t n, int64_t d, int dtype, int64_t gbudget, int* b
   const int64_t min_rows = is_pairs(dtype) ? 2 * kTargetMinRows : kTargetMinRows;
   const int64_t target_rows = mult * d > min_rows ? mult * d : min_rows;
   int64_t target = (target_rows + q - 1) / q;
+  // 16-bit: one block from n = 3072 while its matrix stays within the smallest
+  // budget (n <= 11520): one buffer instead of two, so no more memory than two
+  // blocks of half the rows, half the launches, tiles that fill their rounds
+  // better and half the accumulator updates (fp16 6001 x 512, two blocks of 3072
+  // rows -> one: gradient-matrix tiles 72 -> 54 us, contractions 121 -> 86 us)
+  if (dtype != MEC_DTYPE_F32 && !is_pairs(dtype) && n >= 3072 &&
+      g_bytes(tiles, q, tiles, dtype) <= (gbudget < kGradBudgetMin ? gbudget : kGradBudgetMin))
+    target = tiles;
   if (const char* env = std::getenv("MEC_GRAD_BLOCK_TILES")) {
     long v = std::strtol(env, nullptr, 10);
     if (v >= 1 && v <= 4096) target = v;
@@ -915,7 +923,14 @@ static int sumexp_det_run(const void* x, int64_t ldx, const void* y, int64_t ldy
   const int N = (int)n;
   float* rowpart = workspace + det_partials_offset(n);
   float* colpart = rowpart + (int64_t)DET_Q * n;
-  const int P = tiles_m < DET_P ? tiles_m : DET_P, Q = tiles_n < DET_Q ? tiles_n : DET_Q;
+  int P = tiles_m < DET_P ? tiles_m : DET_P, Q = tiles_n < DET_Q ? tiles_n : DET_Q;
+  // 17 to 22 tiles a side (256 x 256 tiles, one workgroup per CU): with 16 column
+  // blocks more than 256 workgroups of one or two tiles start, and the last ones
+  // end a third tile after the first; blocks of two column tiles are at most 256
+  // workgroups and two tiles (pairs 4999 x 640: forward 119 -> 87 us).  A rule
+  // on the tile counts alone, so that the order of the sums is the same on any
+  // device.
+  if (FwdTile<T, true>::BM == 256 && vec && tiles_n > DET_Q && P * ((tiles_n + 1) / 2) <= 256) Q = (tiles_n + 1) / 2;
   const unsigned sum_grid = (unsigned)((n + 255) / 256);
   auto run = [&](auto lit_c, auto norm_c, auto vec_c) {
     constexpr bool LIT = decltype(lit_c)::value, NORM = decltype(norm_c)::value, VEC = decltype(vec_c)::value;
@@ -1518,27 +1533,28 @@ static int postpass_run(const void* x, int64_t ldx, const void* y, int64_t ldy, 
   // fp32 (not the split modes): the accumulators carry the row's inverse norm
   // (the contractions of H = diag(rx) G' diag(ry) with the raw inputs)
   const bool accr = dtype == MEC_DTYPE_F32;
-  // fp32 data with every row 16-byte aligned: 16-byte vectors
-  const bool pvec = data_dtype(dtype) == MEC_DTYPE_F32 && d % 4 == 0 && ldx % 4 == 0 && ldy % 4 == 0 &&
-                    aligned16(x) && aligned16(y) && aligned16(acc_x) && aligned16(acc_y) && aligned16(dx) &&
-                    aligned16(dy);
-  // both sides, 16-byte rows throughout (the accumulators' rows are n d floats:
-  // D a multiple of the vector), up to 2048 features: one wave takes a row of
-  // both.  Measured against a launch over (row, side): see k_postpass_both.
-  const bool both = acc_x && acc_y && d <= 2048 && rows_vec16(x, ldx, y, ldy, d, data_dtype(dtype)) &&
+  // 16-byte rows throughout (the accumulators' rows are n d floats: D a multiple
+  // of the vector), up to 2048 features: one wave takes a row of every side
+  // there is.  Measured against k_postpass: see k_postpass_vec.
+  const bool both = acc_x && acc_y;
+  const bool vec16 = d <= 2048 && rows_vec16(x, ldx, y, ldy, d, data_dtype(dtype)) &&
                     aligned16(acc_x) && aligned16(acc_y) && aligned16(dx) && aligned16(dy) && aligned16(parts);
-  if (both) {
+  if (vec16) {
     const dim3 rows((unsigned)((n + 3) / 4));
     DISPATCH_DTYPE(data_dtype(dtype), T, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(accr, ACCR, {
       if constexpr (std::is_same<T, float>::value || !ACCR) {
         const PostSide<T> px{(const T*)x, ldx, (const T*)y, ldy, rx, ry, acc_x, (T*)dx, parts};
         const PostSide<T> py{(const T*)y, ldy, (const T*)x, ldx, ry, rx, acc_y, (T*)dy,
-                             parts ? parts + (nparts - 1) * n * d : nullptr};
+                             parts ? parts + (acc_x ? (nparts - 1) * n * d : 0) : nullptr};
         constexpr int per = 16 / kVec16<T>;  // vectors of 16 features
-        if (d <= 1024)
-          k_postpass_both<T, NORM, ACCR, per><<<rows, 256, 0, s>>>(px, py, N, D, kap, a, grad_output, nparts);
-        else
-          k_postpass_both<T, NORM, ACCR, 2 * per><<<rows, 256, 0, s>>>(px, py, N, D, kap, a, grad_output, nparts);
+        const PostSide<T>&p0 = acc_x ? px : py, &p1 = acc_x ? py : px;
+        DISPATCH_BOOL(both, BOTH, {
+          if (d <= 1024)
+            k_postpass_vec<T, NORM, ACCR, BOTH, per><<<rows, 256, 0, s>>>(p0, p1, N, D, kap, a, grad_output, nparts);
+          else
+            k_postpass_vec<T, NORM, ACCR, BOTH, 2 * per><<<rows, 256, 0, s>>>(p0, p1, N, D, kap, a, grad_output,
+                                                                             nparts);
+        });
       }
     })));
     return check_launch("postpass");
@@ -1547,10 +1563,7 @@ static int postpass_run(const void* x, int64_t ldx, const void* y, int64_t ldy, 
     const PostSide<T> px{(const T*)x, ldx, (const T*)y, ldy, rx, ry, acc_x, (T*)dx, parts};
     const PostSide<T> py{(const T*)y, ldy, (const T*)x, ldx, ry, rx, acc_y, (T*)dy,
                          parts ? parts + (acc_x ? (nparts - 1) * n * d : 0) : nullptr};
-    if constexpr (std::is_same<T, float>::value) {
-      DISPATCH_BOOL(pvec, VEC,
-          k_postpass<T, NORM, ACCR, VEC><<<grid, 256, 0, s>>>(acc_x ? px : py, py, N, D, kap, a, grad_output, nparts));
-    } else if constexpr (!ACCR) {
+    if constexpr (std::is_same<T, float>::value || !ACCR) {
       k_postpass<T, NORM, ACCR><<<grid, 256, 0, s>>>(acc_x ? px : py, py, N, D, kap, a, grad_output, nparts);
     }
   })));

@@ -315,14 +315,11 @@ struct PostSide {
 // contractions multiply H = diag(rx) G' diag(ry) with the raw inputs.  Then
 // h = a (kappa_i r_i y^_i + acc) = r_i dx^_i, and the normalisation backward
 // r_i (dx^ - x^ <x^, dx^>) is h - x^ <x^, h>: no division by the norm.
-// VEC (fp32; every row of own, oth, acc and out 16-byte aligned, D a multiple
-// of 4): the register path reads and writes 16-byte vectors, four
-// consecutive features per lane.
-template <typename T, bool NORM, bool ACCR = false, bool VEC = false>
+// Rows that are not 16-byte vectors, or longer than k_postpass_vec takes.
+template <typename T, bool NORM, bool ACCR = false>
 __global__ __launch_bounds__(256) void k_postpass(PostSide<T> s0, PostSide<T> s1, int N, int D,
                                                   const float* __restrict__ kappa, float a,
                                                   const float* __restrict__ grad_output, int nparts) {
-  static_assert(!VEC || std::is_same<T, float>::value, "16-byte vectors of fp32");
   const PostSide<T>& sd = blockIdx.y ? s1 : s0;
   const T* __restrict__ own = sd.own;
   const int64_t ld_own = sd.ld_own;
@@ -340,15 +337,10 @@ __global__ __launch_bounds__(256) void k_postpass(PostSide<T> s0, PostSide<T> s1
   const float* ac = acc + (int64_t)row * D;
   const float* pt = sd.part + (int64_t)row * D;
   const int64_t ps = (int64_t)N * D;
-  // accumulated sums of feature d (or d .. d + 3): the parts in order
+  // accumulated sums of feature d: the parts in order
   auto accv = [&](int d) {
     float v = ac[d];
     for (int p = 0; p + 1 < nparts; ++p) v += pt[p * ps + d];
-    return v;
-  };
-  auto accv4 = [&](int d) {
-    f32x4 v = *(const f32x4*)(ac + d);
-    for (int p = 0; p + 1 < nparts; ++p) v += *(const f32x4*)(pt + p * ps + d);
     return v;
   };
   T* o = out + (int64_t)row * D;
@@ -358,39 +350,6 @@ __global__ __launch_bounds__(256) void k_postpass(PostSide<T> s0, PostSide<T> s1
   if (NORM) {
     float dot = 0.f;
     const bool clamped = ro >= 1e12f;
-    if (VEC && D <= 64 * POST_REG) {
-      constexpr int NV = POST_REG / 4;
-      f32x4 g[NV], xr[NV];
-#pragma unroll
-      for (int k = 0; k < NV; ++k) {
-        const int d = 4 * lane + 256 * k;
-        g[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-        xr[k] = g[k];
-        if (d < D) {
-          const f32x4 yv = *(const f32x4*)(yo + d), av = accv4(d), xv = *(const f32x4*)(xo + d);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            g[k][u] = a * fmaf(kq, yv[u], av[u]);
-            xr[k][u] = xv[u] * ro;
-            dot = fmaf(xr[k][u], g[k][u], dot);
-          }
-        }
-      }
-      dot = wave_sum(dot);
-#pragma unroll
-      for (int k = 0; k < NV; ++k) {
-        const int d = 4 * lane + 256 * k;
-        if (d < D) {
-          f32x4 v;
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            v[u] = go * (ACCR ? (clamped ? g[k][u] : g[k][u] - xr[k][u] * dot)
-                              : (clamped ? ro * g[k][u] : ro * (g[k][u] - xr[k][u] * dot)));
-          *(f32x4*)((float*)o + d) = v;
-        }
-      }
-      return;
-    }
     if (D <= 64 * POST_REG) {
       // the row stays in registers between the reduction and the stores
       float g[POST_REG], xr[POST_REG];
@@ -435,17 +394,20 @@ __global__ __launch_bounds__(256) void k_postpass(PostSide<T> s0, PostSide<T> s1
   }
 }
 
-// k_postpass of both sides at once, on 16-byte vectors: one wave per row takes x_i,
-// y_i and both accumulator rows (with their parts), so that x and y are read once
-// instead of once per side.  HBM-bound.  Rows of up to NV x 64 vectors, 16-byte
+// k_postpass on 16-byte vectors, BOTH: both sides at once (else side s0, s1 naming
+// the other side's input): one wave per row takes x_i, y_i and the accumulator
+// rows (with their parts), so that x and y are read once instead of once per
+// side.  HBM-bound: bf16 4096 x 768 with two parts 23 -> 12.5 us, 16384 x 1024 78
+// -> 42 us (268 MB, 6.4 TB/s with the Infinity Cache's help), fp32 32768 x 1152
+// 215 -> 146 us; one side, bf16 2048 x 768 with eight parts 14.7 -> 6.1 us.  Rows of up to NV x 64 vectors, 16-byte
 // aligned (own, other, accumulators, parts and outputs; D a multiple of the
 // vector).  The same arithmetic as k_postpass; only the order of the feature sum
 // <x^, h> differs.  NV sizes the registers: 16 features per lane up to D = 1024,
 // 32 up to D = 2048.
-template <typename T, bool NORM, bool ACCR, int NV>
-__global__ __launch_bounds__(256) void k_postpass_both(PostSide<T> s0, PostSide<T> s1, int N, int D,
-                                                       const float* __restrict__ kappa, float a,
-                                                       const float* __restrict__ grad_output, int nparts) {
+template <typename T, bool NORM, bool ACCR, bool BOTH, int NV>
+__global__ __launch_bounds__(256) void k_postpass_vec(PostSide<T> s0, PostSide<T> s1, int N, int D,
+                                                      const float* __restrict__ kappa, float a,
+                                                      const float* __restrict__ grad_output, int nparts) {
   constexpr int V = kVec16<T>;
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -474,7 +436,7 @@ __global__ __launch_bounds__(256) void k_postpass_both(PostSide<T> s0, PostSide<
       load_vec<T>(x + d, xv[k]);
       load_vec<T>(y + d, yv[k]);
       load_acc(s0.acc + ro + d, hx[k]);
-      load_acc(s1.acc + ro + d, hy[k]);
+      if (BOTH) load_acc(s1.acc + ro + d, hy[k]);
     } else {
 #pragma unroll
       for (int e = 0; e < V; ++e) xv[k][e] = yv[k][e] = hx[k][e] = hy[k][e] = 0.f;
@@ -487,11 +449,11 @@ __global__ __launch_bounds__(256) void k_postpass_both(PostSide<T> s0, PostSide<
       if (64 * V * k < D && d < D) {
         float u[V], w[V];
         load_acc(s0.part + p * ps + ro + d, u);
-        load_acc(s1.part + p * ps + ro + d, w);
+        if (BOTH) load_acc(s1.part + p * ps + ro + d, w);
 #pragma unroll
         for (int e = 0; e < V; ++e) {
           hx[k][e] += u[e];
-          hy[k][e] += w[e];
+          if (BOTH) hy[k][e] += w[e];
         }
       }
     }
@@ -502,18 +464,20 @@ __global__ __launch_bounds__(256) void k_postpass_both(PostSide<T> s0, PostSide<
 #pragma unroll
     for (int e = 0; e < V; ++e) {
       hx[k][e] = a * fmaf(kx, yv[k][e], hx[k][e]);
-      hy[k][e] = a * fmaf(ky, xv[k][e], hy[k][e]);
+      if (BOTH) hy[k][e] = a * fmaf(ky, xv[k][e], hy[k][e]);
       if (NORM) {
         xv[k][e] *= rx;
-        yv[k][e] *= ry;
         dx = fmaf(xv[k][e], hx[k][e], dx);
-        dy = fmaf(yv[k][e], hy[k][e], dy);
+        if (BOTH) {
+          yv[k][e] *= ry;
+          dy = fmaf(yv[k][e], hy[k][e], dy);
+        }
       }
     }
   }
   if (NORM) {
     dx = wave_sum(dx);
-    dy = wave_sum(dy);
+    if (BOTH) dy = wave_sum(dy);
   }
   const bool cx = rx >= 1e12f, cy = ry >= 1e12f;
 #pragma unroll
@@ -524,13 +488,15 @@ __global__ __launch_bounds__(256) void k_postpass_both(PostSide<T> s0, PostSide<
 #pragma unroll
       for (int e = 0; e < V; ++e) {
         u[e] = NORM && !cx ? hx[k][e] - xv[k][e] * dx : hx[k][e];
-        w[e] = NORM && !cy ? hy[k][e] - yv[k][e] * dy : hy[k][e];
         // (grad_output last, as k_postpass)
         u[e] = NORM && !ACCR ? go * (rx * u[e]) : go * u[e];
-        w[e] = NORM && !ACCR ? go * (ry * w[e]) : go * w[e];
+        if (BOTH) {
+          w[e] = NORM && !cy ? hy[k][e] - yv[k][e] * dy : hy[k][e];
+          w[e] = NORM && !ACCR ? go * (ry * w[e]) : go * w[e];
+        }
       }
       store_vec<T>(s0.out + ro + d, u);
-      store_vec<T>(s1.out + ro + d, w);
+      if (BOTH) store_vec<T>(s1.out + ro + d, w);
     }
   }
 }
