@@ -523,6 +523,18 @@ bool f32_small_fwd_tiles(int64_t n, int64_t d, int cus) {
   const int e = small_tiles_env();
   return e >= 0 ? e == 1 : f32_small_fwd(n, d, cus);
 }
+// 128 x 128 tiles of the 16-bit kernels (small16_n; not bf16x3, whose
+// operands and planes keep the 256 x 256 ones); MEC_16BIT_SMALL_TILES=0 or 1
+// overrides, and forced contraction tiles keep the large ones (tests)
+bool contract_forced() { return std::getenv("MEC_NARROW_CONTRACT") || std::getenv("MEC_WIDE_CONTRACT"); }
+bool small16_tiles(int64_t n, int dtype) {
+  if (dtype == MEC_DTYPE_F32 || is_x3(dtype)) return false;
+  if (const char* env = std::getenv("MEC_16BIT_SMALL_TILES")) {
+    if (env[0] == '0') return false;
+    if (env[0] == '1') return true;
+  }
+  return !contract_forced() && small16_n(n, dtype);
+}
 bool f32_small_bwd_tiles(int64_t n, int64_t d, int64_t bs, int cus) {
   const int e = small_tiles_env();
   return e >= 0 ? e == 1 : f32_small_bwd(n, d, bs, cus);
@@ -580,7 +592,7 @@ BlockGrid block_grid(int64_t d, int dtype, int sides, int bs, int nb, int64_t ld
   const int D = (int)d;
   BlockGrid bg{bs, nb, bs / tf.bm, bs / tf.bn, bs / tc.bm, (D + tc.bn - 1) / tc.bn, 0};
   *w384 = false;
-  if (separate_contractions(dtype) && !is_pairs(dtype)) {
+  if (separate_contractions(dtype) && !is_pairs(dtype) && tc.bm == 256) {
     const int64_t nsides = ((sides & kSideX) ? 1 : 0) + ((sides & kSideY) ? 1 : 0);
     const int64_t wide = nsides * nb * bg.ctm * bg.ctd;
     int64_t tiles = wide;
@@ -621,7 +633,6 @@ struct ConSplit {
 };
 constexpr int kMaxParts = 8;
 constexpr int64_t kPartsBytes = int64_t(256) << 20;  // at most this much for the parts
-bool contract_forced() { return std::getenv("MEC_NARROW_CONTRACT") || std::getenv("MEC_WIDE_CONTRACT"); }
 // bg, w384: the unsplit choice (block_grid)
 ConSplit contract_split(int64_t n, int64_t d, int dtype, int sides, const BlockGrid& bg, bool w384, int64_t ldt,
                         int cus) {
@@ -632,14 +643,17 @@ ConSplit contract_split(int64_t n, int64_t d, int dtype, int sides, const BlockG
   if (contract_forced() && force <= 0) return best;
   const int nsides = ((sides & kSideX) ? 1 : 0) + ((sides & kSideY) ? 1 : 0);
   const int64_t rows = n < bg.bs ? n : bg.bs;  // k rows of a block
-  const double per_k = is_pairs(dtype) ? 0.060 : 0.020;
+  // (128 x 128 tiles: two workgroups per CU, each a quarter of the work)
+  const bool small = small16_tiles(n, dtype);
+  const int slots = small ? 2 * cus : cus;
+  const double per_k = (is_pairs(dtype) ? 0.060 : 0.020) * (small ? 0.6 : 1.0);
   const int64_t tiles1 = (int64_t)nsides * bg.nb * (bg.cnw ? (bg.ctm / 2) * (2 * bg.ctd + 1) : bg.ctm * bg.ctd);
   const int64_t t384 = (int64_t)nsides * bg.nb * bg.ctm * ((d + 383) / 384);
-  const bool can384 = !is_pairs(dtype) && wide_contract_fits(ldt, bg.bs);
+  const bool can384 = !is_pairs(dtype) && !small && wide_contract_fits(ldt, bg.bs);
   auto cost = [&](int ks, bool w) {
     const int64_t tiles = (w && !w384 ? t384 : tiles1) * ks;
     const double k = (double)((rows + ks - 1) / ks) * per_k * (w ? 1.4 : 1.0);
-    return (double)bg.nb * ((double)((tiles + cus - 1) / cus) * (k + 4.0) +
+    return (double)bg.nb * ((double)((tiles + slots - 1) / slots) * (k + 4.0) +
                             (double)(ks - 1) * n * d * nsides * 4.0 * (1.0 + 1.0 / bg.nb) / 2.5e6);
   };
   const int most = force > 0 ? (force < kMaxParts ? force : kMaxParts) : kMaxParts;
@@ -669,8 +683,9 @@ ConSplit backward_split(int64_t n, int64_t d, int dtype, int sides, const Scratc
   if (!separate_contractions(dtype) || is_x3(dtype)) return ConSplit{1, L.bs, false};
   const int gdt = is_split(dtype) ? MEC_DTYPE_BF16 : dtype;
   bool w384 = false;
-  const BlockGrid bg = block_grid(d, gdt, sides, L.bs, L.nb, L.ldt, cus, fwd_tile_dims(gdt, true, false),
-                                  con_tile_dims(gdt, false), &w384);
+  const bool small = small16_tiles(n, dtype);
+  const BlockGrid bg = block_grid(d, gdt, sides, L.bs, L.nb, L.ldt, cus, fwd_tile_dims(gdt, true, small),
+                                  con_tile_dims(gdt, small), &w384);
   return contract_split(n, d, dtype, sides, bg, w384, L.ldt, cus);
 }
 // compute units of the device for the size queries (which also run without one)
@@ -715,14 +730,15 @@ int plan_units() {
 // "high" precision (bf16x3): always (three products as well, more exact, fewer
 // operand bytes; step at 2048 x 512 248 -> 201 us, 4999 x 640 655 -> 567 us,
 // 8192 x 768 1194 -> 1127 us, 32768 x 1152 the same).
-// fp32: above the kept similarity matrix's range.  Measured, CLIP step, fp32
-// MFMA -> pairs: 2500 x 64 129 -> 131 us, 4096 x 64 153 -> 126 us, 8192 x 128
-// 695 -> 384 us, 4096 x 512 554 -> 243 us, 4999 x 640 1171 -> 460 us, 8192 x 768
-// 3028 -> 1090 us, 32768 x 1152 71.9 -> 23.8 ms; the loss alone, 16384 x 64 390
-// -> 164 us, 2500 x 512 80 -> 52 us.  Up to n = 2048 the kept matrix takes three
-// launches (1024 x 512 107 -> 150 us, 1500 x 768 140 -> 156 us, 2048 x 512 131 ->
-// 137 us; only its corner past 1800 x 1152 is slower, 258 -> 234 us), and the
-// loss alone is no faster (2048 x 512 50 us either way).
+// fp32: above the kept similarity matrix's range, and in its larger corner.
+// Measured, CLIP step, fp32 MFMA -> pairs: 4096 x 64 153 -> 126 us, 8192 x 128 695
+// -> 384 us, 4096 x 512 554 -> 243 us, 4999 x 640 1171 -> 416 us, 8192 x 768 3028
+// -> 1090 us, 32768 x 1152 71.9 -> 23.8 ms; the loss alone, 16384 x 64 390 -> 164
+// us, 2500 x 512 80 -> 52 us.  Up to n = 2048 the kept matrix takes three
+// launches: GPU time of a step, kept -> pairs: 1024 x 512 48 -> 74 us, 1024 x 1152
+// 93 -> 117, 1500 x 256 65 -> 65, 2048 x 512 134 -> 100, 1500 x 768 139 -> 112,
+// 2048 x 1152 280 -> 177.  The line is where the kept step outlasts the host work
+// of the pairs' eight launches (about 130 us).
 bool pairs_preferred(int64_t n, int64_t d, int dtype) {
   if (dtype != MEC_DTYPE_F32 && dtype != MEC_DTYPE_F32_BF16X3) return false;
   if (n < 1 || d < 1 || n > kMaxNPairs || d > kMaxD) return false;
@@ -732,7 +748,7 @@ bool pairs_preferred(int64_t n, int64_t d, int dtype) {
   }
   if (dtype == MEC_DTYPE_F32_BF16X3) return true;
   if (small_tiles_env() >= 0) return false;  // (the fp32 tiles are asked for)
-  return n > MEC_KEEP_EXP_MAX_N;
+  return n > MEC_KEEP_EXP_MAX_N || (n >= 1400 && n * n * d >= 2500000000LL);
 }
 
 }  // namespace
@@ -825,7 +841,7 @@ int mec_backward_plan(int64_t n, int64_t d, int dtype, int mode, int sides, int 
   plan->scratch_bytes = L.total;
   // the tiles of a launch with contractions (16-byte rows assumed)
   const int gdt = is_split(dtype) ? MEC_DTYPE_BF16 : dtype;  // (block_grid: no special tiles for the pairs)
-  const bool small = gdt == MEC_DTYPE_F32 && f32_small_bwd_tiles(n, d, L.bs, cus);
+  const bool small = gdt == MEC_DTYPE_F32 ? f32_small_bwd_tiles(n, d, L.bs, cus) : small16_tiles(n, dtype);
   bool w384 = false;
   const BlockGrid bg = block_grid(d, gdt, sides, L.bs, L.nb, L.ldt, cus, fwd_tile_dims(gdt, true, small),
                                   con_tile_dims(gdt, small), &w384);
@@ -918,7 +934,7 @@ struct DetPartials {
 };
 template <typename T>
 static int sumexp_det_run(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int D, bool lit,
-                          bool normalize, bool vec, float c, float* workspace, const float* scl, int tiles_m,
+                          bool normalize, bool vec, bool small, float c, float* workspace, const float* scl, int tiles_m,
                           int tiles_n, hipStream_t s, DetPartials* dp) {
   const int N = (int)n;
   float* rowpart = workspace + det_partials_offset(n);
@@ -930,12 +946,21 @@ static int sumexp_det_run(const void* x, int64_t ldx, const void* y, int64_t ldy
   // workgroups and two tiles (pairs 4999 x 640: forward 119 -> 87 us).  A rule
   // on the tile counts alone, so that the order of the sums is the same on any
   // device.
-  if (FwdTile<T, true>::BM == 256 && vec && tiles_n > DET_Q && P * ((tiles_n + 1) / 2) <= 256) Q = (tiles_n + 1) / 2;
+  if (FwdTile<T, true>::BM == 256 && vec && !small && tiles_n > DET_Q && P * ((tiles_n + 1) / 2) <= 256) Q = (tiles_n + 1) / 2;
   const unsigned sum_grid = (unsigned)((n + 255) / 256);
   auto run = [&](auto lit_c, auto norm_c, auto vec_c) {
     constexpr bool LIT = decltype(lit_c)::value, NORM = decltype(norm_c)::value, VEC = decltype(vec_c)::value;
+    if constexpr (Is16<T>::value && VEC) {
+      if (small) {
+        if constexpr (!IsSplit<T>::value || !NORM)
+          k_sumexp_det<T, LIT, NORM, VEC, true><<<(unsigned)(P * Q), GemmTile<T, VEC, true>::NT, 0, s>>>(
+              (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace + WS_RX * n, workspace + WS_RY * n, rowpart,
+              colpart, tiles_m, tiles_n, P, Q, scl);
+      }
+    }
     if constexpr (!IsSplit<T>::value || (VEC && !NORM)) {
-      k_sumexp_det<T, LIT, NORM, VEC><<<(unsigned)(P * Q), FwdTile<T, VEC>::NT, 0, s>>>(
+      if (!small || !VEC || !Is16<T>::value)
+        k_sumexp_det<T, LIT, NORM, VEC><<<(unsigned)(P * Q), FwdTile<T, VEC>::NT, 0, s>>>(
           (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace + WS_RX * n, workspace + WS_RY * n, rowpart,
           colpart, tiles_m, tiles_n, P, Q, scl);
       if (dp)
@@ -968,6 +993,7 @@ static int sumexp_run(const void* x, int64_t ldx, const void* y, int64_t ldy, in
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   const float c = (float)(1.4426950408889634 / (double)temperature);
+  const int sdtype = dtype;  // as asked for
   // split modes: the bf16 sums over the copies (K = terms * dp) that mec_prepass
   // wrote, already normalized when normalize is set
   GemmOperands g{x, ldx, y, ldy, d, dtype};
@@ -977,8 +1003,10 @@ static int sumexp_run(const void* x, int64_t ldx, const void* y, int64_t ldy, in
   }
   if (is_pairs(dtype)) {
     const PairRows pr = pair_rows(workspace, n, d);
-    const int tiles = (int)((n + 255) / 256), dk = 2 * pr.dp;
-    return sumexp_det_run<F16S>(pr.a, dk, pr.b, dk, n, dk, is_lit(mode), false, true, c, workspace, pr.scl, tiles,
+    const bool small = small16_tiles(n, dtype);
+    const int bm = fwd_tile_dims(dtype, true, small).bm;
+    const int tiles = (int)((n + bm - 1) / bm), dk = 2 * pr.dp;
+    return sumexp_det_run<F16S>(pr.a, dk, pr.b, dk, n, dk, is_lit(mode), false, true, small, c, workspace, pr.scl, tiles,
                                 tiles, s, dp);
   }
   x = g.x, ldx = g.ldx, y = g.y, ldy = g.ldy, d = g.d, dtype = g.dtype;
@@ -997,14 +1025,14 @@ static int sumexp_run(const void* x, int64_t ldx, const void* y, int64_t ldy, in
     rc = compute_units(&cus);
     if (rc) return rc;
   }
-  const bool small = dtype == MEC_DTYPE_F32 && vec && !det && f32_small_fwd_tiles(n, d, cus);
+  const bool small = vec && (dtype == MEC_DTYPE_F32 ? !det && f32_small_fwd_tiles(n, d, cus) : small16_tiles(n, sdtype));
   const TileDims td = fwd_tile_dims(dtype, vec, small);
   const int tiles_m = (int)((n + td.bm - 1) / td.bm), tiles_n = (int)((n + td.bn - 1) / td.bn);
   const int64_t nwg = (int64_t)tiles_m * tiles_n;
   if (nwg > 0x7fffffff) return fail(MEC_ERR_UNSUPPORTED, "forward grid too large");
   const bool lit = is_lit(mode);
   if (det) {
-    DISPATCH_DTYPE(dtype, T, rc = sumexp_det_run<T>(x, ldx, y, ldy, n, D, lit, normalize != 0, vec, c, workspace,
+    DISPATCH_DTYPE(dtype, T, rc = sumexp_det_run<T>(x, ldx, y, ldy, n, D, lit, normalize != 0, vec, small, c, workspace,
                                                     nullptr, tiles_m, tiles_n, s, dp));
     return rc;
   }
@@ -1012,7 +1040,7 @@ static int sumexp_run(const void* x, int64_t ldx, const void* y, int64_t ldy, in
   DISPATCH_DTYPE(dtype, T, DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(vec, VEC, {
     if constexpr (!FwdChain<T, VEC, NORM>::value) {
       if (small) {
-        if constexpr (std::is_same<T, float>::value && VEC)
+        if constexpr (VEC)
           k_sumexp<T, LIT, NORM, VEC, true><<<grid, GemmTile<T, VEC, true>::NT, 0, s>>>(
               (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace, tiles_m, tiles_n);
       } else {
@@ -1196,7 +1224,9 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
   const GemmOperands go = split ? split_operands(workspace, n, d, dtype) : GemmOperands{x, ldx, y, ldy, d, dtype};
   const bool vec = pairs || vec_ok(go.x, go.ldx, go.y, go.ldy, go.d, go.dtype);
   if (split && !vec) return fail(MEC_ERR_UNSUPPORTED, "split operands beyond the direct-load range");
-  const bool small = dtype == MEC_DTYPE_F32 && vec && f32_small_bwd_tiles(n, d, bs, cus);
+  // (16-bit: of the contractions; the gradient-matrix tiles too where the rows allow)
+  const bool small16 = small16_tiles(n, dtype);
+  const bool small = dtype == MEC_DTYPE_F32 ? vec && f32_small_bwd_tiles(n, d, bs, cus) : small16;
   bool w384 = false;  // 16-bit contractions in 256 x 384 tiles
   BlockGrid bg = block_grid(d, dtype, a.sides(), bs, nb, L.ldt, cus, fwd_tile_dims(dtype, vec, small),
                             con_tile_dims(dtype, small), &w384);
@@ -1297,13 +1327,17 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
     const PairRows pr = pair_rows(workspace, n, d);
     const int dk = 2 * pr.dp;
     if (grid_c > 0) {
-      k_grad_contract<T><<<(unsigned)grid_c, ConTileX<T>::NT, 0, s>>>(N, D, gb, bg, sp_c, acc_x, acc_y);
+      if (small16)
+        k_grad_contract<T, false, false, true><<<(unsigned)grid_c, 256, 0, s>>>(N, D, gb, bg, sp_c, acc_x, acc_y);
+      else
+        k_grad_contract<T><<<(unsigned)grid_c, ConTileX<T>::NT, 0, s>>>(N, D, gb, bg, sp_c, acc_x, acc_y);
       rc = check_launch("grad_contract");
     }
     if (!rc && grid > 0) {
-      DISPATCH_BOOL(lit, LIT,
-          k_grad_g_chain<T, LIT, false><<<(unsigned)(grid < cus ? grid : cus), FwdTile<T, true>::NT, 0, s>>>(
-              (const T*)pr.a, dk, (const T*)pr.b, dk, N, dk, dk, c, workspace, gb, bg, sp_g));
+      const unsigned wgs = (unsigned)(grid < cus * (small16 ? 2 : 1) ? grid : cus * (small16 ? 2 : 1));
+      DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(small16, SM,
+          k_grad_g_chain<T, LIT, false, false, SM><<<wgs, GemmTile<T, true, SM>::NT, 0, s>>>(
+              (const T*)pr.a, dk, (const T*)pr.b, dk, N, dk, dk, c, workspace, gb, bg, sp_g)));
       rc = check_launch("grad_step");
     }
     return rc;
@@ -1315,15 +1349,19 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
     const int DK = (int)go.d;
     DISPATCH_BOOL(x3, X3, {
       if (grid_c > 0) {
-        DISPATCH_BOOL(w384, W, k_grad_contract<T, X3, W><<<(unsigned)grid_c, ConTileX<T>::NT, 0, s>>>(
-                                   N, D, gb, bg, sp_c, acc_x, acc_y));
+        if (!X3 && small16)
+          k_grad_contract<T, false, false, true><<<(unsigned)grid_c, 256, 0, s>>>(N, D, gb, bg, sp_c, acc_x, acc_y);
+        else
+          DISPATCH_BOOL(w384, W, k_grad_contract<T, X3, W><<<(unsigned)grid_c, ConTileX<T>::NT, 0, s>>>(
+                                     N, D, gb, bg, sp_c, acc_x, acc_y));
         rc = check_launch("grad_contract");
       }
       if (!rc && grid > 0) {
         // (the copies are already normalized: no norm scaling in the tiles; chained tiles)
-        DISPATCH_BOOL(lit, LIT,
-            k_grad_g_chain<T, LIT, false, X3><<<(unsigned)(grid < cus ? grid : cus), FwdTile<T, true>::NT, 0, s>>>(
-                (const T*)go.x, go.ldx, (const T*)go.y, go.ldy, N, DK, DK, c, workspace, gb, bg, sp_g));
+        const unsigned wgs = (unsigned)(grid < cus * (small16 ? 2 : 1) ? grid : cus * (small16 ? 2 : 1));
+        DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(!X3 && small16, SM,
+            k_grad_g_chain<T, LIT, false, X3, SM && !X3><<<wgs, GemmTile<T, true, SM && !X3>::NT, 0, s>>>(
+                (const T*)go.x, go.ldx, (const T*)go.y, go.ldy, N, DK, DK, c, workspace, gb, bg, sp_g)));
       }
     });
     if (rc) return rc;
@@ -1332,8 +1370,11 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
   DISPATCH_DTYPE(dtype, T, {
     if (grid_c > 0) {
       if constexpr (Is16<T>::value) {
-        DISPATCH_BOOL(w384, W, k_grad_contract<T, false, W><<<(unsigned)grid_c, ConTileX<T>::NT, 0, s>>>(
-                                   N, D, gb, bg, sp_c, acc_x, acc_y));
+        if (small16)
+          k_grad_contract<T, false, false, true><<<(unsigned)grid_c, 256, 0, s>>>(N, D, gb, bg, sp_c, acc_x, acc_y);
+        else
+          DISPATCH_BOOL(w384, W, k_grad_contract<T, false, W><<<(unsigned)grid_c, ConTileX<T>::NT, 0, s>>>(
+                                     N, D, gb, bg, sp_c, acc_x, acc_y));
         rc = check_launch("grad_contract");
       }
     }
@@ -1342,9 +1383,14 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
         if (vec && !normalize) {
           // direct-to-LDS tiles: persistent workgroups, one per CU, chained tiles
           // (the normalising epilogue would spill registers in the tile loop)
-          DISPATCH_BOOL(lit, LIT,
-              k_grad_g_chain<T, LIT, false><<<(unsigned)(grid < cus ? grid : cus), FwdTile<T, true>::NT, 0, s>>>(
-                  (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace, gb, bg, sp_g));
+          const unsigned wgs = (unsigned)(grid < cus * (small16 ? 2 : 1) ? grid : cus * (small16 ? 2 : 1));
+          DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(small16, SM,
+              k_grad_g_chain<T, LIT, false, false, SM><<<wgs, GemmTile<T, true, SM>::NT, 0, s>>>(
+                  (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace, gb, bg, sp_g)));
+        } else if (vec && small16) {
+          DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(normalize, NORM,
+              k_grad_step<T, LIT, NORM, true, false, true><<<(unsigned)grid, GemmTile<T, true, true>::NT, 0, s>>>(
+                  (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace, gb, bg, sp_g, acc_x, acc_y)));
         } else {
           DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(vec, VEC,
               k_grad_step<T, LIT, NORM, VEC><<<(unsigned)grid, FwdTile<T, VEC>::NT, 0, s>>>(

@@ -112,8 +112,8 @@ struct Geo {
   static __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
   static constexpr int MPB = KIND == K_F32 ? 4 : 1;    // MFMAs per block and k-step
   static constexpr bool TA = TA_;                      // A stored k-row-major
-  static_assert(!TA || (ESZ == 2 ? (BM == 256 || BM == 512) : (BM == 64 || BM == 128)),
-                "transposed A: 16-bit with 512- or 1024-byte k-rows, fp32 with 256- or 512-byte k-rows");
+  static_assert(!TA || (ESZ == 2 ? (BM == 256 || BM == 512 || (GB_ && BM == 128)) : (BM == 64 || BM == 128)),
+                "transposed A: 16-bit with 512- or 1024-byte k-rows (blocked: any), fp32 with 256- or 512-byte k-rows");
   static constexpr int TKPB = TA ? 1024 / (BM * ESZ) : 1;  // transposed A: k-rows per 1 KB load block
   // B stored k-row-major (fp32): 0 no, 1 with 16-byte lanes, 2 with 4-byte lanes
   static constexpr int TB = TB_;

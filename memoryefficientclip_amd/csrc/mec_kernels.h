@@ -199,6 +199,11 @@ template <typename T, bool VEC, bool SMALL> struct GemmTileSel { using type = Fw
 template <> struct GemmTileSel<float, true, true> {
   using type = TileD<64, 64, false, 2, 2, gdma::K_F32, 2, false, false, 0, SMALL_STAGES>;
 };
+// 16-bit at a small N (small16_n): 128 x 128 tiles of 2 x 2 waves, 64 KB of LDS,
+// two workgroups per CU
+template <typename T> struct GemmTileSel<T, true, true> {
+  using type = TileD<128, 128, false, 2, 2, kind16<T>(), 2, false, false, 0, 2, 1, IsSplit<T>::value>;
+};
 template <typename T, bool VEC, bool SMALL> using GemmTile = typename GemmTileSel<T, VEC, SMALL>::type;
 // Contractions.  fp32 stores each gradient-matrix block once, row-major and
 // scaled by both norms (H = diag(rx) G' diag(ry)), and runs the contractions
@@ -234,6 +239,8 @@ template <typename T, bool VEC> struct ConTileSel<T, VEC, true> {
   using ny = TileD<512, 128, false, 4, 2, kind16<T>(), 2, true>;
   using wx = TileD<256, 384, true, 2, 4, kind16<T>(), 4, true, true>;
   using wy = TileD<256, 384, false, 2, 4, kind16<T>(), 4, true, true>;
+  using sx = TileD<128, 128, true, 2, 2, kind16<T>(), 2, true>;  // (small16_n)
+  using sy = TileD<128, 128, false, 2, 2, kind16<T>(), 2, true>;
 };
 // (split pairs: 256 x 256, three A stages; a chunk of them has 1.5 times the MFMAs)
 template <bool VEC> struct ConTileSel<F16S, VEC, true> {
@@ -243,6 +250,8 @@ template <bool VEC> struct ConTileSel<F16S, VEC, true> {
   using ny = y;
   using wx = x;
   using wy = y;
+  using sx = TileD<128, 128, true, 2, 2, gdma::K_F16, 2, true, false, 0, 2, 1, true>;
+  using sy = TileD<128, 128, false, 2, 2, gdma::K_F16, 2, true, false, 0, 2, 1, true>;
 };
 template <typename T, bool VEC = true> using ConTileX = typename ConTileSel<T, VEC>::x;
 template <typename T, bool VEC = true> using ConTileY = typename ConTileSel<T, VEC>::y;
@@ -281,8 +290,9 @@ __device__ __forceinline__ float exp_mul(float c, const float* __restrict__ scl)
 
 // workgroups per CU the launch bounds promise (the 16-bit direct-load tiles
 // use 96 KB of LDS or more: one per CU)
-template <typename T, bool VEC> struct Occ {
-  static constexpr int fwd = Is16<T>::value ? (VEC ? 1 : 2) : 2, bwd = Is16<T>::value ? (VEC ? 1 : 2) : 2;
+// (SMALL: two)
+template <typename T, bool VEC, bool SMALL = false> struct Occ {
+  static constexpr int fwd = Is16<T>::value && VEC && !SMALL ? 1 : 2, bwd = fwd;
 };
 
 // Operand of a tile core from a typed pointer (the 16-bit cores address bits)
@@ -451,7 +461,7 @@ template <typename T, bool VEC, bool NORM> struct FwdChain {
 // (XCD-grouped order).  The chain-eligible 16-bit tiles (FwdChain) run
 // k_sumexp_det instead.
 template <typename T, bool LIT, bool NORM, bool VEC, bool SMALL = false>
-__global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC>::fwd)) void k_sumexp(
+__global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>::fwd)) void k_sumexp(
     const T* __restrict__ X, int64_t ldx, const T* __restrict__ Y, int64_t ldy, int N, int D, int kmax, float c,
     float* __restrict__ ws, int tiles_m, int tiles_n) {
   using TL = GemmTile<T, VEC, SMALL>;
@@ -493,12 +503,12 @@ __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC>::fwd)) 
 // index in order.  Every sum is a fixed function of the inputs and of the
 // tile shape, E is computed once, and the partials take (DET_P + DET_Q) * N
 // floats of the workspace.
-template <typename T, bool LIT, bool NORM, bool VEC>
-__global__ __launch_bounds__((FwdTile<T, VEC>::NT), (Occ<T, VEC>::fwd)) void k_sumexp_det(
+template <typename T, bool LIT, bool NORM, bool VEC, bool SMALL = false>
+__global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>::fwd)) void k_sumexp_det(
     const T* __restrict__ X, int64_t ldx, const T* __restrict__ Y, int64_t ldy, int N, int D, int kmax, float c,
     const float* __restrict__ rx, const float* __restrict__ ry, float* __restrict__ rowpart,
     float* __restrict__ colpart, int tiles_m, int tiles_n, int P, int Q, const float* __restrict__ scl) {
-  using TL = FwdTile<T, VEC>;
+  using TL = GemmTile<T, VEC, SMALL>;
   const float cm = exp_mul<T>(c, scl);
   static_assert(TL::FM == 2, "row reduction assumes 64-row wave sub-tiles");
   static_assert(TL::WN == 2, "two row-sum slots per row");
@@ -1068,19 +1078,23 @@ __device__ __forceinline__ void grad_contract_dispatch(int sub, int N, int D, co
 
 // 16-bit (and bf16x3) contractions of one pipeline step (the x side of
 // diagonal diag_c, then the y side).
-// W: the 256 x 384 tiles (ConTileSel::wx / wy; no narrow tiles)
-template <typename T, bool X3 = false, bool W = false>
-__global__ __launch_bounds__(ConTileX<T>::NT, 1) void k_grad_contract(int N, int D, GradBufs gb, BlockGrid bg,
+// W: the 256 x 384 tiles (ConTileSel::wx / wy; no narrow tiles); SM: the
+// 128 x 128 tiles (sx / sy), two workgroups per CU
+template <typename T, bool X3 = false, bool W = false, bool SM = false>
+__global__ __launch_bounds__(SM ? 256 : ConTileX<T>::NT, SM ? 2 : 1) void k_grad_contract(int N, int D, GradBufs gb, BlockGrid bg,
                                                                      StepPlan sp, float* __restrict__ acc_x,
                                                                      float* __restrict__ acc_y) {
   using Sel = ConTileSel<T, true>;
-  using TCX = typename std::conditional<W, typename Sel::wx, typename Sel::x>::type;
-  using TCY = typename std::conditional<W, typename Sel::wy, typename Sel::y>::type;
-  using TNX = typename std::conditional<W, TCX, typename Sel::nx>::type;
-  using TNY = typename std::conditional<W, TCY, typename Sel::ny>::type;
-  static_assert(TCX::BM == TCY::BM && TCX::BN == TCY::BN && TCX::NT == TCY::NT && TCX::NT == ConTileX<T>::NT,
+  using TCX = typename std::conditional<SM, typename Sel::sx,
+                                        typename std::conditional<W, typename Sel::wx, typename Sel::x>::type>::type;
+  using TCY = typename std::conditional<SM, typename Sel::sy,
+                                        typename std::conditional<W, typename Sel::wy, typename Sel::y>::type>::type;
+  using TNX = typename std::conditional<W || SM, TCX, typename Sel::nx>::type;
+  using TNY = typename std::conditional<W || SM, TCY, typename Sel::ny>::type;
+  static_assert(TCX::BM == TCY::BM && TCX::BN == TCY::BN && TCX::NT == TCY::NT &&
+                    TCX::NT == (SM ? 256 : ConTileX<T>::NT),
                 "one contraction tile shape and workgroup size");
-  static_assert(W || IsSplit<T>::value || (TNX::NT == TCX::NT && TNY::NT == TCX::NT && TNX::BM == 2 * TCX::BM && 2 * TNX::BN == TCX::BN),
+  static_assert(W || SM || IsSplit<T>::value || (TNX::NT == TCX::NT && TNY::NT == TCX::NT && TNX::BM == 2 * TCX::BM && 2 * TNX::BN == TCX::BN),
                 "narrow tiles: two row tiles high, half a feature tile wide");
   __shared__ __attribute__((aligned(1024)))
   char lds[CMax<CMax<TCX::LDS_BYTES, TCY::LDS_BYTES>::value, CMax<TNX::LDS_BYTES, TNY::LDS_BYTES>::value>::value];
@@ -1093,7 +1107,7 @@ __global__ __launch_bounds__(ConTileX<T>::NT, 1) void k_grad_contract(int N, int
 // selecting 16-byte or 4-byte load lanes for them).  X3: bf16 split operands
 // (K = 3 dp), G'^T written as hi and lo planes.
 template <typename T, bool LIT, bool NORM, bool VEC, bool X3 = false, bool SMALL = false>
-__global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC>::bwd)) void k_grad_step(
+__global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>::bwd)) void k_grad_step(
     const T* __restrict__ X, int64_t ldx, const T* __restrict__ Y, int64_t ldy, int N, int D, int kmax, float c,
     const float* __restrict__ ws, GradBufs gb, BlockGrid bg, StepPlan sp, float* __restrict__ acc_x,
     float* __restrict__ acc_y) {
@@ -1143,13 +1157,15 @@ __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC>::bwd)) 
 // (rx, ry, 1/R, 1/C) reach LDS by direct loads into one of two buffers,
 // issued right after the previous tile's first barrier (when every wave is
 // done with that buffer).
-template <typename T, bool LIT, bool NORM, bool X3 = false>
-__global__ __launch_bounds__((FwdTile<T, true>::NT), 1) void k_grad_g_chain(
+template <typename T, bool LIT, bool NORM, bool X3 = false, bool SMALL = false>
+__global__ __launch_bounds__((GemmTile<T, true, SMALL>::NT), (SMALL ? 2 : 1)) void k_grad_g_chain(
     const T* __restrict__ X, int64_t ldx, const T* __restrict__ Y, int64_t ldy, int N, int D, int kmax, float c,
     const float* __restrict__ ws, GradBufs gb, BlockGrid bg, StepPlan sp) {
-  using TL = FwdTile<T, true>;
+  using TL = GemmTile<T, true, SMALL>;
   static_assert(TL::CHAIN && GtOnly<T>::value, "chained 16-bit direct-to-LDS tiles");
-  static_assert(TL::BM == 256 && TL::BN == 256 && TL::NT == 512, "one 64-float quarter per vector load, 8 waves");
+  static_assert(TL::BM == TL::BN && TL::BM % 64 == 0, "64 floats per vector load");
+  constexpr int QN = TL::BM / 64, NW = TL::NT / 64;  // loads per vector, waves
+  static_assert(4 * QN % NW == 0, "the vector loads split evenly over the waves");
   enum { V_RX = 0, V_RY = 1, V_IR = 2, V_IC = 3 };
   __shared__ __attribute__((aligned(1024))) char lds[TL::LDS_BYTES];
   __shared__ __attribute__((aligned(16))) float s_vec[2][4][TL::BM];
@@ -1180,14 +1196,14 @@ __global__ __launch_bounds__((FwdTile<T, true>::NT), 1) void k_grad_g_chain(
   };
   auto op_a = [&](int i0) { return tile_op<TL>(X + (int64_t)i0 * ldx, ldx, min(N - i0, TL::BM), kmax); };
   auto op_b = [&](int j0) { return tile_op<TL>(Y + (int64_t)j0 * ldy, ldy, min(N - j0, TL::BN), kmax); };
-  // The vectors of tile (i0, j0) into s_vec[b]: load k (of 16) fills quarter
-  // k % 4 of vector k / 4; wave w issues loads w and w + 8.  Entries past N
+  // The vectors of tile (i0, j0) into s_vec[b]: load k (of 4 QN) fills 64
+  // floats, part k % QN of vector k / QN; wave w issues loads w, w + NW, ...  Entries past N
   // read as 0 (the buffer descriptor ends at N); 1/R and 1/C carry the
   // storage scale of G' in the epilogue.
   auto vec_loads = [&](int i0, int j0, int b) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int k = w + 8 * u, v = k >> 2, qr = k & 3;
+    for (int u = 0; u < 4 * QN / NW; ++u) {
+      const int k = w + NW * u, v = k / QN, qr = k % QN;
       const bool need = v == V_IR || (v == V_IC && !LIT) || ((v == V_RX || v == V_RY) && NORM);
       if (!need) continue;
       const int slot = v == V_RX ? WS_RX : v == V_RY ? WS_RY : v == V_IR ? WS_INV_ROW : WS_INV_COL;

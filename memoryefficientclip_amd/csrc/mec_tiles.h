@@ -73,17 +73,31 @@ inline bool f32_small_bwd(int64_t n, int64_t d, int64_t bs, int cus) {
   const int64_t g = ((n + 127) / 128) * ((bs + 127) / 128);
   return g * d <= ((int64_t)1 << 17) || round_fill(g, cus) < 0.9;
 }
+// 16-bit (and pairs) problems whose 128 x 128 grid is at most two tiles per CU
+// of a 256-CU device (n <= 2816; pairs, three products a tile, n <= 2560) run
+// 128 x 128 tiles, two workgroups per CU, throughout: of 256 x 256 tiles they
+// have 16 (n = 1024) to 121 (n = 2816), and each one's k-loop waits for its
+// loads.  Measured, GPU time of a CLIP step, 256 x 256 -> 128 x 128: bf16 256 x
+// 512 63 -> 42 us, 1024 x 512 73 -> 52, 2048 x 768 94 -> 72, 2500 x 768 104 -> 90,
+// 2816 x 512 88 -> 84, but 3072 x 768 112 -> 133; pairs 2048 x 1152 234 -> 177,
+// 2500 x 512 151 -> 146, but 2816 x 1024 256 -> 274.
+inline bool small16_n(int64_t n, int dtype) {
+  const int64_t t = (n + 127) / 128;
+  return t * t < (dtype == kDtypePairs ? 401 : 512);
+}
 // forward sums and gradient-matrix tiles (x rows x y rows)
 inline TileDims fwd_tile_dims(int dtype, bool vec, bool small = false) {
-  if (dtype == kDtypeX3 || dtype == kDtypeF32B || dtype == kDtypePairs) return {256, 256};
+  if (dtype == kDtypeX3) return {256, 256};
+  if (dtype == kDtypeF32B || dtype == kDtypePairs) return small ? TileDims{128, 128} : TileDims{256, 256};
   if (dtype == kDtypeF32 && vec && small) return {64, 64};
+  if (dtype != kDtypeF32 && vec && small) return {128, 128};
   if (dtype == kDtypeF32 || !vec) return {128, 128};
   return {256, 256};
 }
 // contraction tiles (output rows x feature columns)
 inline TileDims con_tile_dims(int dtype, bool small = false) {
   if (dtype == kDtypeF32) return small ? TileDims{64, 64} : TileDims{128, 128};
-  return {256, 256};
+  return small ? TileDims{128, 128} : TileDims{256, 256};
 }
 // contractions run in their own kernel (k_grad_contract) rather than inside k_grad_step
 inline bool separate_contractions(int dtype) { return dtype != kDtypeF32; }

@@ -588,6 +588,7 @@ def test_pairs_sizes_and_rule(monkeypatch):
         assert lib.mec_product_dtype(32768, 1152, dt) == dt
     assert lib.mec_product_dtype(32768, 1152, 0) == P and lib.mec_product_dtype(2048, 512, 0) == 0
     assert lib.mec_product_dtype(2049, 3, 0) == P
+    assert lib.mec_product_dtype(2048, 1152, 0) == P and lib.mec_product_dtype(1300, 1500, 0) == 0
     assert lib.mec_product_dtype(10, 3, x3) == P
     for dt in (0, x3):
         assert lib.mec_product_dtype((1 << 20) + 1, 1152, dt) == dt
@@ -598,3 +599,22 @@ def test_pairs_sizes_and_rule(monkeypatch):
     assert lib.mec_product_dtype(1, 1, 0) == P
     monkeypatch.setenv("MEC_F32_PAIRS", "0")
     assert lib.mec_product_dtype(10, 3, x3) == x3
+
+
+def test_small_16bit_tile_rule(monkeypatch):
+    # 128 x 128 tiles while their grid is at most two per CU of 256 (n <= 2816;
+    # pairs n <= 2560; never bf16x3), unless contraction tiles are forced
+    for v in ("MEC_16BIT_SMALL_TILES", "MEC_NARROW_CONTRACT", "MEC_WIDE_CONTRACT"):
+        monkeypatch.delenv(v, raising=False)
+
+    def rows(n, dt):
+        return _lib.backward_plan(n, 512, dt, compute_units=256).contract_tile_rows
+
+    for dt in (1, 2, 4):
+        assert rows(1, dt) == rows(2816, dt) == 128 and rows(2817, dt) == 256
+    assert rows(2560, _lib.DTYPE_F32_PAIRS) == 128 and rows(2561, _lib.DTYPE_F32_PAIRS) == 256
+    assert rows(1024, 3) == 256
+    monkeypatch.setenv("MEC_WIDE_CONTRACT", "0")
+    assert rows(1024, 1) == 256
+    monkeypatch.setenv("MEC_16BIT_SMALL_TILES", "1")
+    assert rows(4096, 1) == 128
