@@ -199,6 +199,15 @@ int64_t mec_workspace_floats_mode(int64_t n, int64_t d, int dtype, int mode);
  * is returned as it is).  Host-only.  No counterpart in the reference. */
 int mec_product_dtype(int64_t n, int64_t d, int dtype);
 
+/* mec_product_dtype, mec_keep_exp_supported (asked only when `keep` is not 0)
+ * and mec_workspace_floats_mode for these inputs in one call: bits 0-2 the
+ * dtype code to run with, bit 3 set when MEC_FLAG_KEEP_EXP is to be passed, the
+ * rest the workspace's floats; < 0 on bad arguments.  Host-only (at small n a
+ * caller's host time is a large part of a step).  No counterpart in the
+ * reference. */
+int64_t mec_forward_plan(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
+                         int keep);
+
 /* 1 if mec_forward / mec_backward accept MEC_FLAG_KEEP_EXP for these inputs
  * (MEC_DTYPE_F32, n <= MEC_KEEP_EXP_MAX_N, 16-byte aligned rows: x and y
  * 16-byte aligned, d, ldx and ldy multiples of 4), else 0 (also for invalid

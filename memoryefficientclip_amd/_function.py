@@ -75,28 +75,16 @@ def _stream(index: int) -> int:
     return torch.cuda.current_stream(index).cuda_stream
 
 
-class _on_device:
-    """Make device `index` current for the C-ABI calls (which launch on the
-    current device), restoring the previous one; nothing to do, and no
-    device switch, in the common case where it already is."""
+_raw_alloc = getattr(torch._C, "_cuda_cudaCachingAllocator_raw_alloc", None)
 
-    __slots__ = ("index", "prev")
 
-    def __init__(self, index: int):
-        self.index = index
-        self.prev = -1
-
-    def __enter__(self):
-        cur = torch.cuda.current_device()
-        if cur != self.index:
-            self.prev = cur
-            torch.cuda.set_device(self.index)
-        return self
-
-    def __exit__(self, *exc):
-        if self.prev >= 0:
-            torch.cuda.set_device(self.prev)
-        return False
+def _alloc(nbytes: int, index: int) -> int:
+    """Stream-ordered scratch from PyTorch's caching allocator on the current
+    device `index` (torch.cuda.caching_allocator_alloc without its stream and
+    device objects, about 2 us of host time)."""
+    if _raw_alloc is not None and _raw_stream is not None:
+        return _raw_alloc(nbytes, _raw_stream(index))
+    return torch.cuda.caching_allocator_alloc(nbytes, index, torch.cuda.current_stream(index))
 
 
 def refuse_graph_capture() -> None:
@@ -137,26 +125,38 @@ def forward(ctx, x: torch.Tensor, y: torch.Tensor, temperature: float, mode: int
     y, ldy = _rows(y)
     n, d = x.shape
     dev = x.device
-    di = x.get_device()
-    dt = compute_dtype(x.dtype)
+    di = dev.index
     lib = _lib.load()
-    dt = lib.mec_product_dtype(n, d, dt)
-    # small fp32 problems keep the similarity matrix for the backward (three
-    # launches per step instead of six, no gradient scratch), when a gradient
-    # will be asked for
-    if (ctx.needs_input_grad[0] or ctx.needs_input_grad[1]) and \
-            lib.mec_keep_exp_supported(x.data_ptr(), ldx, y.data_ptr(), ldy, n, d, dt):
+    px, py = x.data_ptr(), y.data_ptr()
+    need = ctx.needs_input_grad
+    # the dtype code, the workspace, and whether a small fp32 problem keeps the
+    # similarity matrix for the backward (three launches per step, no gradient
+    # scratch), which it does when a gradient will be asked for
+    plan = lib.mec_forward_plan(px, ldx, py, ldy, n, d, compute_dtype(x.dtype), int(need[0] or need[1]))
+    if plan < 0:
+        raise RuntimeError(f"MemoryEfficientCLIP: unsupported problem size {n} x {d}")
+    dt = plan & 7
+    if plan & 8:
         mode |= _lib.FLAG_KEEP_EXP
-    ws = torch.empty(lib.mec_workspace_floats_mode(n, d, dt, mode), dtype=torch.float32, device=dev)
+    ws = torch.empty(plan >> 4, dtype=torch.float32, device=dev)
     loss = torch.empty((), dtype=torch.float32, device=dev)
     # under torch.use_deterministic_algorithms(True) the forward sums are
     # formed without atomics (the backward is deterministic either way)
     fmode = mode | (_lib.FLAG_DETERMINISTIC if torch.are_deterministic_algorithms_enabled() else 0)
-    with _on_device(di):
-        _lib.call("mec_forward", x.data_ptr(), ldx, y.data_ptr(), ldy, n, d, dt, fmode, int(normalize),
-                  temperature, ws.data_ptr(), loss.data_ptr(), _stream(di))
+    # (the C-ABI calls launch on the current device)
+    cur = torch.cuda.current_device()
+    if cur != di:
+        torch.cuda.set_device(di)
+    try:
+        rc = lib.mec_forward(px, ldx, py, ldy, n, d, dt, fmode, normalize, temperature, ws.data_ptr(),
+                             loss.data_ptr(), _stream(di))
+    finally:
+        if cur != di:
+            torch.cuda.set_device(cur)
+    if rc:
+        raise _lib.error("mec_forward", rc)
     ctx.save_for_backward(x, y, ws)
-    ctx.mec = (ldx, ldy, n, d, dt, mode, bool(normalize), temperature,
+    ctx.mec = (ldx, ldy, n, d, dt, mode, int(normalize), temperature,
                math.sqrt(n / temperature) if stable else 1.0 / temperature)
     return loss
 
@@ -171,39 +171,49 @@ def backward(ctx, grad_output: torch.Tensor, need_x: bool, need_y: bool):
     if not (need_x or need_y):
         return None, None
     dev = x.device
-    di = x.get_device()
+    di = dev.index
     lib = _lib.load()
     go = grad_output
     if go.dtype != torch.float32 or go.device != dev or go.dim() != 0:
         go = go.detach().to(device=dev, dtype=torch.float32).reshape(())
-    acc_x = torch.empty((n, d), dtype=torch.float32, device=dev) if need_x else None
-    acc_y = torch.empty((n, d), dtype=torch.float32, device=dev) if need_y else None
-    if x.dtype == torch.float32:
-        dx, dy = acc_x, acc_y  # the post-pass runs in place
-    else:
-        dx = torch.empty((n, d), dtype=x.dtype, device=dev) if need_x else None
-        dy = torch.empty((n, d), dtype=y.dtype, device=dev) if need_y else None
+    dx = torch.empty((n, d), dtype=x.dtype, device=dev) if need_x else None
+    dy = torch.empty((n, d), dtype=x.dtype, device=dev) if need_y else None
+    pdx = dx.data_ptr() if need_x else None
+    pdy = dy.data_ptr() if need_y else None
     # The gradient scratch comes straight from PyTorch's caching allocator
     # (stream-ordered, like a tensor): the kernels write every byte of it
     # before reading it, so the NaN fill that torch.empty performs under
     # torch.use_deterministic_algorithms(True) (gigabytes at large N) would
-    # be wasted work.
-    sides = (_lib.SIDE_X if need_x else 0) | (_lib.SIDE_Y if need_y else 0)
-    nbytes = lib.mec_backward_scratch_bytes(n, d, dt, mode, sides)  # 0 with the kept exponentials
-
-    def ptr(t):
-        return None if t is None else t.data_ptr()
-
-    with _on_device(di):
-        scratch = torch.cuda.caching_allocator_alloc(nbytes, di, torch.cuda.current_stream(di)) if nbytes > 0 \
-            else None
-        try:
-            _lib.call("mec_backward", x.data_ptr(), ldx, y.data_ptr(), ldy, n, d, dt, mode, int(normalize),
-                      temperature, grad_scale, ws.data_ptr(), go.data_ptr(), scratch, nbytes,
-                      ptr(acc_x), ptr(acc_y), ptr(dx), ptr(dy), _stream(di))
-        finally:
-            if scratch is not None:
-                torch.cuda.caching_allocator_delete(scratch)
+    # be wasted work.  fp32 accumulates in the outputs (the post-pass runs in
+    # place); the 16-bit types' fp32 accumulators are the scratch's first part.
+    nbytes = off = 0
+    if not mode & _lib.FLAG_KEEP_EXP:
+        sides = (_lib.SIDE_X if need_x else 0) | (_lib.SIDE_Y if need_y else 0)
+        nbytes = lib.mec_backward_scratch_bytes(n, d, dt, mode, sides)
+        if x.dtype != torch.float32:
+            side = (4 * n * d + 255) & ~255
+            off = side * (int(need_x) + int(need_y))
+    cur = torch.cuda.current_device()
+    if cur != di:
+        torch.cuda.set_device(di)
+    scratch = None
+    try:
+        pax, pay = pdx, pdy
+        if nbytes + off > 0:
+            scratch = _alloc(nbytes + off, di)
+        if off:
+            pax = scratch if need_x else None
+            pay = scratch + (side if need_x else 0) if need_y else None
+        rc = lib.mec_backward(x.data_ptr(), ldx, y.data_ptr(), ldy, n, d, dt, mode, normalize, temperature,
+                              grad_scale, ws.data_ptr(), go.data_ptr(), None if scratch is None else scratch + off,
+                              nbytes, pax, pay, pdx, pdy, _stream(di))
+    finally:
+        if scratch is not None:
+            torch.cuda.caching_allocator_delete(scratch)
+        if cur != di:
+            torch.cuda.set_device(cur)
+    if rc:
+        raise _lib.error("mec_backward", rc)
     return dx, dy
 
 

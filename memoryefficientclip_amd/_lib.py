@@ -45,6 +45,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "mec_workspace_floats_for": (_i64, [_i64, _i64, _int]),
     "mec_workspace_floats_mode": (_i64, [_i64, _i64, _int, _int]),
     "mec_product_dtype": (_int, [_i64, _i64, _int]),
+    "mec_forward_plan": (_i64, [_vp, _i64, _vp, _i64, _i64, _i64, _int, _int]),
     "mec_keep_exp_supported": (_int, [_vp, _i64, _vp, _i64, _i64, _i64, _int]),
     "mec_grad_scratch_bytes": (_i64, [_i64, _i64, _int]),
     "mec_grad_scratch_bytes_for": (_i64, [_i64, _i64, _int, _int, _int]),
@@ -130,6 +131,11 @@ def backward_plan(n: int, d: int, dtype: int, mode: int = MODE_CLIP, sides: int 
 
 def last_error() -> str:
     return load().mec_last_error().decode()
+
+
+def error(name: str, code: int) -> MecError:
+    """The exception for status `code` of entry point `name` on this thread."""
+    return MecError(name, code, last_error())
 
 
 def call(name: str, *args) -> int:

@@ -780,6 +780,14 @@ int mec_product_dtype(int64_t n, int64_t d, int dtype) {
   return pairs_preferred(n, d, dtype) ? MEC_DTYPE_F32_PAIRS : dtype;
 }
 
+int64_t mec_forward_plan(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d, int dtype,
+                         int keep) {
+  dtype = mec_product_dtype(n, d, dtype);
+  if (n < 1 || n > max_n(dtype) || d < 1 || d > kMaxD || !known_dtype(dtype)) return -1;
+  const int flag = keep && keep_supported(x, ldx, y, ldy, n, d, dtype) ? MEC_FLAG_KEEP_EXP : 0;
+  return workspace_floats_mode(n, d, dtype, flag) << 4 | (flag ? 8 : 0) | dtype;
+}
+
 int mec_keep_exp_supported(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t n, int64_t d,
                            int dtype) {
   return keep_supported(x, ldx, y, ldy, n, d, dtype) ? 1 : 0;
@@ -804,6 +812,7 @@ int64_t mec_backward_scratch_bytes(int64_t n, int64_t d, int dtype, int mode, in
   const int64_t base = mec_grad_scratch_bytes_for(n, d, dtype, mode, sides);
   if (base <= 0 || keep_flag(mode)) return base;
   if (is_lit(mode)) sides &= kSideX;
+  if (!separate_contractions(dtype)) return base;
   const ConSplit cs = backward_split(n, d, dtype, sides, scratch_layout(n, d, dtype, sides), plan_units());
   return cs.ks > 1 ? align256(base) + parts_bytes(n, d, sides, cs.ks) : base;
 }

@@ -618,3 +618,23 @@ def test_small_16bit_tile_rule(monkeypatch):
     assert rows(1024, 1) == 256
     monkeypatch.setenv("MEC_16BIT_SMALL_TILES", "1")
     assert rows(4096, 1) == 128
+
+
+def test_forward_plan_is_the_separate_queries(monkeypatch):
+    # mec_forward_plan packs mec_product_dtype, mec_keep_exp_supported and
+    # mec_workspace_floats_mode
+    for v in ("MEC_F32_PAIRS", "MEC_F32_SMALL_TILES", "MEC_KEEP_EXP"):
+        monkeypatch.delenv(v, raising=False)
+    lib = _lib.load()
+    A = 1 << 20
+    for n, d, ld, dt in [(1, 1, 1, 0), (1000, 64, 64, 0), (1000, 64, 66, 0), (2048, 1152, 1152, 0), (5000, 512, 512, 0),
+                         (1024, 512, 512, 1), (4096, 768, 768, 2), (700, 96, 96, 3), (700, 96, 96, 4),
+                         ((1 << 20) + 1, 64, 64, 3)]:
+        for keep in (0, 1):
+            run = lib.mec_product_dtype(n, d, dt)
+            k = keep and lib.mec_keep_exp_supported(A, ld, A, ld, n, d, run)
+            floats = lib.mec_workspace_floats_mode(n, d, run, _lib.FLAG_KEEP_EXP if k else 0)
+            assert lib.mec_forward_plan(A, ld, A, ld, n, d, dt, keep) == floats << 4 | (8 if k else 0) | run
+    assert lib.mec_forward_plan(A, 64, A, 64, 1024, 64, 0, 1) & 8
+    for n, d, dt in [(0, 4, 0), (4, 0, 0), (4, 4, 5), ((1 << 22) + 1, 64, 1)]:
+        assert lib.mec_forward_plan(A, 64, A, 64, n, d, dt, 1) < 0
