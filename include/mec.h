@@ -123,10 +123,10 @@ extern "C" {
  * gradients are bitwise reproducible for the same inputs on the same device.
  * The backward is deterministic in either mode.  The similarity tiles are
  * still visited once (in P x Q blocks), with the partial sums combined in a
- * fixed order by a second, O(n) launch.  The 16-bit forward with 16-byte rows
- * and normalize = 0, and the forward of MEC_DTYPE_F32_BF16X3 /
- * MEC_DTYPE_F32_BF16 (on normalized copies), always run this way (chained
- * tiles; faster than the atomic forward there), with or without the flag. */
+ * fixed order by a second, O(n) launch.  The 16-bit forward with 16-byte rows, and the forward of
+ * MEC_DTYPE_F32_BF16X3 / MEC_DTYPE_F32_BF16 / MEC_DTYPE_F32_PAIRS (on copies
+ * in the workspace), always run this way (chained tiles; faster than the atomic
+ * forward there), with or without the flag. */
 #define MEC_FLAG_DETERMINISTIC 0x100
 /* OR into `mode` of mec_forward and of the matching mec_grad / mec_backward
  * (mec_backward_noalloc) for a small problem that mec_keep_exp_supported

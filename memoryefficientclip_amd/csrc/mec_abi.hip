@@ -748,7 +748,10 @@ bool pairs_preferred(int64_t n, int64_t d, int dtype) {
   }
   if (dtype == MEC_DTYPE_F32_BF16X3) return true;
   if (small_tiles_env() >= 0) return false;  // (the fp32 tiles are asked for)
-  return n > MEC_KEEP_EXP_MAX_N || (n >= 1400 && n * n * d >= 2500000000LL);
+  // (from n = 2049 to 4096 both are bound by the host at a small d, where the fp32
+  // kernels have two launches fewer: LiT 3757 x 64 134 us, pairs 142 us)
+  if (n > MEC_KEEP_EXP_MAX_N) return n > 4096 || n * n * d >= 1000000000LL;
+  return n >= 1400 && n * n * d >= 2500000000LL;
 }
 
 }  // namespace
@@ -1022,8 +1025,8 @@ static int sumexp_run(const void* x, int64_t ldx, const void* y, int64_t ldy, in
   const int N = (int)n, D = (int)d;
   const bool vec = vec_ok(x, ldx, y, ldy, d, dtype);
   // Deterministic sums on request, and always for the 16-bit direct-to-LDS
-  // tiles without the norm scaling (FwdChain), whose chained block walk is
-  // faster than the atomic forward.  They keep the default tile size.
+  // tiles (FwdChain), whose chained block walk is faster than the atomic
+  // forward.
   bool chain = false;
   DISPATCH_DTYPE(dtype, T, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(vec, VEC, {
     chain = FwdChain<T, VEC, NORM>::value;
@@ -1389,21 +1392,18 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
     }
     if (!rc && grid > 0) {
       if constexpr (Is16<T>::value) {
-        if (vec && !normalize) {
-          // direct-to-LDS tiles: persistent workgroups, one per CU, chained tiles
-          // (the normalising epilogue would spill registers in the tile loop)
+        if (vec) {
+          // direct-to-LDS tiles: persistent workgroups, chained tiles (with the norm
+          // scaling, unchained -> chained: 16384 x 1024 490 -> 472 us, 65536 x 768 1.68
+          // -> 1.57 ms per step with the transposes)
           const unsigned wgs = (unsigned)(grid < cus * (small16 ? 2 : 1) ? grid : cus * (small16 ? 2 : 1));
-          DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(small16, SM,
-              k_grad_g_chain<T, LIT, false, false, SM><<<wgs, GemmTile<T, true, SM>::NT, 0, s>>>(
-                  (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace, gb, bg, sp_g)));
-        } else if (vec && small16) {
-          DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(normalize, NORM,
-              k_grad_step<T, LIT, NORM, true, false, true><<<(unsigned)grid, GemmTile<T, true, true>::NT, 0, s>>>(
-                  (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace, gb, bg, sp_g, acc_x, acc_y)));
+          DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(small16, SM, DISPATCH_BOOL(normalize, NORM,
+              k_grad_g_chain<T, LIT, NORM, false, SM><<<wgs, GemmTile<T, true, SM>::NT, 0, s>>>(
+                  (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace, gb, bg, sp_g))));
         } else {
-          DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(vec, VEC,
-              k_grad_step<T, LIT, NORM, VEC><<<(unsigned)grid, FwdTile<T, VEC>::NT, 0, s>>>(
-                  (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace, gb, bg, sp_g, acc_x, acc_y))));
+          DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(normalize, NORM,
+              k_grad_step<T, LIT, NORM, false><<<(unsigned)grid, FwdTile<T, false>::NT, 0, s>>>(
+                  (const T*)x, ldx, (const T*)y, ldy, N, D, D, c, workspace, gb, bg, sp_g, acc_x, acc_y)));
         }
       } else if (small) {
         DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(normalize, NORM,

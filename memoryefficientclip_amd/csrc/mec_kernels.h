@@ -16,8 +16,8 @@
 //                       contractions without contending atomics
 //                       (clip_loss.py:127-156, lit_loss.py:123-148); fp32
 //                       runs both kinds of tile in this launch.
-//   k_grad_g_chain  the 16-bit gradient-matrix tiles of inputs already
-//                       normalized, chained in persistent workgroups.
+//   k_grad_g_chain  the 16-bit gradient-matrix tiles on 16-byte rows, chained
+//                       in persistent workgroups.
 //   k_grad_contract the 16-bit types' contractions of one pipeline step, in
 //                       a launch of their own with larger tiles (256 x 256,
 //                       or 256 x 384 where that takes fewer rounds, and
@@ -307,17 +307,16 @@ template <int A, int B> struct CMax { static constexpr int value = A > B ? A : B
 // E = exp2(S cm - c) of this wave's TM x TN accumulators (S scaled by rx_i ry_j
 // when NORM; cm = c, exp_mul of split pairs); rowv[bm * 16 + r] and colv[bn] collect this lane's partial row
 // and column sums.  MASK zeroes the diagonal and entries outside [0, N).
-// Eb (not null): every entry of the tile, masked ones as 0, is also stored at
-// Eb[row * ldE + column] (tile-relative; each 32-lane half writes 128 bytes
-// of one row); STORE_S stores the exponent's row-scaled similarity S_ij rx_i
-// there instead (unmasked), from which E is exp2(s c ry_j - c) as here.
-template <class TL, bool NORM, bool MASK, bool STORE_S = false>
+template <class TL, bool NORM, bool MASK>
 __device__ __forceinline__ void sumexp_epilogue(const f32x16 (&acc)[TL::FM][TL::FN], float cm, float c, int m0,
                                                 int n0, int N, const float* s_rx, const float* s_ry, float (&rowv)[TL::FM * 16],
-                                                float (&colv)[TL::FN], float* __restrict__ Eb = nullptr,
-                                                int ldE = 0) {
+                                                float (&colv)[TL::FN]) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w / TL::WN, wn = w % TL::WN;
-  float sv[STORE_S ? TL::FN : 1][STORE_S ? TL::FM * 16 : 1];  // STORE_S: the similarities to store
+  // row of accumulator (bm, r): mb + 32 bm + 8 (r / 4) + r % 4, so that the scales
+  // are read with one base and immediate offsets (as separate indices they were
+  // hoisted out of the chained tile loop, 32 registers that spilled)
+  const int mb = wm * TL::TM + 4 * (lane >> 5);
+  const float* rxb = s_rx + mb;
 #pragma unroll
   for (int k = 0; k < TL::FM * 16; ++k) rowv[k] = 0.f;
 #pragma unroll
@@ -330,35 +329,16 @@ __device__ __forceinline__ void sumexp_epilogue(const f32x16 (&acc)[TL::FM][TL::
     for (int bm = 0; bm < TL::FM; ++bm) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int ml = wm * TL::TM + bm * 32 + acc_row(r, lane);
-        const int i = m0 + ml;
-        const float sc = NORM ? acc[bm][bn][r] * s_rx[ml] : acc[bm][bn][r];
+        const int mo = bm * 32 + 8 * (r >> 2) + (r & 3);
+        const int i = m0 + mb + mo;
+        const float sc = NORM ? acc[bm][bn][r] * rxb[mo] : acc[bm][bn][r];
         float e = fast_exp2(fmaf(sc, cy, -c));
         if (MASK) e = (i < N && j < N && i != j) ? e : 0.f;
-        if constexpr (STORE_S)
-          sv[bn][bm * 16 + r] = sc;
-        else if (Eb)
-          Eb[(int64_t)ml * ldE + nl] = e;
         rowv[bm * 16 + r] += e;
         cs += e;
       }
     }
     colv[bn] = cs;
-  }
-  // STORE_S: the stores after every LDS read of the scales (a store through a
-  // generic pointer may alias LDS, so each store interleaved with the reads
-  // made the next read wait for it), at device scope (the next launch reads
-  // them)
-  if constexpr (STORE_S) {
-#pragma unroll
-    for (int bn = 0; bn < TL::FN; ++bn)
-#pragma unroll
-      for (int bm = 0; bm < TL::FM; ++bm)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          store_device(&Eb[(int64_t)(wm * TL::TM + bm * 32 + acc_row(r, lane)) * ldE + wn * TL::TN + bn * 32 +
-                           (lane & 31)],
-                       sv[bn][bm * 16 + r]);
   }
 }
 
@@ -372,12 +352,15 @@ __device__ __forceinline__ void lds_barrier() {
 
 // Row and column sums of E over one tile: thread t gets the sums of row m0 + t
 // (rs) and column n0 + t (cs), which sums_flush adds into ws.  rxv / ryv:
-// 1/|x| of row m0 + t and 1/|y| of column n0 + t (NORM).
+// 1/|x| of row m0 + t and 1/|y| of column n0 + t (NORM).  STORE_S: the exponent's
+// row-scaled similarity S_ij rx_i of every entry (unmasked) is also stored at
+// Sb[row * ldS + column] (tile-relative; each 32-lane half writes 128 bytes of
+// one row), from which E is exp2(s c ry_j - c) as here.
 template <class TL, bool LIT, bool NORM, bool STORE_S = false>
 __device__ __forceinline__ void sumexp_tile(const f32x16 (&acc)[TL::FM][TL::FN], float c, int m0, int n0, int N,
                                             float rxv, float ryv, float* s_rx, float* s_ry, float* s_row,
-                                            float* s_col, float& rs_out, float& cs_out, float* __restrict__ Eb = nullptr,
-                                            int ldE = 0, bool active = true) {
+                                            float* s_col, float& rs_out, float& cs_out, float* __restrict__ Sb = nullptr,
+                                            int ldS = 0, bool active = true) {
   static_assert(TL::NT >= TL::BM && TL::NT >= TL::BN, "one row and one column per thread");
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, wm = w / TL::WN, wn = w % TL::WN;
   if (t < TL::BM) {
@@ -397,9 +380,26 @@ __device__ __forceinline__ void sumexp_tile(const f32x16 (&acc)[TL::FM][TL::FN],
     // interior tiles (no diagonal entry, no row or column beyond N) need no mask
     const bool diag = m0 < n0 + TL::BN && n0 < m0 + TL::BM;
     if (!diag && m0 + TL::BM <= N && n0 + TL::BN <= N)
-      sumexp_epilogue<TL, NORM, false, STORE_S>(acc, c, c, m0, n0, N, s_rx, s_ry, rowv, colv, Eb, ldE);
+      sumexp_epilogue<TL, NORM, false>(acc, c, c, m0, n0, N, s_rx, s_ry, rowv, colv);
     else
-      sumexp_epilogue<TL, NORM, true, STORE_S>(acc, c, c, m0, n0, N, s_rx, s_ry, rowv, colv, Eb, ldE);
+      sumexp_epilogue<TL, NORM, true>(acc, c, c, m0, n0, N, s_rx, s_ry, rowv, colv);
+    if constexpr (STORE_S) {
+      // every scale first, then the stores (a store through a generic pointer may
+      // alias LDS, so a store between the reads made the next read wait for it),
+      // at device scope (the next launch reads them)
+      const int mb = wm * TL::TM + 4 * (lane >> 5);
+      float sv[TL::FM * 16];
+#pragma unroll
+      for (int k = 0; k < TL::FM * 16; ++k)
+        sv[k] = NORM ? s_rx[mb + (k >> 4) * 32 + 8 * ((k & 15) >> 2) + (k & 3)] : 1.f;
+#pragma unroll
+      for (int bn = 0; bn < TL::FN; ++bn)
+#pragma unroll
+        for (int k = 0; k < TL::FM * 16; ++k)
+          store_device(&Sb[(int64_t)(mb + (k >> 4) * 32 + 8 * ((k & 15) >> 2) + (k & 3)) * ldS + wn * TL::TN + bn * 32 +
+                           (lane & 31)],
+                       NORM ? acc[k >> 4][bn][k & 15] * sv[k] : acc[k >> 4][bn][k & 15]);
+    }
     if constexpr (TL::FM == 1) {
       // one 32-row block: its 16 row sums padded to the 32 of the reduction
       float v[32];
@@ -443,22 +443,24 @@ __device__ __forceinline__ void sums_flush(float* __restrict__ ws, int m0, int n
     __hip_atomic_fetch_add(&ws[WS_COL_OFF * n64 + n0 + t], cs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Forward tiles that chain (FwdChain): the 16-bit direct-to-LDS tiles
-// without the norm scaling, which always take the deterministic forward's
-// block walk (k_sumexp_det) with chained tiles.  Measured: the 16-bit forward
-// (one workgroup per CU, nothing else to overlap its epilogue) is 7% faster
-// chained, and the block walk with its fixed-order sums another 2-7% faster
-// than chained tiles with atomic sums; fp32 (two workgroups per CU, one's
-// epilogue already overlaps the other's k-loop) was 4% slower chained; the
-// normalizing 16-bit epilogue spills registers in the chained loop, or is
-// slower when kept from spilling.
+// Forward tiles that chain (FwdChain): the 16-bit direct-to-LDS tiles, which
+// always take the deterministic forward's block walk (k_sumexp_det) with
+// chained tiles.  Measured: the 16-bit forward (one workgroup per CU, nothing
+// else to overlap its epilogue) is 7% faster chained, and the block walk with
+// its fixed-order sums another 2-7% faster than chained tiles with atomic sums;
+// fp32 (two workgroups per CU, one's epilogue already overlaps the other's
+// k-loop) was 4% slower chained.  With the norm scaling (bf16, unchained atomic
+// -> chained): 16384 x 1024 456 -> 446 us, 65536 x 768 5.64 -> 5.29 ms, 32768 x
+// 256 703 -> 578 us, 131072 x 128 8.83 -> 6.09 ms; its scales reach LDS by one
+// direct load per wave during the tile before.  (It spilled until the epilogue
+// addressed its rows from one base.)
 template <typename T, bool VEC, bool NORM> struct FwdChain {
-  static constexpr bool value = FwdTile<T, VEC>::CHAIN && Is16<T>::value && !NORM;
+  static constexpr bool value = FwdTile<T, VEC>::CHAIN && Is16<T>::value;
 };
 
 // Forward sums with relaxed atomics into ws (as the reference,
 // clip_loss.py:63-64): one tile per workgroup of the tiles_m x tiles_n grid
-// (XCD-grouped order).  The chain-eligible 16-bit tiles (FwdChain) run
+// (XCD-grouped order).  The 16-bit tiles on 16-byte rows (FwdChain) run
 // k_sumexp_det instead.
 template <typename T, bool LIT, bool NORM, bool VEC, bool SMALL = false>
 __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>::fwd)) void k_sumexp(
@@ -514,7 +516,10 @@ __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>:
   static_assert(TL::WN == 2, "two row-sum slots per row");
   static_assert(TL::NT >= TL::BM && TL::NT >= TL::BN, "one row and one column per thread");
   __shared__ __attribute__((aligned(1024))) char lds[TL::LDS_BYTES];
-  __shared__ float s_rx[TL::BM], s_ry[TL::BN], s_row[TL::WN][TL::BM], s_col[TL::WM][TL::BN];
+  // (row and column scales; chained tiles: the next tile's land in the other half)
+  constexpr int NV = FwdChain<T, VEC, NORM>::value && NORM ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) float s_vec[NV][TL::BM + TL::BN];
+  __shared__ float s_row[TL::WN][TL::BM], s_col[TL::WM][TL::BN];
   __shared__ __attribute__((aligned(16))) float s_cold[TL::BN];
   const int nbm = tiles_m / P, rbm = tiles_m % P, nbn = tiles_n / Q, rbn = tiles_n % Q;
   // Workgroup -> block.  Even blocks (no remainder tiles): XCD x = blockIdx % 8
@@ -556,7 +561,9 @@ __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>:
   // tile (tm, tn) of the block: its sums into the slots, then thread t's row
   // sum into rs and its column partial into colpart (cold: the partial so far
   // was prefetched into s_cold)
-  auto tile_sums = [&](const f32x16 (&acc)[TL::FM][TL::FN], int tm, int tn, float& rs, bool cold = false) {
+  auto tile_sums = [&](const f32x16 (&acc)[TL::FM][TL::FN], int tm, int tn, float& rs, bool cold = false,
+                       int vb = 0) {
+    const float *s_rx = s_vec[vb], *s_ry = s_vec[vb] + TL::BM;
     const int m0 = tm * TL::BM, n0 = tn * TL::BN;
     float rowv[TL::FM * 16];
     float colv[TL::FN];
@@ -584,7 +591,7 @@ __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>:
     }
   };
   if constexpr (FwdChain<T, VEC, NORM>::value) {
-    // chained tiles (no norm scaling: s_rx, s_ry unused): the last chunk of
+    // chained tiles: the last chunk of
     // each tile's k-loop loads chunk 0 of the next, which lands during the
     // epilogue.  The k-loop's barriers order one tile's slot reads before the
     // next tile's slot writes.
@@ -596,6 +603,23 @@ __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>:
     // With a single k-chunk there is no such barrier: the partials are read
     // from global memory in the epilogue instead.
     const bool pf = !LIT && D > TL::G::BK;
+    // NORM: the scales of tile (tm, tn) into half b, 64 floats per wave (entries
+    // past N read as 0 and are masked)
+    const int wu = __builtin_amdgcn_readfirstlane(w);
+    auto vec_loads = [&](int tm, int tn, int b) {
+      if constexpr (NORM) {
+        constexpr int RQ = TL::BM / 64;
+        static_assert(RQ + TL::BN / 64 == TL::NT / 64, "one load per wave");
+        const bool isr = wu < RQ;
+        const int o = isr ? tm * TL::BM + wu * 64 : tn * TL::BN + (wu - RQ) * 64;
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)((isr ? rx : ry) + o), 0,
+                                                                           max(N - o, 0) * 4, 0x00020000);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            r, (__attribute__((address_space(3))) void*)(&s_vec[b][wu * 64]), 4, (uint32_t)lane * 4, 0, 0, 0);
+      }
+    };
+    int vb = 0;
+    vec_loads(tm0, tn0, 0);
     typename TL::Plan lp;
     TL::start(op_a(tm0), op_b(tn0), lds, lp);
     int p0 = 0;
@@ -605,6 +629,7 @@ __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>:
       const bool has_next = k + 1 < K;
       const int tmn = has_next ? tm0 + (k + 1) / ntn : tm, tnn = has_next ? tn0 + (k + 1) % ntn : tn;
       auto hook = [&] {
+        if (NORM && has_next) vec_loads(tmn, tnn, vb ^ 1);
         if (pf && tm > tm0 && w < TL::BN / 64) {
           const int n0 = tn * TL::BN;
           const __amdgpu_buffer_rsrc_t r =
@@ -615,7 +640,8 @@ __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>:
       };
       f32x16 acc[TL::FM][TL::FN];
       TL::chain(lp, op_a(tmn), op_b(tnn), has_next, D, lds, p0, acc, hook);
-      tile_sums(acc, tm, tn, rs, pf);
+      tile_sums(acc, tm, tn, rs, pf, vb);
+      if (NORM) vb ^= 1;
       if (tn == tn1 - 1) {
         if (t < TL::BM && tm * TL::BM + t < N) rowpart[(int64_t)q * n64 + tm * TL::BM + t] = rs;
         rs = 0.f;
@@ -630,6 +656,7 @@ __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>:
       for (int tn = tn0; tn < tn1; ++tn) {
         const int n0 = tn * TL::BN;
         __syncthreads();  // the previous tile's epilogue is done with the LDS stages and slots
+        float *s_rx = s_vec[0], *s_ry = s_vec[0] + TL::BM;
         if (t < TL::BM) s_rx[t] = (NORM && m0 + t < N) ? rx[m0 + t] : 1.f;
         if (t < TL::BN) s_ry[t] = (NORM && n0 + t < N) ? ry[n0 + t] : 1.f;
         f32x16 acc[TL::FM][TL::FN];
@@ -781,6 +808,7 @@ __device__ __forceinline__ void grad_gt_store_direct(const f32x16 (&acc)[TL::FM]
   constexpr int NP = X3 || SPL ? 2 : 1;  // planes
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w / TL::WN, wn = w % TL::WN;
   const int64_t rowb = (int64_t)(bs >> 4) * (SPL ? 1024 : 512);  // elements per row of blocks
+  const int mb = wm * TL::TM + 4 * (lane >> 5);  // (as in sumexp_epilogue)
   // Non-temporal stores through buffer descriptors at the tile's planes (the
   // write-once G'^T should not displace the operand panels from the caches).
   // __builtin_nontemporal_store lost its hint in this function for the
@@ -791,6 +819,9 @@ __device__ __forceinline__ void grad_gt_store_direct(const f32x16 (&acc)[TL::FM]
       __builtin_amdgcn_make_buffer_rsrc((void*)(X3 ? GTl : GTb), 0, 0x7fffffff, 0x00020000);
 #pragma unroll
   for (int bn = 0; bn < TL::FN; ++bn) {
+    // (the row vectors are read again for every column block: kept in registers
+    // across them they spill beside the accumulators)
+    if constexpr (NORM && TL::FN > 2) asm volatile("" ::: "memory");
     const int nl = wn * TL::TN + bn * 32 + (lane & 31);
     const int j = j0 + nl;
     const float cy = NORM ? cm * s_ry[nl] : cm;
@@ -807,11 +838,11 @@ __device__ __forceinline__ void grad_gt_store_direct(const f32x16 (&acc)[TL::FM]
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int r = 4 * (2 * p + q) + e;
-            const int ml = wm * TL::TM + bm * 32 + acc_row(r, lane);
-            const int i = i0 + ml;
-            const float sc = NORM ? acc[bm][bn][r] * s_rx[ml] : acc[bm][bn][r];
+            const int mo = bm * 32 + 8 * (r >> 2) + (r & 3);
+            const int i = i0 + mb + mo;
+            const float sc = NORM ? acc[bm][bn][r] * s_rx[mb + mo] : acc[bm][bn][r];
             const float ex = fast_exp2(fmaf(sc, cy, -c));
-            float g = LIT ? ex * s_ir[ml] : ex * (s_ir[ml] + icj);
+            float g = LIT ? ex * s_ir[mb + mo] : ex * (s_ir[mb + mo] + icj);
             if (GSC != 1) g *= (float)GSC;  // storage scale (exact: a power of two)
             if (MASK) g = (i < N && j < N && i != j) ? g : 0.f;
             gv[e] = g;

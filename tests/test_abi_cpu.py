@@ -587,7 +587,8 @@ def test_pairs_sizes_and_rule(monkeypatch):
     for dt in (1, 2, 4, P, 7):
         assert lib.mec_product_dtype(32768, 1152, dt) == dt
     assert lib.mec_product_dtype(32768, 1152, 0) == P and lib.mec_product_dtype(2048, 512, 0) == 0
-    assert lib.mec_product_dtype(2049, 3, 0) == P
+    assert lib.mec_product_dtype(2049, 3, 0) == 0 and lib.mec_product_dtype(2049, 256, 0) == P
+    assert lib.mec_product_dtype(4097, 3, 0) == P
     assert lib.mec_product_dtype(2048, 1152, 0) == P and lib.mec_product_dtype(1300, 1500, 0) == 0
     assert lib.mec_product_dtype(10, 3, x3) == P
     for dt in (0, x3):

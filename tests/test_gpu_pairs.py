@@ -195,7 +195,7 @@ def test_noalloc_and_one_side(pairs):
 
 def test_rule_reaches_the_module():
     os.environ.pop("MEC_F32_PAIRS", None)
-    for n, d, want in [(2048, 512, _lib.DTYPE_F32), (2049, 64, _lib.DTYPE_F32_PAIRS), (4999, 640, _lib.DTYPE_F32_PAIRS)]:
+    for n, d, want in [(2048, 512, _lib.DTYPE_F32), (2049, 64, _lib.DTYPE_F32), (4097, 64, _lib.DTYPE_F32_PAIRS), (4999, 640, _lib.DTYPE_F32_PAIRS)]:
         x = torch.randn(n, d, device=DEV).requires_grad_(True)
         loss = MemoryEfficientCLIPLoss()(x, torch.randn(n, d, device=DEV))
         assert loss.grad_fn.mec[4] == want, (n, d)
