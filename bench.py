@@ -15,7 +15,8 @@ benchmark table for exploration.  Rank 0 prints ONE JSON line:
 * ``roofline``: the dominant kernel's algorithmic flop per launch over its
   average launch time, measured with HIP events on the stream the library
   launches on (torch's current stream), against the dense MFMA peak of the
-  input dtype;
+  arithmetic (fp32 from fp16 pairs: three fp16 products per fp32 one, so the
+  flop count three times against the fp16 peak);
 * ``cpu_baseline``: the dense PyTorch loss (fp32) on the host cores at the
   same workload (same N, D and generator; a smaller N only with
   ``--cpu-n``), timed forward and backward, reported as the flop the dense
@@ -23,16 +24,19 @@ benchmark table for exploration.  Rank 0 prints ONE JSON line:
   4 N^2 D for LiT) per second, with the core count and CPU model;
 * ``configs``: every benchmark configuration (1-5) timed for a few steps
   through the same module (the headline's row repeats its numbers), with
-  forward / backward / step ms, TFLOP/s, fraction of the input dtype's MFMA
-  peak and peak extra HBM bytes (``--no-table`` skips the other four).
+  forward / backward / step ms, TFLOP/s, fraction of the MFMA peak of its
+  arithmetic and peak extra HBM bytes (``--no-table`` skips the other four).
 
-``--precision high`` runs fp32 inputs under
-``torch.set_float32_matmul_precision("high")``: the products are formed from
-bf16 terms (hi*hi + lo*hi + hi*lo) on the bf16 MFMA.  ``dtype`` is then
-"bf16x3", ``value`` stays in algorithmic (fp32-equivalent) flop, and the
-roofline counts the three MFMA products per algorithmic one against the bf16
-peak.  ``--precision medium`` multiplies bf16-rounded values ("bf16").  The
-default, "highest", is IEEE fp32 on the fp32 MFMA.
+fp32 inputs of this size run on the fp16 MFMA from pairs: each value, scaled
+by a power of two, is hi + lo of two fp16 terms (about 22 significant bits),
+and a product is hi*hi + lo*hi + hi*lo, accumulated in fp32 (errors against
+64-bit values no larger than those of the IEEE fp32 kernels).  ``dtype`` is
+then "f16x2", ``value`` stays in algorithmic (fp32) flop, and the fractions
+count the three MFMA products per algorithmic one against the fp16 peak.
+Under ``--precision high`` the same kernels run; ``--precision medium``
+multiplies bf16-rounded values ("bf16").  Smaller fp32 problems run on the
+fp32 MFMA ("f32"); ``fp32_mfma`` in the JSON is the default workload on those
+kernels, for comparison.
 """
 from __future__ import annotations
 
@@ -51,6 +55,8 @@ if ROOT not in sys.path:
 METRIC = "CLIP fwd+bwd ms & TFLOP/s (% MFMA peak) at N=32768 D=1152, 1 MI355X"
 # MI355X published dense MFMA peaks (256 CUs at 2.4 GHz), TFLOP/s.
 PEAK_TFLOPS = {"f32": 157.3, "bf16": 2516.6, "f16": 2516.6}
+# the MFMA peak and the MFMA products per algorithmic product of each arithmetic
+ARITH = {"f32": (157.3, 1), "bf16": (2516.6, 1), "f16": (2516.6, 1), "bf16x3": (2516.6, 3), "f16x2": (2516.6, 3)}
 TORCH_DTYPE = {"f32": "float32", "bf16": "bfloat16", "f16": "float16"}
 
 # config -> (mode, n, d, dtype, normalized_inputs, temperature, generator, CPU baseline n)
@@ -67,6 +73,18 @@ CONFIGS = {
 # a step is ~0.1 ms of host-bound work, so 300 of them, 30 ms, for a stable
 # mean)
 TABLE_STEPS = {1: (300, 20), 2: (5, 2), 3: (5, 2), 4: (5, 2), 5: (3, 1)}
+
+
+def arithmetic(n, d, dt, precision):
+    """(C-ABI dtype code, name in ARITH) the module runs n x d inputs of dtype
+    `dt` with under float32 matmul precision `precision`."""
+    from memoryefficientclip_amd import _lib
+    code = {"f32": _lib.DTYPE_F32, "bf16": _lib.DTYPE_BF16, "f16": _lib.DTYPE_F16}[dt]
+    if dt == "f32" and precision != "highest":
+        code = _lib.DTYPE_F32_BF16X3 if precision == "high" else _lib.DTYPE_F32_BF16
+    code = _lib.load().mec_product_dtype(n, d, code)
+    return code, {_lib.DTYPE_F32: "f32", _lib.DTYPE_BF16: "bf16", _lib.DTYPE_F16: "f16",
+                  _lib.DTYPE_F32_BF16X3: "bf16x3", _lib.DTYPE_F32_BF16: "bf16", _lib.DTYPE_F32_PAIRS: "f16x2"}[code]
 
 
 def log(*a):
@@ -336,14 +354,14 @@ def main():
     ap.add_argument("--dtype", choices=sorted(PEAK_TFLOPS), default=None,
                     help="input dtype instead of the config's own (e.g. --config 4 --dtype f16)")
     ap.add_argument("--precision", choices=["highest", "high", "medium"], default="highest",
-                    help="float32 matmul precision for fp32 inputs: highest = IEEE fp32 MFMA, "
-                         "high = three bf16 MFMA products per fp32 product (bf16x3), medium = bf16 products")
+                    help="float32 matmul precision for fp32 inputs: highest and high = fp32 accuracy (fp16 pairs, or "
+                         "the fp32 MFMA where that is faster), medium = bf16 products")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--cpu-n", type=int, default=0,
                     help="N of the CPU baseline sample (default: the configuration's own N, at most 32768)")
     ap.add_argument("--no-table", action="store_true", help="skip timing the other benchmark configurations")
     ap.add_argument("--no-alt", action="store_true",
-                    help="skip the fp32 'high' precision side leg (e.g. for per-kernel profiles of the IEEE path)")
+                    help="skip the side leg on the fp32 MFMA kernels (e.g. for per-kernel profiles)")
     ap.add_argument("--kernel-reps", type=int, default=0, help="launches per stage in the kernel leg (default: steps)")
     ap.add_argument("--probe", choices=["copy", "gemm"], default=None,
                     help="copy: only run 5 plain device copies of 1 GiB (calibrates the rocprofv3 byte counters); "
@@ -398,20 +416,12 @@ def main():
     dt = args.dtype or dt
     dev = torch.device("cuda:0")
     torch.cuda.set_device(dev)
-    # arithmetic: the input dtype's MFMA, or for fp32 inputs below "highest"
-    # precision bf16x3 (three bf16 products per fp32 product) or bf16
-    x3 = args.precision == "high"
-    lowp = args.precision != "highest"
-    if lowp and dt != "f32":
+    if args.precision != "highest" and dt != "f32":
         print(f"bench.py: --precision {args.precision} applies to fp32 inputs only", file=sys.stderr)
         sys.exit(2)
     torch.set_float32_matmul_precision(args.precision)
-    arith = "bf16x3" if x3 else "bf16" if lowp else dt
-    mfma_per_flop = 3 if x3 else 1
-    peak = PEAK_TFLOPS["bf16" if lowp else dt]
-    dtc = {"f32": _lib.DTYPE_F32, "bf16": _lib.DTYPE_BF16, "f16": _lib.DTYPE_F16}[dt]
-    if lowp:
-        dtc = _lib.DTYPE_F32_BF16X3 if x3 else _lib.DTYPE_F32_BF16
+    dtc, arith = arithmetic(n, d, dt, args.precision)
+    peak, mfma_per_flop = ARITH[arith]
     log(f"bench: config {args.config} {mode} n={n} d={d} {dt} normalized_inputs={normalized} T={temperature}"
         f" arithmetic={arith}")
     head, a, b = measure(args.config, dt, args.steps, args.warmup)
@@ -422,18 +432,19 @@ def main():
     log(f"bench: {args.steps} steps, {ms:.3f} ms/step (fwd {fwd_ms:.3f}, bwd {bwd_ms:.3f}), {tflops:.2f} TFLOP/s, "
         f"loss {loss_val:.6f}")
 
-    # fp32 inputs at "highest" precision: the same steps once more under "high"
-    # (bf16x3), reported beside the IEEE line (not as its value)
+    # fp32 inputs that run as pairs: the same steps once more on the fp32 MFMA
+    # kernels, reported beside the line (not as its value)
     alt = None
-    if dt == "f32" and not lowp and not args.no_alt:
-        torch.set_float32_matmul_precision("high")
-        hi, _, _ = measure(args.config, dt, args.steps, args.warmup, with_events=False)
+    if dt == "f32" and arith == "f16x2" and not args.no_alt and "MEC_F32_PAIRS" not in os.environ:
+        os.environ["MEC_F32_PAIRS"] = "0"
         torch.set_float32_matmul_precision("highest")
-        ms_hi = hi["ms_per_step"]
-        alt = {"float32_matmul_precision": "high", "dtype": "bf16x3", "ms_per_step": round(ms_hi, 4),
-               "value": round(flop / (ms_hi * 1e-3) / 1e12, 3), "unit": "TFLOP/s",
-               "frac_of_bf16_peak": round(3 * flop / (ms_hi * 1e-3) / 1e12 / PEAK_TFLOPS["bf16"], 4)}
-        log(f"bench: float32 matmul precision high (bf16x3): {ms_hi:.3f} ms/step, {alt['value']:.2f} TFLOP/s")
+        ie, _, _ = measure(args.config, dt, min(args.steps, 5), min(args.warmup, 2), with_events=False)
+        torch.set_float32_matmul_precision(args.precision)
+        del os.environ["MEC_F32_PAIRS"]
+        alt = {"dtype": "f32", "ms_per_step": ie["ms_per_step"], "value": ie["tflops"], "unit": "TFLOP/s",
+               "frac_of_fp32_peak": round(ie["tflops"] / PEAK_TFLOPS["f32"], 4), "loss": ie["loss"]}
+        log(f"bench: fp32 MFMA kernels: {ie['ms_per_step']:.3f} ms/step, {ie['tflops']:.2f} TFLOP/s, "
+            f"loss {ie['loss']:.6f}")
 
     # kernel leg: per-stage launch times on the library's stream
     x = a.detach()
@@ -443,17 +454,14 @@ def main():
     for k, (t, nl, fl) in stages.items():
         log(f"bench: stage {k:9s} {t:9.3f} ms x {nl:3d}" + (f"  {fl / (t * 1e-3) / 1e12:8.2f} TFLOP/s" if fl else ""))
     log(f"bench: backward blocking {blocking}")
-    # dominant kernel: the backward pipeline step, nb + 1 launches of mec_grad_step per
-    # step, about 3/4 of the step's flop: k_grad_step (fp32: gradient-matrix tiles and
-    # contractions in one kernel; 16-bit: the gradient-matrix tiles, chained in
-    # k_grad_g_chain for normalized inputs, with the contractions in k_grad_contract
-    # before them)
-    # (bf16x3: MFMA flop = 3 x algorithmic flop, against the bf16 peak)
+    # dominant kernels: the backward pipeline steps, nb + 1 launches of mec_grad_step
+    # per step, about 3/4 of the step's flop: k_grad_step (fp32: gradient-matrix
+    # tiles and contractions in one kernel), else the chained gradient-matrix
+    # tiles with the contractions in k_grad_contract before them
+    # (three products: MFMA flop = 3 x algorithmic flop, against the 16-bit peak)
     t_k, nl_k, f_k = stages["grad_step"]
     achieved = mfma_per_flop * f_k / (t_k * 1e-3) / 1e12
-    # (16-bit data with normalized inputs: the gradient-matrix tiles run chained, in k_grad_g_chain)
-    gkern = "k_grad_g_chain" if (normalized and not x3) else "k_grad_step"
-    kernels = ["k_grad_step"] if arith == "f32" else ["k_grad_contract", gkern]
+    kernels = ["k_grad_step"] if arith == "f32" else ["k_grad_contract", "k_grad_g_chain"]
     traffic = measured_traffic(f"{mode}_n{n}_d{d}_{arith}", kernels)
     if traffic is not None and len(kernels) > 1:
         # each kernel runs in nb of the nb + 1 pipeline launches
@@ -463,9 +471,8 @@ def main():
                 "unit": "TFLOP/s", "frac": round(achieved / peak, 4), "traffic": traffic,
                 "launch_ms": round(t_k, 4), "flop_per_launch": mfma_per_flop * f_k, "launches_per_step": nl_k}
     t_f, _, f_f = stages["sumexp"]
-    # (bf16/fp16 products on inputs already normalized: the forward runs the
-    # chained block walk, k_sumexp_det, with its O(N) reduction)
-    fkern = "k_sumexp_det+k_det_reduce" if (arith != "f32" and normalized) else "k_sumexp"
+    # (16-bit products: the chained block walk, k_sumexp_det, with its O(N) reduction)
+    fkern = "k_sumexp" if arith == "f32" else "k_sumexp_det+k_det_reduce"
     roofline_fwd = {"kernel": fkern, "achieved": round(mfma_per_flop * f_f / (t_f * 1e-3) / 1e12, 3),
                     "frac": round(mfma_per_flop * f_f / (t_f * 1e-3) / 1e12 / peak, 4), "launch_ms": round(t_f, 4),
                     "flop_per_launch": mfma_per_flop * f_f}
@@ -485,7 +492,9 @@ def main():
                 row, ta, tb = measure(cfg, CONFIGS[cfg][3], st, wu)
                 del ta, tb
                 torch.cuda.empty_cache()
-            row["frac_of_peak"] = round(row["tflops"] / PEAK_TFLOPS[row["dtype"]], 4)
+            row["arithmetic"] = arithmetic(row["n"], row["d"], row["dtype"], "highest")[1]
+            row_peak, row_mfma = ARITH[row["arithmetic"]]
+            row["frac_of_peak"] = round(row_mfma * row["tflops"] / row_peak, 4)
             if CONFIGS[cfg][1] <= 4096:
                 # small N: the host, not the GPU, sets the step; the same loop with
                 # the backward on the calling thread shows how much of it is the
@@ -496,7 +505,7 @@ def main():
             table.append(row)
             log(f"bench: table config {cfg}: {row['ms_per_step']:.3f} ms/step (fwd {row['fwd_ms']:.3f}, "
                 f"bwd {row['bwd_ms']:.3f}), {row['tflops']:.1f} TFLOP/s, {100 * row['frac_of_peak']:.1f}% of "
-                f"{row['dtype']} peak, extra HBM {row['peak_extra_hbm_bytes'] / 1e9:.2f} GB")
+                f"the peak ({row['arithmetic']}), extra HBM {row['peak_extra_hbm_bytes'] / 1e9:.2f} GB")
             if "ms_per_step_backward_on_calling_thread" in row:
                 log(f"bench: table config {cfg}, backward on the calling thread: "
                     f"{row['ms_per_step_backward_on_calling_thread']:.3f} ms/step")
@@ -525,6 +534,8 @@ def main():
         "config": {"workload": f"{mode}_loss_fwd_bwd", "n": n, "d": d, "temperature": temperature,
                    "normalized_inputs": normalized, "input_dtype": dt, "float32_matmul_precision": args.precision,
                    "parallelism": "none (1 GPU)"},
+        "arithmetic": ("fp32 values as scaled fp16 pairs (hi + lo, about 22 significant bits), three fp16 MFMA "
+                       "products per fp32 product, fp32 accumulation" if arith == "f16x2" else arith),
         "fwd_ms": round(fwd_ms, 4),
         "bwd_ms": round(bwd_ms, 4),
         "frac_of_peak": round(mfma_per_flop * tflops / peak, 4),
@@ -537,7 +548,7 @@ def main():
         "roofline": roofline,
         "roofline_forward": roofline_fwd,
         "backward_blocking": blocking,
-        "precision_high": alt,
+        "fp32_mfma": alt,
         "cpu_baseline": cpu,
         "configs": table,
     }
