@@ -15,12 +15,16 @@
 //                             kernel of their own, a last column of at most
 //                             128 features in 512 x 128 tiles where faster;
 //                             256 x 384 where those take fewer rounds of work
+//                             128 x 128 tiles for all of them at a small n
+//                             (small16_n)
 //   bf16 / fp16, other        forward sums and gradient-matrix tiles 128 x 128
 //   layouts                   staged through registers (mec_gemm_16.h); the
 //                             contractions read internal buffers, which are
 //                             always 16-byte vectors, so they keep 256 x 256
 //   fp32 data with bf16       the bf16 tiles on internal bf16 / split copies
 //   products (bf16, bf16x3)   of the inputs (always 16-byte vectors)
+//   fp32 data as fp16 pairs   the 16-bit tiles, contractions 256 x 256 (128 x
+//                             128 at a small n), on internal copies
 //
 // The backward's block decomposition uses blocks of a multiple of
 // block_quantum(dtype) rows, so that every tile kind divides a block.
