@@ -457,6 +457,7 @@ struct ScratchLayout {
   int64_t ldt;         // elements
   int64_t gbuf, tbuf;  // bytes of one diagonal plane / one transposed plane
   int64_t xt, yt;      // byte offsets of XT and YT (-1: not held)
+  int64_t gs;          // of the scale of the pairs' gradient matrix (GradBufs::gscl)
   int64_t total;
 };
 ScratchLayout scratch_layout_blocks(int64_t n, int64_t d, int dtype, int sides, int bs, int nb) {
@@ -480,6 +481,8 @@ ScratchLayout scratch_layout_blocks(int64_t n, int64_t d, int dtype, int sides, 
     L.yt = off;
     off += L.ntp * L.tbuf;
   }
+  L.gs = off;
+  if (is_pairs(dtype)) off += 256;
   L.total = off;
   return L;
 }
@@ -1296,7 +1299,10 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
     if (x3) gb.yt_lo = base + L.yt + L.tbuf;
   }
   gb.ldt = L.ldt;
-  if (pairs) gb.scl = pair_scl(workspace, n);
+  if (pairs) {
+    gb.scl = pair_scl(workspace, n);
+    gb.gscl = (const float*)(base + L.gs);
+  }
   hipStream_t s = (hipStream_t)stream;
   if (step == 0 && dtype != MEC_DTYPE_F32) {
     // transposed normalised operands of the 16-bit contractions: YT for the
@@ -1312,7 +1318,7 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
       const TS tx{(const float*)x, ldx, workspace + WS_RX * n64, (uint16_t*)gb.xt, nullptr};
       DISPATCH_BOOL(normalize, NORM, k_transpose_pairs<NORM><<<tgrid, 256, 0, s>>>(
                                          acc_x ? ty : tx, tx, N, D, L.ldt, gb.scl + (acc_x ? SCL_Y : SCL_X),
-                                         gb.scl + SCL_X));
+                                         gb.scl + SCL_X, workspace + WS_KAPPA * n64, (float*)(base + L.gs)));
     } else if (split) {
       using TS = TransSide<float, uint16_t>;
       const TS ty{(const float*)y, ldy, workspace + WS_RY * n64, (uint16_t*)gb.yt, (uint16_t*)gb.yt_lo};

@@ -273,7 +273,6 @@ template <typename T> struct GtOnly { static constexpr bool value = Is16<T>::val
 // the fp16 maximum 65504) and the contractions scale back by 2^-14 (exact).
 template <typename T> struct GScale { static constexpr float value = 1.f; };
 template <> struct GScale<_Float16> { static constexpr float value = 16384.f; };
-template <> struct GScale<F16S> { static constexpr float value = 16384.f; };
 
 // The scales of the split pairs: x and y are multiplied by the powers of two
 // scl[0] and scl[1] before they are split (so that the lo parts stay within
@@ -724,7 +723,8 @@ struct GradBufs {
   void* gt_lo[2];
   const void* xt_lo;
   const void* yt_lo;
-  const float* scl;  // scales of split pairs (F16S)
+  const float* scl;   // scales of split pairs (F16S)
+  const float* gscl;  // of their gradient matrix: the scale, its inverse
 };
 
 // One pipeline step of the backward (launch t = 0 .. nb):
@@ -802,7 +802,7 @@ template <class TL, bool LIT, bool NORM, bool MASK, int GSC, bool X3 = false>
 __device__ __forceinline__ void grad_gt_store_direct(const f32x16 (&acc)[TL::FM][TL::FN], float cm, float c, int i0,
                                                      int j0, int N, uint16_t* __restrict__ GTb, int bs, const float* s_rx,
                                                      const float* s_ry, const float* s_ir, const float* s_ic,
-                                                     uint16_t* __restrict__ GTl = nullptr) {
+                                                     uint16_t* __restrict__ GTl = nullptr, float gs = 1.f) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   constexpr bool SPL = TL::SPL;
   constexpr int NP = X3 || SPL ? 2 : 1;  // planes
@@ -843,7 +843,9 @@ __device__ __forceinline__ void grad_gt_store_direct(const f32x16 (&acc)[TL::FM]
             const float sc = NORM ? acc[bm][bn][r] * s_rx[mb + mo] : acc[bm][bn][r];
             const float ex = fast_exp2(fmaf(sc, cy, -c));
             float g = LIT ? ex * s_ir[mb + mo] : ex * (s_ir[mb + mo] + icj);
-            if (GSC != 1) g *= (float)GSC;  // storage scale (exact: a power of two)
+            // storage scale (exact: a power of two)
+            if constexpr (SPL) g *= gs;
+            else if (GSC != 1) g *= (float)GSC;
             if (MASK) g = (i < N && j < N && i != j) ? g : 0.f;
             gv[e] = g;
           }
@@ -899,6 +901,7 @@ __device__ __forceinline__ void grad_g_tile(const T* __restrict__ X, int64_t ldx
   f32x16 acc[TL::FM][TL::FN];
   TL::template run<VEC, VEC>(A, B, D, lds, acc);
   // 1/R_i and 1/C_j carry the storage scale of G' (a power of two: exact)
+  static_assert(!IsSplit<T>::value, "split pairs run in k_grad_g_chain");
   constexpr float GS = GScale<T>::value;
   for (int u = t; u < TL::BM; u += TL::NT) {
     const bool ok = i0 + u < N;
@@ -1032,7 +1035,7 @@ __device__ __forceinline__ void grad_contract_dispatch(int sub, int N, int D, co
   const int64_t blk = (int64_t)bg.bs * bg.bs * (IsSplit<T>::value ? 2 : 1);  // elements per G' block
   const bool is_x = sub < sp.cx_pad;
   float osc = 1.f / GScale<T>::value;
-  if constexpr (IsSplit<T>::value) osc *= gb.scl[is_x ? SCL_INVY : SCL_INVX];
+  if constexpr (IsSplit<T>::value) osc = gb.gscl[1] * gb.scl[is_x ? SCL_INVY : SCL_INVX];
   if (!is_x) sub -= sp.cx_pad;
   const int pid = xcd_remap(sub, is_x ? sp.cx_pad : sp.cy_pad);
   if (pid >= (is_x ? sp.cx_n : sp.cy_n)) return;
@@ -1206,6 +1209,7 @@ __global__ __launch_bounds__((GemmTile<T, true, SMALL>::NT), (SMALL ? 2 : 1)) vo
   const int64_t blk = (int64_t)bg.bs * bg.bs * E;
   const int buf = sp.diag_g & 1;
   const float cm = exp_mul<T>(c, gb.scl);
+  const float gs = IsSplit<T>::value ? gb.gscl[0] : 1.f;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   // tile -> (i0, j0, its place in the G'^T block); false for padding ids and tiles wholly past N
   auto coords = [&](int tile, int& i0, int& j0, uint16_t*& gt) {
@@ -1275,11 +1279,11 @@ __global__ __launch_bounds__((GemmTile<T, true, SMALL>::NT), (SMALL ? 2 : 1)) vo
     if (!diag && i0 + TL::BM <= N && j0 + TL::BN <= N)
       grad_gt_store_direct<TL, LIT, NORM, false, (int)GScale<T>::value, X3>(
           acc, cm, c, i0, j0, N, gt, bg.bs, sv + V_RX * TL::BM, sv + V_RY * TL::BM, sv + V_IR * TL::BM,
-          sv + V_IC * TL::BM, gtl);
+          sv + V_IC * TL::BM, gtl, gs);
     else
       grad_gt_store_direct<TL, LIT, NORM, true, (int)GScale<T>::value, X3>(
           acc, cm, c, i0, j0, N, gt, bg.bs, sv + V_RX * TL::BM, sv + V_RY * TL::BM, sv + V_IR * TL::BM,
-          sv + V_IC * TL::BM, gtl);
+          sv + V_IC * TL::BM, gtl, gs);
     if (!has_next) break;
     tile = next;
     i0 = i1;

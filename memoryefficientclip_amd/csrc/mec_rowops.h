@@ -893,6 +893,30 @@ __global__ __launch_bounds__(256) void k_pair_rows(const float* __restrict__ X, 
   }
 }
 
+// The scale of the gradient matrix's pairs, for one workgroup of 256 threads:
+// gscl = {2^k, 2^-k}, the largest with 2^k G'_ij <= 2^15 that the row sums
+// allow, at least 2^14 (G' <= 2).  G'_ij = E_ij (1/R_i + 1/C_j) <= row_off_i /
+// R_i + col_off_j / C_j <= 2 max |kappa|.  Where the pairs match well (small
+// off-diagonal sums) the entries are small against 2, and under the fixed scale
+// 2^14 their lo parts, then their hi parts, fell below fp16's range.
+constexpr int PAIR_G_MIN_EXP = -26;
+__device__ __forceinline__ void pair_grad_scale(int N, const float* __restrict__ kappa, float* gscl) {
+  __shared__ float s_m[4];
+  float m = 0.f;
+#pragma unroll 8
+  for (int k = threadIdx.x; k < N; k += 256) m = fmaxf(m, -kappa[k]);
+  for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int e = 0;  // 2 max |kappa| < 2^(e + 1)
+    m = fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3]));
+    if (m < 0.5f) (void)frexpf(fmaxf(m, ldexpf(1.f, PAIR_G_MIN_EXP)), &e);
+    gscl[0] = ldexpf(1.f, 14 - e);
+    gscl[1] = ldexpf(1.f, e - 14);
+  }
+}
+
 // k_transpose_split into pairs: row d of XT (pitch 2 ldt) holds, for every 32
 // rows i, 32 hi and then 32 lo values of scale_i x_i[d] (NORM) times the side's
 // pair scale, zero for N <= i < ldt (ldt a multiple of 64).  Two values of i
@@ -900,7 +924,8 @@ __global__ __launch_bounds__(256) void k_pair_rows(const float* __restrict__ X, 
 template <bool NORM>
 __global__ __launch_bounds__(256) void k_transpose_pairs(TransSide<float, uint16_t> s0, TransSide<float, uint16_t> s1,
                                                          int N, int D, int64_t ldt, const float* scl0,
-                                                         const float* scl1) {
+                                                         const float* scl1, const float* __restrict__ kappa,
+                                                         float* gscl) {
   const TransSide<float, uint16_t>& sd = blockIdx.z ? s1 : s0;
   const float ps = blockIdx.z ? *scl1 : *scl0;
   const float* __restrict__ X = sd.X;
@@ -931,6 +956,7 @@ __global__ __launch_bounds__(256) void k_transpose_pairs(TransSide<float, uint16
     *(uint32_t*)o = pack2_f16(ha, hb);
     *(uint32_t*)(o + 32) = pack2_f16(__builtin_isinf(ha) ? 0.f : a - ha, __builtin_isinf(hb) ? 0.f : b - hb);
   }
+  if (blockIdx.x + blockIdx.y + blockIdx.z == 0) pair_grad_scale(N, kappa, gscl);
 }
 
 }  // namespace mec
