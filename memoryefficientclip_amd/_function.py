@@ -91,7 +91,7 @@ def refuse_graph_capture() -> None:
     """Raise instead of enqueueing work into a CUDA/HIP graph capture.
 
     Capturing a step that calls this loss ended in a host segmentation fault
-    inside ``torch.cuda.graph``'s ``capture_end`` on the MI355X box, with no
+    inside ``torch.cuda.graph``'s ``capture_end`` on an MI355X, with no
     cause found in this library's launches; a clear error is better than a
     crashed training process."""
     if torch.cuda.is_current_stream_capturing():

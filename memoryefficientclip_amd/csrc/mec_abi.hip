@@ -93,7 +93,7 @@ int check_launch(const char* what) {
 // Launches into a stream that is being captured into a HIP graph are
 // refused (MEC_ERR_UNSUPPORTED, before any launch): capturing a step of the
 // loss ended in a host segmentation fault during graph instantiation on the
-// MI355X box, with no cause found in these launches.  A legacy default
+// MI355X, with no cause found in these launches.  A legacy default
 // stream implicitly joined to another stream's capture counts as capturing.
 // MEC_TEST_ASSUME_CAPTURING=1 makes the check report a capture without
 // asking HIP (tests of this refusal on machines without a GPU).
