@@ -387,9 +387,8 @@ void grad_blocks_budget(int64_t n, int64_t d, int dtype, int64_t gbudget, int* b
   if (dtype != MEC_DTYPE_F32 && !is_pairs(dtype) && n >= 8192 && n < 16 * 8 * d) mult = 16;
   // at least 1024 rows (below that the pipeline's launches and accumulator
   // updates dominate), where the budget allows
-  // (pairs: twice the fp32 kernels' rows throughout.  A sum over more rows
-  // rounds more, and at twice the rows their sums are still no further from 64
-  // bits than the fp32 kernels', at four times 1.5 times as far: 4097 x 192)
+  // (pairs: twice the fp32 kernels' rows throughout; the sums over a block's rows
+  // are taken in pieces of those kernels' blocks: StepPlan::seg)
   const int64_t min_rows = is_pairs(dtype) ? 2 * kTargetMinRows : kTargetMinRows;
   const int64_t target_rows = mult * d > min_rows ? mult * d : min_rows;
   int64_t target = (target_rows + q - 1) / q;
@@ -1257,6 +1256,13 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
   StepPlan sp{};
   sp.ks = ks;
   sp.kl = cs ? cs->kl : bs;
+  sp.seg = bs;
+  if (pairs) {
+    // (sums no longer than the fp32 kernels': grad_contract_tile)
+    int bs32, nb32;
+    grad_blocks(n, d, MEC_DTYPE_F32, &bs32, &nb32);
+    if (bs32 < bs) sp.seg = bs32;
+  }
   sp.px = parts;
   sp.py = parts ? parts + (acc_x ? (int64_t)(ks - 1) * n * d : 0) : nullptr;
   sp.diag_g = step < nb ? (int)step : -1;

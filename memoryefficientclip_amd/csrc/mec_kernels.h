@@ -746,6 +746,7 @@ struct StepPlan {
   // part p into px / py + (p - 1) N D
   int ks, kl;
   float *px, *py;
+  int seg;  // split pairs: the most k rows that one sum runs over (grad_contract_tile)
 };
 
 // fp32 gradient-matrix tile: H_ij = rx_i G'_ij ry_j (G'_ij without the norm
@@ -935,6 +936,65 @@ __device__ __forceinline__ void grad_g_tile(const T* __restrict__ X, int64_t ldx
   }
 }
 
+// The tile's sums times osc into rows r0.. and columns d0.. of out (N x D),
+// added to what is there (accumulate) or in its place.  The adds are
+// fire-and-forget in L2 instead of a load-add-store round trip; the tile has one
+// owner per launch, so the summation order (program and launch order) and the
+// result are deterministic.
+template <class TC>
+__device__ __forceinline__ void contract_store(const f32x16 (&acc)[TC::FM][TC::FN], int r0, int d0, int N, int D,
+                                               bool accumulate, float* __restrict__ out, float osc) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w / TC::WN, wn = w % TC::WN;
+#pragma unroll
+  for (int bm = 0; bm < TC::FM; ++bm) {
+#pragma unroll
+    for (int bn = 0; bn < TC::FN; ++bn) {
+      const int d = d0 + wn * TC::TN + bn * 32 + (lane & 31);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = r0 + wm * TC::TM + bm * 32 + acc_row(r, lane);
+        if (row < N && d < D) {
+          float* p = out + (int64_t)row * D + d;
+          const float v = acc[bm][bn][r] * osc;
+          if (accumulate)
+            __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          else
+            *p = v;
+        }
+      }
+    }
+  }
+}
+// contract_store in a loop: the addresses and masks of the 128 elements are
+// formed anew each time, with one branch on `accumulate` (kept across the k-loop
+// between, and with a branch per element, they spilled; once per tile the branch
+// per element takes fewer registers).
+template <class TC>
+__device__ __forceinline__ void contract_store_again(const f32x16 (&acc)[TC::FM][TC::FN], int r0, int d0, int N, int D,
+                                                     bool accumulate, float* __restrict__ out, float osc) {
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));
+  const int w = threadIdx.x >> 6, wm = w / TC::WN, wn = w % TC::WN;
+  auto each = [&](auto put) {
+#pragma unroll
+    for (int bm = 0; bm < TC::FM; ++bm) {
+#pragma unroll
+      for (int bn = 0; bn < TC::FN; ++bn) {
+        const int d = d0 + wn * TC::TN + bn * 32 + (lane & 31);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int row = r0 + wm * TC::TM + bm * 32 + acc_row(r, lane);
+          if (row < N && d < D) put(out + (int64_t)row * D + d, acc[bm][bn][r] * osc);
+        }
+      }
+    }
+  };
+  if (accumulate)
+    each([](float* p, float v) { __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); });
+  else
+    each([](float* p, float v) { *p = v; });
+}
+
 // One BM x BN output tile of a contraction: rows r0.. of block P, feature
 // columns d0..:
 //   x side: acc_x[i, d] (+)= sum_{j in Q} G'(P,Q)[i, j]  * YT[d, j]   (Q = P + s)
@@ -952,13 +1012,14 @@ __device__ __forceinline__ void grad_g_tile(const T* __restrict__ X, int64_t ldx
 // X3 (bf16x3): Gblk/OT are the hi planes and Glo/OTlo the lo planes; the
 // tile is hi.hi + hi.lo + lo.hi, three passes over K into one accumulator.
 // osc: the inverse of the operands' storage scales (a power of two).
+// Only k rows [kbeg, kbeg + klen) of the block.
 template <class TC, typename T, bool X3 = false>
-__device__ __forceinline__ void grad_contract_tile(int N, int D, const T* __restrict__ Gblk,
+__device__ __forceinline__ void grad_contract_piece(int N, int D, const T* __restrict__ Gblk,
                                                    const T* __restrict__ Glo, const T* __restrict__ OT,
                                                    const T* __restrict__ OTlo, int64_t ldt, const BlockGrid& bg,
                                                    int P, int Q, int tm, int td, bool accumulate,
-                                                   float* __restrict__ out, char* lds, float osc, int kbeg = 0,
-                                                   int klen = 1 << 30) {
+                                                   float* __restrict__ out, char* lds, float osc, int kbeg,
+                                                   int klen) {
   const int r0 = P * bg.bs + tm * TC::BM;
   if (r0 >= N) return;
   const int d0 = td * TC::BN;
@@ -999,28 +1060,39 @@ __device__ __forceinline__ void grad_contract_tile(int N, int D, const T* __rest
     __syncthreads();
     TC::template run<true, true, false>(tile_op<TC>(Glo + a_off, bg.bs, TC::BM, kq), B, kq, lds, acc);
   }
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w / TC::WN, wn = w % TC::WN;
-#pragma unroll
-  for (int bm = 0; bm < TC::FM; ++bm) {
-#pragma unroll
-    for (int bn = 0; bn < TC::FN; ++bn) {
-      const int d = d0 + wn * TC::TN + bn * 32 + (lane & 31);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = r0 + wm * TC::TM + bm * 32 + acc_row(r, lane);
-        if (row < N && d < D) {
-          float* p = out + (int64_t)row * D + d;
-          // a fire-and-forget add in L2 instead of a load-add-store round trip;
-          // the tile has one owner per launch, so the summation order (launch
-          // order) and the result are deterministic
-          const float v = acc[bm][bn][r] * osc;
-          if (accumulate)
-            __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          else
-            *p = v;
-        }
-      }
+  if constexpr (SPL)
+    contract_store_again<TC>(acc, r0, d0, N, D, accumulate, out, osc);
+  else
+    contract_store<TC>(acc, r0, d0, N, D, accumulate, out, osc);
+}
+
+// grad_contract_piece over the k rows [kbeg, kbeg + klen).
+// seg (split pairs): a sum over more than seg k rows is taken in
+// pieces of seg, each added to the accumulators as another block's would be: a
+// longer sum rounds more.  With seg the block rows of the fp32 kernels the
+// sums are no longer than theirs, and round 3 times per 8 k where the fp32
+// MFMA rounds 4 times; unlimited (one sum per block), positive features came
+// out up to 1.9 times as far from 64 bits as the fp32 kernels' (4200 x 512).
+template <class TC, typename T, bool X3 = false>
+__device__ __forceinline__ void grad_contract_tile(int N, int D, const T* __restrict__ Gblk,
+                                                   const T* __restrict__ Glo, const T* __restrict__ OT,
+                                                   const T* __restrict__ OTlo, int64_t ldt, const BlockGrid& bg,
+                                                   int P, int Q, int tm, int td, bool accumulate,
+                                                   float* __restrict__ out, char* lds, float osc, int kbeg, int klen,
+                                                   int seg) {
+  if constexpr (IsSplit<T>::value) {
+    const int kend = min(min(bg.bs, N - Q * bg.bs), kbeg + klen);
+    for (int k = kbeg;;) {
+      grad_contract_piece<TC, T, X3>(N, D, Gblk, Glo, OT, OTlo, ldt, bg, P, Q, tm, td, accumulate || k > kbeg, out,
+                                     lds, osc, k, min(seg, klen));
+      k += seg;
+      if (k >= kend) break;
+      klen -= seg;
+      __syncthreads();  // every wave is past its last read of the ring
     }
+  } else {
+    grad_contract_piece<TC, T, X3>(N, D, Gblk, Glo, OT, OTlo, ldt, bg, P, Q, tm, td, accumulate, out, lds, osc, kbeg,
+                                   klen);
   }
 }
 
@@ -1074,7 +1146,16 @@ __device__ __forceinline__ void grad_contract_dispatch(int sub, int N, int D, co
   } else {
     group_tile(pid, bg.nb * bg.ctm, bg.ctd, 8, tmg, td);
   }
-  const int P = tmg / rows, tm = tmg - P * rows;  // P: block owning the output rows
+  if constexpr (IsSplit<T>::value) {
+    // (the divisions above run on the VALU: without this the buffer descriptors
+    // in the loop over the sums' pieces end in vector registers)
+    tmg = __builtin_amdgcn_readfirstlane(tmg);
+    td = __builtin_amdgcn_readfirstlane(td);
+    part = __builtin_amdgcn_readfirstlane(part);
+  }
+  int P = tmg / rows;
+  if constexpr (IsSplit<T>::value) P = __builtin_amdgcn_readfirstlane(P);
+  const int tm = tmg - P * rows;  // P: block owning the output rows
   const int buf = sp.diag_c & 1;
   const int kbeg = part * sp.kl, klen = sp.ks > 1 ? sp.kl : 1 << 30;
   if (part > 0) {
@@ -1082,31 +1163,33 @@ __device__ __forceinline__ void grad_contract_dispatch(int sub, int N, int D, co
     acc_y = sp.py + (int64_t)(part - 1) * N * D;
   }
   if (is_x) {
-    const int Q = (P + sp.diag_c) % bg.nb;
+    int Q = (P + sp.diag_c) % bg.nb;
+    if constexpr (IsSplit<T>::value) Q = __builtin_amdgcn_readfirstlane(Q);
     const T* gx = (const T*)(GtOnly<T>::value ? gb.gt[buf] : gb.g[buf]) + P * blk;
     const T* gxl = X3 ? (const T*)gb.gt_lo[buf] + P * blk : nullptr;
-    if (narrow)
+    if (!IsSplit<T>::value && narrow)
       grad_contract_tile<TNX, T, X3>(N, D, gx, gxl, (const T*)gb.yt, (const T*)gb.yt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_x, lds, osc, kbeg, klen);
+                                     sp.accumulate != 0, acc_x, lds, osc, kbeg, klen, sp.seg);
     else if constexpr (TCX::TB)
       grad_contract_tile<TCX, T, X3>(N, D, gx, gxl, Y, nullptr, ldy, bg, P, Q, tm, td, sp.accumulate != 0, acc_x,
-                                     lds, osc, kbeg, klen);
+                                     lds, osc, kbeg, klen, sp.seg);
     else
       grad_contract_tile<TCX, T, X3>(N, D, gx, gxl, (const T*)gb.yt, (const T*)gb.yt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_x, lds, osc, kbeg, klen);
+                                     sp.accumulate != 0, acc_x, lds, osc, kbeg, klen, sp.seg);
   } else {
-    const int Q = (P - sp.diag_c + bg.nb) % bg.nb;
+    int Q = (P - sp.diag_c + bg.nb) % bg.nb;
+    if constexpr (IsSplit<T>::value) Q = __builtin_amdgcn_readfirstlane(Q);
     const T* gy = (const T*)(GtOnly<T>::value ? gb.gt[buf] : gb.g[buf]) + Q * blk;
     const T* gyl = X3 ? (const T*)gb.gt_lo[buf] + Q * blk : nullptr;
-    if (narrow)
+    if (!IsSplit<T>::value && narrow)
       grad_contract_tile<TNY, T, X3>(N, D, gy, gyl, (const T*)gb.xt, (const T*)gb.xt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_y, lds, osc, kbeg, klen);
+                                     sp.accumulate != 0, acc_y, lds, osc, kbeg, klen, sp.seg);
     else if constexpr (TCY::TB)
       grad_contract_tile<TCY, T, X3>(N, D, gy, gyl, X, nullptr, ldx, bg, P, Q, tm, td, sp.accumulate != 0, acc_y,
-                                     lds, osc, kbeg, klen);
+                                     lds, osc, kbeg, klen, sp.seg);
     else
       grad_contract_tile<TCY, T, X3>(N, D, gy, gyl, (const T*)gb.xt, (const T*)gb.xt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_y, lds, osc, kbeg, klen);
+                                     sp.accumulate != 0, acc_y, lds, osc, kbeg, klen, sp.seg);
   }
 }
 

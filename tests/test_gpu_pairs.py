@@ -174,6 +174,63 @@ def test_off_diagonal_sums_are_as_exact_as_in_fp32(n, d, t, noise):
         assert p <= 1.1 * f
 
 
+def stages(x, y, t, dt, mode):
+    """acc_x, acc_y of mec_forward + mec_grad on normalized x, y."""
+    lib, (n, d) = _lib.load(), x.shape
+    st = torch.cuda.current_stream().cuda_stream
+    ws = torch.empty(lib.mec_workspace_floats_for(n, d, dt), device=DEV)
+    loss = torch.empty((), device=DEV)
+    nbytes = lib.mec_grad_scratch_bytes(n, d, dt)
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    acc = torch.empty(n, d, device=DEV), torch.empty(n, d, device=DEV)
+    _lib.call("mec_forward", x.data_ptr(), d, y.data_ptr(), d, n, d, dt, mode, 0, t, ws.data_ptr(), loss.data_ptr(), st)
+    _lib.call("mec_grad", x.data_ptr(), d, y.data_ptr(), d, n, d, dt, mode, 0, t, ws.data_ptr(), scratch.data_ptr(),
+              nbytes, acc[0].data_ptr(), acc[1].data_ptr(), st)
+    torch.cuda.synchronize()
+    return acc if mode == _lib.MODE_CLIP else acc[:1]
+
+
+def dense_sums(x, y, t, mode):
+    """The off-diagonal sums of stages() by definition, in 64 bits."""
+    xh, yh = x.double(), y.double()
+    e = torch.exp((xh @ yh.T - 1.0) / t)
+    gm = e / e.sum(1, keepdim=True)
+    if mode == _lib.MODE_CLIP:
+        gm += e / e.sum(0, keepdim=True)
+    gm.fill_diagonal_(0.0)
+    if mode == _lib.MODE_CLIP:
+        return gm @ yh, gm.T.contiguous() @ xh
+    return (gm @ yh,)
+
+
+def features(kind, n, d):
+    """Unit rows x and y, a pair's cosine about 0.3: of either sign, positive,
+    or at least 0 with half the values 0 (what follows a ReLU)."""
+    g = torch.Generator(device=DEV).manual_seed(n + d)
+    f = {"normal": lambda v: v, "positive": torch.abs, "relu": torch.relu}[kind]
+    x, z = (torch.nn.functional.normalize(f(torch.randn(n, d, generator=g, device=DEV)), dim=1) for _ in range(2))
+    return x, torch.nn.functional.normalize(x + 3.0 * z, dim=1)
+
+
+# (4200 and 8192 rows: one block of pairs, three and two blocks of the fp32
+# kernels; 4999 with its contractions split over k; 2300 in 128 x 128 tiles)
+@pytest.mark.parametrize("mode", ["clip", "lit"])
+@pytest.mark.parametrize("kind,n,d", [("positive", 4200, 512), ("relu", 4200, 512), ("normal", 4200, 512),
+                                      ("positive", 8192, 256), ("positive", 4999, 640), ("positive", 2300, 128)])
+def test_no_further_from_64_bits_than_fp32(kind, n, d, mode):
+    """Sums that grow with every term round the most, and the more the longer
+    they are: those of the pairs, in pieces of the fp32 kernels' blocks, end no
+    further from 64 bits than the fp32 kernels' (one sum per block of pairs:
+    1.9 times as far)."""
+    m = _lib.MODE_CLIP if mode == "clip" else _lib.MODE_LIT
+    x, y = features(kind, n, d)
+    ref = dense_sums(x, y, 0.07, m)
+    f, p = ([((a.double() - r).norm() / r.norm()).item() for a, r in zip(stages(x, y, 0.07, dt, m), ref)]
+            for dt in (_lib.DTYPE_F32, _lib.DTYPE_F32_PAIRS))
+    say(f"{kind} {mode} n={n} d={d}: fp32 {f}, pairs {p}")
+    assert all(a <= b for a, b in zip(p, f))
+
+
 def test_noalloc_and_one_side(pairs):
     """mec_backward_noalloc and a frozen tower, bitwise as mec_backward with both
     sides (unsplit: each chooses its own split of the contractions)."""
