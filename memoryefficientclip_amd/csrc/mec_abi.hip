@@ -1020,8 +1020,12 @@ static int sumexp_run(const void* x, int64_t ldx, const void* y, int64_t ldy, in
     const bool small = small16_tiles(n, dtype);
     const int bm = fwd_tile_dims(dtype, true, small).bm;
     const int tiles = (int)((n + bm - 1) / bm), dk = 2 * pr.dp;
-    return sumexp_det_run<F16S>(pr.a, dk, pr.b, dk, n, dk, is_lit(mode), false, true, small, c, workspace, pr.scl, tiles,
-                                tiles, s, dp);
+    rc = sumexp_det_run<F16S>(pr.a, dk, pr.b, dk, n, dk, is_lit(mode), false, true, small, c, workspace, pr.scl, tiles,
+                              tiles, s, dp);
+    if (rc || dp) return rc;
+    DISPATCH_BOOL(is_lit(mode), LIT, k_pair_range<LIT><<<(unsigned)((n + 255) / 256), 256, 0, s>>>(
+                                         (int)n, 1.0 / (double)temperature, workspace, pr.scl));
+    return check_launch("pair range");
   }
   x = g.x, ldx = g.ldx, y = g.y, ldy = g.ldy, d = g.d, dtype = g.dtype;
   const int N = (int)n, D = (int)d;
@@ -1149,7 +1153,8 @@ int mec_forward(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t 
   double* partial = (double*)(workspace + (int64_t)WS_NSLOTS * n);
   DISPATCH_BOOL(is_lit(mode), LIT, DISPATCH_BOOL(dp.Q > 0, DET, {
     k_finalize_all<LIT, DET><<<blocks, DET ? 4 * FIN_ROWS : FIN_ROWS, 0, (hipStream_t)stream>>>(
-        (int)n, inv_t, workspace, dp.rowpart, dp.Q, dp.colpart, dp.P, partial, counter, loss);
+        (int)n, inv_t, workspace, dp.rowpart, dp.Q, dp.colpart, dp.P, partial, counter, loss,
+        is_pairs(dtype) ? pair_scl(workspace, n) : nullptr);
   }));
   return check_launch("finalize");
 }
@@ -1324,7 +1329,7 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
       const TS tx{(const float*)x, ldx, workspace + WS_RX * n64, (uint16_t*)gb.xt, nullptr};
       DISPATCH_BOOL(normalize, NORM, k_transpose_pairs<NORM><<<tgrid, 256, 0, s>>>(
                                          acc_x ? ty : tx, tx, N, D, L.ldt, gb.scl + (acc_x ? SCL_Y : SCL_X),
-                                         gb.scl + SCL_X, workspace + WS_KAPPA * n64, (float*)(base + L.gs)));
+                                         gb.scl + SCL_X, gb.scl, (float*)(base + L.gs)));
     } else if (split) {
       using TS = TransSide<float, uint16_t>;
       const TS ty{(const float*)y, ldy, workspace + WS_RY * n64, (uint16_t*)gb.yt, (uint16_t*)gb.yt_lo};

@@ -52,6 +52,12 @@ constexpr int FIN_ROWS = 256;  // rows per workgroup of the loss finalize (one p
 // column)
 constexpr int DET_P = 32, DET_Q = 16;
 
+// The words that go with the pairs in the workspace (PairRows::scl): the
+// scales of x and y, their inverses, and of the finalize's rows the largest
+// |kappa_i| and the smallest off-diagonal share, row_off_i / R_i or col_off_i /
+// C_i (CLIP), as the bits of floats that are not negative (integer atomics).
+enum { SCL_X = 0, SCL_Y = 1, SCL_INVX = 2, SCL_INVY = 3, SCL_KMAX = 4, SCL_SMIN = 5 };
+
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) {

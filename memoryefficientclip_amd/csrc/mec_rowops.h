@@ -55,6 +55,67 @@ __device__ __forceinline__ void store_vec(T* __restrict__ p, const float (&v)[kV
   }
 }
 
+// How the gradient matrix of split pairs is stored: its scale, the scale's
+// inverse, and whether as fp32 values (wide) instead of pairs.
+//
+// A pair holds v with an error of at most 2^-23 |v| or 2^-25, whichever is
+// larger, so a matrix of pairs has one scale for all of it: the largest 2^k with
+// 2^k G'_ij <= 2^15 that the row sums allow, at least 2^14 (G' <= 2): G'_ij =
+// E_ij (1/R_i + 1/C_j) <= row_off_i / R_i + col_off_j / C_j <= 2 max |kappa|.
+// Row i of the gradient is a sum of terms whose sizes add up to at least its
+// share s_i = row_off_i / R_i (columns: col_off_j / C_j), to which N entries
+// off by 2^-25-k each (of either sign) add an error of about sqrt(N) 2^-25-k.
+// With 2^k s_i >= sqrt(N) that is no more than 2^-25 s_i, an fp32 rounding.
+// Where one row has less (pairs that match well beside one that does not: the
+// small shares' entries fall below fp16's range, the lo parts first), or the
+// scale stops at 2^40, the matrix is held wide, at fp32's range and precision,
+// and contracted as three bf16 terms (mec_gemm_wide.h).  Distance of a row's
+// off-diagonal sum from 64 bits, the largest over the rows, fp32 kernels, pairs
+// throughout, this rule: 4097 x 768, T = 0.03, two y rows swapped: 3.9e-6, 1.0
+// (nothing left of it), 3.5e-6; 4200 x 512, T = 0.02, all pairs matching (loss
+// 4e-16) 9.0e-6, 0.12, 8.9e-6.
+struct PairGrad {
+  float scale, inv;
+  bool wide;
+};
+constexpr int PAIR_G_MIN_EXP = -26;
+__device__ __forceinline__ PairGrad pair_grad_scale(int N, const float* __restrict__ scl) {
+  const float m = scl[SCL_KMAX], smin = scl[SCL_SMIN];
+  int e = 0;  // 2 max |kappa| < 2^(e + 1)
+  if (m < 0.5f) (void)frexpf(fmaxf(m, ldexpf(1.f, PAIR_G_MIN_EXP)), &e);
+  PairGrad g{ldexpf(1.f, 14 - e), ldexpf(1.f, e - 14), false};
+  if (!(g.scale * smin >= sqrtf((float)N))) {
+    // (2^40: entries down to fp32's smallest keep their lower terms)
+    g = PairGrad{ldexpf(1.f, 40), ldexpf(1.f, -40), true};
+  }
+  return g;
+}
+// The rows of a workgroup's first NW waves into SCL_KMAX and SCL_SMIN (k: |kappa|,
+// s: share; 0 and infinity without a row; every thread calls it): one atomic of
+// each per workgroup (one per wave was 10 us of atomics at n = 32768).
+template <int NW>
+__device__ __forceinline__ void pair_grad_range(float k, float s, float* __restrict__ scl) {
+  __shared__ float s_k[NW], s_s[NW];
+  for (int o = 32; o >= 1; o >>= 1) {
+    k = fmaxf(k, __shfl_xor(k, o, 64));
+    s = fminf(s, __shfl_xor(s, o, 64));
+  }
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0 && w < NW) {
+    s_k[w] = k;
+    s_s[w] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int q = 1; q < NW; ++q) {
+      k = fmaxf(k, s_k[q]);
+      s = fminf(s, s_s[q]);
+    }
+    atomicMax((unsigned int*)(scl + SCL_KMAX), __float_as_uint(k));
+    atomicMin((unsigned int*)(scl + SCL_SMIN), __float_as_uint(s));
+  }
+}
+
 // Per row i: rx = 1/max(||x_i||, 1e-12) (or 1), ry likewise, diag = x_i . y_i.
 // Also clears the off-diagonal sum accumulators used by the sum-exp kernel.
 // Follows F.normalize(dim=1) as applied at clip_loss.py:266-268 and the
@@ -137,10 +198,19 @@ __device__ __forceinline__ double softplus_log_ratio(double off, double t) {
   return u > 0.0 ? u + log1p(exp(-u)) : log1p(exp(u));
 }
 
-// The loss term of row i (a CLIP row and column, or a LiT row), and 1/R_i,
-// 1/C_i and kappa_i into the workspace.
+// The off-diagonal share of row i's sum, and of column i's where that is less
+// (CLIP): the smallest of what pair_grad_scale is told of.
 template <bool LIT>
-__device__ __forceinline__ double finalize_row(int i, int64_t n, double inv_t, float* __restrict__ ws) {
+__device__ __forceinline__ float least_share(double ro, double R, double co, double C) {
+  const float r = (float)(ro / R);
+  return LIT ? r : fminf(r, (float)(co / C));
+}
+
+// The loss term of row i (a CLIP row and column, or a LiT row), and 1/R_i,
+// 1/C_i and kappa_i into the workspace; -kappa_i and least_share.
+template <bool LIT>
+__device__ __forceinline__ double finalize_row(int i, int64_t n, double inv_t, float* __restrict__ ws, float& kout,
+                                               float& sout) {
   const double s = (double)ws[WS_DIAG * n + i] * (double)ws[WS_RX * n + i] * (double)ws[WS_RY * n + i];
   const double t = (s - 1.0) * inv_t;
   const double e = exp(t);
@@ -149,14 +219,17 @@ __device__ __forceinline__ double finalize_row(int i, int64_t n, double inv_t, f
   double acc = softplus_log_ratio(ro, t);
   ws[WS_INV_ROW * n + i] = (float)(1.0 / R);
   double kap = -(ro / R);
+  double co = 0.0, C = 1.0;
   if (!LIT) {
-    const double co = ws[WS_COL_OFF * n + i];
-    const double C = co + e;
+    co = ws[WS_COL_OFF * n + i];
+    C = co + e;
     acc += softplus_log_ratio(co, t);
     ws[WS_INV_COL * n + i] = (float)(1.0 / C);
     kap -= co / C;
   }
   ws[WS_KAPPA * n + i] = (float)kap;
+  kout = -(float)kap;
+  sout = least_share<LIT>(ro, R, co, C);
   return acc;
 }
 
@@ -178,7 +251,8 @@ __global__ __launch_bounds__(SINGLE ? FIN_SINGLE_ROWS : FIN_ROWS) void k_finaliz
   __shared__ double red[NT / 64];
   const int64_t n = N;
   const int i = blockIdx.x * NT + threadIdx.x;
-  double acc = i < N ? finalize_row<LIT>(i, n, inv_t, ws) : 0.0;
+  float kap, share;
+  double acc = i < N ? finalize_row<LIT>(i, n, inv_t, ws, kap, share) : 0.0;
   acc = wave_sum_f64(acc);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if (lane == 0) red[w] = acc;
@@ -218,13 +292,15 @@ __global__ __launch_bounds__(1024) void k_finalize_sum(int N, int nparts, const 
 // and the last workgroup to arrive at `counter` (zeroed by the pre-pass) adds
 // the partials in order and writes the loss.  The counter is the loss word
 // itself, which nobody reads before the launch ends.  The handshake is a
-// release / acquire of one thread per workgroup.  Latency-bound: as separate
+// release / acquire of one thread per workgroup.  pair_scl (split pairs, else
+// null) gets the rows' range (pair_grad_range).  Latency-bound: as separate
 // launches (k_det_reduce with one thread per row adding 48 partials one after
 // the other, rows, sum) it took 11 + 5 + 5 us at n = 6001, 16 + 5 + 5 us at 8192.
 template <bool LIT, bool DET>
 __global__ __launch_bounds__(DET ? 4 * FIN_ROWS : FIN_ROWS) void k_finalize_all(
     int N, double inv_t, float* __restrict__ ws, const float* __restrict__ rowpart, int Q,
-    const float* __restrict__ colpart, int P, double* partial, uint32_t* counter, float* loss) {
+    const float* __restrict__ colpart, int P, double* partial, uint32_t* counter, float* loss,
+    float* __restrict__ pair_scl) {
   constexpr int NT = DET ? 4 * FIN_ROWS : FIN_ROWS;
   constexpr int MQ = DET_Q / 4, MP = DET_P / 4;
   __shared__ float s_r[DET ? 4 : 1][FIN_ROWS], s_c[DET ? 4 : 1][FIN_ROWS];
@@ -259,7 +335,9 @@ __global__ __launch_bounds__(DET ? 4 * FIN_ROWS : FIN_ROWS) void k_finalize_all(
     }
   }
   // (the same thread reads back what it wrote)
-  double acc = q == 0 && i < N ? finalize_row<LIT>(i, n, inv_t, ws) : 0.0;
+  float kap = 0.f, share = __builtin_inff();
+  double acc = q == 0 && i < N ? finalize_row<LIT>(i, n, inv_t, ws, kap, share) : 0.0;
+  if (pair_scl) pair_grad_range<FIN_ROWS / 64>(kap, share, pair_scl);
   acc = wave_sum_f64(acc);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if (lane == 0) red[w] = acc;
@@ -759,6 +837,10 @@ __global__ __launch_bounds__(256) void k_pair_prepass(const float* __restrict__ 
                                                       uint32_t* __restrict__ counter) {
   __shared__ float s_mx[2][4];
   if (counter && blockIdx.x == 0 && threadIdx.x == 0) *counter = 0u;  // (k_finalize_all)
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // (pair_grad_range)
+    pr.scl[SCL_KMAX] = 0.f;
+    pr.scl[SCL_SMIN] = __builtin_inff();
+  }
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int row = blockIdx.x * 4 + w;
   const int64_t n = N;
@@ -893,38 +975,34 @@ __global__ __launch_bounds__(256) void k_pair_rows(const float* __restrict__ X, 
   }
 }
 
-// The scale of the gradient matrix's pairs, for one workgroup of 256 threads:
-// gscl = {2^k, 2^-k}, the largest with 2^k G'_ij <= 2^15 that the row sums
-// allow, at least 2^14 (G' <= 2).  G'_ij = E_ij (1/R_i + 1/C_j) <= row_off_i /
-// R_i + col_off_j / C_j <= 2 max |kappa|.  Where the pairs match well (small
-// off-diagonal sums) the entries are small against 2, and under the fixed scale
-// 2^14 their lo parts, then their hi parts, fell below fp16's range.
-constexpr int PAIR_G_MIN_EXP = -26;
-__device__ __forceinline__ void pair_grad_scale(int N, const float* __restrict__ kappa, float* gscl) {
-  __shared__ float s_m[4];
-  float m = 0.f;
-#pragma unroll 8
-  for (int k = threadIdx.x; k < N; k += 256) m = fmaxf(m, -kappa[k]);
-  for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int e = 0;  // 2 max |kappa| < 2^(e + 1)
-    m = fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3]));
-    if (m < 0.5f) (void)frexpf(fmaxf(m, ldexpf(1.f, PAIR_G_MIN_EXP)), &e);
-    gscl[0] = ldexpf(1.f, 14 - e);
-    gscl[1] = ldexpf(1.f, e - 14);
+// pair_grad_range of the rows' sums for a forward run stage by stage
+// (mec_sumexp; mec_forward's finalize does it on the way): one thread per row.
+template <bool LIT>
+__global__ __launch_bounds__(256) void k_pair_range(int N, double inv_t, const float* __restrict__ ws,
+                                                    float* __restrict__ scl) {
+  const int64_t n = N;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  float k = 0.f, s = __builtin_inff();
+  if (i < N) {
+    const double e = exp(((double)ws[WS_DIAG * n + i] * (double)ws[WS_RX * n + i] * (double)ws[WS_RY * n + i] - 1.0) *
+                         inv_t);
+    const double ro = ws[WS_ROW_OFF * n + i], co = LIT ? 0.0 : (double)ws[WS_COL_OFF * n + i];
+    k = (float)(ro / (ro + e)) + (LIT ? 0.f : (float)(co / (co + e)));
+    s = least_share<LIT>(ro, ro + e, co, co + e);
   }
+  pair_grad_range<4>(k, s, scl);
 }
 
 // k_transpose_split into pairs: row d of XT (pitch 2 ldt) holds, for every 32
 // rows i, 32 hi and then 32 lo values of scale_i x_i[d] (NORM) times the side's
 // pair scale, zero for N <= i < ldt (ldt a multiple of 64).  Two values of i
-// per thread: 4-byte stores, 64 contiguous bytes per part.
+// per thread: 4-byte stores, 64 contiguous bytes per part.  Where the gradient
+// matrix is held wide: the values themselves, fp32, row d of pitch ldt.  The
+// first workgroup leaves the gradient matrix's scale in gscl (GradBufs).
 template <bool NORM>
 __global__ __launch_bounds__(256) void k_transpose_pairs(TransSide<float, uint16_t> s0, TransSide<float, uint16_t> s1,
                                                          int N, int D, int64_t ldt, const float* scl0,
-                                                         const float* scl1, const float* __restrict__ kappa,
+                                                         const float* scl1, const float* __restrict__ scl,
                                                          float* gscl) {
   const TransSide<float, uint16_t>& sd = blockIdx.z ? s1 : s0;
   const float ps = blockIdx.z ? *scl1 : *scl0;
@@ -945,7 +1023,18 @@ __global__ __launch_bounds__(256) void k_transpose_pairs(TransSide<float, uint16
     }
     tile[r][tx] = v;
   }
+  const PairGrad pg = pair_grad_scale(N, scl);
+  if (blockIdx.x + blockIdx.y + blockIdx.z + threadIdx.x == 0) {
+    gscl[0] = pg.scale;
+    gscl[1] = pg.inv;
+    gscl[2] = pg.wide ? 1.f : 0.f;
+  }
   __syncthreads();
+  if (pg.wide) {
+    float* __restrict__ XW = (float*)XT;
+    for (int r = ty; r < 64 && d0 + r < D; r += 4) XW[(int64_t)(d0 + r) * ldt + i0 + tx] = tile[tx][r];
+    return;
+  }
   const int il = 2 * (threadIdx.x & 31);
   for (int r = threadIdx.x >> 5; r < 64; r += 8) {
     const int d = d0 + r;
@@ -956,7 +1045,6 @@ __global__ __launch_bounds__(256) void k_transpose_pairs(TransSide<float, uint16
     *(uint32_t*)o = pack2_f16(ha, hb);
     *(uint32_t*)(o + 32) = pack2_f16(__builtin_isinf(ha) ? 0.f : a - ha, __builtin_isinf(hb) ? 0.f : b - hb);
   }
-  if (blockIdx.x + blockIdx.y + blockIdx.z == 0) pair_grad_scale(N, kappa, gscl);
 }
 
 }  // namespace mec

@@ -191,16 +191,21 @@ def stages(x, y, t, dt, mode):
 
 
 def dense_sums(x, y, t, mode):
-    """The off-diagonal sums of stages() by definition, in 64 bits."""
+    """The off-diagonal sums of stages() by definition, in 64 bits, and the
+    diagonal coefficient kappa."""
     xh, yh = x.double(), y.double()
     e = torch.exp((xh @ yh.T - 1.0) / t)
     gm = e / e.sum(1, keepdim=True)
     if mode == _lib.MODE_CLIP:
         gm += e / e.sum(0, keepdim=True)
+    # kappa from the off-diagonal shares (as 1 - p_ii it would cancel)
+    r, c = e.sum(1), e.sum(0)
+    e.fill_diagonal_(0.0)
+    kappa = -e.sum(1) / r - (e.sum(0) / c if mode == _lib.MODE_CLIP else 0.0)
     gm.fill_diagonal_(0.0)
     if mode == _lib.MODE_CLIP:
-        return gm @ yh, gm.T.contiguous() @ xh
-    return (gm @ yh,)
+        return (gm @ yh, gm.T.contiguous() @ xh), kappa
+    return (gm @ yh,), kappa
 
 
 def features(kind, n, d):
@@ -224,11 +229,106 @@ def test_no_further_from_64_bits_than_fp32(kind, n, d, mode):
     1.9 times as far)."""
     m = _lib.MODE_CLIP if mode == "clip" else _lib.MODE_LIT
     x, y = features(kind, n, d)
-    ref = dense_sums(x, y, 0.07, m)
+    ref, _ = dense_sums(x, y, 0.07, m)
     f, p = ([((a.double() - r).norm() / r.norm()).item() for a, r in zip(stages(x, y, 0.07, dt, m), ref)]
             for dt in (_lib.DTYPE_F32, _lib.DTYPE_F32_PAIRS))
     say(f"{kind} {mode} n={n} d={d}: fp32 {f}, pairs {p}")
     assert all(a <= b for a, b in zip(p, f))
+
+
+def held_wide(ws, n):
+    """The rule of pair_grad_scale on what the forward left in its workspace:
+    the largest |kappa| and the smallest off-diagonal share."""
+    off = (_lib.load().mec_workspace_floats(n) + 63) // 64 * 64
+    kmax, smin = ws[off + 4:off + 6].cpu().numpy().astype(np.float64)
+    e = 0 if kmax >= 0.5 else np.frexp(max(kmax, 2.0 ** -26))[1]
+    return not 2.0 ** (14 - e) * smin >= np.sqrt(n)
+
+
+def matching(kind, n, d, seed=1):
+    """Unit rows whose pairs match well: all of them, all but two that are
+    swapped, or all but one that has nothing to do with any other."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+
+    def unit(v):
+        return torch.nn.functional.normalize(v, dim=1)
+
+    x, z = (unit(torch.randn(n, d, generator=g, device=DEV)) for _ in range(2))
+    y = unit(x + 0.4 * z)
+    if kind == "swapped":
+        y[[0, n // 2]] = y[[n // 2, 0]]
+    elif kind == "stray":
+        y[n // 3] = unit(torch.randn(1, d, generator=g, device=DEV))[0]
+    return x, y
+
+
+def row_errors(a, ref):
+    return ((a.double() - ref).norm(dim=1) / ref.norm(dim=1)).cpu()
+
+
+@pytest.mark.parametrize("mode", ["clip", "lit"])
+@pytest.mark.parametrize("kind,n,d,t", [("swapped", 4097, 768, 0.03), ("swapped", 4097, 768, 0.02),
+                                        ("stray", 4200, 512, 0.03), ("matching", 4200, 512, 0.02),
+                                        ("swapped", 2300, 200, 0.03), ("swapped", 8192, 320, 0.04)])
+def test_every_row_is_as_exact_as_in_fp32(kind, n, d, t, mode):
+    """Batches whose rows' off-diagonal shares lie far apart, or are all tiny:
+    under one scale the small rows' entries fell below fp16's range (4097 x 768,
+    T = 0.03: nothing was left of most rows' sums).  Every row's sum on its own,
+    against 64 bits."""
+    m = _lib.MODE_CLIP if mode == "clip" else _lib.MODE_LIT
+    x, y = matching(kind, n, d)
+    ref, _ = dense_sums(x, y, t, m)
+    for side in range(len(ref)):
+        f, p = (row_errors(stages(x, y, t, dt, m)[side], ref[side]) for dt in (_lib.DTYPE_F32, _lib.DTYPE_F32_PAIRS))
+        say(f"{kind} {mode} n={n} d={d} T={t} side {side}: rows' errors, median and largest: "
+            f"fp32 {f.median():.2e} {f.max():.2e}, pairs {p.median():.2e} {p.max():.2e}")
+        # (the largest of n rows: two draws of the same rounding differ)
+        assert p.median() <= f.median() and p.max() <= 1.5 * f.max()
+
+
+# as CASES, with the parts of the contractions (0: the default)
+WIDE = [("clip", 2, 33, False, 0, 0, 0), ("clip", 31, 31, False, 3, 0, 0), ("lit", 255, 32, True, 0, 0, 0),
+        ("clip", 257, 130, False, 1, 0, 0), ("lit", 513, 255, True, 0, 1, 3), ("clip", 1300, 257, False, 0, 2, 0),
+        ("clip", 2049, 320, True, 5, 3, 2), ("clip", 2600, 512, False, 0, 0, 4), ("clip", 3001, 100, False, 0, 4, 8),
+        ("lit", 4097, 600, False, 0, 0, 0)]
+
+
+@pytest.mark.parametrize("mode,n,d,normed,pad,tb,parts", WIDE, ids=[f"{c[0]}-{c[1]}x{c[2]}" for c in WIDE])
+def test_wide_matrix_against_the_definition(pairs, mode, n, d, normed, pad, tb, parts):
+    """Gradient matrices that are held wide, at the edges of tiles, chunks, blocks
+    and parts.  Bar, row by row: S of unit rows, sums that stay below 1, is off by
+    about 2 x 2^-24 and the exponent (S - 1) / T by 2^-24 of itself (S > -0.5), an
+    entry of G' by twice their sum (its E and its R), and a row that matches well
+    loses up to 2 / |x^ - y^| (about 5 here) to the normalisation backward."""
+    lit = mode == "lit"
+    t = 0.03
+    if tb:
+        pairs.setenv("MEC_GRAD_BLOCK_TILES", str(tb))
+    if parts:
+        pairs.setenv("MEC_CONTRACT_PARTS", str(parts))
+    x, y = matching("swapped" if n > 2 else "matching", n, d)
+    if not normed:
+        g = torch.Generator(device=DEV).manual_seed(7)
+        x, y = (v * torch.exp(torch.randn(n, 1, generator=g, device=DEV)) for v in (x, y))
+    wx, wy = torch.zeros(n, d + pad, device=DEV), torch.zeros(n, d + pad, device=DEV)
+    wx[:, pad:], wy[:, pad:] = x, y
+    gx, gy = wx[:, pad:].requires_grad_(True), wy[:, pad:].requires_grad_(not lit)
+    say(f"wide {mode} n={n} d={d} normed={normed} pad={pad} blocks={tb} parts={parts}")
+    loss = (MemoryEfficientLiTLoss if lit else MemoryEfficientCLIPLoss)(t, normed)(gx, gy)
+    assert loss.grad_fn.mec[4] == _lib.DTYPE_F32_PAIRS
+    assert held_wide(loss.grad_fn.saved_tensors[2], n)
+    loss.backward()
+    norms = [torch.ones(n, 1, device=DEV).double() if normed else v.double().norm(dim=1, keepdim=True) for v in (x, y)]
+    xh, yh = x.double() / norms[0], y.double() / norms[1]
+    sums, kappa = dense_sums(xh, yh, t, _lib.MODE_LIT if lit else _lib.MODE_CLIP)
+    bar = 5 * 2 * (2 + 1.5) * 2.0 ** -24 / t
+    for a, own, oth, nrm, acc in zip([gx.grad, gy.grad], [xh, yh], [yh, xh], norms, sums):
+        r = (acc + kappa[:, None] * oth) / (n * t * (1 if lit else 2))
+        if not normed:
+            r = (r - own * (own * r).sum(1, keepdim=True)) / nrm
+        e = row_errors(a, r)
+        say(f"  rows' errors: median {e.median():.2e}, largest {e.max():.2e} (bar {bar:.2e})")
+        assert e.max() <= bar
 
 
 def test_noalloc_and_one_side(pairs):
