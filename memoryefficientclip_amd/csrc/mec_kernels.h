@@ -281,14 +281,20 @@ template <> struct GScale<_Float16> { static constexpr float value = 16384.f; };
 // The scales of the split pairs: x and y are multiplied by the powers of two
 // scl[0] and scl[1] before they are split (so that the lo parts stay within
 // fp16's range), scl[2] and scl[3] are their inverses.  Exponent multiplier of
-// the accumulated similarities: c, times the inverse scales of split pairs.
+// the accumulated similarities: c, times the inverse scales of split pairs.  Two
+// sides of very large values can take that product past fp32: the largest finite
+// number then, so that rows with no product (S = 0) keep S = 0, and any other S
+// is an overflow as in fp32.  (Two of very small values: 0, where S < 2^-90.)
 template <typename T>
 __device__ __forceinline__ float exp_mul(float c, const float* __restrict__ scl) {
   if constexpr (IsSplit<T>::value)
-    return c * scl[SCL_INVX] * scl[SCL_INVY];
+    return fminf(c * (scl[SCL_INVX] * scl[SCL_INVY]), 3.402823466e38f);
   else
     return c;
 }
+
+// k of 2^k, a normal number
+__device__ __forceinline__ int exp_of(float p) { return (int)(__float_as_uint(p) >> 23) - 127; }
 
 // workgroups per CU the launch bounds promise (the 16-bit direct-load tiles
 // use 96 KB of LDS or more: one per CU)
@@ -1008,10 +1014,11 @@ __device__ __forceinline__ void contract_store(const f32x16 (&acc)[TC::FM][TC::F
 // contract_store in a loop: the addresses and masks of the 128 elements are
 // formed anew each time, with one branch on `accumulate` (kept across the k-loop
 // between, and with a branch per element, they spilled; once per tile the branch
-// per element takes fewer registers).
+// per element takes fewer registers).  Times 2^oe: the inverse scales of the
+// gradient matrix and of an input, whose product may be no fp32 number.
 template <class TC>
 __device__ __forceinline__ void contract_store_again(const f32x16 (&acc)[TC::FM][TC::FN], int r0, int d0, int N, int D,
-                                                     bool accumulate, float* __restrict__ out, float osc) {
+                                                     bool accumulate, float* __restrict__ out, int oe) {
   int lane = threadIdx.x & 63;
   asm volatile("" : "+v"(lane));
   const int w = threadIdx.x >> 6, wm = w / TC::WN, wn = w % TC::WN;
@@ -1024,7 +1031,7 @@ __device__ __forceinline__ void contract_store_again(const f32x16 (&acc)[TC::FM]
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int row = r0 + wm * TC::TM + bm * 32 + acc_row(r, lane);
-          if (row < N && d < D) put(out + (int64_t)row * D + d, acc[bm][bn][r] * osc);
+          if (row < N && d < D) put(out + (int64_t)row * D + d, __builtin_ldexpf(acc[bm][bn][r], oe));
         }
       }
     }
@@ -1051,15 +1058,16 @@ __device__ __forceinline__ void contract_store_again(const f32x16 (&acc)[TC::FM]
 // atomics, clip_loss.py:148-156).
 // X3 (bf16x3): Gblk/OT are the hi planes and Glo/OTlo the lo planes; the
 // tile is hi.hi + hi.lo + lo.hi, three passes over K into one accumulator.
-// osc: the inverse of the operands' storage scales (a power of two).
+// osc, or 2^oe (split pairs): the inverse of the operands' storage scales (a
+// power of two).
 // Only k rows [kbeg, kbeg + klen) of the block.
 template <class TC, typename T, bool X3 = false>
 __device__ __forceinline__ void grad_contract_piece(int N, int D, const T* __restrict__ Gblk,
                                                    const T* __restrict__ Glo, const T* __restrict__ OT,
                                                    const T* __restrict__ OTlo, int64_t ldt, const BlockGrid& bg,
                                                    int P, int Q, int tm, int td, bool accumulate,
-                                                   float* __restrict__ out, char* lds, float osc, int kbeg,
-                                                   int klen) {
+                                                   float* __restrict__ out, char* lds, float osc, int oe,
+                                                   int kbeg, int klen) {
   const int r0 = P * bg.bs + tm * TC::BM;
   if (r0 >= N) return;
   const int d0 = td * TC::BN;
@@ -1101,7 +1109,7 @@ __device__ __forceinline__ void grad_contract_piece(int N, int D, const T* __res
     TC::template run<true, true, false>(tile_op<TC>(Glo + a_off, bg.bs, TC::BM, kq), B, kq, lds, acc);
   }
   if constexpr (SPL)
-    contract_store_again<TC>(acc, r0, d0, N, D, accumulate, out, osc);
+    contract_store_again<TC>(acc, r0, d0, N, D, accumulate, out, oe);
   else
     contract_store<TC>(acc, r0, d0, N, D, accumulate, out, osc);
 }
@@ -1118,21 +1126,21 @@ __device__ __forceinline__ void grad_contract_tile(int N, int D, const T* __rest
                                                    const T* __restrict__ Glo, const T* __restrict__ OT,
                                                    const T* __restrict__ OTlo, int64_t ldt, const BlockGrid& bg,
                                                    int P, int Q, int tm, int td, bool accumulate,
-                                                   float* __restrict__ out, char* lds, float osc, int kbeg, int klen,
-                                                   int seg) {
+                                                   float* __restrict__ out, char* lds, float osc, int oe,
+                                                   int kbeg, int klen, int seg) {
   if constexpr (IsSplit<T>::value) {
     const int kend = min(min(bg.bs, N - Q * bg.bs), kbeg + klen);
     for (int k = kbeg;;) {
       grad_contract_piece<TC, T, X3>(N, D, Gblk, Glo, OT, OTlo, ldt, bg, P, Q, tm, td, accumulate || k > kbeg, out,
-                                     lds, osc, k, min(seg, klen));
+                                     lds, osc, oe, k, min(seg, klen));
       k += seg;
       if (k >= kend) break;
       klen -= seg;
       __syncthreads();  // every wave is past its last read of the ring
     }
   } else {
-    grad_contract_piece<TC, T, X3>(N, D, Gblk, Glo, OT, OTlo, ldt, bg, P, Q, tm, td, accumulate, out, lds, osc, kbeg,
-                                   klen);
+    grad_contract_piece<TC, T, X3>(N, D, Gblk, Glo, OT, OTlo, ldt, bg, P, Q, tm, td, accumulate, out, lds, osc, oe,
+                                   kbeg, klen);
   }
 }
 
@@ -1143,7 +1151,7 @@ template <int B>
 __device__ __forceinline__ void grad_contract_wide(bool xside, int N, int D, const float* __restrict__ G,
                                                    const float* __restrict__ OT, int64_t ldt, const BlockGrid& bg,
                                                    int P, int Q, int tm, int td, bool accumulate,
-                                                   float* __restrict__ out, char* lds, float osc, int kbeg, int klen,
+                                                   float* __restrict__ out, char* lds, int oe, int kbeg, int klen,
                                                    int seg) {
   using TL = gwide::Tile<B>;
   const int r0 = P * bg.bs + tm * B, d0 = td * B, q0 = Q * bg.bs;
@@ -1165,7 +1173,7 @@ __device__ __forceinline__ void grad_contract_wide(bool xside, int N, int D, con
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     }
-    contract_store_again<TL>(acc, r0, d0, N, D, accumulate || k > kbeg, out, osc);
+    contract_store_again<TL>(acc, r0, d0, N, D, accumulate || k > kbeg, out, oe);
     if (k + seg >= kend) break;
   }
 }
@@ -1181,7 +1189,9 @@ __device__ __forceinline__ void grad_contract_dispatch(int sub, int N, int D, co
   const int64_t blk = (int64_t)bg.bs * bg.bs * (IsSplit<T>::value ? 2 : 1);  // elements per G' block
   const bool is_x = sub < sp.cx_pad;
   float osc = 1.f / GScale<T>::value;
-  if constexpr (IsSplit<T>::value) osc = gb.gscl[1] * gb.scl[is_x ? SCL_INVY : SCL_INVX];
+  int oe = 0;
+  if constexpr (IsSplit<T>::value)
+    oe = __builtin_amdgcn_readfirstlane(exp_of(gb.gscl[1]) + exp_of(gb.scl[is_x ? SCL_INVY : SCL_INVX]));
   if (!is_x) sub -= sp.cx_pad;
   const int pid = xcd_remap(sub, is_x ? sp.cx_pad : sp.cy_pad);
   if (pid >= (is_x ? sp.cx_n : sp.cy_n)) return;
@@ -1244,7 +1254,7 @@ __device__ __forceinline__ void grad_contract_dispatch(int sub, int N, int D, co
           __builtin_amdgcn_readfirstlane(is_x ? (P + sp.diag_c) % bg.nb : (P - sp.diag_c + bg.nb) % bg.nb);
       const float* g = (const float*)gb.gt[buf] + (is_x ? P : Q) * wblk;
       grad_contract_wide<TCX::BM>(is_x, N, D, g, (const float*)(is_x ? gb.yt : gb.xt), gb.ldt, bg, P, Q, tm, td,
-                                  sp.accumulate != 0, is_x ? acc_x : acc_y, lds, osc, kbeg, klen, sp.seg);
+                                  sp.accumulate != 0, is_x ? acc_x : acc_y, lds, oe, kbeg, klen, sp.seg);
       return;
     }
   }
@@ -1255,13 +1265,13 @@ __device__ __forceinline__ void grad_contract_dispatch(int sub, int N, int D, co
     const T* gxl = X3 ? (const T*)gb.gt_lo[buf] + P * blk : nullptr;
     if (!IsSplit<T>::value && narrow)
       grad_contract_tile<TNX, T, X3>(N, D, gx, gxl, (const T*)gb.yt, (const T*)gb.yt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_x, lds, osc, kbeg, klen, sp.seg);
+                                     sp.accumulate != 0, acc_x, lds, osc, oe, kbeg, klen, sp.seg);
     else if constexpr (TCX::TB)
       grad_contract_tile<TCX, T, X3>(N, D, gx, gxl, Y, nullptr, ldy, bg, P, Q, tm, td, sp.accumulate != 0, acc_x,
-                                     lds, osc, kbeg, klen, sp.seg);
+                                     lds, osc, oe, kbeg, klen, sp.seg);
     else
       grad_contract_tile<TCX, T, X3>(N, D, gx, gxl, (const T*)gb.yt, (const T*)gb.yt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_x, lds, osc, kbeg, klen, sp.seg);
+                                     sp.accumulate != 0, acc_x, lds, osc, oe, kbeg, klen, sp.seg);
   } else {
     int Q = (P - sp.diag_c + bg.nb) % bg.nb;
     if constexpr (IsSplit<T>::value) Q = __builtin_amdgcn_readfirstlane(Q);
@@ -1269,13 +1279,13 @@ __device__ __forceinline__ void grad_contract_dispatch(int sub, int N, int D, co
     const T* gyl = X3 ? (const T*)gb.gt_lo[buf] + Q * blk : nullptr;
     if (!IsSplit<T>::value && narrow)
       grad_contract_tile<TNY, T, X3>(N, D, gy, gyl, (const T*)gb.xt, (const T*)gb.xt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_y, lds, osc, kbeg, klen, sp.seg);
+                                     sp.accumulate != 0, acc_y, lds, osc, oe, kbeg, klen, sp.seg);
     else if constexpr (TCY::TB)
       grad_contract_tile<TCY, T, X3>(N, D, gy, gyl, X, nullptr, ldx, bg, P, Q, tm, td, sp.accumulate != 0, acc_y,
-                                     lds, osc, kbeg, klen, sp.seg);
+                                     lds, osc, oe, kbeg, klen, sp.seg);
     else
       grad_contract_tile<TCY, T, X3>(N, D, gy, gyl, (const T*)gb.xt, (const T*)gb.xt_lo, gb.ldt, bg, P, Q, tm, td,
-                                     sp.accumulate != 0, acc_y, lds, osc, kbeg, klen, sp.seg);
+                                     sp.accumulate != 0, acc_y, lds, osc, oe, kbeg, klen, sp.seg);
   }
 }
 

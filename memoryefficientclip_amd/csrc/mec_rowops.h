@@ -788,11 +788,13 @@ __device__ __forceinline__ void split_pair4(const f32x4& v, uint2& hi, uint2& lo
   lo = uint2{pack2_f16(l[0], l[1]), pack2_f16(l[2], l[3])};
 }
 // the power of two that puts m (the largest finite magnitude) into [2^14,
-// 2^15), kept between 2^-100 and 2^100 (its square must be a number); 1 for 0
+// 2^15), at most 2^126 (2^-113 at the least: m < 2^128); 1 for 0.  It and its
+// inverse are normal numbers; a product of two need not be one (exp_mul,
+// contract_store_again).
 __device__ __forceinline__ float pair_scale(float m) {
   if (!(m > 0.f)) return 1.f;
   int s = 14 - ((int)(__float_as_uint(m) >> 23) - 127);
-  s = s < -100 ? -100 : s > 100 ? 100 : s;
+  s = s > 126 ? 126 : s;
   return __uint_as_float((uint32_t)(s + 127) << 23);
 }
 constexpr float PAIR_UNIT_SCALE = 16384.f;  // of rows that are normalized here (|v| <= 1)

@@ -42,7 +42,7 @@ def pairs(monkeypatch):
 def scale_of(v):
     """The power of two that puts the largest finite magnitude into [2^14, 2^15)."""
     m = np.abs(v[np.isfinite(v)]).max(initial=0.0)
-    return np.float32(2.0 ** (14 - np.floor(np.log2(m)))) if m > 0 else np.float32(1)
+    return np.float32(2.0 ** min(14 - np.floor(np.log2(m)), 126)) if m > 0 else np.float32(1)
 
 
 def pair_rows(v):
@@ -329,6 +329,32 @@ def test_wide_matrix_against_the_definition(pairs, mode, n, d, normed, pad, tb, 
         e = row_errors(a, r)
         say(f"  rows' errors: median {e.median():.2e}, largest {e.max():.2e} (bar {bar:.2e})")
         assert e.max() <= bar
+
+
+@pytest.mark.parametrize("ex,ey", [(118, -118), (-118, 118), (119, 119), (-100, -100)])
+@pytest.mark.parametrize("mode", ["clip", "lit"])
+def test_scales_at_the_ends_of_fp32(pairs, mode, ex, ey):
+    """Rows that come as they are, 2^ex and 2^ey times unit rows: with the exponents
+    opposed the products are those of unit rows; with both large, rows of x and y
+    without a common feature (S = 0); with both small, S = 0 to fp32 too.  The
+    gradients of 2^e x scale as 2^-e times those of x."""
+    n, d, t = 300, 64, 0.1
+    lit = mode == "lit"
+    a, b = (torch.nn.functional.normalize(v, dim=1) for v in randn_pair(n, d, seed=3))
+    if ex == ey:
+        a[:, d // 2:] = 0
+        b[:, :d // 2] = 0
+    x, y = (a * 2.0 ** ex).to(DEV).requires_grad_(True), (b * 2.0 ** ey).to(DEV).requires_grad_(not lit)
+    say(f"scales {mode} 2^{ex} 2^{ey}")
+    loss = (MemoryEfficientLiTLoss if lit else MemoryEfficientCLIPLoss)(t, True)(x, y)
+    assert loss.grad_fn.mec[4] == _lib.DTYPE_F32_PAIRS
+    loss.backward()
+    f = oracle.lit_loss_and_grads if lit else oracle.clip_loss_and_grads
+    ref = f(a, b, t, normalized_inputs=True)
+    assert rel_err(loss.detach().cpu(), ref[0]) <= BAR
+    # (d loss / d x_i is a sum of rows of y)
+    for g, r, e in [(x.grad, ref[1], ey)] + ([] if lit else [(y.grad, ref[2], ex)]):
+        assert max_rel(g.double() * 2.0 ** -e, r) <= BAR
 
 
 def test_noalloc_and_one_side(pairs):
