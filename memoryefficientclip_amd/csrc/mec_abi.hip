@@ -393,13 +393,25 @@ void grad_blocks_budget(int64_t n, int64_t d, int dtype, int64_t gbudget, int* b
   const int64_t target_rows = mult * d > min_rows ? mult * d : min_rows;
   int64_t target = (target_rows + q - 1) / q;
   // 16-bit: one block from n = 3072 while its matrix stays within the smallest
-  // budget (n <= 11520): one buffer instead of two, so no more memory than two
-  // blocks of half the rows, half the launches, tiles that fill their rounds
-  // better and half the accumulator updates (fp16 6001 x 512, two blocks of 3072
-  // rows -> one: gradient-matrix tiles 72 -> 54 us, contractions 121 -> 86 us)
-  if (dtype != MEC_DTYPE_F32 && !is_pairs(dtype) && n >= 3072 &&
-      g_bytes(tiles, q, tiles, dtype) <= (gbudget < kGradBudgetMin ? gbudget : kGradBudgetMin))
-    target = tiles;
+  // budget (n <= 11520) and within 64 times the two inputs (256 n d bytes; 64 MiB
+  // below that): one launch of each kind instead of several, tiles that fill
+  // their rounds, one accumulator update.  One block of n rows takes the memory
+  // of two double-buffered blocks of half the rows, and n / (2 bs) times that of
+  // blocks of bs rows.  CLIP step and peak memory beyond the inputs, blocks of
+  // the target's rows -> one: fp16 6001 x 512 (two) 279 -> 225 us, 132 MB both;
+  // bf16 8192 x 256 (two) 250 -> 206 us, 186 -> 202 MB; 10007 x 128 (five) 428 ->
+  // 273 us, 116 -> 236 MB; 8192 x 64 (eight) 291 -> 146 us, 48 -> 148 MB.  Past
+  // the second bound the memory grows faster than the time falls: 11520 x 64
+  // (nine) 389 -> 278 us, 73 -> 287 MB for 3 MB of inputs; it keeps its blocks.
+  // Below n = 3072 the blocks of the target are left: one block there is 7-12 us
+  // less GPU time (2048 x 64 84 -> 77 us, 2816 x 64 89 -> 77 us) of a step that the
+  // host bounds.
+  if (dtype != MEC_DTYPE_F32 && !is_pairs(dtype) && n >= 3072) {
+    int64_t most = 256 * n * d > (int64_t(64) << 20) ? 256 * n * d : int64_t(64) << 20;
+    if (most > kGradBudgetMin) most = kGradBudgetMin;
+    if (most > gbudget) most = gbudget;
+    if (g_bytes(tiles, q, tiles, dtype) <= most) target = tiles;
+  }
   if (const char* env = std::getenv("MEC_GRAD_BLOCK_TILES")) {
     long v = std::strtol(env, nullptr, 10);
     if (v >= 1 && v <= 4096) target = v;

@@ -639,3 +639,18 @@ def test_forward_plan_is_the_separate_queries(monkeypatch):
     assert lib.mec_forward_plan(A, 64, A, 64, 1024, 64, 0, 1) & 8
     for n, d, dt in [(0, 4, 0), (4, 0, 0), (4, 4, 5), ((1 << 22) + 1, 64, 1)]:
         assert lib.mec_forward_plan(A, 64, A, 64, n, d, dt, 1) < 0
+
+
+def test_one_16bit_block_is_bounded_by_the_inputs():
+    # one backward block from n = 3072 while its matrix is within 256 MiB and
+    # within 64 times the two inputs (or 64 MiB): the scratch of a small d stays
+    # a multiple of the inputs
+    for n, d, one in [(3072, 64, True), (5632, 16, True), (5889, 16, False), (6001, 512, True), (8192, 64, True),
+                      (8193, 64, False), (11520, 64, False), (11520, 90, True), (11521, 512, False)]:
+        p = _lib.backward_plan(n, d, 1, compute_units=256)
+        assert (p.num_blocks == 1) == one, (n, d, p.num_blocks)
+    for n in range(3072, 11600, 509):
+        for d in (8, 33, 64, 100, 256):
+            p = _lib.backward_plan(n, d, 1, compute_units=256)
+            matrix = p.scratch_bytes - 2 * 2 * d * ((n + 127) // 128 * 128)
+            assert matrix <= max(64 << 20, 256 * n * d), (n, d, matrix)
