@@ -187,17 +187,18 @@ def backward(ctx, grad_output: torch.Tensor, need_x: bool, need_y: bool):
     # be wasted work.  fp32 accumulates in the outputs (the post-pass runs in
     # place); the 16-bit types' fp32 accumulators are the scratch's first part.
     nbytes = off = 0
-    if not mode & _lib.FLAG_KEEP_EXP:
-        sides = (_lib.SIDE_X if need_x else 0) | (_lib.SIDE_Y if need_y else 0)
-        nbytes = lib.mec_backward_scratch_bytes(n, d, dt, mode, sides)
-        if x.dtype != torch.float32:
-            side = (4 * n * d + 255) & ~255
-            off = side * (int(need_x) + int(need_y))
     cur = torch.cuda.current_device()
     if cur != di:
         torch.cuda.set_device(di)
     scratch = None
     try:
+        # (the size depends on the current device's compute units)
+        if not mode & _lib.FLAG_KEEP_EXP:
+            sides = (_lib.SIDE_X if need_x else 0) | (_lib.SIDE_Y if need_y else 0)
+            nbytes = lib.mec_backward_scratch_bytes(n, d, dt, mode, sides)
+            if x.dtype != torch.float32:
+                side = (4 * n * d + 255) & ~255
+                off = side * (int(need_x) + int(need_y))
         pax, pay = pdx, pdy
         if nbytes + off > 0:
             scratch = _alloc(nbytes + off, di)

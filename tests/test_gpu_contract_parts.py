@@ -87,3 +87,18 @@ def test_parts_match_the_unsplit_contractions(monkeypatch, kind, n, d, parts, mo
         finally:
             torch.use_deterministic_algorithms(False)
     assert all(torch.equal(u, v) for u, v in zip(*r))
+
+
+def test_the_scratch_is_sized_on_the_tensors_device(monkeypatch):
+    """The parts follow the compute units of the current device: with another one
+    current, the size is asked for after the switch and the switch undone."""
+    x, y = (torch.randn(300, 64, device=DEV, dtype=torch.bfloat16, requires_grad=True) for _ in range(2))
+    loss = MemoryEfficientCLIPLoss(0.07)(x, y)
+    lib, seen = _lib.load(), []
+    size = lib.mec_backward_scratch_bytes
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(torch.cuda, "set_device", lambda i: seen.append(i))
+    monkeypatch.setattr(lib, "mec_backward_scratch_bytes", lambda *a: (seen.append("size"), size(*a))[1])
+    loss.backward()
+    assert seen == [0, "size", 1]
+    assert x.grad is not None and y.grad is not None
