@@ -761,7 +761,6 @@ bool pairs_preferred(int64_t n, int64_t d, int dtype) {
     if (env[0] == '1') return true;
   }
   if (dtype == MEC_DTYPE_F32_BF16X3) return true;
-  if (small_tiles_env() >= 0) return false;  // (the fp32 tiles are asked for)
   // (from n = 2049 to 4096 both are bound by the host at a small d, where the fp32
   // kernels have two launches fewer: LiT 3757 x 64 134 us, pairs 142 us)
   if (n > MEC_KEEP_EXP_MAX_N) return n > 4096 || n * n * d >= 1000000000LL;

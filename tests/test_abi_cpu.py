@@ -581,8 +581,7 @@ def test_pairs_sizes_and_rule(monkeypatch):
     rc = lib.mec_prepass(16, 64, 16, 64, 10, 64, P, 1, 8, None)
     assert rc == _lib.MEC_ERR_INVALID and "16-byte" in _lib.last_error()
     # which problems run as pairs
-    for v in ("MEC_F32_PAIRS", "MEC_F32_SMALL_TILES"):
-        monkeypatch.delenv(v, raising=False)
+    monkeypatch.delenv("MEC_F32_PAIRS", raising=False)
     x3 = _lib.DTYPE_F32_BF16X3
     for dt in (1, 2, 4, P, 7):
         assert lib.mec_product_dtype(32768, 1152, dt) == dt
@@ -594,8 +593,9 @@ def test_pairs_sizes_and_rule(monkeypatch):
     for dt in (0, x3):
         assert lib.mec_product_dtype((1 << 20) + 1, 1152, dt) == dt
         assert lib.mec_product_dtype(0, 1152, dt) == dt
+    # (asking for tiles of the fp32 kernels does not ask for the fp32 kernels)
     monkeypatch.setenv("MEC_F32_SMALL_TILES", "1")
-    assert lib.mec_product_dtype(32768, 1152, 0) == 0
+    assert lib.mec_product_dtype(32768, 1152, 0) == P
     monkeypatch.setenv("MEC_F32_PAIRS", "1")
     assert lib.mec_product_dtype(1, 1, 0) == P
     monkeypatch.setenv("MEC_F32_PAIRS", "0")
@@ -624,7 +624,7 @@ def test_small_16bit_tile_rule(monkeypatch):
 def test_forward_plan_is_the_separate_queries(monkeypatch):
     # mec_forward_plan packs mec_product_dtype, mec_keep_exp_supported and
     # mec_workspace_floats_mode
-    for v in ("MEC_F32_PAIRS", "MEC_F32_SMALL_TILES", "MEC_KEEP_EXP"):
+    for v in ("MEC_F32_PAIRS", "MEC_KEEP_EXP"):
         monkeypatch.delenv(v, raising=False)
     lib = _lib.load()
     A = 1 << 20

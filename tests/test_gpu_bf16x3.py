@@ -1,6 +1,9 @@
-"""The bf16x3 mode for fp32 inputs (torch.set_float32_matmul_precision("high")):
+"""The bf16x3 mode for fp32 inputs (torch.set_float32_matmul_precision("high")
+beyond the size limit of the fp16 pairs, and MEC_DTYPE_F32_BF16X3 of the C ABI):
 every product of the similarity GEMMs and the gradient contractions is formed
-as hi*hi + lo*hi + hi*lo from bf16 terms on the bf16 MFMA.
+as hi*hi + lo*hi + hi*lo from bf16 terms on the bf16 MFMA.  Up to N = 2^20 "high"
+runs as pairs (mec_product_dtype): MEC_F32_PAIRS=0 turns that off here, and
+every run asserts the mode that ran; test_high_runs_as_pairs is the rule itself.
 
 * The split copies of x and y that mec_prepass writes into the workspace are
   checked bit for bit against a numpy restatement of the split (round to
@@ -33,10 +36,17 @@ def say(*a):
     print(*a, flush=True)
 
 
+@pytest.fixture(autouse=True)
+def no_pairs(monkeypatch):
+    monkeypatch.setenv("MEC_F32_PAIRS", "0")
+
+
 def run(module, a, b, grad_b=True):
     ga = a.to(DEV).requires_grad_(True)
     gb = b.to(DEV).requires_grad_(grad_b)
     loss = module(ga, gb)
+    high = torch.get_float32_matmul_precision() == "high"
+    assert loss.grad_fn.mec[4] == (_lib.DTYPE_F32_BF16X3 if high else _lib.DTYPE_F32)
     loss.backward()
     torch.cuda.synchronize()
     return loss.detach().cpu(), ga.grad.cpu(), (gb.grad.cpu() if grad_b else None)
@@ -137,6 +147,7 @@ def test_frozen_tower_and_grad_output():
     say(f"bf16x3 frozen text tower, grad_output -1.5, n={n} d={d}")
     with matmul_precision("high"):
         loss = MemoryEfficientCLIPLoss(0.07)(ga, gb)
+        assert loss.grad_fn.mec[4] == _lib.DTYPE_F32_BF16X3
         (loss * -1.5).backward()
     torch.cuda.synchronize()
     rl, rda, _ = oracle.clip_loss_and_grads(a, b, 0.07, grad_output=-1.5)
@@ -199,3 +210,19 @@ def test_full_size(mode):
     say(f"  loss {float(loss):.7f} ref {rl.item():.7f} rel {le:.2e}; grads {ea:.2e} {eb:.2e}")
     assert math.isfinite(float(loss))
     assert le <= F32["loss"] and ea <= F32["grad"] and eb <= F32["grad"]
+
+
+@pytest.mark.parametrize("n,d", [(5, 3), (1024, 512), (3000, 100)])
+def test_high_runs_as_pairs(monkeypatch, n, d):
+    """Under "high" the modules run fp32 data as fp16 pairs at any size up to
+    2^20, within the tolerance of the fp32 kernels."""
+    monkeypatch.delenv("MEC_F32_PAIRS")
+    a, b = randn_pair(n, d, seed=n)
+    ga, gb = a.to(DEV).requires_grad_(True), b.to(DEV).requires_grad_(True)
+    with matmul_precision("high"):
+        loss = MemoryEfficientCLIPLoss(0.07)(ga, gb)
+        assert loss.grad_fn.mec[4] == _lib.DTYPE_F32_PAIRS
+        loss.backward()
+    rl, rda, rdb = oracle.clip_loss_and_grads(a, b, 0.07)
+    assert rel_err(loss.detach().cpu(), rl) <= 4e-6
+    assert max_rel(ga.grad, rda) <= 4e-6 and max_rel(gb.grad, rdb) <= 4e-6

@@ -14,6 +14,9 @@ small for its K or fill its rounds of CUs poorly (the forward and each
 backward step choose on their own); MEC_F32_SMALL_TILES=0 / 1 forces either
 tile size, so both are checked on both sides of those bounds, with the kept
 similarity matrix (which takes over at N <= 2048) turned off.
+
+Above that range fp32 runs as fp16 pairs (mec_product_dtype); here
+MEC_F32_PAIRS=0 keeps the fp32 kernels, and every run says which kernels ran.
 """
 import os
 
@@ -22,6 +25,7 @@ import torch
 
 import oracle
 from helpers import max_rel, randn_pair, rel_err
+from memoryefficientclip_amd import _lib
 from memoryefficientclip_amd.clip_loss import MemoryEfficientCLIPLoss
 from memoryefficientclip_amd.lit_loss import MemoryEfficientLiTLoss
 
@@ -34,10 +38,16 @@ def say(*a):
     print(*a, flush=True)
 
 
+@pytest.fixture(autouse=True)
+def fp32_kernels(monkeypatch):
+    monkeypatch.setenv("MEC_F32_PAIRS", "0")
+
+
 def run(module, a, b, grad_b=True):
     ga = a.to(DEV).requires_grad_(True)
     gb = b.to(DEV).requires_grad_(grad_b)
     loss = module(ga, gb)
+    assert loss.grad_fn.mec[4] == _lib.DTYPE_F32
     loss.backward()
     torch.cuda.synchronize()
     return loss.detach().cpu(), ga.grad.cpu(), (gb.grad.cpu() if grad_b else None)
@@ -68,6 +78,7 @@ def test_f32_unaligned_rows(lit, n, d, ld):
     ga = strided(a, ld).requires_grad_(True)
     gb = strided(b, ld).requires_grad_(not lit)
     loss = mod(ga, gb)
+    assert loss.grad_fn.mec[4] == _lib.DTYPE_F32
     loss.backward()
     torch.cuda.synchronize()
     l_un, da_un = loss.detach().cpu(), ga.grad.cpu()

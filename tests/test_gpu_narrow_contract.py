@@ -22,6 +22,7 @@ import torch
 
 import oracle
 from helpers import TOL, matmul_precision, max_rel, randn_pair, rel_err
+from memoryefficientclip_amd import _lib
 from memoryefficientclip_amd.clip_loss import MemoryEfficientCLIPLoss
 from memoryefficientclip_amd.lit_loss import MemoryEfficientLiTLoss
 
@@ -33,7 +34,7 @@ def say(*a):
     print(*a, flush=True)
 
 
-def run(module, a, b, grad_b, env):
+def run(module, a, b, grad_b, env, code=None):
     old = {k: os.environ.get(k) for k in env}
     os.environ.update(env)
     det = torch.are_deterministic_algorithms_enabled()
@@ -42,6 +43,7 @@ def run(module, a, b, grad_b, env):
         ga = a.to(DEV).requires_grad_(True)
         gb = b.to(DEV).requires_grad_(grad_b)
         loss = module(ga, gb)
+        assert code in (None, loss.grad_fn.mec[4])
         loss.backward()
         torch.cuda.synchronize()
         return loss.detach().cpu(), ga.grad.cpu(), (gb.grad.cpu() if grad_b else None)
@@ -90,17 +92,23 @@ def test_narrow_contraction_tiles(dt, lit, n, d, normed):
                          ids=["bf16x3", "bf16-products"])
 @pytest.mark.parametrize("lit", [False, True], ids=["clip", "lit"])
 @pytest.mark.parametrize("n,d", [(1024, 300), (2048, 100)])
-def test_narrow_contraction_tiles_fp32_split(prec, tol, lit, n, d):
+def test_narrow_contraction_tiles_fp32_split(monkeypatch, prec, tol, lit, n, d):
     """fp32 inputs under matmul precision "high" (bf16x3: three passes over
     hi / lo planes) and "medium" (bf16 products) run the same contraction
     kernel on their bf16 copies."""
+    # the two settings do choose different tiles ("high" runs this mode only without the pairs)
+    monkeypatch.setenv("MEC_F32_PAIRS", "0")
+    dt = _lib.DTYPE_F32_BF16X3 if prec == "high" else _lib.DTYPE_F32_BF16
+    for v in "10":
+        monkeypatch.setenv("MEC_NARROW_CONTRACT", v)
+        assert _lib.backward_plan(n, d, dt, int(lit), 1 if lit else 3).narrow_tiles == int(v)
     a, b = randn_pair(n, d, seed=11 * n + d)
     kind = "LiT" if lit else "CLIP"
     mod = (MemoryEfficientLiTLoss if lit else MemoryEfficientCLIPLoss)(0.1)
     say(f"fp32 ({prec}) {kind} n={n} d={d}: narrow vs wide contraction tiles")
     with matmul_precision(prec):
-        l_n, da_n, db_n = run(mod, a, b, not lit, {"MEC_NARROW_CONTRACT": "1"})
-        l_w, da_w, db_w = run(mod, a, b, not lit, {"MEC_NARROW_CONTRACT": "0"})
+        l_n, da_n, db_n = run(mod, a, b, not lit, {"MEC_NARROW_CONTRACT": "1"}, dt)
+        l_w, da_w, db_w = run(mod, a, b, not lit, {"MEC_NARROW_CONTRACT": "0"}, dt)
     assert torch.equal(l_n, l_w) and torch.equal(da_n, da_w)
     if not lit:
         assert torch.equal(db_n, db_w)

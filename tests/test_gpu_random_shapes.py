@@ -1,5 +1,6 @@
 """Randomised GPU parity sweep: shapes, dtypes (fp32, bf16, fp16, and fp32
-under float32 matmul precision "high", "f32x3"), modes and layouts drawn from
+in the bf16x3 mode, "f32x3": matmul precision "high" without the fp16 pairs that
+it otherwise runs as), modes and layouts drawn from
 a fixed seed, each checked against the fp64 CPU oracle on the same
 (dtype-rounded) inputs at the task's tolerances.  It covers the
 masking of ragged tiles and short last backward blocks, D that is or is not a
@@ -13,7 +14,7 @@ import torch
 
 import oracle
 from helpers import TOL, max_rel, rel_err
-from memoryefficientclip_amd import MemoryEfficientCLIPLoss, MemoryEfficientLiTLoss
+from memoryefficientclip_amd import MemoryEfficientCLIPLoss, MemoryEfficientLiTLoss, _lib
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -40,7 +41,7 @@ CASES = (draw_cases() + [(20 + c[0],) + c[1:] for c in draw_cases(seed=777, coun
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(v) for v in c[:6]))
-def test_random_case(case):
+def test_random_case(monkeypatch, case):
     k, n, d, dt, mode, normed, pad, go, temp = case
     torch_dt = {"f32": torch.float32, "f32x3": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dt]
     g = torch.Generator().manual_seed(1000 + k)
@@ -56,6 +57,8 @@ def test_random_case(case):
     wb[:, pad:pad + d] = b
     ga = wa.to(DEV)[:, pad:pad + d].requires_grad_(True)
     gb = wb.to(DEV)[:, pad:pad + d].requires_grad_(mode == "clip")
+    if dt == "f32x3":
+        monkeypatch.setenv("MEC_F32_PAIRS", "0")
     print(f"case {case}", flush=True)
     old_precision = torch.get_float32_matmul_precision()
     torch.set_float32_matmul_precision("high" if dt == "f32x3" else "highest")
@@ -64,6 +67,7 @@ def test_random_case(case):
             loss = MemoryEfficientCLIPLoss(temp, normed)(ga, gb)
         else:
             loss = MemoryEfficientLiTLoss(temp, normed)(ga, gb)
+        assert dt != "f32x3" or loss.grad_fn.mec[4] == _lib.DTYPE_F32_BF16X3
         (loss * go).backward()
         torch.cuda.synchronize()
     finally:
