@@ -968,9 +968,10 @@ static int sumexp_det_run(const void* x, int64_t ldx, const void* y, int64_t ldy
   // 17 to 22 tiles a side (256 x 256 tiles, one workgroup per CU): with 16 column
   // blocks more than 256 workgroups of one or two tiles start, and the last ones
   // end a third tile after the first; blocks of two column tiles are at most 256
-  // workgroups and two tiles (pairs 4999 x 640: forward 119 -> 87 us).  A rule
-  // on the tile counts alone, so that the order of the sums is the same on any
-  // device.
+  // workgroups and two tiles.  The loss alone at n = 4400-5632, d = 128, 512 and
+  // 1152, bf16, fp16 and pairs: 14-30% less time at every one (bf16 4400 x 512 54
+  // -> 41 us, 5632 x 1152 99 -> 85 us; pairs 4999 x 512 117 -> 89 us).  A rule on the
+  // tile counts alone, so that the order of the sums is the same on any device.
   if (FwdTile<T, true>::BM == 256 && vec && !small && tiles_n > DET_Q && P * ((tiles_n + 1) / 2) <= 256) Q = (tiles_n + 1) / 2;
   const unsigned sum_grid = (unsigned)((n + 255) / 256);
   auto run = [&](auto lit_c, auto norm_c, auto vec_c) {
@@ -1046,7 +1047,7 @@ static int sumexp_run(const void* x, int64_t ldx, const void* y, int64_t ldy, in
   // forward.
   bool chain = false;
   DISPATCH_DTYPE(dtype, T, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(vec, VEC, {
-    chain = FwdChain<T, VEC, NORM>::value;
+    chain = FwdChain<T, VEC>::value;
   })));
   const bool det = (mode & MEC_FLAG_DETERMINISTIC) || chain;
   int cus = 0;
@@ -1067,7 +1068,7 @@ static int sumexp_run(const void* x, int64_t ldx, const void* y, int64_t ldy, in
   }
   dim3 grid((unsigned)nwg);
   DISPATCH_DTYPE(dtype, T, DISPATCH_BOOL(lit, LIT, DISPATCH_BOOL(normalize, NORM, DISPATCH_BOOL(vec, VEC, {
-    if constexpr (!FwdChain<T, VEC, NORM>::value) {
+    if constexpr (!FwdChain<T, VEC>::value) {
       if (small) {
         if constexpr (VEC)
           k_sumexp<T, LIT, NORM, VEC, true><<<grid, GemmTile<T, VEC, true>::NT, 0, s>>>(

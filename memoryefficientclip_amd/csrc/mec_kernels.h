@@ -462,7 +462,7 @@ __device__ __forceinline__ void sums_flush(float* __restrict__ ws, int m0, int n
 // 256 703 -> 578 us, 131072 x 128 8.83 -> 6.09 ms; its scales reach LDS by one
 // direct load per wave during the tile before.  (It spilled until the epilogue
 // addressed its rows from one base.)
-template <typename T, bool VEC, bool NORM> struct FwdChain {
+template <typename T, bool VEC> struct FwdChain {
   static constexpr bool value = FwdTile<T, VEC>::CHAIN && Is16<T>::value;
 };
 
@@ -525,7 +525,7 @@ __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>:
   static_assert(TL::NT >= TL::BM && TL::NT >= TL::BN, "one row and one column per thread");
   __shared__ __attribute__((aligned(1024))) char lds[TL::LDS_BYTES];
   // (row and column scales; chained tiles: the next tile's land in the other half)
-  constexpr int NV = FwdChain<T, VEC, NORM>::value && NORM ? 2 : 1;
+  constexpr int NV = FwdChain<T, VEC>::value && NORM ? 2 : 1;
   __shared__ __attribute__((aligned(16))) float s_vec[NV][TL::BM + TL::BN];
   __shared__ float s_row[TL::WN][TL::BM], s_col[TL::WM][TL::BN];
   __shared__ __attribute__((aligned(16))) float s_cold[TL::BN];
@@ -598,7 +598,7 @@ __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>:
       *cp = tm == tm0 ? v : (cold ? s_cold[t] : *cp) + v;
     }
   };
-  if constexpr (FwdChain<T, VEC, NORM>::value) {
+  if constexpr (FwdChain<T, VEC>::value) {
     // chained tiles: the last chunk of
     // each tile's k-loop loads chunk 0 of the next, which lands during the
     // epilogue.  The k-loop's barriers order one tile's slot reads before the

@@ -56,6 +56,8 @@ inline double round_fill(int64_t tiles, int cus) {
   const int64_t rounds = (tiles + cus - 1) / cus;
   return (double)tiles / ((double)rounds * cus);
 }
+// (fp32 data above n = 4096, and above 2048 at a larger d, runs as fp16 pairs, up to
+// n = 2^20, unless MEC_DTYPE_F32 is asked for through the C ABI: mec_product_dtype)
 // fp32 forward tiles: 64 x 64 for f32_small_n, and for D >= 512 where the
 // 128 x 128 grid fills its rounds below 90% (measured on one MI355X: the
 // forward 7-23% faster at N = 3072 and 5120, D = 512-1024; at D = 128-256 and
