@@ -1371,18 +1371,19 @@ __global__ __launch_bounds__((GemmTile<T, VEC, SMALL>::NT), (Occ<T, VEC, SMALL>:
 // (rx, ry, 1/R, 1/C) reach LDS by direct loads into one of two buffers,
 // issued right after the previous tile's first barrier (when every wave is
 // done with that buffer).
-template <typename T, bool LIT, bool NORM, bool X3 = false, bool SMALL = false>
-__global__ __launch_bounds__((GemmTile<T, true, SMALL>::NT), (SMALL ? 2 : 1)) void k_grad_g_chain(
-    const T* __restrict__ X, int64_t ldx, const T* __restrict__ Y, int64_t ldy, int N, int D, int kmax, float c,
-    const float* __restrict__ ws, GradBufs gb, BlockGrid bg, StepPlan sp) {
+// WIDE: split pairs whose gradient matrix is held wide (GradBufs).
+template <typename T, bool LIT, bool NORM, bool X3, bool SMALL, bool WIDE>
+__device__ __forceinline__ void grad_g_chain(const T* __restrict__ X, int64_t ldx, const T* __restrict__ Y,
+                                             int64_t ldy, int N, int D, int kmax, float c,
+                                             const float* __restrict__ ws, const GradBufs& gb, const BlockGrid& bg,
+                                             const StepPlan& sp, char* lds,
+                                             float (&s_vec)[2][4][GemmTile<T, true, SMALL>::BM]) {
   using TL = GemmTile<T, true, SMALL>;
   static_assert(TL::CHAIN && GtOnly<T>::value, "chained 16-bit direct-to-LDS tiles");
   static_assert(TL::BM == TL::BN && TL::BM % 64 == 0, "64 floats per vector load");
   constexpr int QN = TL::BM / 64, NW = TL::NT / 64;  // loads per vector, waves
   static_assert(4 * QN % NW == 0, "the vector loads split evenly over the waves");
   enum { V_RX = 0, V_RY = 1, V_IR = 2, V_IC = 3 };
-  __shared__ __attribute__((aligned(1024))) char lds[TL::LDS_BYTES];
-  __shared__ __attribute__((aligned(16))) float s_vec[2][4][TL::BM];
   constexpr int NST = gt_chain_stores<TL>() * (X3 || IsSplit<T>::value ? 2 : 1);  // G'^T stores per lane and tile (two parts)
   const int64_t n64 = N;
   constexpr int E = IsSplit<T>::value ? 2 : 1;  // stored elements per value
@@ -1390,7 +1391,6 @@ __global__ __launch_bounds__((GemmTile<T, true, SMALL>::NT), (SMALL ? 2 : 1)) vo
   const int buf = sp.diag_g & 1;
   const float cm = exp_mul<T>(c, gb.scl);
   const float gs = IsSplit<T>::value ? gb.gscl[0] : 1.f;
-  const bool wide = IsSplit<T>::value && gb.gscl[2] != 0.f;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   // tile -> (i0, j0, its place in the G'^T block); false for padding ids and tiles wholly past N
   auto coords = [&](int tile, int& i0, int& j0, uint16_t*& gt) {
@@ -1404,7 +1404,7 @@ __global__ __launch_bounds__((GemmTile<T, true, SMALL>::NT), (SMALL ? 2 : 1)) vo
     j0 = J * bg.bs + tn * TL::BN;
     // (wide: fp32 values, row-major, in the bytes of the pairs)
     gt = (uint16_t*)gb.gt[buf] + I * blk +
-         (wide ? 2 * ((int64_t)(tm * TL::BM) * bg.bs + tn * TL::BN)
+         (WIDE ? 2 * ((int64_t)(tm * TL::BM) * bg.bs + tn * TL::BN)
                : E * gdma::gb_offset(tn * TL::BN, tm * TL::BM, bg.bs));
     return i0 < N && j0 < N;
   };
@@ -1460,16 +1460,14 @@ __global__ __launch_bounds__((GemmTile<T, true, SMALL>::NT), (SMALL ? 2 : 1)) vo
     const bool diag = i0 < j0 + TL::BN && j0 < i0 + TL::BM;
     // (X3: the lo plane at the same offset in gt_lo)
     uint16_t* gtl = X3 ? (uint16_t*)gb.gt_lo[buf] + (gt - (uint16_t*)gb.gt[buf]) : nullptr;
-    if (wide) {
+    if constexpr (WIDE) {
       // (more stores than NST: the next tile's first barrier waits for some of them too)
-      if constexpr (IsSplit<T>::value) {
-        if (!diag && i0 + TL::BM <= N && j0 + TL::BN <= N)
-          grad_gw_store<TL, LIT, NORM, false>(acc, cm, c, i0, j0, N, (float*)gt, bg.bs, sv + V_IR * TL::BM,
-                                              sv + V_IC * TL::BM, gs);
-        else
-          grad_gw_store<TL, LIT, NORM, true>(acc, cm, c, i0, j0, N, (float*)gt, bg.bs, sv + V_IR * TL::BM,
-                                             sv + V_IC * TL::BM, gs);
-      }
+      if (!diag && i0 + TL::BM <= N && j0 + TL::BN <= N)
+        grad_gw_store<TL, LIT, NORM, false>(acc, cm, c, i0, j0, N, (float*)gt, bg.bs, sv + V_IR * TL::BM,
+                                            sv + V_IC * TL::BM, gs);
+      else
+        grad_gw_store<TL, LIT, NORM, true>(acc, cm, c, i0, j0, N, (float*)gt, bg.bs, sv + V_IR * TL::BM,
+                                           sv + V_IC * TL::BM, gs);
     } else if (!diag && i0 + TL::BM <= N && j0 + TL::BN <= N)
       grad_gt_store_direct<TL, LIT, NORM, false, (int)GScale<T>::value, X3>(
           acc, cm, c, i0, j0, N, gt, bg.bs, sv + V_RX * TL::BM, sv + V_RY * TL::BM, sv + V_IR * TL::BM,
@@ -1486,6 +1484,23 @@ __global__ __launch_bounds__((GemmTile<T, true, SMALL>::NT), (SMALL ? 2 : 1)) vo
     vb ^= 1;
   }
   gdma::drain_loads();
+}
+
+template <typename T, bool LIT, bool NORM, bool X3 = false, bool SMALL = false>
+__global__ __launch_bounds__((GemmTile<T, true, SMALL>::NT), (SMALL ? 2 : 1)) void k_grad_g_chain(
+    const T* __restrict__ X, int64_t ldx, const T* __restrict__ Y, int64_t ldy, int N, int D, int kmax, float c,
+    const float* __restrict__ ws, GradBufs gb, BlockGrid bg, StepPlan sp) {
+  using TL = GemmTile<T, true, SMALL>;
+  __shared__ __attribute__((aligned(1024))) char lds[TL::LDS_BYTES];
+  __shared__ __attribute__((aligned(16))) float s_vec[2][4][TL::BM];
+  if constexpr (IsSplit<T>::value) {
+    // (a loop of its own: the branch inside the tile loop cost the pairs 2%)
+    if (gb.gscl[2] != 0.f) {
+      grad_g_chain<T, LIT, NORM, X3, SMALL, true>(X, ldx, Y, ldy, N, D, kmax, c, ws, gb, bg, sp, lds, s_vec);
+      return;
+    }
+  }
+  grad_g_chain<T, LIT, NORM, X3, SMALL, false>(X, ldx, Y, ldy, N, D, kmax, c, ws, gb, bg, sp, lds, s_vec);
 }
 
 }  // namespace mec
