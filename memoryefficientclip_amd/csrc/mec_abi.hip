@@ -1275,7 +1275,7 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
   sp.kl = cs ? cs->kl : bs;
   sp.seg = bs;
   if (pairs) {
-    // (sums no longer than the fp32 kernels': grad_contract_tile)
+    // (sums about as long as the fp32 kernels': grad_contract_tile)
     int bs32, nb32;
     grad_blocks(n, d, MEC_DTYPE_F32, &bs32, &nb32);
     if (bs32 < bs) sp.seg = bs32;

@@ -1114,13 +1114,34 @@ __device__ __forceinline__ void grad_contract_piece(int N, int D, const T* __res
     contract_store<TC>(acc, r0, d0, N, D, accumulate, out, osc);
 }
 
+// The pieces of a sum over k rows [kbeg, kend) (split pairs; StepPlan::seg): as
+// few of about the same length as seg allows, the boundaries moved by up to 3/16
+// of it either way by `phase`, the tile's row.  The tiles of a launch run in step:
+// with the same boundaries for all they add to the accumulators at one time and
+// wait for HBM at one time.  CLIP step against unlimited sums, boundaries in step
+// -> moved: 32768 x 1152 +1.9 -> +1.6%, 16384 x 512 +3.7 -> +1.6%, 8192 x 768 +1.2 ->
+// +0.8%; moved by feature tile as well, which parts the tiles that share a panel
+// of the gradient matrix: +2.3, +2.4, +1.7%.  A fixed function of the tile's place,
+// so that the order of the sums is too.
+struct Pieces {
+  int n, first, len, kbeg, kend;
+  __device__ __forceinline__ Pieces(int kb, int ke, int seg, int phase) : kbeg(kb), kend(ke) {
+    const int l = ke - kb;
+    n = l > seg ? (l + seg - 1) / seg : 1;
+    len = n > 1 ? ((l + n - 1) / n + 63) & ~63 : l;
+    first = n > 1 ? len + (2 * (phase & 3) - 3) * ((len / 16) & ~63) : l;
+  }
+  // the end of piece i
+  __device__ __forceinline__ int end(int i) const { return i + 1 < n ? min(kbeg + first + i * len, kend) : kend; }
+};
+
 // grad_contract_piece over the k rows [kbeg, kbeg + klen).
-// seg (split pairs): a sum over more than seg k rows is taken in
-// pieces of seg, each added to the accumulators as another block's would be: a
-// longer sum rounds more.  With seg the block rows of the fp32 kernels the
-// sums are no longer than theirs, and round 3 times per 8 k where the fp32
-// MFMA rounds 4 times; unlimited (one sum per block), positive features came
-// out up to 1.9 times as far from 64 bits as the fp32 kernels' (4200 x 512).
+// seg (split pairs): a sum over more than seg k rows is taken in pieces
+// (Pieces), each added to the accumulators as another block's would be: a longer
+// sum rounds more.  With seg the block rows of the fp32 kernels the sums are
+// hardly longer than theirs, and round 3 times per 8 k where the fp32 MFMA
+// rounds 4 times; unlimited (one sum per block), positive features came out up
+// to 1.9 times as far from 64 bits as the fp32 kernels' (4200 x 512).
 template <class TC, typename T, bool X3 = false>
 __device__ __forceinline__ void grad_contract_tile(int N, int D, const T* __restrict__ Gblk,
                                                    const T* __restrict__ Glo, const T* __restrict__ OT,
@@ -1130,12 +1151,13 @@ __device__ __forceinline__ void grad_contract_tile(int N, int D, const T* __rest
                                                    int kbeg, int klen, int seg) {
   if constexpr (IsSplit<T>::value) {
     const int kend = min(min(bg.bs, N - Q * bg.bs), kbeg + klen);
-    for (int k = kbeg;;) {
-      grad_contract_piece<TC, T, X3>(N, D, Gblk, Glo, OT, OTlo, ldt, bg, P, Q, tm, td, accumulate || k > kbeg, out,
-                                     lds, osc, oe, k, min(seg, klen));
-      k += seg;
-      if (k >= kend) break;
-      klen -= seg;
+    const Pieces pc(kbeg, kend, seg, tm);
+    for (int i = 0, k = kbeg;; ++i) {
+      const int ke = pc.end(i);
+      grad_contract_piece<TC, T, X3>(N, D, Gblk, Glo, OT, OTlo, ldt, bg, P, Q, tm, td, accumulate || i > 0, out, lds,
+                                     osc, oe, k, ke - k);
+      if (i + 1 >= pc.n) break;
+      k = ke;
       __syncthreads();  // every wave is past its last read of the ring
     }
   } else {
@@ -1157,9 +1179,10 @@ __device__ __forceinline__ void grad_contract_wide(bool xside, int N, int D, con
   const int r0 = P * bg.bs + tm * B, d0 = td * B, q0 = Q * bg.bs;
   if (r0 >= N) return;
   const int kend = min(min(bg.bs, N - q0), kbeg + klen);
-  for (int k = kbeg;; k += seg) {
-    // (k >= kend: a part past a short last block)
-    const int kl = min(seg, kend - k);
+  const Pieces pc(kbeg, kend, seg, tm);
+  for (int i = 0, k = kbeg;; ++i) {
+    // (kl <= 0: a part past a short last block)
+    const int ke = pc.end(i), kl = ke - k;
     if (kl <= 0 && accumulate) return;
     f32x16 acc[TL::FM][TL::FN];
     if (kl > 0) {
@@ -1167,14 +1190,15 @@ __device__ __forceinline__ void grad_contract_wide(bool xside, int N, int D, con
       gwide::run<TL>(xside, a, bg.bs, OT + (int64_t)d0 * ldt + q0 + k, ldt, min(D - d0, B), kl, lds, acc);
     } else {
 #pragma unroll
-      for (int i = 0; i < TL::FM; ++i)
+      for (int i1 = 0; i1 < TL::FM; ++i1)
 #pragma unroll
         for (int j = 0; j < TL::FN; ++j)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+          for (int r = 0; r < 16; ++r) acc[i1][j][r] = 0.f;
     }
-    contract_store_again<TL>(acc, r0, d0, N, D, accumulate || k > kbeg, out, oe);
-    if (k + seg >= kend) break;
+    contract_store_again<TL>(acc, r0, d0, N, D, accumulate || i > 0, out, oe);
+    if (i + 1 >= pc.n) break;
+    k = ke;
   }
 }
 
