@@ -106,10 +106,20 @@ extern "C" {
  * contractions (x^, y^, G') held as a pair of fp16 values, hi = fp16(v) and lo
  * = fp16(v - hi) (about 22 significant bits, after a power-of-two scaling that
  * keeps lo within fp16's range), and every product formed as hi_a hi_b + lo_a
- * hi_b + hi_a lo_b on the fp16 MFMA, accumulated in fp32.  The loss and the
- * gradients are as close to the 64-bit values as those of MEC_DTYPE_F32 (the
- * rounding of the fp32 sums is larger than what the pairs leave out), at a
- * multiple of its speed for larger problems.  n <= 2^20.  Workspace
+ * hi_b + hi_a lo_b on the fp16 MFMA, accumulated in fp32.  G' has one scale for
+ * all its entries; where that cannot hold the smallest row's to an fp32 rounding
+ * (rows whose off-diagonal shares lie far apart, or below sqrt(n) 2^-39), which the
+ * kernels find from the forward's sums, G' and the transposed inputs are held in
+ * fp32 instead, and the contractions split them into three bf16 terms: six
+ * products, up to twice the time of a step.  The loss and the gradients, each row
+ * on its own, are as close to the 64-bit values as those of MEC_DTYPE_F32 (the
+ * fp32 sums, of about the same length, round off more than what the pairs leave
+ * out), at a multiple of its speed for larger problems.  A value below 2^-17 of the
+ * largest of its side (of 1, for rows that are normalized here) has fewer than 22
+ * bits as a pair, down to 2^-39 of the largest: an input of that size adds as
+ * little to every product, but a gradient that is made of such values alone (of
+ * a feature that is that small in every row) has as few.
+ * n <= 2^20.  Workspace
  * (mec_workspace_floats_for, 16-byte aligned) and scratch are larger; any row
  * stride and alignment is accepted.  mec_product_dtype names the problems that
  * are better run this way.  No counterpart dtype in the reference. */
@@ -179,8 +189,10 @@ int64_t mec_workspace_floats(int64_t n);
 /* Number of floats of the workspace for (n, d, dtype): mec_workspace_floats(n)
  * for fp32, bf16 and fp16; for MEC_DTYPE_F32_BF16X3 (MEC_DTYPE_F32_BF16) that,
  * rounded up to 4 floats, plus split copies of x and y: 2 n rows of
- * 3 * round8(d) (round8(d)) bf16.  Returns < 0 on bad args.  No counterpart
- * in the reference. */
+ * 3 * round8(d) (round8(d)) bf16; for MEC_DTYPE_F32_PAIRS that, rounded up to 64
+ * floats, 64 floats (scales, and the range of the gradient matrix's rows) and
+ * the pairs of x and y, 2 n round32(d) x 4 bytes.  Returns < 0 on bad args.  No
+ * counterpart in the reference. */
 int64_t mec_workspace_floats_for(int64_t n, int64_t d, int dtype);
 
 /* Number of floats of the workspace for (n, d, dtype, mode):
@@ -194,9 +206,10 @@ int64_t mec_workspace_floats_for(int64_t n, int64_t d, int dtype);
 int64_t mec_workspace_floats_mode(int64_t n, int64_t d, int dtype, int mode);
 
 /* The dtype code to run MEC_DTYPE_F32 or MEC_DTYPE_F32_BF16X3 data of this
- * size with: MEC_DTYPE_F32_PAIRS where that is faster (it is as exact as the
- * first and more exact than the second), else `dtype` itself (any other dtype
- * is returned as it is).  Host-only.  No counterpart in the reference. */
+ * size with: MEC_DTYPE_F32_PAIRS where that is faster (as exact as the first,
+ * with the limit stated there, and more exact than the second), else `dtype`
+ * itself (any other dtype is returned as it is).  Host-only.  No counterpart in
+ * the reference. */
 int mec_product_dtype(int64_t n, int64_t d, int dtype);
 
 /* mec_product_dtype, mec_keep_exp_supported (asked only when `keep` is not 0)
@@ -218,21 +231,24 @@ int mec_keep_exp_supported(const void* x, int64_t ldx, const void* y, int64_t ld
 /* Bytes of gradient scratch that mec_grad / mec_grad_step / mec_backward
  * need for (n, d, dtype, mode, sides), sides a mask of MEC_SIDE_X and
  * MEC_SIDE_Y (LiT: the x side only).  The layout, in the scratch element type
- * (fp32 for MEC_DTYPE_F32, 16 bits for every other dtype):
+ * (4 bytes for MEC_DTYPE_F32 and MEC_DTYPE_F32_PAIRS, 2 for every other dtype):
  *   - the gradient-matrix buffers: one block diagonal of the off-diagonal
  *     gradient matrix (nb blocks of bs x bs), double-buffered (one buffer
- *     when a single block covers n).  fp32 keeps H = diag(rx) G' diag(ry)
- *     once, row-major; the 16-bit types keep G'^T in a blocked layout
- *     (bf16x3: hi and lo planes);
- *   - the 16-bit types (and the bf16-product modes) only: transposed
- *     normalised copies of the inputs, [d][n rounded up to 128], one for each
- *     side computed (bf16x3: hi and lo planes).  fp32 reads its raw inputs.
- * bs targets ~4d rows for fp32 and ~8d for the other dtypes (~16d when
- * n >= 8192 and 8d would give fewer than 16 blocks; at most 16384 rows for
- * fp32 and 32512 for the 16-bit kernels), and is shortened, never below 128
- * (fp32) or 256 rows, until the gradient-matrix buffers fit
- * min(16 GiB, max(64 n d elem, 256 MiB)): O(n*d).  Examples: n = 32768,
- * d = 1152 fp32 CLIP 1.07 GB; LiT the same; n = 1024, d = 512 fp32 4.2 MB.
+ *     when a single block covers n, and for MEC_DTYPE_F32_PAIRS).  fp32 keeps H =
+ *     diag(rx) G' diag(ry) once, row-major; the 16-bit types and the pairs keep
+ *     G'^T in a blocked layout (bf16x3: hi and lo planes);
+ *   - every dtype but MEC_DTYPE_F32: transposed normalised copies of the inputs,
+ *     [d][n rounded up to 128], one for each side computed (bf16x3: hi and lo
+ *     planes).  fp32 reads its raw inputs;
+ *   - MEC_DTYPE_F32_PAIRS: 256 bytes for the gradient matrix's scale.
+ * bs targets ~4d rows for fp32 (at least 1024), ~8d for the pairs (at least 2048)
+ * and ~8d for the other dtypes (at least 1024; ~16d when n >= 8192 and 8d would
+ * give fewer than 16 blocks), at most 16384 rows for fp32, 23040 for the pairs and
+ * 32512 for the others.  The others take one block of all n rows from n = 3072
+ * while that matrix is within 256 MiB and within 256 n d bytes or 64 MiB.  bs is
+ * shortened, never below 128 (fp32) or 256 rows, until the gradient-matrix buffers
+ * fit min(16 GiB, max(64 n d elem, 256 MiB)): O(n*d).  Examples, CLIP: n = 32768,
+ * d = 1152 fp32 1.07 GB, pairs 1.38 GB; n = 1024, d = 512 fp32 4.2 MB.
  * With MEC_FLAG_KEEP_EXP in mode: 0 (the backward contracts the kept
  * matrix); < 0 where the flag does not apply (dtype, n).
  * Returns < 0 on bad args or n outside [1, 2^22]. */
@@ -251,10 +267,13 @@ int64_t mec_grad_scratch_bytes(int64_t n, int64_t d, int dtype);
  * are assumed where there is none).  No counterpart in the reference. */
 int64_t mec_backward_scratch_bytes(int64_t n, int64_t d, int dtype, int mode, int sides);
 
-/* The backward's plan for (n, d, dtype, mode, sides) on a device of
- * `compute_units` CUs (<= 0: the current device's), for 16-byte aligned rows.
- * No counterpart in the reference; for callers sizing buffers and for tests
- * of the selection rules without a GPU. */
+/* The plan of mec_grad for (n, d, dtype, mode, sides) on a device of
+ * `compute_units` CUs (<= 0: the current device's), for 16-byte aligned rows:
+ * also that of mec_backward with no more scratch than mec_grad_scratch_bytes_for.
+ * With the scratch of mec_backward_scratch_bytes the blocks are the same, but the
+ * contractions may be split over k and their tiles 384 features wide where these
+ * are not.  No counterpart in the reference; for callers sizing buffers and for
+ * tests of the selection rules without a GPU. */
 typedef struct mec_backward_plan_t {
   int64_t block_rows;            /* rows per block of the gradient matrix */
   int64_t num_blocks;            /* blocks (mec_grad runs num_blocks + 1 steps) */

@@ -68,7 +68,7 @@ __device__ __forceinline__ void store_vec(T* __restrict__ p, const float (&v)[kV
 // With 2^k s_i >= sqrt(N) that is no more than 2^-25 s_i, an fp32 rounding.
 // Where one row has less (pairs that match well beside one that does not: the
 // small shares' entries fall below fp16's range, the lo parts first), or the
-// scale stops at 2^40, the matrix is held wide, at fp32's range and precision,
+// scale stops at 2^39, the matrix is held wide, at fp32's range and precision,
 // and contracted as three bf16 terms (mec_gemm_wide.h).  Distance of a row's
 // off-diagonal sum from 64 bits, the largest over the rows, fp32 kernels, pairs
 // throughout, this rule: 4097 x 768, T = 0.03, two y rows swapped: 3.9e-6, 1.0
