@@ -13,8 +13,10 @@
 // the MFMA (12 per 32 x 32 block and chunk, against the pairs' 6) and the split
 // (about 10 VALU operations a value), one after the other between barriers.
 // CLIP step with wide contractions (one swapped pair at T = 0.02), pairs -> wide,
-// and on the fp32 kernels: 4999 x 640 371 -> 679 us, 1166; 8192 x 768 951 -> 2027
-// us, 3028; 32768 x 1152 21.2 -> 44.0 ms, 70.5.
+// and on the fp32 kernels: 4999 x 640 371 -> 641 us, 1154; 8192 x 768 951 -> 1892
+// us, 3021; 32768 x 1152 21.2 -> 44.0 ms, 70.5.  At d = 64 they take longer than
+// the fp32 kernels (8192 x 64 504 us, 437): three quarters of a tile are columns
+// past d.
 #pragma once
 #include "mec_common.h"
 
@@ -44,17 +46,19 @@ struct Tile {
 template <class TL>
 struct Source {
   __amdgpu_buffer_rsrc_t r;
-  uint32_t vo, estep, kstep;  // byte steps of a load's element (row, k) and of k (k-row-major: both the k-row)
-  __device__ __forceinline__ Source(bool km, const float* p, int64_t ld, int rows, int klen) {
+  bool km;
+  uint32_t estep, kstep;  // byte steps of a load's element (row, k) and of k (k-row-major: both the k-row)
+  __device__ __forceinline__ Source(bool km_, const float* p, int64_t ld, int rows, int klen) : km(km_) {
     const int64_t n = km ? (rows - 1) * ld + klen : (klen - 1) * ld + TL::BM;
     r = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)(n * 4), 0x00020000);
     estep = (uint32_t)ld * 4;
     kstep = km ? 4 : estep;
-    const uint32_t t = threadIdx.x;
-    vo = km ? (t >> 3) * 4 * estep + (t & 7) * 16 : t / (TL::BM / 4) * 4 * estep + t % (TL::BM / 4) * 16;
   }
   __device__ __forceinline__ void load(int k, f32x4 (&v)[4]) const {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));  // (the addresses are formed here: kept across the loop they spill)
+    const uint32_t vo = km ? (t >> 3) * 4 * estep + (t & 7) * 16 : t / (TL::BM / 4) * 4 * estep + t % (TL::BM / 4) * 16;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const u32x4 u = __builtin_amdgcn_raw_buffer_load_b128(r, vo, k * kstep + e * estep, 0);
@@ -79,7 +83,8 @@ __device__ __forceinline__ void split4(float f0, float f1, float f2, float f3, c
 // A chunk as three planes of K-major rows at `lds`
 template <class TL>
 __device__ __forceinline__ void split_store(bool km, const f32x4 (&v)[4], char* lds) {
-  const int t = threadIdx.x;
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));  // (as in Source::load)
   if (km) {
     char* o = lds + (t >> 3) * 4 * TL::PITCH + 8 * (t & 7);
 #pragma unroll
@@ -99,9 +104,6 @@ __device__ __forceinline__ void run(bool akm, const float* __restrict__ a, int64
                                     int64_t ldb, int b_rows, int klen, char* lds, f32x16 (&acc)[TL::FM][TL::FN]) {
   klen = (klen + 31) & ~31;
   const Source<TL> sa(akm, a, lda, TL::BM, klen), sb(true, b, ldb, b_rows, klen);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w / TL::WN, wn = w % TL::WN;
-  const char* ra = lds + (wm * TL::TM + (lane & 31)) * TL::PITCH + 16 * (lane >> 5);
-  const char* rb = lds + 3 * TL::PLANE + (wn * TL::TN + (lane & 31)) * TL::PITCH + 16 * (lane >> 5);
 #pragma unroll
   for (int i = 0; i < TL::FM; ++i)
 #pragma unroll
@@ -120,6 +122,13 @@ __device__ __forceinline__ void run(bool akm, const float* __restrict__ a, int64
       sb.load(k + TL::KC, vb);
     }
     __syncthreads();
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));  // (as in Source::load)
+    const int lane = t & 63, w = t >> 6, wm = w / TL::WN, wn = w % TL::WN;
+    // (a wave whose columns hold no row of B leaves its sums at 0)
+    if (__builtin_amdgcn_readfirstlane(b_rows - wn * TL::TN) <= 0) continue;
+    const char* ra = lds + (wm * TL::TM + (lane & 31)) * TL::PITCH + 16 * (lane >> 5);
+    const char* rb = lds + 3 * TL::PLANE + (wn * TL::TN + (lane & 31)) * TL::PITCH + 16 * (lane >> 5);
 #pragma unroll
     for (int s = 0; s < TL::KC / 16; ++s) {
       i16x8 fa[TL::FM][3];
@@ -136,13 +145,13 @@ __device__ __forceinline__ void run(bool akm, const float* __restrict__ a, int64
         constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
         for (int i = 0; i < TL::FM; ++i) {
-          f32x16 t;
+          f32x16 u;
 #pragma unroll
-          for (int r = 0; r < 16; ++r) t[r] = 0.f;
+          for (int r = 0; r < 16; ++r) u[r] = 0.f;
 #pragma unroll
-          for (int q = 0; q < 6; ++q) t = mfma16_32x32x16<false>(fa[i][PA[q]], fb[PB[q]], t);
+          for (int q = 0; q < 6; ++q) u = mfma16_32x32x16<false>(fa[i][PA[q]], fb[PB[q]], u);
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][j][r] += t[r];
+          for (int r = 0; r < 16; ++r) acc[i][j][r] += u[r];
         }
         // (the next block's reads stay behind: with all of them ahead the
         // registers do not last)
