@@ -999,11 +999,16 @@ __device__ __forceinline__ void split_step(const i16x8 (&a)[G::FM], const i16x8 
   });
   sched_fence();
 }
-template <class G, bool ZERO, bool CHAIN, class Hook = NoHook, int VMF = 0>
+// PIECE: the chunks [kt0, kt1) of a longer k-loop, whose loads run on across the
+// calls (the first call's kt0 is 0, a call's kt0 the last one's kt1).  vmf_first:
+// between two calls come at least 63 stores of every wave, so that with at most 63
+// memory operations left the loads before them have landed.
+template <class G, bool ZERO, bool CHAIN, class Hook = NoHook, int VMF = 0, bool PIECE = false>
 __device__ __forceinline__ void mainloop_split(LoadPlan<G>& lp, __amdgpu_buffer_rsrc_t ra_next,
                                                __amdgpu_buffer_rsrc_t rb_next, bool has_next, int K, char* lds,
                                                int& p0, f32x16 (&acc)[G::FM][G::FN], const Hook& hook = Hook(),
-                                               bool vmf_first = false) {
+                                               bool vmf_first = false, int kt0 = 0, int kt1 = 0) {
+  static_assert(!PIECE || !CHAIN, "pieces of one tile");
   static_assert(G::SPL && G::NS == 4 && G::MPB == 1 && G::S == 2, "16-bit pairs, four k-steps, two stages");
   static_assert(G::SA == 2 || (G::SA == 3 && !CHAIN && VMF == 0), "three A stages: one tile per call");
   if constexpr (ZERO) {
@@ -1021,10 +1026,15 @@ __device__ __forceinline__ void mainloop_split(LoadPlan<G>& lp, __amdgpu_buffer_
   // the loads; three, chunk kt + 1's B loads, then chunk kt + 2's A loads
   constexpr int S0A = G::SA == 2 ? 0 : LA, S0B = G::SA == 2 ? L1 : L2;
   constexpr int S1A = G::SA == 2 ? L1 : 0, S1B = G::SA == 2 ? L2 : LA;
-  const int nk = (K + BK - 1) / BK;
+  const int nk = PIECE ? kt1 : (K + BK - 1) / BK;
   i16x8 a0[G::FM], a1[G::FM], bh[G::FN], bl[G::FN];
-  for (int kt = 0; kt < nk; ++kt) {
-    if constexpr (G::SA == 3)
+  for (int kt = kt0; kt < nk; ++kt) {
+    if (PIECE && kt == kt0 && kt > 0) {
+      if (vmf_first)
+        wait_barrier<63>();
+      else
+        wait_barrier<0>();
+    } else if constexpr (G::SA == 3)
       wait_barrier<LA>();
     else if (VMF > 0 && kt == 0 && vmf_first)
       wait_barrier<VMF>();
@@ -1054,7 +1064,7 @@ __device__ __forceinline__ void mainloop_split(LoadPlan<G>& lp, __amdgpu_buffer_
     }
     const int k2 = G::SA == 2 ? k1 : (kt + 2) * BK;
     const FragReader<G> h0(ca, cb, 0), h1(ca, cb, 1), l0(ca, cb, 2), l1(ca, cb, 3);
-    if (kt > 0) {
+    if (kt > kt0) {
       split_step<G, S0A, S0B, true>(a0, bl, acc, lp, k1, na, nb, h0, a1, bh);  // P3 of the chunk before
     } else {
       static_for<frag_reads<G>()>([&](auto r) { h0.template read_to<r>(a1, bh); });

@@ -123,6 +123,27 @@ struct TileD : PackOf<KIND>::type {
       gdma::mainloop<G, ZERO>(a, b, K, (char*)lds, acc);
     }
   }
+  // run() of split operands with the sum in pieces: flush(acc) takes the
+  // sums up to each end of a piece but the last (end: the chunk at which piece i
+  // ends, at most the tile's last); full: with at least 63 stores of every wave
+  template <class Ends, class Flush>
+  static __device__ __forceinline__ void run_pieces(const Op& a, const Op& b, int K, void* lds,
+                                                    f32x16 (&acc)[FM][FN], const Ends& end, bool full,
+                                                    const Flush& flush) {
+    gdma::LoadPlan<G> lp;
+    gdma::prologue<G>(a, b, (char*)lds, lp);
+    const int nk = (K + G::BK - 1) / G::BK;
+    int p0 = 0;
+    for (int i = 0, k0 = 0;; ++i) {
+      const int k1 = end(i);
+      gdma::mainloop_split<G, true, false, gdma::NoHook, 0, true>(lp, lp.ra, lp.rb, false, K, (char*)lds, p0, acc,
+                                                                  gdma::NoHook(), full, k0, k1);
+      if (k1 >= nk) break;
+      flush(acc);
+      k0 = k1;
+    }
+    gdma::drain_loads();
+  }
   // run() with a hook on the operand values (gdma::NormHook; fp32 tiles)
   template <class FH>
   static __device__ __forceinline__ void run_fh(const Op& a, const Op& b, int K, void* lds, f32x16 (&acc)[FM][FN],
@@ -758,7 +779,7 @@ struct StepPlan {
   // part p into px / py + (p - 1) N D
   int ks, kl;
   float *px, *py;
-  int seg;  // split pairs: the most k rows that one sum runs over (grad_contract_tile)
+  int seg;  // split pairs: about the most k rows that one sum runs over (Pieces)
 };
 
 // fp32 gradient-matrix tile: H_ij = rx_i G'_ij ry_j (G'_ij without the norm
@@ -1011,36 +1032,78 @@ __device__ __forceinline__ void contract_store(const f32x16 (&acc)[TC::FM][TC::F
     }
   }
 }
-// contract_store in a loop: the addresses and masks of the 128 elements are
-// formed anew each time, with one branch on `accumulate` (kept across the k-loop
-// between, and with a branch per element, they spilled; once per tile the branch
-// per element takes fewer registers).  Times 2^oe: the inverse scales of the
-// gradient matrix and of an input, whose product may be no fp32 number.
-template <class TC>
-__device__ __forceinline__ void contract_store_again(const f32x16 (&acc)[TC::FM][TC::FN], int r0, int d0, int N, int D,
-                                                     bool accumulate, float* __restrict__ out, int oe) {
-  int lane = threadIdx.x & 63;
-  asm volatile("" : "+v"(lane));
-  const int w = threadIdx.x >> 6, wm = w / TC::WN, wn = w % TC::WN;
-  auto each = [&](auto put) {
-#pragma unroll
-    for (int bm = 0; bm < TC::FM; ++bm) {
+// contract_store for the sums of split pairs, which are stored several times a
+// tile: through a buffer of the tile's rows (rows past N are outside it, columns
+// past D are sent there), the addresses formed anew each time from one lane offset
+// (kept across the k-loop between, they spill).  Times 2^oe: the inverse scales of
+// the gradient matrix and of an input, whose product may be no fp32 number.
+struct PairOut {
+  __amdgpu_buffer_rsrc_t rs;
+  int d0, D, oe;
+  __device__ __forceinline__ PairOut(float* out, int r0, int rows, int d0_, int N, int D_, int oe_)
+      : rs(__builtin_amdgcn_make_buffer_rsrc((void*)(out + (int64_t)r0 * D_), 0, min(rows, N - r0) * D_ * 4,
+                                             0x00020000)),
+        d0(d0_), D(D_), oe(oe_) {}
+  template <class TC>
+  __device__ __forceinline__ void put(const f32x16 (&acc)[TC::FM][TC::FN], bool accumulate) const {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    const int lane = t & 63, w = t >> 6, wm = w / TC::WN, wn = w % TC::WN;
+    const int d = d0 + wn * TC::TN + (lane & 31);
+    // this wave's 32-column blocks that hold any column
+    const int fn = __builtin_amdgcn_readfirstlane((D - d0 - wn * TC::TN + 31) >> 5);
+    auto each = [&](auto st) {
+      // (from values of its own: what both kinds of store share would be formed
+      // ahead of the branch, for all elements at once)
+      uint32_t vo = (uint32_t)((wm * TC::TM + acc_row(0, lane)) * D + d) * 4;
+      int e = oe;
+      asm volatile("" : "+v"(vo), "+s"(e));
 #pragma unroll
       for (int bn = 0; bn < TC::FN; ++bn) {
-        const int d = d0 + wn * TC::TN + bn * 32 + (lane & 31);
+        if (bn >= fn) break;
+        // (past D: at least 2^31, the buffer is smaller)
+        const uint32_t vb = d + 32 * bn < D ? vo + 128 * bn : 0x80000000u;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int row = r0 + wm * TC::TM + bm * 32 + acc_row(r, lane);
-          if (row < N && d < D) put(out + (int64_t)row * D + d, __builtin_ldexpf(acc[bm][bn][r], oe));
-        }
+        for (int bm = 0; bm < TC::FM; ++bm)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            if (r % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+            st(__builtin_ldexpf(acc[bm][bn][r], e), vb + (uint32_t)((bm * 32 + acc_row(r, 0)) * D) * 4);
+          }
       }
-    }
-  };
-  if (accumulate)
-    each([](float* p, float v) { __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); });
-  else
-    each([](float* p, float v) { *p = v; });
-}
+    };
+    if (accumulate)
+      each([&](float v, uint32_t o) { (void)__builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(v, rs, o, 0, 0); });
+    else
+      each([&](float v, uint32_t o) { __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rs, o, 0, 0); });
+  }
+};
+
+// The pieces of a sum over k rows [kbeg, kend) (split pairs; StepPlan::seg): as
+// few of about the same length as 9/8 of seg allows, the boundaries moved by up to
+// 3/16 of it either way, and to at most 6/5 of seg, by `phase`, the tile's row.  The
+// tiles of a launch run in step: with the same boundaries for all they add to the
+// accumulators at one time and wait for HBM at one time (32768 x 1152 1% slower,
+// 16384 x 512 2%; moved by feature tile as well, which parts the tiles that share a
+// panel of the gradient matrix, 1% slower again).  A fixed function of the tile's
+// place, so that the order of the sums is too.
+// What the pieces cost, CLIP step against unlimited sums: 8192 x 768 1.1%, 32768 x
+// 1152 2.2%, 50000 x 1000 3.5%, 32768 x 256 and 30000 x 256 4-7% (twice the traffic
+// of the accumulators), 65536 x 64 0.4%.  With the k-loop started anew for each
+// piece and stores under a branch per element 65536 x 64 took 1.6% more.
+struct Pieces {
+  int n, first, len, kbeg, kend;
+  __device__ __forceinline__ Pieces(int kb, int ke, int seg, int phase) : kbeg(kb), kend(ke) {
+    const int l = ke - kb, most = seg + seg / 8;
+    // (divisions run on the VALU; the loops that ask for the ends are scalar)
+    n = l > most ? __builtin_amdgcn_readfirstlane((l + most - 1) / most) : 1;
+    len = n > 1 ? __builtin_amdgcn_readfirstlane(((l + n - 1) / n + 63) & ~63) : l;
+    const int by = min(len / 16, max(seg + seg / 5 - len, 0) / 3) & ~63;
+    first = n > 1 ? len + (2 * (phase & 3) - 3) * by : l;
+  }
+  // the end of piece i
+  __device__ __forceinline__ int end(int i) const { return i + 1 < n ? min(kbeg + first + i * len, kend) : kend; }
+};
 
 // One BM x BN output tile of a contraction: rows r0.. of block P, feature
 // columns d0..:
@@ -1061,13 +1124,19 @@ __device__ __forceinline__ void contract_store_again(const f32x16 (&acc)[TC::FM]
 // osc, or 2^oe (split pairs): the inverse of the operands' storage scales (a
 // power of two).
 // Only k rows [kbeg, kbeg + klen) of the block.
+// seg (split pairs): a sum over more than seg k rows is taken in pieces
+// (Pieces), each added to the accumulators as another block's would be: a longer
+// sum rounds more.  With seg the block rows of the fp32 kernels the sums are
+// hardly longer than theirs, and round 3 times per 8 k where the fp32 MFMA
+// rounds 4 times; unlimited (one sum per block), positive features came out up
+// to 1.9 times as far from 64 bits as the fp32 kernels' (4200 x 512).
 template <class TC, typename T, bool X3 = false>
-__device__ __forceinline__ void grad_contract_piece(int N, int D, const T* __restrict__ Gblk,
+__device__ __forceinline__ void grad_contract_tile(int N, int D, const T* __restrict__ Gblk,
                                                    const T* __restrict__ Glo, const T* __restrict__ OT,
                                                    const T* __restrict__ OTlo, int64_t ldt, const BlockGrid& bg,
                                                    int P, int Q, int tm, int td, bool accumulate,
                                                    float* __restrict__ out, char* lds, float osc, int oe,
-                                                   int kbeg, int klen) {
+                                                   int kbeg, int klen, int seg) {
   const int r0 = P * bg.bs + tm * TC::BM;
   if (r0 >= N) return;
   const int d0 = td * TC::BN;
@@ -1099,6 +1168,18 @@ __device__ __forceinline__ void grad_contract_piece(int N, int D, const T* __res
       for (int bn = 0; bn < TC::FN; ++bn)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[bm][bn][r] = 0.f;
+  } else if constexpr (SPL) {
+    const PairOut po(out, r0, TC::BM, d0, N, D, oe);
+    const Pieces pc(kbeg, kbeg + qk, seg, tm);
+    // (two of its 32-column blocks: 64 stores)
+    const int wn = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) % TC::WN;
+    static_assert(TC::FM == 2, "32 stores a column block");
+    TC::run_pieces(
+        A, B, kq, lds, acc, [&](int i) { return (pc.end(i) - kbeg + 31) >> 5; }, D - d0 - wn * TC::TN > 32,
+        [&](const f32x16 (&sums)[TC::FM][TC::FN]) {
+          po.template put<TC>(sums, accumulate);
+          accumulate = true;
+        });
   } else {
     TC::template run<true, true>(A, B, kq, lds, acc);
   }
@@ -1109,61 +1190,9 @@ __device__ __forceinline__ void grad_contract_piece(int N, int D, const T* __res
     TC::template run<true, true, false>(tile_op<TC>(Glo + a_off, bg.bs, TC::BM, kq), B, kq, lds, acc);
   }
   if constexpr (SPL)
-    contract_store_again<TC>(acc, r0, d0, N, D, accumulate, out, oe);
+    PairOut(out, r0, TC::BM, d0, N, D, oe).template put<TC>(acc, accumulate);
   else
     contract_store<TC>(acc, r0, d0, N, D, accumulate, out, osc);
-}
-
-// The pieces of a sum over k rows [kbeg, kend) (split pairs; StepPlan::seg): as
-// few of about the same length as seg allows, the boundaries moved by up to 3/16
-// of it either way by `phase`, the tile's row.  The tiles of a launch run in step:
-// with the same boundaries for all they add to the accumulators at one time and
-// wait for HBM at one time.  CLIP step against unlimited sums, boundaries in step
-// -> moved: 32768 x 1152 +1.9 -> +1.6%, 16384 x 512 +3.7 -> +1.6%, 8192 x 768 +1.2 ->
-// +0.8%; moved by feature tile as well, which parts the tiles that share a panel
-// of the gradient matrix: +2.3, +2.4, +1.7%.  A fixed function of the tile's place,
-// so that the order of the sums is too.
-struct Pieces {
-  int n, first, len, kbeg, kend;
-  __device__ __forceinline__ Pieces(int kb, int ke, int seg, int phase) : kbeg(kb), kend(ke) {
-    const int l = ke - kb;
-    n = l > seg ? (l + seg - 1) / seg : 1;
-    len = n > 1 ? ((l + n - 1) / n + 63) & ~63 : l;
-    first = n > 1 ? len + (2 * (phase & 3) - 3) * ((len / 16) & ~63) : l;
-  }
-  // the end of piece i
-  __device__ __forceinline__ int end(int i) const { return i + 1 < n ? min(kbeg + first + i * len, kend) : kend; }
-};
-
-// grad_contract_piece over the k rows [kbeg, kbeg + klen).
-// seg (split pairs): a sum over more than seg k rows is taken in pieces
-// (Pieces), each added to the accumulators as another block's would be: a longer
-// sum rounds more.  With seg the block rows of the fp32 kernels the sums are
-// hardly longer than theirs, and round 3 times per 8 k where the fp32 MFMA
-// rounds 4 times; unlimited (one sum per block), positive features came out up
-// to 1.9 times as far from 64 bits as the fp32 kernels' (4200 x 512).
-template <class TC, typename T, bool X3 = false>
-__device__ __forceinline__ void grad_contract_tile(int N, int D, const T* __restrict__ Gblk,
-                                                   const T* __restrict__ Glo, const T* __restrict__ OT,
-                                                   const T* __restrict__ OTlo, int64_t ldt, const BlockGrid& bg,
-                                                   int P, int Q, int tm, int td, bool accumulate,
-                                                   float* __restrict__ out, char* lds, float osc, int oe,
-                                                   int kbeg, int klen, int seg) {
-  if constexpr (IsSplit<T>::value) {
-    const int kend = min(min(bg.bs, N - Q * bg.bs), kbeg + klen);
-    const Pieces pc(kbeg, kend, seg, tm);
-    for (int i = 0, k = kbeg;; ++i) {
-      const int ke = pc.end(i);
-      grad_contract_piece<TC, T, X3>(N, D, Gblk, Glo, OT, OTlo, ldt, bg, P, Q, tm, td, accumulate || i > 0, out, lds,
-                                     osc, oe, k, ke - k);
-      if (i + 1 >= pc.n) break;
-      k = ke;
-      __syncthreads();  // every wave is past its last read of the ring
-    }
-  } else {
-    grad_contract_piece<TC, T, X3>(N, D, Gblk, Glo, OT, OTlo, ldt, bg, P, Q, tm, td, accumulate, out, lds, osc, oe,
-                                   kbeg, klen);
-  }
 }
 
 // The contraction of gradient-matrix blocks that are held wide (GradBufs): G at
@@ -1196,7 +1225,7 @@ __device__ __forceinline__ void grad_contract_wide(bool xside, int N, int D, con
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[i1][j][r] = 0.f;
     }
-    contract_store_again<TL>(acc, r0, d0, N, D, accumulate || i > 0, out, oe);
+    PairOut(out, r0, B, d0, N, D, oe).template put<TL>(acc, accumulate || i > 0);
     if (i + 1 >= pc.n) break;
     k = ke;
   }
