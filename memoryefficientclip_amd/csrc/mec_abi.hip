@@ -361,6 +361,14 @@ int64_t default_gbudget(int64_t n, int64_t d, int dtype) {
   if (b < kGradBudgetMin) b = kGradBudgetMin;
   return b < kGradBudgetCap ? b : kGradBudgetCap;
 }
+// rows that a block is to have: 4 d (fp32) or 8 d, and at least 1024 (below that
+// the pipeline's launches and accumulator updates dominate), where the budget
+// allows (pairs: twice the fp32 kernels' rows throughout; the sums over a block's
+// rows are taken in pieces: StepPlan::seg)
+int64_t target_rows(int64_t d, int dtype) {
+  const int64_t rows = (dtype == MEC_DTYPE_F32 ? 4 : 8) * d, least = (is_pairs(dtype) ? 2 : 1) * kTargetMinRows;
+  return rows > least ? rows : least;
+}
 void grad_blocks_budget(int64_t n, int64_t d, int dtype, int64_t gbudget, int* bs, int* nb) {
   const int64_t q = block_quantum(dtype);
   const int64_t tiles = (n + q - 1) / q;
@@ -383,15 +391,9 @@ void grad_blocks_budget(int64_t n, int64_t d, int dtype, int64_t gbudget, int* b
     }
     cap = tb;
   }
-  int64_t mult = dtype == MEC_DTYPE_F32 ? 4 : 8;
-  if (dtype != MEC_DTYPE_F32 && !is_pairs(dtype) && n >= 8192 && n < 16 * 8 * d) mult = 16;
-  // at least 1024 rows (below that the pipeline's launches and accumulator
-  // updates dominate), where the budget allows
-  // (pairs: twice the fp32 kernels' rows throughout; the sums over a block's rows
-  // are taken in pieces of those kernels' blocks: StepPlan::seg)
-  const int64_t min_rows = is_pairs(dtype) ? 2 * kTargetMinRows : kTargetMinRows;
-  const int64_t target_rows = mult * d > min_rows ? mult * d : min_rows;
-  int64_t target = (target_rows + q - 1) / q;
+  int64_t rows = target_rows(d, dtype);
+  if (dtype != MEC_DTYPE_F32 && !is_pairs(dtype) && n >= 8192 && n < 16 * 8 * d && rows < 16 * d) rows = 16 * d;
+  int64_t target = (rows + q - 1) / q;
   // 16-bit: one block from n = 3072 while its matrix stays within the smallest
   // budget (n <= 11520) and within 64 times the two inputs (256 n d bytes; 64 MiB
   // below that): one launch of each kind instead of several, tiles that fill
@@ -1275,10 +1277,19 @@ static int grad_step_run(const StepArgs& a, int64_t step, const ScratchLayout& L
   sp.kl = cs ? cs->kl : bs;
   sp.seg = bs;
   if (pairs) {
-    // (sums about as long as the fp32 kernels': grad_contract_tile)
+    // Sums as long as the fp32 kernels' blocks (grad_contract_tile).  Where no
+    // divisor lets those be as long as they aim to be, that length if the sums round
+    // no more for it: the square of the error that roundings leave in a sum of n
+    // positive terms, in pieces of l, goes as r l^2 + n^2 / l, with r the roundings
+    // a term (1/2; pairs 3/8) and one a piece.  (n = 30000, d = 256: blocks of 640
+    // rows; pieces of 683 and 1024 took 6.57 and 5.77 ms a step, one of 2048 5.51; the
+    // sums of 1024 are 0.43-0.77 times as far from 64 bits as the fp32 kernels'.)
     int bs32, nb32;
     grad_blocks(n, d, MEC_DTYPE_F32, &bs32, &nb32);
-    if (bs32 < bs) sp.seg = bs32;
+    const double b = bs32, aim = (double)target_rows(d, MEC_DTYPE_F32), n2 = (double)n * n;
+    int64_t seg = bs32;
+    if (aim > b && 0.375 * aim * aim + n2 / aim <= 0.5 * b * b + n2 / b) seg = (int64_t)aim;
+    if (seg < bs) sp.seg = (int)seg;
   }
   sp.px = parts;
   sp.py = parts ? parts + (acc_x ? (int64_t)(ks - 1) * n * d : 0) : nullptr;

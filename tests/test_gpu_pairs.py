@@ -218,10 +218,12 @@ def features(kind, n, d):
 
 
 # (4200 and 8192 rows: one block of pairs, three and two blocks of the fp32
-# kernels; 4999 with its contractions split over k; 2300 in 128 x 128 tiles)
+# kernels; 4999 with its contractions split over k; 2300 in 128 x 128 tiles; 30000
+# where the fp32 kernels' blocks are shorter than the pieces of the pairs' sums)
 @pytest.mark.parametrize("mode", ["clip", "lit"])
 @pytest.mark.parametrize("kind,n,d", [("positive", 4200, 512), ("relu", 4200, 512), ("normal", 4200, 512),
-                                      ("positive", 8192, 256), ("positive", 4999, 640), ("positive", 2300, 128)])
+                                      ("positive", 8192, 256), ("positive", 4999, 640), ("positive", 2300, 128),
+                                      ("normal", 30000, 256)])
 def test_no_further_from_64_bits_than_fp32(kind, n, d, mode):
     """Sums that grow with every term round the most, and the more the longer
     they are: those of the pairs, in pieces of the fp32 kernels' blocks, end no
