@@ -14,7 +14,7 @@
 // (about 10 VALU operations a value), one after the other between barriers.
 // CLIP step with wide contractions (one swapped pair at T = 0.02), pairs -> wide,
 // and on the fp32 kernels: 4999 x 640 371 -> 641 us, 1154; 8192 x 768 951 -> 1892
-// us, 3021; 32768 x 1152 21.2 -> 44.0 ms, 70.5.  At d = 64 they take longer than
+// us, 3021; 32768 x 1152 21.2 -> 42.7 ms, 70.5.  At d = 64 they take longer than
 // the fp32 kernels (8192 x 64 504 us, 437): three quarters of a tile are columns
 // past d.
 #pragma once
