@@ -758,7 +758,9 @@ int plan_units() {
 bool pairs_preferred(int64_t n, int64_t d, int dtype) {
   if (dtype != MEC_DTYPE_F32 && dtype != MEC_DTYPE_F32_BF16X3) return false;
   if (n < 1 || d < 1 || n > kMaxNPairs || d > kMaxD) return false;
-  if (const char* env = std::getenv("MEC_F32_PAIRS")) {  // (tests)
+  // (0: for callers who need the memory, or every bit of features below 2^-17 of
+  // their rows, more than the time; 1: for tests)
+  if (const char* env = std::getenv("MEC_F32_PAIRS")) {
     if (env[0] == '0') return false;
     if (env[0] == '1') return true;
   }
